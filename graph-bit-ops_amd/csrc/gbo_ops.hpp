@@ -80,12 +80,21 @@ class AsyncAllocs {
   }
 
  private:
-  static constexpr int kMax = 16;
+  static constexpr int kMax = 24;
   hipStream_t st_;
   void* ptrs_[kMax] = {};
   int n_ = 0;
 };
 int validate_bsr(const gbo_bsr* A, int want_dir, const char* who);
+
+// The nonzeros of a row-direction bit-BSR as CSR (rows in order, columns
+// ascending), in device memory owned by `mem`; one host read of the total.
+struct CsrList {
+  const int64_t* rowptr = nullptr;  // [nrows + 1]
+  const int32_t* col = nullptr;     // [nnz]
+  int64_t nnz = 0;
+};
+int expand_csr(const gbo_bsr* A, AsyncAllocs& mem, CsrList* out, hipStream_t st);
 
 template <class TI, class TO>
 int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st);

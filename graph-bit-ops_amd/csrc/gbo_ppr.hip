@@ -10,21 +10,27 @@
 // for L = sum_k w_k . p_k.  The adjoint needs only the converged p (no
 // checkpointing of the forward iterates).
 //
-// The product is a bit-BSR SpMM with a dense K-column right-hand side in
-// vertex-major layout X[n][K]: every set bit (r, c) of a tile costs one
-// 4K-byte row read X[j][0..K), taken by the wave together.  At bs 8 X
-// carries the per-source scale (one elementwise pass).  With whole blocks of
-// 64 columns (k_ppr_spmm8r) lane l holds tile row l / 8 and columns
-// 8 (l % 8) .. +7: the set bits are listed per tile row and the eight rows'
-// lists are walked in step, 32 bytes of a row read per lane.  Otherwise
-// (k_ppr_spmm8) lane k owns column k, and the set bits are listed in LDS
-// and read back 8 at a time.  Both add each row's terms in the same order,
-// so they give the same bits.  At bs 16/32 (k_ppr_spmm) tile
-// row words are fetched by lanes r < bs, the rows with bits are found by a
-// ballot and set bits are read one at a time.  Each row's partial sum lives
-// in register acc[r] (uniform index).  Waves take tile-balanced chunks;
-// rows cut by a chunk boundary leave partials that a fix-up kernel adds in
-// chunk order, so results are bitwise reproducible.
+// Both solves run some tens of products over one matrix, so a call lists the
+// nonzeros of its tiles once as CSR (expand_csr) and every product streams 4
+// bytes per nonzero and gathers one row of X per nonzero.  Walking the tiles
+// in each product instead (a wave per 1024 tiles, its set bits listed in LDS
+// or taken one at a time) left most of the chip idle on matrices of a few
+// million nonzeros and one wave at work on the densest tiles.
+//
+// The product (k_spmm): the rows are cut into segments of at most 64
+// nonzeros (longer for hub rows), a unit of 16 lanes takes a segment.  X is
+// kept with its rows padded to a multiple of four columns, so a lane gathers
+// 16 bytes: at K > 32 the 16 lanes span a row of X and the unit takes one
+// nonzero at a time, eight gathers in flight; at smaller K the unit takes 2
+// to 16 nonzeros at a time.  Sums are FP64.  A segment that is its whole row
+// finishes it in place: Y, the next product's scaled row, and its part of
+// the convergence measure.  Rows of several segments leave FP64 partials
+// that k_spmm_fix adds in a fixed order, so results are bitwise reproducible
+// and independent of the block size and of the operands' alignment.
+//
+// The solves decide on convergence on the device (k_colsum): each kernel
+// returns at once when the flag is up, and the host queues kBatch iterations
+// between two looks at it.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -33,474 +39,368 @@
 #include "gbo_ops.hpp"
 
 namespace gbo {
+namespace {
 
-struct PprArgs {
-  const int32_t* rowptr;
-  const int32_t* colind;
-  const void* tiles;
-  int32_t nrows, nbr;
-  int64_t T;
-  const int32_t* plan;
-  int32_t chunk, nchunks;
-  int32_t K;                 // columns (<= 64 per launch; ld is the row stride)
-  int32_t ld;                // row stride of X/Y/Z (total columns)
-  const float* X;            // [n][ld] right-hand side (column block offset applied)
-  const float* colscale;     // per source vertex factor on X (nullable -> 1)
-  const float* rowscale;     // per output row factor (nullable -> 1)
-  float a;                   // Y = a * rowscale * (A X) + b * Z
-  float b;
-  const float* Z;            // nullable
-  float* Y;
-  float* partial;            // [nchunks][2][bs][64] split-row partials (sum + compensation)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kUnit = 16;        // lanes per segment
+constexpr int kBlk = 256;        // threads per workgroup
+constexpr int kUnits = kBlk / kUnit;
+constexpr int kMainBlocks = 2048;  // most workgroups of k_spmm (fixed, so that the order of the measure is too)
+constexpr int kFixBlocks = 2048;   // and of k_spmm_fix
+// Iterations queued between two host reads of the flag: a read costs about
+// 30 us of idle GPU, an iteration after convergence three empty launches
+// (about 9 us), and a solve takes 30 to 120 iterations.
+constexpr int kBatch = 8;
+
+// Nonzeros per segment of a row of `deg`: 64 keeps the units of a wave close
+// to equal; hub rows take longer ones so that at most some hundred partials
+// of a row are added one after another.
+__host__ __device__ inline int64_t seg_len(int64_t deg) { return deg <= 4096 ? 64 : deg <= 65536 ? 256 : 1024; }
+
+// A segment: row, start | length << 48 | (its row has several) << 63, and
+// then the slot of its partial.
+struct alignas(16) Seg {
+  uint64_t sl;
+  int32_t row;
+  uint32_t slot;
 };
 
-// First tile of chunk c (c <= nchunks; chunk nchunks starts at T).
-__device__ __forceinline__ int64_t chunk_start(const PprArgs& A, int64_t c) {
-  const int64_t b = c * A.chunk;
-  return b < A.T ? b : A.T;
+__device__ __forceinline__ int64_t row_segs(int64_t deg) {
+  const int64_t L = seg_len(deg);
+  return deg <= L ? 1 : (deg + L - 1) / L;  // an empty row has one empty segment
 }
 
-__device__ __forceinline__ void nadd(float& s, float& c, float v) {
-  const float t = s + v;
-  if (fabsf(s) >= fabsf(v)) c += (s - t) + v;
-  else c += (v - t) + s;
-  s = t;
+// Per row: segments in the low half, partial slots (rows of several segments
+// only) in the high half; and whether it has several.
+__global__ __launch_bounds__(256) void k_seg_count(const int64_t* __restrict__ rowptr, int32_t n,
+                                                   int64_t* __restrict__ cnt, int32_t* __restrict__ multi) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t s = row_segs(rowptr[i + 1] - rowptr[i]);
+  cnt[i] = s | (s > 1 ? s << 32 : 0);
+  multi[i] = s > 1;
 }
 
-template <int BS>
-__device__ __forceinline__ void ppr_store_row(const PprArgs& A, int64_t R, int lane, const float* acc, const float* cmp,
-                                              bool full, int slot, int c) {
-  for (int r = 0; r < BS; ++r) {
-    const int64_t i = R * BS + r;
-    if (i >= A.nrows) break;
-    const float v = acc[r] + cmp[r];
-    if (full) {
-      if (lane < A.K) {
-        const float rs = A.rowscale ? A.rowscale[i] : 1.0f;
-        float y = A.a * rs * v;
-        if (A.Z) y += A.b * A.Z[i * A.ld + lane];
-        A.Y[i * A.ld + lane] = y;
+__global__ __launch_bounds__(256) void k_seg_fill(const int64_t* __restrict__ rowptr, int32_t n,
+                                                  const int64_t* __restrict__ off, const int64_t* __restrict__ moff,
+                                                  Seg* __restrict__ segs, int32_t* __restrict__ mrow) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t r0 = rowptr[i], deg = rowptr[i + 1] - r0;
+  const int64_t s = row_segs(deg), L = seg_len(deg);
+  const int64_t at = off[i] & 0xFFFFFFFF;
+  const uint32_t slot = (uint32_t)(off[i] >> 32);
+  for (int64_t k = 0; k < s; ++k) {
+    Seg g;
+    g.sl = (uint64_t)(r0 + k * L) | ((uint64_t)min(L, deg - k * L) << 48) | (s > 1 ? 1ull << 63 : 0ull);
+    g.row = (int32_t)i;
+    g.slot = slot + (uint32_t)k;
+    segs[at + k] = g;
+  }
+  if (s > 1) mrow[moff[i]] = (int32_t)i;
+}
+
+// Device-side state of a solve.
+struct Ctl {
+  unsigned long long done;  // 1: converged, later kernels return
+  unsigned long long iters;
+  unsigned long long ticket;
+  double dmax;
+  double val[64];   // the last column sums
+  double norm[64];  // the columns' norms
+};
+
+struct SpmmArgs {
+  const Seg* segs;
+  int64_t nseg;
+  const int32_t* mrow;   // rows of several segments
+  int64_t nmulti;
+  const int64_t* off;    // per row, as k_seg_count's scan
+  const int32_t* col;
+  int32_t K, ld;         // columns; row stride of the padded arrays (a multiple of 4)
+  const float* X;        // [n][ld], already carrying any per-source scale
+  const float* rowscale; // per output row factor (nullable -> 1)
+  float a, b;            // Y = a * rowscale * (A X) + b * Z
+  const float* Z;        // [n][K] (nullable)
+  int zvec;              // Z rows are 16-byte aligned and K % 4 == 0
+  float* Y;              // [n][ld] (nullable: measure only)
+  const float* P;        // measure: [n][ld], against which Y is measured; may be Y itself
+  const float* L;        // nullable: measure = sum |Y - P| per column; else sum L * (Y - Z'), Z' = P [n][K]
+  float* Xs;             // nullable: next product's operand, Y * xscale
+  const float* xscale;
+  double* partial;       // [slots][ld]
+  double* part;          // measure: [64][kMainBlocks + kFixBlocks]
+  Ctl* ctl;
+};
+
+// Row i, columns 4 cl .. 4 cl + 3 from their sums; adds to the measure.
+__device__ __forceinline__ void finish_row(const SpmmArgs& A, int64_t i, int cl, const double* acc, double* d) {
+  const int k0 = cl * 4;
+  float z[4] = {0.f, 0.f, 0.f, 0.f};
+  if (A.Z) {
+    if (A.zvec) {
+      const f32x4 v = *(const f32x4*)(A.Z + i * A.K + k0);
+      z[0] = v.x, z[1] = v.y, z[2] = v.z, z[3] = v.w;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (k0 + q < A.K) z[q] = A.Z[i * A.K + k0 + q];
+    }
+  }
+  const double rs = A.rowscale ? (double)A.rowscale[i] : 1.0;
+  float y[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    double t = (double)A.a * rs * acc[q];
+    if (A.Z) t += (double)A.b * (double)z[q];
+    y[q] = k0 + q < A.K ? (float)t : 0.f;
+  }
+  if (A.L) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (k0 + q < A.K) d[q] += (double)A.L[i * A.ld + k0 + q] * ((double)y[q] - (double)A.P[i * A.K + k0 + q]);
+    return;
+  }
+  const f32x4 p = *(const f32x4*)(A.P + i * A.ld + k0);
+  d[0] += fabs((double)y[0] - (double)p.x);
+  d[1] += fabs((double)y[1] - (double)p.y);
+  d[2] += fabs((double)y[2] - (double)p.z);
+  d[3] += fabs((double)y[3] - (double)p.w);
+  *(f32x4*)(A.Y + i * A.ld + k0) = f32x4{y[0], y[1], y[2], y[3]};
+  if (A.Xs) {
+    const float s = A.xscale[i];
+    *(f32x4*)(A.Xs + i * A.ld + k0) = f32x4{y[0] * s, y[1] * s, y[2] * s, y[3] * s};
+  }
+}
+
+// The workgroup's measure: d of every unit's column lanes, added over the
+// units in order, to column k's partial `slot`.
+template <int LPR>
+__device__ __forceinline__ void store_measure(const SpmmArgs& A, const double* d, int slot) {
+  __shared__ double sh[kUnits][4 * LPR];
+  const int unit = threadIdx.x / kUnit, l = threadIdx.x % kUnit;
+  if (l < LPR) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sh[unit][4 * l + q] = d[q];
+  }
+  __syncthreads();
+  const int k = threadIdx.x;
+  if (k < 4 * LPR && k < A.K) {
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) s += sh[u][k];
+    A.part[(int64_t)k * (kMainBlocks + kFixBlocks) + slot] = s;
+  }
+}
+
+// Lane n of the calling lane's row of 16 lanes (all 16 active): DPP
+// row_newbcast, no LDS trip.
+template <int N>
+__device__ __forceinline__ int row_lane(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0x150 + N, 0xF, 0xF, false);
+}
+
+// Eight nonzeros of a segment, H .. H + 7 of the 16 whose columns the unit's
+// lanes hold: eight gathers in flight, then the sums in order.
+template <int H>
+__device__ __forceinline__ void add8(const float* __restrict__ X, int64_t ld, int c, int nl, double* acc) {
+  f32x4 x[8];
+  const int v[8] = {row_lane<H>(c),     row_lane<H + 1>(c), row_lane<H + 2>(c), row_lane<H + 3>(c),
+                    row_lane<H + 4>(c), row_lane<H + 5>(c), row_lane<H + 6>(c), row_lane<H + 7>(c)};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = *(const f32x4*)(X + v[j] * ld);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (H + j < nl) {
+      acc[0] += (double)x[j].x;
+      acc[1] += (double)x[j].y;
+      acc[2] += (double)x[j].z;
+      acc[3] += (double)x[j].w;
+    }
+  }
+}
+
+// LPR lanes span the (padded) columns of a row of X, kUnit / LPR nonzeros
+// are taken at a time.
+// Bound by the row gathers: R-MAT 2^17 vertices, 3.9M nonzeros, K = 64, a
+// product of 1.0 GB of gathered rows and 0.13 GB of streamed ones takes 110
+// us (10 TB/s out of L2 and the Infinity Cache), k_spmm_fix 11 us, k_colsum
+// 7 us.  The kernels that walked the tiles took 556 us at bs 8 (chunks of
+// 1024 tiles, the densest one set the time) and 1.7 ms at bs 16 already on
+// 1007 vertices; forward and adjoint together 82.5 -> 21.7 ms, at 2^22
+// vertices 980 -> 838 ms.
+template <int LPR>
+__global__ __launch_bounds__(kBlk) void k_spmm(const SpmmArgs A) {
+  if (A.ctl->done) return;
+  constexpr int EP = kUnit / LPR;
+  const int unit = threadIdx.x / kUnit, l = threadIdx.x % kUnit;
+  const int cl = l % LPR, el = l / LPR;
+  const bool col_ok = cl * 4 < A.ld;
+  const float* __restrict__ X = A.X + (col_ok ? cl * 4 : 0);
+  const int64_t ld = A.ld;
+  double d[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int64_t u = (int64_t)blockIdx.x * kUnits + unit; u < A.nseg; u += (int64_t)gridDim.x * kUnits) {
+    const Seg s = A.segs[u];
+    const int len = (int)(s.sl >> 48) & 0x7FFF;
+    const int32_t* __restrict__ col = A.col + (s.sl & 0xFFFFFFFFFFFFull);
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if constexpr (LPR == kUnit) {
+      for (int e = 0; e < len; e += kUnit) {
+        // lanes past the end repeat the last column: their gathers hit the
+        // line of the last nonzero and are not added
+        const int c = col[min(e + l, len - 1)];
+        add8<0>(X, ld, c, len - e, acc);
+        if (e + 8 < len) add8<8>(X, ld, c, len - e, acc);
       }
     } else {
-      A.partial[(((int64_t)c * 2 + slot) * BS + r) * kWave + lane] = v;
+      constexpr int U = 4;
+      for (int e = el; e < len; e += U * EP) {
+        int c[U];
+        f32x4 x[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) c[j] = col[min(e + j * EP, len - 1)];
+#pragma unroll
+        for (int j = 0; j < U; ++j) x[j] = *(const f32x4*)(X + c[j] * ld);
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+          if (e + j * EP < len) {
+            acc[0] += (double)x[j].x;
+            acc[1] += (double)x[j].y;
+            acc[2] += (double)x[j].z;
+            acc[3] += (double)x[j].w;
+          }
+        }
+      }
+#pragma unroll
+      for (int off = LPR; off < kUnit; off <<= 1) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] += __shfl_xor(acc[q], off);
+      }
+    }
+    if (el == 0 && col_ok) {
+      if (s.sl >> 63) {
+        double* p = A.partial + (int64_t)s.slot * ld + cl * 4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) p[q] = acc[q];
+      } else {
+        finish_row(A, s.row, cl, acc, d);
+      }
     }
   }
+  store_measure<LPR>(A, d, blockIdx.x);
 }
 
-template <int BS>
-__global__ __launch_bounds__(256) void k_ppr_spmm(const PprArgs A) {
-  using W = word_t<BS>;
+// Rows of several segments: a wave adds a row's partials, its four units (and
+// the unit's spare lanes) each every (4 EP)-th of them in order, then the
+// lanes' sums in a fixed tree.
+template <int LPR>
+__global__ __launch_bounds__(kBlk) void k_spmm_fix(const SpmmArgs A) {
+  if (A.ctl->done) return;
+  constexpr int EP = kUnit / LPR, W = (kWave / kUnit) * EP;
   const int lane = lane_id();
-  const int c = wave_index();
-  if (c >= A.nchunks) return;
-  const int64_t cb = chunk_start(A, c);
-  const int64_t ce = chunk_start(A, c + 1);
-  const bool last = (c == A.nchunks - 1);
-  const W* __restrict__ tiles = (const W*)A.tiles;
-  const bool col_ok = lane < A.K;
-
-  for (int32_t R0 = A.plan[c]; R0 < A.nbr;) {
-    const int32_t Rl = R0 + lane;
-    int32_t rsl = 0, rel = 0;
-    if (Rl < A.nbr) {
-      rsl = A.rowptr[Rl];
-      rel = A.rowptr[Rl + 1];
-    }
-    const bool belong = (Rl < A.nbr) && (last || (int64_t)rsl < ce);
-    const uint64_t bmask = __ballot(belong);
-    uint64_t todo = bmask;  // empty rows are written with the epilogue too
-    while (todo) {
-      const int j = __builtin_ctzll(todo);
-      todo &= todo - 1;
-      const int64_t R = R0 + j;
-      const int64_t rs = __builtin_amdgcn_readlane(rsl, j), re = __builtin_amdgcn_readlane(rel, j);
-      const int64_t s = rs > cb ? rs : cb;
-      const int64_t te = re < ce ? re : ce;
-      const bool full = (rs >= cb) && (re <= ce);
-      float acc[BS], cmp[BS];
+  const int cl = lane % LPR, el = lane / LPR;  // el in [0, W)
+  const bool col_ok = cl * 4 < A.ld;
+  double d[4] = {0.0, 0.0, 0.0, 0.0};
+  const int64_t nw = (int64_t)gridDim.x * (kBlk / kWave);
+  for (int64_t w = wave_index(); w < A.nmulti; w += nw) {  // wave-uniform
+    const int32_t i = A.mrow[w];
+    const int64_t s0 = A.off[i] >> 32, s1 = A.off[i + 1] >> 32;
+    const double* __restrict__ P = A.partial + (col_ok ? cl * 4 : 0);
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    constexpr int U = 4;
+    for (int64_t s = s0 + el; s < s1; s += U * W) {
+      double v[U][4];
 #pragma unroll
-      for (int r = 0; r < BS; ++r) acc[r] = cmp[r] = 0.0f;
-      for (int64_t t = s; t < te; ++t) {
-        const int32_t col = A.colind[t];
-        const uint64_t word = (lane < BS) ? (uint64_t)tiles[t * BS + lane] : 0ull;
-        uint64_t rows = __ballot(word != 0);
-        while (rows) {
-          const int r = __builtin_ctzll(rows);
-          rows &= rows - 1;
-          uint64_t wr = (uint64_t)__shfl((long long)word, r);
-          while (wr) {
-            const int p = __builtin_ctzll(wr);
-            wr &= wr - 1;
-            const int64_t v = (int64_t)col * BS + (BS - 1 - p);
-            float x = col_ok ? A.X[v * A.ld + lane] : 0.0f;
-            if (A.colscale) x *= A.colscale[v];
-            nadd(acc[r], cmp[r], x);  // r is wave-uniform
-          }
+      for (int j = 0; j < U; ++j) {
+        const double* p = P + min(s + j * W, s1 - 1) * A.ld;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[j][q] = p[q];
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        if (s + j * W < s1) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[q] += v[j][q];
         }
       }
-      ppr_store_row<BS>(A, R, lane, acc, cmp, full, (rs < cb) ? 0 : 1, c);
     }
-    if (__popcll(bmask) < kWave) break;
-    R0 += kWave;
+#pragma unroll
+    for (int off = LPR; off < kWave; off <<= 1) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] += __shfl_xor(acc[q], off);
+    }
+    if (el == 0 && col_ok) finish_row(A, i, cl, acc, d);
   }
+  // one measure per wave: only its first unit's lanes hold any
+  if (lane >= kUnit) d[0] = d[1] = d[2] = d[3] = 0.0;
+  store_measure<LPR>(A, d, kMainBlocks + blockIdx.x);
 }
 
-// bs 8 SpMM with batched row gathers.  Lanes are columns, so every set bit
-// (r, c) of a tile is one coalesced row read X[v][0..K) for the whole wave.
-// The bits are listed in parallel: lane i takes tile b + i of a 64-tile
-// block of the row segment, a wave prefix sum of the tiles' popcounts gives
-// each bit its slot, and each lane writes (r << 29 | v) for its bits into a
-// per-wave LDS list (in tile order, then bit order, so the summation order
-// is fixed).  The wave then walks the list 8 entries at a time, issuing the
-// 8 row reads together.  Sums are FP64, one register per tile row indexed
-// by the wave-uniform row.  X must already carry any per-source scale.
-constexpr int kPprCap = 1024;  // list entries per wave and pass
-
-__global__ __launch_bounds__(256) void k_ppr_spmm8(const PprArgs A) {
-  constexpr int BS = 8, NB = 8;
-  __shared__ uint32_t lists[256 / kWave][kPprCap];
-  const int lane = lane_id();
-  uint32_t* __restrict__ list = lists[threadIdx.x / kWave];
-  const int c = wave_index();
-  if (c >= A.nchunks) return;
-  const int64_t cb = chunk_start(A, c);
-  const int64_t ce = chunk_start(A, c + 1);
-  const bool last = (c == A.nchunks - 1);
-  const uint64_t* __restrict__ tw = (const uint64_t*)A.tiles;
-  const bool col_ok = lane < A.K;
-
-  for (int32_t R0 = A.plan[c]; R0 < A.nbr;) {
-    const int32_t Rl = R0 + lane;
-    int32_t rsl = 0, rel = 0;
-    if (Rl < A.nbr) {
-      rsl = A.rowptr[Rl];
-      rel = A.rowptr[Rl + 1];
-    }
-    const bool belong = (Rl < A.nbr) && (last || (int64_t)rsl < ce);
-    const uint64_t bmask = __ballot(belong);
-    uint64_t todo = bmask;  // empty rows are written with the epilogue too
-    while (todo) {
-      const int j = __builtin_ctzll(todo);
-      todo &= todo - 1;
-      const int64_t R = R0 + j;
-      const int64_t rs = __builtin_amdgcn_readlane(rsl, j), re = __builtin_amdgcn_readlane(rel, j);
-      const int64_t s = rs > cb ? rs : cb;
-      const int64_t te = re < ce ? re : ce;
-      const bool full = (rs >= cb) && (re <= ce);
-      double acc[BS];
-#pragma unroll
-      for (int r = 0; r < BS; ++r) acc[r] = 0.0;
-      for (int64_t b = s; b < te; b += kWave) {
-        const int64_t nt = min((int64_t)kWave, te - b);
-        const uint64_t word = lane < nt ? tw[b + lane] : 0ull;
-        const uint32_t vb = lane < nt ? (uint32_t)A.colind[b + lane] * BS + (BS - 1) : 0u;
-        const int cnt = __popcll(word);
-        const int incl = wave_incl_scan(cnt);  // inclusive prefix sum of the popcounts over the lanes
-        const int excl = incl - cnt;
-        const int tot = __builtin_amdgcn_readlane(incl, kWave - 1);
-        for (int base = 0; base < tot; base += kPprCap) {
-          // list entries [base, base + kPprCap) of this block
-          uint64_t w = word;
-          int idx = excl;
-          while (w) {
-            const int p = __builtin_ctzll(w);
-            w &= w - 1;
-            if (idx >= base && idx < base + kPprCap)
-              list[idx - base] = ((uint32_t)(p >> 3) << 29) | (vb - (uint32_t)(p & 7));  // row p/8, column 7 - p%8
-            ++idx;
-          }
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-          const int nl = min(kPprCap, tot - base);
-          for (int i = 0; i < nl; i += NB) {
-            uint32_t e[NB];
-#pragma unroll
-            for (int k = 0; k < NB; ++k) e[k] = __builtin_amdgcn_readfirstlane(list[min(i + k, nl - 1)]);
-            // the NB row reads are unconditional (e[k] is a valid entry,
-            // lanes past K read column 0) so they are in flight together;
-            // conditional reads were each waited for in turn
-            const int lc = col_ok ? lane : 0;
-            float xk[NB];
-#pragma unroll
-            for (int k = 0; k < NB; ++k) {
-              const float xv = A.X[(int64_t)(e[k] & 0x1FFFFFFFu) * A.ld + lc];
-              xk[k] = (i + k < nl && col_ok) ? xv : 0.0f;
-            }
-#pragma unroll
-            for (int k = 0; k < NB; ++k)
-              if (i + k < nl) acc[e[k] >> 29] += (double)xk[k];
-          }
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        }
-      }
-      for (int r = 0; r < BS; ++r) {
-        const int64_t i = R * BS + r;
-        if (i >= A.nrows) break;
-        if (full) {
-          if (col_ok) {
-            const double rsc = A.rowscale ? (double)A.rowscale[i] : 1.0;
-            double y = (double)A.a * rsc * acc[r];
-            if (A.Z) y += (double)A.b * (double)A.Z[i * A.ld + lane];
-            A.Y[i * A.ld + lane] = (float)y;
-          }
-        } else {
-          A.partial[(((int64_t)c * 2 + ((rs < cb) ? 0 : 1)) * BS + r) * kWave + lane] = (float)acc[r];
-        }
-      }
-    }
-    if (__popcll(bmask) < kWave) break;
-    R0 += kWave;
-  }
-}
-
-// bs 8 SpMM for a block of 64 columns, lane = (tile row lane / 8, columns
-// 8 (lane % 8) .. +7).  A 64-tile block's set bits are listed per tile row
-// (eight LDS sublists; offsets from wave prefix sums of the rows' popcounts,
-// two rows to a 32-bit word as 16-bit fields), and the eight rows' sublists
-// are walked in step: each lane reads its row's next entry v and its 32
-// bytes of row v of X (two 16-byte loads), and adds them into eight FP64
-// registers of its own.  A row's entries keep the order of the flat list
-// (tile, then bit), so the sums are those of k_ppr_spmm8, with no
-// per-entry scalar work and no indexed register file access.
-constexpr int kPprRowCap = 128;  // sublist entries per tile row and pass
-// Entries per lane and step: four (eight 16-byte loads in flight per lane)
-// measured 8.2 ms per R-MAT s22 K = 64 iteration against 8.4 with two, at
-// 4 waves per SIMD (96-110 VGPRs); the flat-list kernel took 12.1.
-constexpr int kPprRowStep = 4;
-
-__device__ __forceinline__ uint32_t field16(uint32_t w, int hi) { return hi ? (w >> 16) : (w & 0xFFFFu); }
-
-__global__ __launch_bounds__(256) void k_ppr_spmm8r(const PprArgs A) {
-  constexpr int BS = 8, U = kPprRowStep, CAP = kPprRowCap;
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  __shared__ uint32_t lists[256 / kWave][BS * CAP];
-  const int lane = lane_id();
-  const int row = lane >> 3, cg = lane & 7;
-  uint32_t* __restrict__ list = lists[threadIdx.x / kWave];
-  const int c = wave_index();
-  if (c >= A.nchunks) return;
-  const int64_t cb = chunk_start(A, c);
-  const int64_t ce = chunk_start(A, c + 1);
-  const bool last = (c == A.nchunks - 1);
-  const uint64_t* __restrict__ tw = (const uint64_t*)A.tiles;
-
-  for (int32_t R0 = A.plan[c]; R0 < A.nbr;) {
-    const int32_t Rl = R0 + lane;
-    int32_t rsl = 0, rel = 0;
-    if (Rl < A.nbr) {
-      rsl = A.rowptr[Rl];
-      rel = A.rowptr[Rl + 1];
-    }
-    const bool belong = (Rl < A.nbr) && (last || (int64_t)rsl < ce);
-    const uint64_t bmask = __ballot(belong);
-    uint64_t todo = bmask;  // empty rows are written with the epilogue too
-    while (todo) {
-      const int j = __builtin_ctzll(todo);
-      todo &= todo - 1;
-      const int64_t R = R0 + j;
-      const int64_t rs = __builtin_amdgcn_readlane(rsl, j), re = __builtin_amdgcn_readlane(rel, j);
-      const int64_t s = rs > cb ? rs : cb;
-      const int64_t te = re < ce ? re : ce;
-      const bool full = (rs >= cb) && (re <= ce);
-      double acc[8];
-#pragma unroll
-      for (int m = 0; m < 8; ++m) acc[m] = 0.0;
-      for (int64_t b = s; b < te; b += kWave) {
-        const int64_t nt = min((int64_t)kWave, te - b);
-        const uint64_t word = lane < nt ? tw[b + lane] : 0ull;
-        const uint32_t vb = lane < nt ? (uint32_t)A.colind[b + lane] * BS + (BS - 1) : 0u;
-        int maxlen = 0, mylen = 0;
-        {
-          // row totals of the block (sublist lengths)
-          uint32_t tot[4];
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            const uint32_t qh = (uint32_t)__popc((uint32_t)(word >> (16 * h)) & 0xFFu) |
-                                ((uint32_t)__popc((uint32_t)(word >> (16 * h + 8)) & 0xFFu) << 16);
-            tot[h] = __builtin_amdgcn_readlane((uint32_t)wave_incl_scan((int)qh), kWave - 1);
-          }
-#pragma unroll
-          for (int r = 0; r < BS; ++r) {
-            const int l = (int)field16(tot[r >> 1], r & 1);
-            maxlen = l > maxlen ? l : maxlen;
-            mylen = (row == r) ? l : mylen;
-          }
-        }
-        for (int pass = 0; pass < maxlen; pass += CAP) {
-          // this lane's bits of every row whose sublist index is in the pass
-          // (offsets recomputed per pass, so that they are not live across
-          // the gathers)
-#pragma unroll
-          for (int r = 0; r < BS; ++r) {
-            uint32_t byte = (uint32_t)(word >> (8 * r)) & 0xFFu;
-            const uint32_t qr = (uint32_t)__popc(byte);
-            int k = wave_incl_scan((int)qr) - (int)qr - pass;
-            while (byte) {
-              const int bit = __builtin_ctz(byte);  // column 7 - bit
-              byte &= byte - 1;
-              if (k >= 0 && k < CAP) list[r * CAP + k] = vb - (uint32_t)bit;
-              ++k;
-            }
-          }
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-          const int lr = min(max(mylen - pass, 0), CAP);
-          const int kmax = min(maxlen - pass, CAP);
-          for (int k0 = 0; k0 < kmax; k0 += U) {
-            f32x4 xa[U], xb[U];
-            bool ok[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              ok[u] = k0 + u < lr;
-              const uint32_t v = ok[u] ? list[row * CAP + k0 + u] : 0u;  // row 0 stands in
-              const f32x4* px = (const f32x4*)(A.X + (int64_t)v * A.ld + cg * 8);
-              xa[u] = px[0];
-              xb[u] = px[1];
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              if (ok[u]) {
-                acc[0] += (double)xa[u].x;
-                acc[1] += (double)xa[u].y;
-                acc[2] += (double)xa[u].z;
-                acc[3] += (double)xa[u].w;
-                acc[4] += (double)xb[u].x;
-                acc[5] += (double)xb[u].y;
-                acc[6] += (double)xb[u].z;
-                acc[7] += (double)xb[u].w;
-              }
-            }
-          }
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        }
-      }
-      const int64_t i = R * BS + row;
-      if (i < A.nrows) {
-        if (full) {
-          const double rsc = A.rowscale ? (double)A.rowscale[i] : 1.0;
-          f32x4 za = {0.f, 0.f, 0.f, 0.f}, zb = za;
-          if (A.Z) {
-            const f32x4* pz = (const f32x4*)(A.Z + i * A.ld + cg * 8);
-            za = pz[0];
-            zb = pz[1];
-          }
-          const float zz[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
-          float y[8];
-#pragma unroll
-          for (int m = 0; m < 8; ++m) {
-            double t = (double)A.a * rsc * acc[m];
-            if (A.Z) t += (double)A.b * (double)zz[m];
-            y[m] = (float)t;
-          }
-          f32x4* py = (f32x4*)(A.Y + i * A.ld + cg * 8);
-          py[0] = f32x4{y[0], y[1], y[2], y[3]};
-          py[1] = f32x4{y[4], y[5], y[6], y[7]};
-        } else {
-          float* pp = A.partial + (((int64_t)c * 2 + ((rs < cb) ? 0 : 1)) * BS + row) * kWave + cg * 8;
-#pragma unroll
-          for (int m = 0; m < 8; ++m) pp[m] = (float)acc[m];
-        }
-      }
-    }
-    if (__popcll(bmask) < kWave) break;
-    R0 += kWave;
-  }
-}
-
-// Xs[i][k] = X[i][k] * scale[i] over K columns of a row stride ld.
-__global__ __launch_bounds__(256) void k_row_scale(const float* __restrict__ X, const float* __restrict__ scale,
-                                                   float* __restrict__ Xs, int32_t n, int32_t K, int32_t ld) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)n * K) return;
-  const int64_t i = idx / K, k = idx % K;
-  Xs[i * ld + k] = X[i * ld + k] * scale[i];
-}
-
-template <int BS>
-__global__ __launch_bounds__(256) void k_ppr_fixup(const PprArgs A) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = (int)(idx % kWave);
-  const int64_t cr = idx / kWave;  // (chunk, row) pairs
-  const int64_t c = cr / BS;
-  const int r = (int)(cr % BS);
-  if (c + 1 >= A.nchunks) return;
-  const int64_t nb = chunk_start(A, c + 1);
-  const int32_t R = A.plan[c + 1];
-  const int64_t rs = A.rowptr[R], re = A.rowptr[R + 1];
-  if (!(rs < nb) || rs < chunk_start(A, c)) return;
-  float s = A.partial[((c * 2 + 1) * BS + r) * kWave + lane], cmp = 0.0f;
-  for (int64_t c2 = c + 1; c2 < A.nchunks && chunk_start(A, c2) < re; ++c2)
-    nadd(s, cmp, A.partial[((c2 * 2 + 0) * BS + r) * kWave + lane]);
-  const int64_t i = (int64_t)R * BS + r;
-  if (i < A.nrows && lane < A.K) {
-    const float rsc = A.rowscale ? A.rowscale[i] : 1.0f;
-    float y = A.a * rsc * (s + cmp);
-    if (A.Z) y += A.b * A.Z[i * A.ld + lane];
-    A.Y[i * A.ld + lane] = y;
-  }
-}
-
-// Deterministic column-wise reduction over a [n][ld] column block of
-// `cols` <= 64 columns; mode 0: sum |Y - P|, mode 1: sum L * (Y - P),
-// mode 2: sum |Y|.  Each block writes 64 partials; k_colred_final adds
-// them in a fixed order.
-constexpr int kColredBlocks = 2048;  // fixed, so the reduction order is the same on every GPU
-
-__global__ __launch_bounds__(256) void k_colred(const float* __restrict__ Y, const float* __restrict__ P,
-                                                const float* __restrict__ L, int32_t n, int32_t ld, int32_t cols,
-                                                int mode, double* __restrict__ part) {
-  const int col = threadIdx.x & 63, rsub = threadIdx.x >> 6;
-  // four rows per step into four accumulators (loads of a step in flight
-  // together), combined in a fixed order: deterministic for a fixed grid
-  double acc4[4] = {0.0, 0.0, 0.0, 0.0};
-  if (col < cols) {
-    const int64_t S = (int64_t)gridDim.x * 4;
-    for (int64_t i0 = (int64_t)blockIdx.x * 4 + rsub; i0 < n; i0 += 4 * S) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int64_t i = i0 + q * S;
-        if (i < n) {
-          const int64_t o = i * ld + col;
-          if (mode == 0) acc4[q] += fabs((double)Y[o] - (double)P[o]);
-          else if (mode == 1) acc4[q] += (double)L[o] * ((double)Y[o] - (double)P[o]);
-          else acc4[q] += fabs((double)Y[o]);
-        }
-      }
-    }
-  }
-  const double acc = (acc4[0] + acc4[1]) + (acc4[2] + acc4[3]);
-  __shared__ double sh[256];
-  sh[threadIdx.x] = acc;
-  __syncthreads();
-  if (threadIdx.x < 64)
-    part[(int64_t)blockIdx.x * 64 + threadIdx.x] =
-        sh[threadIdx.x] + sh[threadIdx.x + 64] + sh[threadIdx.x + 128] + sh[threadIdx.x + 192];
-}
-
-// One block of 1024 threads: 16 per column, thread (s, k) adds the partials
-// of blocks s, s+16, s+32, ... in order (eight loads in flight), then the
-// 16 sums of a column are added in s order -- a fixed order for a fixed nb.
-constexpr int kColredFinalThreads = 1024;
-__global__ __launch_bounds__(kColredFinalThreads) void k_colred_final(const double* __restrict__ part, int nb,
-                                                                      double* out) {
-  constexpr int NS = kColredFinalThreads / 64;
-  __shared__ double sh[NS][64];
-  const int k = threadIdx.x & 63, sidx = threadIdx.x >> 6;
+// Column sums of |Y| ([n][K]) into the same partials, kMainBlocks of them.
+__global__ __launch_bounds__(kBlk) void k_col_abs(const float* __restrict__ Y, int32_t n, int32_t K, double* part) {
+  __shared__ double sh[kBlk];
+  const int k = threadIdx.x & 63, sub = threadIdx.x >> 6;
   double s = 0.0;
-  int b = sidx;
-  for (; b + 7 * NS < nb; b += 8 * NS) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)(b + u * NS) * 64 + k];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += v[u];
+  if (k < K) {
+    for (int64_t i = (int64_t)blockIdx.x * 4 + sub; i < n; i += (int64_t)gridDim.x * 4)
+      s += fabs((double)Y[i * K + k]);
   }
-  for (; b < nb; b += NS) s += part[(int64_t)b * 64 + k];
-  sh[sidx][k] = s;
+  sh[threadIdx.x] = s;
   __syncthreads();
-  if (sidx == 0) {
-    double t = 0.0;
-#pragma unroll
-    for (int q = 0; q < NS; ++q) t += sh[q][k];
-    out[k] = t;
+  if (sub == 0 && k < K)
+    part[(int64_t)k * (kMainBlocks + kFixBlocks) + blockIdx.x] = sh[k] + sh[k + 64] + sh[k + 128] + sh[k + 192];
+}
+
+// Workgroup k adds column k's partials [0, n0) and [kMainBlocks, kMainBlocks
+// + n1) in a fixed order.  NORM: they are the columns' norms.  Otherwise the
+// last workgroup to finish compares them with tol: done where max_k val[k] /
+// norm[k] (val[k] where norm[k] is 0) is below it.
+template <bool NORM>
+__global__ __launch_bounds__(kBlk) void k_colsum(const double* __restrict__ part, int n0, int n1, int K, double tol,
+                                                 Ctl* ctl) {
+  if (!NORM && ctl->done) return;
+  __shared__ double sh[kBlk];
+  const int k = blockIdx.x, t = threadIdx.x;
+  const double* __restrict__ p = part + (int64_t)k * (kMainBlocks + kFixBlocks);
+  double s = 0.0;
+#pragma unroll 4
+  for (int i = t; i < n0; i += kBlk) s += p[i];
+  for (int i = t; i < n1; i += kBlk) s += p[kMainBlocks + i];
+  sh[t] = s;
+  __syncthreads();
+  for (int off = kBlk / 2; off > 0; off >>= 1) {
+    if (t < off) sh[t] += sh[t + off];
+    __syncthreads();
+  }
+  __shared__ bool last;
+  if (t == 0) {
+    last = false;
+    if (NORM) {
+      ctl->norm[k] = sh[0];
+    } else {
+      __hip_atomic_store(&ctl->val[k], sh[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = __hip_atomic_fetch_add(&ctl->ticket, 1ull, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 ==
+             (unsigned long long)K;
+    }
+  }
+  __syncthreads();
+  if (!last || t >= kWave) return;
+  double m = 0.0;
+  if (t < K) {
+    const double v = __hip_atomic_load(&ctl->val[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double r = ctl->norm[t] > 0.0 ? v / ctl->norm[t] : v;
+    m = m < r ? r : m;
+  }
+  for (int off = 1; off < kWave; off <<= 1) {
+    const double o = __shfl_xor(m, off);
+    m = m < o ? o : m;
+  }
+  if (t == 0) {
+    ctl->ticket = 0;
+    ctl->dmax = m;
+    ctl->iters += 1;
+    if (m < tol) ctl->done = 1;
   }
 }
 
@@ -509,168 +409,173 @@ __global__ void k_invdeg(const int32_t* __restrict__ deg, float* __restrict__ in
   if (i < n) inv[i] = deg[i] > 0 ? 1.0f / (float)deg[i] : 0.0f;
 }
 
-__global__ void k_scale_copy(const float* __restrict__ src, float* __restrict__ dst, int64_t n, float a) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = a * src[i];
+__global__ void k_ctl_init(Ctl* ctl) {
+  ctl->done = ctl->iters = ctl->ticket = 0;
+  ctl->dmax = 0.0;
 }
 
-// Plans with a chunk sized for the SpMM (one tile costs up to bs*K loads).
-// The SpMM's work plan and scratch, released on every return path.
-struct PprPlan {
-  int32_t* plan = nullptr;
-  int32_t chunk = 0, nchunks = 0;
-  float* partial = nullptr;
-  float* xs = nullptr;  // bs 8: X with the per-source scale applied, [n][K]
-  int64_t xs_len = 0;
-  hipStream_t st = nullptr;
-  explicit PprPlan(hipStream_t s) : st(s) {}
-  ~PprPlan() {
-    if (plan) (void)hipFreeAsync(plan, st);
-    if (partial) (void)hipFreeAsync(partial, st);
-    if (xs) (void)hipFreeAsync(xs, st);
+// dst = src ([n][K] -> [n][ld], zeros in the padding) and, with xs, xs =
+// dst * scale (per row).  dst may be null.
+__global__ __launch_bounds__(256) void k_pad(const float* __restrict__ src, int32_t n, int32_t K, int32_t ld,
+                                             float* __restrict__ dst, const float* __restrict__ scale,
+                                             float* __restrict__ xs) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t q4 = ld / 4;
+  if (idx >= n * q4) return;
+  const int64_t i = idx / q4;
+  const int k0 = (int)(idx % q4) * 4;
+  float v[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = k0 + q < K ? src[i * K + k0 + q] : 0.f;
+  if (dst) *(f32x4*)(dst + i * ld + k0) = f32x4{v[0], v[1], v[2], v[3]};
+  if (xs) {
+    const float s = scale[i];
+    *(f32x4*)(xs + i * ld + k0) = f32x4{v[0] * s, v[1] * s, v[2] * s, v[3] * s};
   }
-  PprPlan(const PprPlan&) = delete;
-  PprPlan& operator=(const PprPlan&) = delete;
+}
+
+// dst [n][K] = a * src [n][ld].
+__global__ __launch_bounds__(256) void k_unpad(const float* __restrict__ src, int32_t n, int32_t K, int32_t ld, float a,
+                                               float* __restrict__ dst) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= (int64_t)n * K) return;
+  const int64_t i = idx / K, k = idx % K;
+  dst[idx] = a * src[i * ld + k];
+}
+
+unsigned grid_of(int64_t items, int per_block) {
+  return (unsigned)std::max<int64_t>(1, (items + per_block - 1) / per_block);
+}
+
+bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// The operand of a solve's products: the matrix as CSR segments.
+struct Operand {
+  CsrList csr;
+  const Seg* segs = nullptr;
+  const int64_t* off = nullptr;
+  const int32_t* mrow = nullptr;
+  int64_t nseg = 0, nslot = 0, nmulti = 0;
 };
 
-__global__ void k_plan_ppr(const int32_t* __restrict__ rowptr, int32_t nbr, int32_t chunk, int32_t nchunks,
-                           int32_t* __restrict__ plan) {
-  const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nchunks) return;
-  const int64_t b = (int64_t)c * chunk;
-  int32_t lo = 0, hi = nbr;
-  while (lo < hi) {
-    const int32_t mid = lo + (hi - lo) / 2;
-    if ((int64_t)rowptr[mid] < b) lo = mid + 1;
-    else hi = mid;
-  }
-  int32_t R = lo;
-  if ((int64_t)rowptr[R] > b) R -= 1;
-  if (R >= nbr) R = nbr > 0 ? nbr - 1 : 0;
-  if (R < 0) R = 0;
-  plan[c] = R;
+int make_operand(const gbo_bsr* M, AsyncAllocs& mem, Operand* o, hipStream_t st) {
+  const char* who = "gbo_ppr";
+  const int32_t n = M->nrows;
+  int rc = expand_csr(M, mem, &o->csr, st);
+  if (rc) return rc;
+  AsyncAllocs tmp(st);
+  int64_t *cnt = nullptr, *moff = nullptr, *off = nullptr;
+  int32_t *multi = nullptr, *mrow = nullptr;
+  if ((rc = tmp.alloc(&cnt, sizeof(int64_t) * (size_t)std::max(n, 1), who)) ||
+      (rc = tmp.alloc(&multi, sizeof(int32_t) * (size_t)std::max(n, 1), who)) ||
+      (rc = tmp.alloc(&moff, sizeof(int64_t) * ((size_t)n + 1), who)) ||
+      (rc = mem.alloc(&off, sizeof(int64_t) * ((size_t)n + 1), who)))
+    return rc;
+  k_seg_count<<<grid_of(n, 256), 256, 0, st>>>(o->csr.rowptr, n, cnt, multi);
+  GBO_LAUNCH_CHECK();
+  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, off, n, st))) return rc;
+  if ((rc = scan_exclusive<int32_t, int64_t>(multi, moff, n, st))) return rc;
+  int64_t tot = 0;
+  GBO_HIP_CHECK(hipMemcpyAsync(&tot, off + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  GBO_HIP_CHECK(hipMemcpyAsync(&o->nmulti, moff + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  o->nseg = tot & 0xFFFFFFFF;
+  o->nslot = tot >> 32;
+  Seg* segs = nullptr;
+  if ((rc = mem.alloc(&segs, sizeof(Seg) * (size_t)std::max<int64_t>(o->nseg, 1), who)) ||
+      (rc = mem.alloc(&mrow, sizeof(int32_t) * (size_t)std::max<int64_t>(o->nmulti, 1), who)))
+    return rc;
+  k_seg_fill<<<grid_of(n, 256), 256, 0, st>>>(o->csr.rowptr, n, off, moff, segs, mrow);
+  GBO_LAUNCH_CHECK();
+  o->segs = segs;
+  o->off = off;
+  o->mrow = mrow;
+  return GBO_OK;
 }
 
-// k_row_scale for K % 4 == 0 and 16-byte aligned X and Xs (ld == K):
-// four columns per thread, n * K < 2^32.
-__global__ __launch_bounds__(256) void k_row_scale4(const float* __restrict__ X, const float* __restrict__ scale,
-                                                    float* __restrict__ Xs, uint32_t n4, uint32_t K4) {
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n4) return;
-  const uint32_t i = t / K4;
-  ((f32x4*)Xs)[t] = ((const f32x4*)X)[t] * scale[i];
-}
+int main_blocks(const Operand& o) { return (int)std::min<int64_t>(kMainBlocks, (o.nseg + kUnits - 1) / kUnits); }
+int fix_blocks(const Operand& o) { return (int)std::min<int64_t>(kFixBlocks, (o.nmulti + kBlk / kWave - 1) / (kBlk / kWave)); }
 
-static int make_ppr_plan(const gbo_bsr* M, PprPlan* P, hipStream_t st) {
-  P->chunk = 1024;
-  P->nchunks = (int32_t)std::max<int64_t>(1, (M->nblocks + P->chunk - 1) / P->chunk);
-  GBO_HIP_CHECK(hipMallocAsync((void**)&P->plan, sizeof(int32_t) * P->nchunks, st));
-  GBO_HIP_CHECK(hipMallocAsync((void**)&P->partial, sizeof(float) * 2 * (size_t)P->nchunks * M->bs * kWave, st));
-  k_plan_ppr<<<(P->nchunks + 255) / 256, 256, 0, st>>>(M->rowptr, M->nblockrows, P->chunk, P->nchunks, P->plan);
+template <int LPR>
+int spmm_t(const Operand& o, const SpmmArgs& A, hipStream_t st) {
+  const int nb = main_blocks(o), nf = fix_blocks(o);
+  if (nb > 0) k_spmm<LPR><<<nb, kBlk, 0, st>>>(A);
+  if (nf > 0) k_spmm_fix<LPR><<<nf, kBlk, 0, st>>>(A);
   GBO_LAUNCH_CHECK();
   return GBO_OK;
 }
 
-// Y = a * rowscale * (M (colscale .* X)) + b * Z over all K columns.
-static int spmm(const gbo_bsr* M, PprPlan& P, int32_t K, const float* X, const float* colscale,
-                const float* rowscale, float a, float b, const float* Z, float* Y, hipStream_t st) {
-  if (M->bs == 8 && M->ncols > (1 << 29))
-    return set_error(GBO_EUNSUPPORTED, "PPR at block size 8 supports up to 2^29 vertices");
-  if (M->bs == 8 && colscale) {
-    // the bs 8 kernel reads pre-scaled rows
-    const int64_t len = (int64_t)M->ncols * K;
-    if (P.xs_len < len) {
-      if (P.xs) GBO_HIP_CHECK(hipFreeAsync(P.xs, st));
-      P.xs = nullptr;
-      GBO_HIP_CHECK(hipMallocAsync((void**)&P.xs, sizeof(float) * std::max<int64_t>(len, 1), st));
-      P.xs_len = len;
-    }
-    if (len > 0) {
-      if (K % 4 == 0 && len < ((int64_t)1 << 32) && ((((uintptr_t)X) | ((uintptr_t)P.xs)) & 15) == 0) {
-        const uint32_t n4 = (uint32_t)(len / 4);
-        k_row_scale4<<<(n4 + 255) / 256, 256, 0, st>>>(X, colscale, P.xs, n4, (uint32_t)(K / 4));
-      } else {
-        k_row_scale<<<(unsigned)((len + 255) / 256), 256, 0, st>>>(X, colscale, P.xs, M->ncols, K, K);
-      }
-      GBO_LAUNCH_CHECK();
-    }
-    X = P.xs;
-    colscale = nullptr;
-  }
-  // bs 8 with whole 64-column blocks and 16-byte aligned rows: the per-row
-  // sublist kernel (the same sums as the flat-list one, fewer instructions)
-  const bool rows8 = M->bs == 8 && K % kWave == 0 && ((((uintptr_t)X) | ((uintptr_t)Y) | ((uintptr_t)Z)) & 15) == 0;
-  for (int32_t k0 = 0; k0 < K; k0 += kWave) {
-    PprArgs A{};
-    A.rowptr = M->rowptr;
-    A.colind = M->colind;
-    A.tiles = M->tiles;
-    A.nrows = M->nrows;
-    A.nbr = M->nblockrows;
-    A.T = M->nblocks;
-    A.plan = P.plan;
-    A.chunk = P.chunk;
-    A.nchunks = P.nchunks;
-    A.K = std::min(kWave, K - k0);
-    A.ld = K;
-    A.X = X + k0;
-    A.colscale = colscale;
-    A.rowscale = rowscale;
-    A.a = a;
-    A.b = b;
-    A.Z = Z ? Z + k0 : nullptr;
-    A.Y = Y + k0;
-    A.partial = P.partial;
-    const unsigned blocks = (unsigned)(((int64_t)P.nchunks + 3) / 4);
-    switch (M->bs) {
-      case 8: {
-        if (rows8) k_ppr_spmm8r<<<blocks, 256, 0, st>>>(A);
-        else k_ppr_spmm8<<<blocks, 256, 0, st>>>(A);
-        break;
-      }
-      case 16: k_ppr_spmm<16><<<blocks, 256, 0, st>>>(A); break;
-      case 32: k_ppr_spmm<32><<<blocks, 256, 0, st>>>(A); break;
-      default: return set_error(GBO_EUNSUPPORTED, "PPR supports block sizes 8, 16, 32");
-    }
-    GBO_LAUNCH_CHECK();
-    if (P.nchunks > 1) {
-      const int64_t thr = (int64_t)(P.nchunks - 1) * M->bs * kWave;
-      const unsigned fb = (unsigned)((thr + 255) / 256);
-      switch (M->bs) {
-        case 8: k_ppr_fixup<8><<<fb, 256, 0, st>>>(A); break;
-        case 16: k_ppr_fixup<16><<<fb, 256, 0, st>>>(A); break;
-        case 32: k_ppr_fixup<32><<<fb, 256, 0, st>>>(A); break;
-      }
-      GBO_LAUNCH_CHECK();
-    }
-  }
+// One product with its measure, and the measure's verdict.
+int spmm(const Operand& o, SpmmArgs A, double tol, hipStream_t st) {
+  A.segs = o.segs;
+  A.nseg = o.nseg;
+  A.mrow = o.mrow;
+  A.nmulti = o.nmulti;
+  A.off = o.off;
+  A.col = o.csr.col;
+  A.zvec = A.K % 4 == 0 && al16(A.Z);
+  int rc = A.ld > 32 ? spmm_t<16>(o, A, st)
+           : A.ld > 16 ? spmm_t<8>(o, A, st)
+           : A.ld > 8 ? spmm_t<4>(o, A, st)
+           : A.ld > 4 ? spmm_t<2>(o, A, st)
+                      : spmm_t<1>(o, A, st);
+  if (rc) return rc;
+  k_colsum<false><<<A.K, kBlk, 0, st>>>(A.part, main_blocks(o), fix_blocks(o), A.K, tol, A.ctl);
+  GBO_LAUNCH_CHECK();
   return GBO_OK;
 }
 
-// Column-wise reduction over [n][K] in column blocks of 64 (deterministic).
-static int colreduce(const float* Y, const float* P, const float* L, int32_t n, int32_t K, int mode, double* d_part,
-                     double* d_out, double* h_out, hipStream_t st) {
-  constexpr int nb = kColredBlocks;
-  for (int32_t k0 = 0; k0 < K; k0 += 64) {
-    const int32_t cols = std::min(64, K - k0);
-    k_colred<<<nb, 256, 0, st>>>(Y + k0, P ? P + k0 : nullptr, L ? L + k0 : nullptr, n, K, cols, mode, d_part);
-    GBO_LAUNCH_CHECK();
-    k_colred_final<<<1, kColredFinalThreads, 0, st>>>(d_part, nb, d_out);
-    GBO_LAUNCH_CHECK();
-    GBO_HIP_CHECK(hipMemcpyAsync(h_out + k0, d_out, sizeof(double) * cols, hipMemcpyDeviceToHost, st));
-  }
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+// Scratch of a solve: padded iterates, measure partials, state.
+struct Scratch {
+  float* inv = nullptr;
+  double *part = nullptr, *partial = nullptr;
+  Ctl* ctl = nullptr;
+};
+
+int make_scratch(const int32_t* d_outdeg, int32_t n, int32_t ld, int64_t nslot, AsyncAllocs& mem, Scratch* s,
+                 hipStream_t st) {
+  const char* who = "gbo_ppr";
+  int rc;
+  if ((rc = mem.alloc(&s->inv, sizeof(float) * (size_t)std::max(n, 1), who)) ||
+      (rc = mem.alloc(&s->part, sizeof(double) * 64 * (kMainBlocks + kFixBlocks), who)) ||
+      (rc = mem.alloc(&s->partial, sizeof(double) * (size_t)std::max<int64_t>(nslot * ld, 1), who)) ||
+      (rc = mem.alloc(&s->ctl, sizeof(Ctl), who)))
+    return rc;
+  k_invdeg<<<grid_of(n, 256), 256, 0, st>>>(d_outdeg, s->inv, n);
+  k_ctl_init<<<1, 1, 0, st>>>(s->ctl);
+  GBO_LAUNCH_CHECK();
   return GBO_OK;
 }
 
-// max over columns of delta[k] / norm[k] (delta[k] itself where norm[k] is 0)
-static double max_relative(const std::vector<double>& delta, const std::vector<double>& norm) {
-  double m = 0.0;
-  for (size_t k = 0; k < delta.size(); ++k) m = std::max(m, norm[k] > 0.0 ? delta[k] / norm[k] : delta[k]);
-  return m;
+// The columns' norms of the driving vectors: the change is measured relative
+// to them (1 for a distribution).
+int col_norms(const float* Y, int32_t n, int32_t K, const Scratch& s, hipStream_t st) {
+  const int nb = (int)std::min<int64_t>(kMainBlocks, grid_of(n, 16));
+  k_col_abs<<<nb, kBlk, 0, st>>>(Y, n, K, s.part);
+  k_colsum<true><<<K, kBlk, 0, st>>>(s.part, nb, 0, K, 0.0, s.ctl);
+  GBO_LAUNCH_CHECK();
+  return GBO_OK;
 }
 
+// Runs step(it) for it = 0, 1, ... until the device says done or max_iter.
+template <class Step>
+int iterate(int32_t max_iter, const Scratch& s, int32_t* iters, double* dmax, hipStream_t st, Step step) {
+  int32_t it = 0;
+  Ctl h{};
+  while (it < max_iter && !h.done) {
+    for (int b = 0; b < kBatch && it < max_iter; ++b, ++it) {
+      const int rc = step(it);
+      if (rc) return rc;
+    }
+    GBO_HIP_CHECK(hipMemcpyAsync(&h, s.ctl, offsetof(Ctl, val), hipMemcpyDeviceToHost, st));
+    GBO_HIP_CHECK(hipStreamSynchronize(st));
+  }
+  *iters = (int32_t)h.iters;
+  *dmax = h.dmax;
+  return GBO_OK;
+}
+
+}  // namespace
 }  // namespace gbo
 
 using namespace gbo;
@@ -686,39 +591,51 @@ int gbo_ppr_forward(const gbo_bsr* AT, const int32_t* d_outdeg, int32_t K, float
   if (!(alpha > 0.0f && alpha < 1.0f) || max_iter < 1) return set_error(GBO_EINVAL, "gbo_ppr_forward: bad alpha/max_iter");
   if (!d_outdeg || !d_s || !d_p) return set_error(GBO_EINVAL, "gbo_ppr_forward: null argument");
   if (AT->bs > 32) return set_error(GBO_EUNSUPPORTED, "gbo_ppr_forward: block sizes 8, 16, 32");
+  if (AT->bs == 8 && AT->ncols > (1 << 29))
+    return set_error(GBO_EUNSUPPORTED, "PPR at block size 8 supports up to 2^29 vertices");
   hipStream_t st = stream;
-  const int32_t n = AT->nrows;
-  const int64_t nk = (int64_t)n * K;
+  const int32_t n = AT->nrows, ld = (K + 3) / 4 * 4;
+  const size_t bytes = sizeof(float) * (size_t)std::max<int64_t>((int64_t)n * ld, 1);
   AsyncAllocs mem(st);
-  float *inv = nullptr, *q = nullptr;
-  double* dpart = nullptr;
-  if ((rc = mem.alloc(&inv, sizeof(float) * std::max(n, 1), "gbo_ppr_forward")) ||
-      (rc = mem.alloc(&q, sizeof(float) * std::max<int64_t>(nk, 1), "gbo_ppr_forward")) ||
-      (rc = mem.alloc(&dpart, sizeof(double) * (kColredBlocks * 64 + 64), "gbo_ppr_forward")))
+  Operand o;
+  Scratch s;
+  if ((rc = make_operand(AT, mem, &o, st)) || (rc = make_scratch(d_outdeg, n, ld, o.nslot, mem, &s, st))) return rc;
+  // the iterate stays in the caller's buffer where its rows can be read 16
+  // bytes at a time; the products read it scaled by 1 / outdeg, from two
+  // buffers in turn
+  float *p = d_p, *xs[2] = {nullptr, nullptr};
+  const bool own = ld != K || !al16(d_p);
+  if ((own && (rc = mem.alloc(&p, bytes, "gbo_ppr_forward"))) ||
+      (rc = mem.alloc(&xs[0], bytes, "gbo_ppr_forward")) || (rc = mem.alloc(&xs[1], bytes, "gbo_ppr_forward")))
     return rc;
-  k_invdeg<<<(n + 255) / 256, 256, 0, st>>>(d_outdeg, inv, n);
+  k_pad<<<grid_of((int64_t)n * (ld / 4), 256), 256, 0, st>>>(d_s, n, K, ld, p, s.inv, xs[0]);  // p_0 = s
   GBO_LAUNCH_CHECK();
-  PprPlan P(st);
-  if ((rc = make_ppr_plan(AT, &P, st))) return rc;
-  // p_0 = s
-  GBO_HIP_CHECK(hipMemcpyAsync(d_p, d_s, sizeof(float) * nk, hipMemcpyDeviceToDevice, st));
-  std::vector<double> delta(K), snorm(K);
-  // the change is measured relative to ||s_k||_1 (1 for a distribution)
-  if ((rc = colreduce(d_s, nullptr, nullptr, n, K, 2, dpart, dpart + kColredBlocks * 64, snorm.data(), st))) return rc;
+  if ((rc = col_norms(d_s, n, K, s, st))) return rc;
+  SpmmArgs A{};
+  A.K = K;
+  A.ld = ld;
+  A.a = alpha;
+  A.b = 1.0f - alpha;
+  A.Z = d_s;
+  A.Y = p;
+  A.P = p;
+  A.xscale = s.inv;
+  A.partial = s.partial;
+  A.part = s.part;
+  A.ctl = s.ctl;
   int32_t it = 0;
   double dmax = 0.0;
-  float* cur = d_p;
-  float* nxt = q;
-  while (it < max_iter) {
-    if ((rc = spmm(AT, P, K, cur, inv, nullptr, alpha, 1.0f - alpha, d_s, nxt, st))) return rc;
-    if ((rc = colreduce(nxt, cur, nullptr, n, K, 0, dpart, dpart + kColredBlocks * 64, delta.data(), st))) return rc;
-    ++it;
-    std::swap(cur, nxt);
-    dmax = max_relative(delta, snorm);
-    if (dmax < tol) break;
+  rc = iterate(max_iter, s, &it, &dmax, st, [&](int32_t i) {
+    A.X = xs[i & 1];
+    A.Xs = xs[(i + 1) & 1];
+    return spmm(o, A, tol, st);
+  });
+  if (rc) return rc;
+  if (own) {
+    k_unpad<<<grid_of((int64_t)n * K, 256), 256, 0, st>>>(p, n, K, ld, 1.0f, d_p);
+    GBO_LAUNCH_CHECK();
+    GBO_HIP_CHECK(hipStreamSynchronize(st));
   }
-  if (cur != d_p) GBO_HIP_CHECK(hipMemcpyAsync(d_p, cur, sizeof(float) * nk, hipMemcpyDeviceToDevice, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
   if (h_iters) *h_iters = it;
   if (h_delta) *h_delta = dmax;
   if (!(dmax < tol))
@@ -738,50 +655,73 @@ int gbo_ppr_adjoint(const gbo_bsr* A, const gbo_bsr* AT, const int32_t* d_outdeg
   if (!(alpha > 0.0f && alpha < 1.0f) || max_iter < 1) return set_error(GBO_EINVAL, "gbo_ppr_adjoint: bad alpha/max_iter");
   if (!d_outdeg || !d_s || !d_p || !d_w || !d_grad_s) return set_error(GBO_EINVAL, "gbo_ppr_adjoint: null argument");
   if (A->bs > 32 || AT->bs > 32) return set_error(GBO_EUNSUPPORTED, "gbo_ppr_adjoint: block sizes 8, 16, 32");
+  if ((A->bs == 8 && A->ncols > (1 << 29)) || (AT->bs == 8 && AT->ncols > (1 << 29)))
+    return set_error(GBO_EUNSUPPORTED, "PPR at block size 8 supports up to 2^29 vertices");
   hipStream_t st = stream;
-  const int32_t n = A->nrows;
-  const int64_t nk = (int64_t)n * K;
-  AsyncAllocs mem(st);
-  float *inv = nullptr, *lam = nullptr;
-  double* dpart = nullptr;
-  if ((rc = mem.alloc(&inv, sizeof(float) * std::max(n, 1), "gbo_ppr_adjoint")) ||
-      (rc = mem.alloc(&lam, sizeof(float) * std::max<int64_t>(nk, 1) * 2, "gbo_ppr_adjoint")) ||
-      (rc = mem.alloc(&dpart, sizeof(double) * (kColredBlocks * 64 + 64), "gbo_ppr_adjoint")))
+  const int32_t n = A->nrows, ld = (K + 3) / 4 * 4;
+  const size_t bytes = sizeof(float) * (size_t)std::max<int64_t>((int64_t)n * ld, 1);
+  const bool same = A->rowptr == AT->rowptr && A->colind == AT->colind && A->tiles == AT->tiles && A->bs == AT->bs &&
+                    A->nblocks == AT->nblocks;
+  AsyncAllocs mem(st), memT(st);
+  Operand o, oT;
+  Scratch s;
+  if ((rc = make_operand(A, mem, &o, st))) return rc;
+  if (same) oT = o;
+  else if ((rc = make_operand(AT, memT, &oT, st))) return rc;
+  if ((rc = make_scratch(d_outdeg, n, ld, std::max(o.nslot, oT.nslot), mem, &s, st))) return rc;
+  float* lam[2] = {nullptr, nullptr};
+  if ((rc = mem.alloc(&lam[0], bytes, "gbo_ppr_adjoint")) || (rc = mem.alloc(&lam[1], bytes, "gbo_ppr_adjoint")))
     return rc;
-  float* q = lam + nk;
-  k_invdeg<<<(n + 255) / 256, 256, 0, st>>>(d_outdeg, inv, n);
+  const unsigned padg = grid_of((int64_t)n * (ld / 4), 256);
+  k_pad<<<padg, 256, 0, st>>>(d_w, n, K, ld, lam[0], nullptr, nullptr);
   GBO_LAUNCH_CHECK();
-  PprPlan PA(st), PT(st);
-  if ((rc = make_ppr_plan(A, &PA, st)) || (rc = make_ppr_plan(AT, &PT, st))) return rc;
-  GBO_HIP_CHECK(hipMemcpyAsync(lam, d_w, sizeof(float) * nk, hipMemcpyDeviceToDevice, st));
-  std::vector<double> delta(K), ga(K), wnorm(K);
-  // the change is measured relative to ||w_k||_1, the scale of lambda_k
-  if ((rc = colreduce(d_w, nullptr, nullptr, n, K, 2, dpart, dpart + kColredBlocks * 64, wnorm.data(), st))) return rc;
+  if ((rc = col_norms(d_w, n, K, s, st))) return rc;
+  // lambda' = alpha * D^-1 A lambda + w
+  SpmmArgs S{};
+  S.K = K;
+  S.ld = ld;
+  S.rowscale = s.inv;
+  S.a = alpha;
+  S.b = 1.0f;
+  S.Z = d_w;
+  S.partial = s.partial;
+  S.part = s.part;
+  S.ctl = s.ctl;
   int32_t it = 0;
-  float* cur = lam;
-  float* nxt = q;
   double dmax = 0.0;
-  while (it < max_iter) {
-    // lambda' = alpha * D^-1 A lambda + w
-    if ((rc = spmm(A, PA, K, cur, nullptr, inv, alpha, 1.0f, d_w, nxt, st))) return rc;
-    if ((rc = colreduce(nxt, cur, nullptr, n, K, 0, dpart, dpart + kColredBlocks * 64, delta.data(), st))) return rc;
-    ++it;
-    std::swap(cur, nxt);
-    dmax = max_relative(delta, wnorm);
-    if (dmax < tol) break;
-  }
+  rc = iterate(max_iter, s, &it, &dmax, st, [&](int32_t i) {
+    S.X = S.P = lam[i & 1];
+    S.Y = lam[(i + 1) & 1];
+    return spmm(o, S, tol, st);
+  });
+  if (rc) return rc;
+  const float* cur = lam[it & 1];
+  float* xs = lam[(it + 1) & 1];
   // grad_s = (1 - alpha) * lambda
-  k_scale_copy<<<(unsigned)((nk + 255) / 256), 256, 0, st>>>(cur, d_grad_s, nk, 1.0f - alpha);
-  GBO_LAUNCH_CHECK();
+  k_unpad<<<grid_of((int64_t)n * K, 256), 256, 0, st>>>(cur, n, K, ld, 1.0f - alpha, d_grad_s);
   // dL/dalpha = sum_k lambda_k . (P^T p_k - s_k)
-  if ((rc = spmm(AT, PT, K, d_p, inv, nullptr, 1.0f, 0.0f, nullptr, nxt, st))) return rc;
-  if ((rc = colreduce(nxt, d_s, cur, n, K, 1, dpart, dpart + kColredBlocks * 64, ga.data(), st))) return rc;
-  if (h_grad_alpha) {
-    double s = 0.0;
-    for (double v : ga) s += v;
-    *h_grad_alpha = s;
-  }
+  k_pad<<<padg, 256, 0, st>>>(d_p, n, K, ld, nullptr, s.inv, xs);
+  k_ctl_init<<<1, 1, 0, st>>>(s.ctl);
+  GBO_LAUNCH_CHECK();
+  SpmmArgs T{};
+  T.K = K;
+  T.ld = ld;
+  T.X = xs;
+  T.a = 1.0f;
+  T.P = d_s;
+  T.L = cur;
+  T.partial = s.partial;
+  T.part = s.part;
+  T.ctl = s.ctl;
+  if ((rc = spmm(oT, T, 0.0, st))) return rc;
+  double ga[64];
+  GBO_HIP_CHECK(hipMemcpyAsync(ga, s.ctl->val, sizeof(double) * K, hipMemcpyDeviceToHost, st));
   GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if (h_grad_alpha) {
+    double g = 0.0;
+    for (int32_t k = 0; k < K; ++k) g += ga[k];
+    *h_grad_alpha = g;
+  }
   if (h_iters) *h_iters = it;
   if (!(dmax < tol))
     return set_error(GBO_ENOCONV, "gbo_ppr_adjoint: not converged after %d iterations (%.3e)", it, dmax);
