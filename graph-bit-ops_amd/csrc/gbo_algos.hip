@@ -180,6 +180,8 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
   a.nbr = nbr;
   a.T = A->nblocks;
   a.plan = pv.plan;
+  a.start = pv.start;
+  a.tail = pv.tail;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -554,6 +556,8 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   a.nbr = AT->nblockrows;
   a.T = AT->nblocks;
   a.plan = pv.plan;
+  a.start = pv.start;
+  a.tail = pv.tail;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -611,6 +615,8 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   a.nbr = AT->nblockrows;
   a.T = AT->nblocks;
   a.plan = pv.plan;
+  a.start = pv.start;
+  a.tail = pv.tail;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -678,6 +684,8 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   a.nbr = A->nblockrows;
   a.T = A->nblocks;
   a.plan = pv.plan;
+  a.start = pv.start;
+  a.tail = pv.tail;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

@@ -27,6 +27,8 @@ struct MsArgs {
   int32_t nrows, nbr;
   int64_t T;
   const int32_t* plan;
+  const int64_t* start;  // as in SpmvArgs
+  const int32_t* tail;
   int32_t chunk, nchunks;
   const uint64_t* F;       // n * KW
   const uint64_t* V;       // n * KW
@@ -42,8 +44,7 @@ __global__ __launch_bounds__(256) void k_msbfs(const MsArgs a) {
   const int g = lane / BS, r = lane % BS;
   const int c = wave_index();
   if (c >= a.nchunks) return;
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const W* __restrict__ tiles = (const W*)a.tiles;
 
@@ -148,8 +149,7 @@ __global__ __launch_bounds__(256) void k_msbfs8r(const MsArgs a) {
   uint32_t* __restrict__ list = lists[threadIdx.x / kWave];
   const int c = wave_index();
   if (c >= a.nchunks) return;
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const uint64_t* __restrict__ tw = (const uint64_t*)a.tiles;
 
@@ -252,11 +252,11 @@ __global__ __launch_bounds__(256) void k_msbfs8r(const MsArgs a) {
 template <int BS, int KW>
 __global__ __launch_bounds__(256) void k_ms_prefill(const MsArgs a) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t c = idx / BS + 1;
+  const int64_t c = idx / BS;
   const int r = (int)(idx % BS);
-  if (c >= a.nchunks) return;
-  const int32_t R = a.plan[c];
-  if ((int64_t)a.rowptr[R] >= c * a.chunk) return;
+  if (c + 1 >= a.nchunks) return;
+  const int32_t R = a.plan[c + 1];
+  if (a.tail[c] == 0) return;
   const int64_t i = (int64_t)R * BS + r;
   if (i < a.nrows)
     for (int w = 0; w < KW; ++w) a.Fn[i * KW + w] = 0;
@@ -339,6 +339,8 @@ static int msbfs_t(const gbo_bsr* A, const int32_t* h_src, int32_t nsrc, int32_t
   a.nbr = A->nblockrows;
   a.T = A->nblocks;
   a.plan = pv.plan;
+  a.start = pv.start;
+  a.tail = pv.tail;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   int32_t lvl = 0;

@@ -88,8 +88,7 @@ __global__ __launch_bounds__(256) void k_spmv(const SpmvArgs a) {
   const int g = BS == 64 ? 0 : lane / BS, r = lane % BS;
   const int c = wave_index();
   if (c >= a.nchunks) return;  // wave-uniform
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const W* __restrict__ tiles = (const W*)a.tiles;
   const int32_t* __restrict__ colind = a.colind;
@@ -502,8 +501,7 @@ __global__ __launch_bounds__(256) void k_spmv_lpt(const SpmvArgs a) {
   const int lane = lane_id();
   const int c = wave_index();
   if (c >= a.nchunks) return;
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const int32_t* __restrict__ colind = a.colind;
   const W* __restrict__ xb = (const W*)a.xbits;
@@ -752,8 +750,7 @@ __device__ __forceinline__ void stream_chunk(const SpmvArgs& a, int c, StreamSlo
   constexpr int LPR = kWave / BS;        // lanes per row after the reduce-scatter
   constexpr int64_t STEP = (int64_t)kWave * TPL;
   const int lane = lane_id();
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const W* __restrict__ xb = (const W*)a.xbits;
   int32_t* __restrict__ y = (int32_t*)a.out;
@@ -868,14 +865,14 @@ __device__ __forceinline__ void stream_chunk(const SpmvArgs& a, int c, StreamSlo
 // First tile of chunk c's first step (a multiple of the tiles per lane).
 template <int BS>
 __device__ __forceinline__ int64_t stream_base(const SpmvArgs& a, int c) {
-  const int64_t cb = (int64_t)c * a.chunk;
+  const int64_t cb = chunk_start(a, c);
   return cb - cb % StreamSlots<BS>::TPL;
 }
 
 template <int BS>
 __device__ __forceinline__ void stream_first(const SpmvArgs& a, int c, int lane, StreamSlots<BS>& s) {
-  const int64_t cb = (int64_t)c * a.chunk;
-  stream_load<BS>(a, stream_base<BS>(a, c), lane, cb, min(cb + (int64_t)a.chunk, a.T), s);
+  const int64_t cb = chunk_start(a, c);
+  stream_load<BS>(a, stream_base<BS>(a, c), lane, cb, chunk_start(a, c + 1), s);
 }
 
 // Variant 2: one wavefront per chunk.  The first step's loads are issued
@@ -997,8 +994,7 @@ __global__ __launch_bounds__(256) void k_count8(const SpmvArgs a) {
   const int lane = lane_id();
   const int c = wave_index();
   if (c >= a.nchunks) return;  // wave-uniform
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   // frame: positions relative to b0 (a multiple of 4); tiles and rowptr are
   // int32-indexed (T < 2^31), so every position fits 32 bits
@@ -1140,8 +1136,7 @@ __global__ __launch_bounds__(256) void k_count16q(const SpmvArgs a) {
   const int slot = lane >> 2, q = lane & 3;
   const int c = wave_index();
   if (c >= a.nchunks) return;  // wave-uniform
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const uint64_t* __restrict__ tw = (const uint64_t*)a.tiles;  // 4 words per tile
   const uint16_t* __restrict__ xb = (const uint16_t*)a.xbits;
@@ -1225,8 +1220,7 @@ __global__ __launch_bounds__(256) void k_count32q(const SpmvArgs a) {
   const int slot = lane >> 3, p = lane & 7;
   const int c = wave_index();
   if (c >= a.nchunks) return;  // wave-uniform
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   const u32x4* __restrict__ tw = (const u32x4*)a.tiles;  // 8 x 16 bytes per tile
@@ -1330,8 +1324,7 @@ __global__ __launch_bounds__(256) void k_value_q(const SpmvArgs a) {
   const int slot = lane / LPT, p = lane % LPT;
   const int c = wave_index();
   if (c >= a.nchunks) return;  // wave-uniform
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const int32_t* __restrict__ colind = a.colind;
   const uint32_t* __restrict__ xv = (const uint32_t*)a.xval;
@@ -1557,8 +1550,7 @@ __global__ __launch_bounds__(256) void k_value_lpt(const SpmvArgs a) {
   const int wv = threadIdx.x / kWave;
   const int c = wave_index();
   if (c >= a.nchunks) return;  // wave-uniform; no workgroup barriers below
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const int32_t* __restrict__ colind = a.colind;
   const uint32_t* __restrict__ xv = (const uint32_t*)a.xval;
@@ -1738,16 +1730,16 @@ __global__ __launch_bounds__(256) void k_value_lpt(const SpmvArgs a) {
   }
 }
 
-// Initializes the outputs of split rows (rows that begin before the chunk
-// that lists them) to the identity of the combining atomic.
+// Initializes the outputs of split rows (rows that go on past the chunk they
+// begin in) to the identity of the combining atomic.
 template <int BS, int OP>
 __global__ __launch_bounds__(256) void k_prefill_split(const SpmvArgs a) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t c = idx / BS + 1;
+  const int64_t c = idx / BS;
   const int r = (int)(idx % BS);
-  if (c >= a.nchunks) return;
-  const int32_t R = a.plan[c];
-  if ((int64_t)a.rowptr[R] >= c * a.chunk) return;
+  if (c + 1 >= a.nchunks) return;
+  const int32_t R = a.plan[c + 1];
+  if (a.tail[c] == 0) return;
   const int64_t i = (int64_t)R * BS + r;
   if constexpr (OP == OP_COUNT) {
     if (i < a.nrows) ((int32_t*)a.out)[i] = 0;
@@ -1760,34 +1752,55 @@ __global__ __launch_bounds__(256) void k_prefill_split(const SpmvArgs a) {
   }
 }
 
-// FP32 sum: the chunk that holds the first tile of a split row adds its own
-// partial and those of the following chunks in chunk order.
+// FP32 sum: the partials of a split row, its first chunk's and those of the
+// tail[c] chunks that go on with it, added in a fixed order.  A thread takes
+// one tile row of one such row, up to kOwnTail chunks of it; what a hub row has
+// beyond them (hundreds) the whole wave adds, one row after another, its 64 /
+// BS lane groups each every (64 / BS)-th chunk in order, eight loads in
+// flight, then the groups' sums in a fixed tree.  No thread leaves early: the
+// shuffles need every lane.
+constexpr int kOwnTail = 5;
+
 template <int BS>
 __global__ __launch_bounds__(256) void k_sum_fixup(const SpmvArgs a) {
+  constexpr int G = kWave / BS, U = 8;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t c = idx / BS;
-  const int r = (int)(idx % BS);
-  if (c + 1 >= a.nchunks) return;
-  const int64_t nb = (c + 1) * a.chunk;
+  const int64_t c = min(idx / BS, (int64_t)a.nchunks - 2);  // nchunks >= 2
+  const int r = (int)(idx % BS), g = lane_id() / BS;
   const int32_t R = a.plan[c + 1];
-  const int64_t rs = a.rowptr[R], re = a.rowptr[R + 1];
-  if (!(rs < nb) || rs < c * a.chunk) return;  // not split here, or not the owner
-  // chunks c+1 .. ce-1 hold the rest of the row (a hub row spans hundreds):
-  // their partials are loaded 16 at a time, so the chain costs one memory
-  // latency per 16 chunks, and added in chunk order
-  const int64_t ce = min((int64_t)a.nchunks, (re + a.chunk - 1) / a.chunk);
-  double s = a.partial[(c * 2 + 1) * BS + r];
-  int64_t c2 = c + 1;
-  for (; c2 + 16 <= ce; c2 += 16) {
-    double v[16];
+  const int n = idx / BS + 1 < a.nchunks ? a.tail[c] : 0;
+  double s = 0.0;
+  if (n > 0) {
+    const double own = a.partial[(c * 2 + 1) * BS + r], next = a.partial[(c + 1) * 2 * BS + r];
+    s = own + next;
+    if (n > 1) {
+      double v[kOwnTail];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = a.partial[((c2 + u) * 2 + 0) * BS + r];
+      for (int u = 1; u < kOwnTail; ++u) v[u] = a.partial[(c + 1 + min(u, n - 1)) * 2 * BS + r];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) s += v[u];
+      for (int u = 1; u < kOwnTail; ++u)
+        if (u < n) s += v[u];
+    }
   }
-  for (; c2 < ce; ++c2) s += a.partial[(c2 * 2 + 0) * BS + r];
+  for (uint64_t more = __ballot(n > kOwnTail); more;) {
+    const int j = __builtin_ctzll(more) / BS;  // lane group of the row taken next
+    more &= ~(low_mask<BS>() << (j * BS));
+    const int64_t c0 = __shfl((long long)c, j * BS) + 1;
+    const int nj = __shfl(n, j * BS);
+    double t = 0.0;
+    for (int k = kOwnTail; k < nj; k += U * G) {  // wave-uniform
+      double v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = a.partial[(c0 + min(k + u * G + g, nj - 1)) * 2 * BS + r];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k + u * G + g < nj) t += v[u];
+    }
+    for (int off = BS; off < kWave; off <<= 1) t += __shfl_xor(t, off);
+    if (g == j) s += t;
+  }
   const int64_t i = (int64_t)R * BS + r;
-  if (i < a.nrows) ((float*)a.out)[i] = (float)((double)a.scale * s + (double)a.bias);
+  if (n > 0 && i < a.nrows) ((float*)a.out)[i] = (float)((double)a.scale * s + (double)a.bias);
 }
 
 // Dense BFS step, second half: next[R] = rows of block row R whose
@@ -1934,6 +1947,8 @@ static SpmvArgs base_args(const gbo_bsr* A, const PlanView& pv) {
   a.nbr = A->nblockrows;
   a.T = A->nblocks;
   a.plan = pv.plan;
+  a.start = pv.start;
+  a.tail = pv.tail;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

@@ -9,13 +9,18 @@
 namespace gbo {
 
 // Work decomposition of a bit-BSR: the tiles [0, nblocks) are cut into
-// chunks of `chunk` consecutive tiles; plan[c] is the first block row that
-// chunk c touches (a row that begins before the chunk is "split" and its
-// partial results are combined across chunks).
+// nchunks chunks of consecutive tiles, chunk c being [start[c], start[c+1]);
+// plan[c] is the first block row that chunk c touches (a row that begins
+// before the chunk is "split" and its partial results are combined across
+// chunks).  A chunk size given by the caller cuts evenly, chunk c starting at
+// tile c * chunk; the library's own plan (plan_create) makes chunks of about
+// equal work, at most `chunk` tiles.
 //
 // The scratch the operations need besides their inputs and outputs is kept
 // in the plan's allocation, after the nchunks plan entries, so that a call
 // on a planned matrix allocates nothing (each part 256-byte aligned):
+//   start       nchunks+1 x i64     first tile of each chunk
+//   tail        nchunks x i32       chunks after c that go on with a row begun in c
 //   slots       kCountSlots x u64   BFS frontier-size slots (zero between calls)
 //   count       1 x int64           the folded frontier size
 //   partial     nchunks*2*bs x f64  split-row partials of the FP32 sum
@@ -23,12 +28,14 @@ namespace gbo {
 // Calls on one matrix therefore share that scratch: they must be ordered
 // (one stream, or synchronised); separately created matrices do not share.
 struct PlanLayout {
-  size_t slots = 0, count = 0, partial = 0, bfs_counts = 0, bytes = 0;
+  size_t start = 0, tail = 0, slots = 0, count = 0, partial = 0, bfs_counts = 0, bytes = 0;
 };
 PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr, bool scratch);
 
 struct PlanView {
   const int32_t* plan = nullptr;
+  const int64_t* start = nullptr;  // null: even chunks of `chunk` tiles
+  const int32_t* tail = nullptr;
   int32_t chunk = 0;
   int32_t nchunks = 0;
   int32_t variant = 0;
@@ -39,11 +46,13 @@ struct PlanView {
   int32_t* bfs_counts = nullptr;  // the dense BFS step's row counts
 };
 
-int default_chunk(int bs);
+// Most tiles per chunk of the library's own plans.
+int default_chunk(int bs, int64_t tiles);
 int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st);
 int release_plan(PlanView* pv, hipStream_t st);
-// Allocates A->plan (chunk tiles per chunk, 0 = default); with `scratch` the
-// allocation also holds the scratch parts above.
+// Allocates A->plan (chunk tiles per chunk, 0 = the library's own plan); with
+// `scratch` the allocation also holds the scratch parts above.  The library's
+// own plan reads the tiles once and synchronizes the stream.
 int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, hipStream_t st);
 
 // A plan acquired for the length of one call, released on every return path.
@@ -117,6 +126,8 @@ struct SpmvArgs {
   int32_t nrows, ncols, nbr;
   int64_t T;
   const int32_t* plan;
+  const int64_t* start;  // first tile of each chunk, nchunks + 1 entries (null: even chunks of `chunk` tiles)
+  const int32_t* tail;   // chunks that go on with a row begun in chunk c (0: no row is cut there)
   int32_t chunk, nchunks;
   int32_t variant;      // bs 8/16 COUNT/BFS kernel variant
   const void* xbits;    // COUNT: x bits; BFS: frontier bits
@@ -135,6 +146,13 @@ struct SpmvArgs {
   int accumulate;       // COUNT: add into y
   float scale, bias;    // SUM: y = scale * (A x) + bias  (scale 1, bias 0 for the plain op)
 };
+
+// First tile of chunk c, for c up to nchunks.  The even form is kept apart
+// because it needs no load before the chunk's tiles can be asked for.
+template <class Args>
+__device__ __forceinline__ int64_t chunk_start(const Args& a, int64_t c) {
+  return a.start ? a.start[c] : min(c * a.chunk, a.T);
+}
 
 int spmv_launch(int bs, int op, const SpmvArgs& a, hipStream_t st);
 

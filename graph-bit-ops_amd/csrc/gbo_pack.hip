@@ -325,14 +325,16 @@ __global__ __launch_bounds__(256) void k_pack_vec(const float* __restrict__ x, w
   xb[j] = (word_t<BS>)w;
 }
 
-// First block row of every chunk of `chunk` tiles: the first row R with
-// rowptr[R] >= b, or the row containing tile b when that row starts before b.
+// First block row of every chunk: the first row R with rowptr[R] >= b, or the
+// row containing tile b when that row starts before b.  tail[c] = how many
+// chunks after c hold tiles of a row that begins in c and is cut by its end
+// (0: none is).
 __global__ __launch_bounds__(256) void k_plan(const int32_t* __restrict__ rowptr, int32_t nbr,
-                                              int32_t chunk, int32_t nchunks,
-                                              int32_t* __restrict__ plan) {
+                                              const int64_t* __restrict__ start, int32_t nchunks,
+                                              int32_t* __restrict__ plan, int32_t* __restrict__ tail) {
   const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= nchunks) return;
-  const int64_t b = (int64_t)c * chunk;
+  const int64_t b = start[c];
   int32_t lo = 0, hi = nbr;  // search in rowptr[0..nbr]
   while (lo < hi) {
     const int32_t mid = lo + (hi - lo) / 2;
@@ -344,17 +346,122 @@ __global__ __launch_bounds__(256) void k_plan(const int32_t* __restrict__ rowptr
   if (R >= nbr) R = nbr > 0 ? nbr - 1 : 0;
   if (R < 0) R = 0;
   plan[c] = R;
+  if (c == nchunks - 1) tail[c] = 0;
+  if (c == 0) return;
+  const int64_t rs = rowptr[R], re = rowptr[R + 1];
+  int32_t n = 0;
+  if (rs < b && rs >= start[c - 1]) {
+    int32_t l = c + 1, h = nchunks;  // first chunk that starts at or past the row's end
+    while (l < h) {
+      const int32_t mid = l + (h - l) / 2;
+      if (start[mid] < re) l = mid + 1;
+      else h = mid;
+    }
+    n = l - c;
+  }
+  tail[c - 1] = n;
 }
 
 __global__ __launch_bounds__(256) void k_fill_u64(unsigned long long* p, int n, unsigned long long v) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
 }
 
-// Tiles per wavefront chunk when the plan call gives none: 256 at every block
-// size.  At bs 64 (one tile per wave instruction, scalar per-tile reads) 256
-// beat 128 for the count (R-MAT s22 4.17-4.30 against 4.28-4.36 ms) and the
-// sum (4.78 against 5.12 ms).
-int default_chunk(int /*bs*/) { return 256; }
+// start[c] = c * chunk, start[nchunks] = T.
+__global__ __launch_bounds__(256) void k_even_starts(int64_t T, int32_t chunk, int32_t nchunks,
+                                                     int64_t* __restrict__ start) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c <= nchunks) start[c] = min(c * chunk, T);
+}
+
+// ---- the library's own plan: chunks of about equal work.  Tiles are taken
+// in units of kUnitTiles.  The work of a unit is kTileWork per tile and one per
+// set bit past kFreeBits per tile (the value products gather one word per set
+// bit, the first few of a tile with its own load; the count and the BFS step,
+// whose tiles all cost the same, lose little to shorter chunks where tiles are
+// dense, and the sparse rest keeps even chunks).  A unit starts a chunk where
+// the prefix sum of the work passes a multiple of chunk * kTileWork.  Cut evenly, a power-law matrix has chunks of ten to
+// fifty times the mean number of bits, and one wave on the densest one sets
+// the time of a sweep: R-MAT 2^18, 256 tiles a chunk, weighted min-plus bs 64
+// 1.52 ms, sum bs 32 0.50 ms, against 0.15 and 0.08 ms of streaming.
+template <int BS>
+constexpr int kUnitTiles = BS == 64 ? 8 : 16;
+template <int BS>
+constexpr int kTileWork = BS >= 32 ? 16 : 8;
+constexpr int kFreeBits = 4;
+
+// Work of every unit.  Lanes take 16 bytes each: a unit is 8 lanes at bs 8,
+// 32 at bs 16, a wave twice over at bs 32.  At bs 64 a wave reads a quarter of
+// each tile, another quarter from tile to tile, and counts it four times: the
+// bits are only a measure of work.
+template <int BS>
+__global__ __launch_bounds__(256) void k_unit_work(const uint4* __restrict__ tiles, int64_t T, int64_t nunits,
+                                                   int32_t* __restrict__ work) {
+  constexpr int UT = kUnitTiles<BS>, UL = BS == 8 ? 8 : BS == 16 ? 32 : 64;  // lanes per unit
+  const int lane = lane_id();
+  const int64_t u = (int64_t)wave_index() * (kWave / UL) + lane / UL;
+  const int l = lane % UL;
+  auto bits = [](uint4 v) { return __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w); };
+  int c = 0;
+  if constexpr (BS == 8) {
+    // lane l: tiles 2l, 2l + 1 of the unit; the last tile may be alone
+    const int64_t t = u * UT + 2 * l;
+    if (t + 1 < T) c = bits(tiles[t / 2]);
+    else if (t < T) c = __popcll(((const uint64_t*)tiles)[t]);
+  } else if constexpr (BS == 16) {
+    const int64_t t = u * UT + l / 2;
+    if (t < T) c = bits(tiles[t * 2 + l % 2]);
+  } else if constexpr (BS == 32) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t t = u * UT + h * 8 + l / 8;
+      if (t < T) c += bits(tiles[t * 8 + l % 8]);
+    }
+  } else {
+    const int64_t t = u * UT + l / 8;
+    if (t < T) c = 4 * bits(tiles[t * 32 + (t % 4) * 8 + l % 8]);
+  }
+  for (int off = 1; off < UL; off <<= 1) c += __shfl_xor(c, off);
+  if (l == 0 && u < nunits) work[u] = UT * kTileWork<BS> + max(c - UT * kFreeBits, 0);
+}
+
+__device__ __forceinline__ bool unit_starts(const int64_t* __restrict__ pre, int64_t u, int64_t target) {
+  return u == 0 || pre[u] / target != pre[u - 1] / target;
+}
+
+__global__ __launch_bounds__(256) void k_unit_heads(const int64_t* __restrict__ pre, int64_t nunits, int64_t target,
+                                                    int32_t* __restrict__ head) {
+  const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (u < nunits) head[u] = unit_starts(pre, u, target);
+}
+
+__global__ __launch_bounds__(256) void k_unit_chunks(const int64_t* __restrict__ pre,
+                                                     const int64_t* __restrict__ rank, int64_t nunits, int64_t target,
+                                                     int unit_tiles, int64_t T, int64_t* __restrict__ start) {
+  const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= nunits) return;
+  if (unit_starts(pre, u, target)) start[rank[u]] = u * unit_tiles;
+  if (u == 0) start[rank[nunits]] = T;
+}
+
+// Most tiles per chunk of the library's own plans: 256 on large matrices, and
+// less where that leaves a sweep short of waves (8192 are resident), down to
+// 16.  At bs 16 to 64 256 tiles make two to four rounds of waves and an
+// uneven last one up to some 12M tiles: R-MAT 2^18 bs 16 (4M) count 67 / 88 us
+// at 128 / 256 tiles, G(n, m) with 3.2M tiles 31 / 31 us, with 16.6M tiles bs
+// 32 sum 512 / 487 us.  At bs 8 a step of the count takes 256 tiles (G(n, m)
+// with 3.2M tiles 20 / 17 us).  Small ones: G(n, m) with 0.5M tiles bs 8 12.6 /
+// 8.3 / 8.1 us at 32 / 128 / 256; G(1024) bs 32 (1024 tiles) sum 9 / 18 / 59 us
+// at 16 / 64 / 256.
+int default_chunk(int bs, int64_t tiles) {
+  if (tiles >= (bs == 8 ? 2ll << 20 : 12ll << 20)) return 256;
+  const int64_t c = (tiles / 4096 + 8) / 16 * 16;
+  return (int)std::min<int64_t>(128, std::max<int64_t>(c, 16));
+}
+
+// Above this many tiles the densest chunk ends long before the sweep does,
+// and even chunks of 256 are best (R-MAT 2^22 bs 8: count 465 us against 472
+// with equal work, min 757 against 774).
+constexpr int64_t kEvenTiles = 32ll << 20;
 
 static bool bs_ok(int bs) { return bs == 8 || bs == 16 || bs == 32 || bs == 64; }
 
@@ -463,6 +570,10 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr, bool scratch) {
   PlanLayout L;
   size_t off = align256(sizeof(int32_t) * (size_t)nchunks);
+  L.start = off;
+  off += align256(sizeof(int64_t) * ((size_t)nchunks + 1));
+  L.tail = off;
+  off += align256(sizeof(int32_t) * (size_t)nchunks);
   if (scratch) {
     L.slots = off;
     off += align256(sizeof(unsigned long long) * kCountSlots);
@@ -478,21 +589,28 @@ PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr, bool scratch) {
 }
 
 // Points the view's scratch pointers into a plan allocation made with scratch.
-static void view_scratch(PlanView* pv, int bs, int32_t nbr) {
+static void view_scratch(PlanView* pv, int bs, int32_t nbr, bool even) {
   const PlanLayout L = plan_layout(bs, pv->nchunks, nbr, true);
   char* base = (char*)const_cast<int32_t*>(pv->plan);
+  if (!even) pv->start = (const int64_t*)(base + L.start);
+  pv->tail = (const int32_t*)(base + L.tail);
   pv->slots = (unsigned long long*)(base + L.slots);
   pv->count = (int64_t*)(base + L.count);
   pv->partial = (double*)(base + L.partial);
   pv->bfs_counts = (int32_t*)(base + L.bfs_counts);
 }
 
-// Plan entries plus (optionally) zeroed count slots in one allocation.
-static int plan_fill(const gbo_bsr* A, int32_t chunk, int64_t nch, bool scratch, int32_t* plan, hipStream_t st) {
-  k_plan<<<(unsigned)((nch + 255) / 256), 256, 0, st>>>(A->rowptr, A->nblockrows, chunk, (int32_t)nch, plan);
+// Plan entries (of the chunks whose starts are in place, or of even chunks of
+// `chunk` tiles) plus (optionally) zeroed count slots in one allocation.
+static int plan_fill(const gbo_bsr* A, int32_t chunk, bool even, int64_t nch, bool scratch, int32_t* plan,
+                     hipStream_t st) {
+  const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, scratch);
+  int64_t* start = (int64_t*)((char*)plan + L.start);
+  if (even) k_even_starts<<<(unsigned)((nch + 256) / 256), 256, 0, st>>>(A->nblocks, chunk, (int32_t)nch, start);
+  k_plan<<<(unsigned)((nch + 255) / 256), 256, 0, st>>>(A->rowptr, A->nblockrows, start, (int32_t)nch, plan,
+                                                       (int32_t*)((char*)plan + L.tail));
   GBO_LAUNCH_CHECK();
   if (scratch) {
-    const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, true);
     unsigned long long* slots = (unsigned long long*)((char*)plan + L.slots);
     k_fill_u64<<<kCountSlots / 256, 256, 0, st>>>(slots, kCountSlots, 0ull);
     GBO_LAUNCH_CHECK();
@@ -500,9 +618,43 @@ static int plan_fill(const gbo_bsr* A, int32_t chunk, int64_t nch, bool scratch,
   return GBO_OK;
 }
 
+// The chunks of about equal work: their number, and (owned by `mem`) the
+// prefix sums and ranks k_unit_chunks writes their starts from.
+struct WorkCut {
+  int64_t *pre = nullptr, *rank = nullptr;
+  int64_t nunits = 0, target = 0, nch = 0, total = 0;
+  int unit = 0;
+};
+
+template <int BS>
+static int work_cut(const gbo_bsr* A, int32_t chunk, AsyncAllocs& mem, WorkCut* w, hipStream_t st) {
+  constexpr int UT = kUnitTiles<BS>, G = BS == 8 ? 8 : BS == 16 ? 2 : 1;  // units per wave
+  w->unit = UT;
+  w->nunits = (A->nblocks + UT - 1) / UT;
+  w->target = (int64_t)chunk * kTileWork<BS>;
+  int32_t* work = nullptr;
+  int rc;
+  if ((rc = mem.alloc(&work, sizeof(int32_t) * (size_t)w->nunits, "gbo_bsr_plan")) ||
+      (rc = mem.alloc(&w->pre, sizeof(int64_t) * ((size_t)w->nunits + 1), "gbo_bsr_plan")) ||
+      (rc = mem.alloc(&w->rank, sizeof(int64_t) * ((size_t)w->nunits + 1), "gbo_bsr_plan")))
+    return rc;
+  const unsigned blocks = (unsigned)((w->nunits + 255) / 256);
+  k_unit_work<BS><<<(unsigned)((w->nunits + 4 * G - 1) / (4 * G)), 256, 0, st>>>((const uint4*)A->tiles, A->nblocks,
+                                                                                  w->nunits, work);
+  GBO_LAUNCH_CHECK();
+  if ((rc = scan_exclusive<int32_t, int64_t>(work, w->pre, w->nunits, st))) return rc;
+  k_unit_heads<<<blocks, 256, 0, st>>>(w->pre, w->nunits, w->target, work);
+  GBO_LAUNCH_CHECK();
+  if ((rc = scan_exclusive<int32_t, int64_t>(work, w->rank, w->nunits, st))) return rc;
+  GBO_HIP_CHECK(hipMemcpyAsync(&w->total, w->pre + w->nunits, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  GBO_HIP_CHECK(hipMemcpyAsync(&w->nch, w->rank + w->nunits, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  return GBO_OK;
+}
+
 // Plan for a matrix: uses A->plan (made by gbo_bsr_plan, with its scratch)
-// when present, else builds a temporary one with scratch (stream-ordered
-// allocation, released by release_plan).
+// when present, else builds a temporary one of even chunks with scratch
+// (stream-ordered allocation, released by release_plan).
 int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
   if (A->plan && A->plan_chunk > 0 && A->plan_nchunks > 0) {
     pv->plan = A->plan;
@@ -510,10 +662,10 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
     pv->nchunks = A->plan_nchunks;
     pv->variant = A->plan_variant;
     pv->owned = false;
-    view_scratch(pv, A->bs, A->nblockrows);
+    view_scratch(pv, A->bs, A->nblockrows, A->plan_even == 1);
     return GBO_OK;
   }
-  const int32_t chunk = default_chunk(A->bs);
+  const int32_t chunk = default_chunk(A->bs, A->nblocks);
   const int64_t nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "too many chunks");
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, true);
@@ -524,13 +676,30 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
   pv->nchunks = (int32_t)nch;
   pv->variant = A->plan_variant;
   pv->owned = true;
-  view_scratch(pv, A->bs, A->nblockrows);
-  return plan_fill(A, chunk, nch, true, plan, st);
+  view_scratch(pv, A->bs, A->nblockrows, true);
+  return plan_fill(A, chunk, true, nch, true, plan, st);
 }
 
 int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, hipStream_t st) {
-  const int32_t chunk = chunk_tiles > 0 ? chunk_tiles : default_chunk(A->bs);
-  const int64_t nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
+  const int32_t chunk = chunk_tiles > 0 ? chunk_tiles : default_chunk(A->bs, A->nblocks);
+  // equal work needs the tiles' bits in 16-byte reads; the kernels that gain
+  // from it need the same alignment
+  bool even = chunk_tiles > 0 || A->nblocks == 0 || A->nblocks >= kEvenTiles || !A->tiles || ((uintptr_t)A->tiles & 15);
+  int64_t nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
+  AsyncAllocs mem(st);
+  WorkCut w;
+  if (!even) {
+    int rc = GBO_OK;
+    switch (A->bs) {
+      case 8: rc = work_cut<8>(A, chunk, mem, &w, st); break;
+      case 16: rc = work_cut<16>(A, chunk, mem, &w, st); break;
+      case 32: rc = work_cut<32>(A, chunk, mem, &w, st); break;
+      case 64: rc = work_cut<64>(A, chunk, mem, &w, st); break;
+    }
+    if (rc) return rc;
+    even = w.total == w.nunits * w.target / chunk * w.unit;  // no unit has more than its tiles' work
+    if (!even) nch = w.nch;
+  }
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "gbo_bsr_plan: too many chunks");
   gbo_bsr_plan_free(A);
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, scratch);
@@ -538,7 +707,17 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, 
   A->plan_chunk = chunk;
   A->plan_nchunks = (int32_t)nch;
   A->plan_variant = variant;
-  const int rc = plan_fill(A, chunk, nch, scratch, A->plan, st);
+  A->plan_even = even ? 1 : 0;
+  if (!even) {
+    k_unit_chunks<<<(unsigned)((w.nunits + 255) / 256), 256, 0, st>>>(w.pre, w.rank, w.nunits, w.target, w.unit,
+                                                                      A->nblocks, (int64_t*)((char*)A->plan + L.start));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      gbo_bsr_plan_free(A);
+      return set_error(GBO_EDEVICE, "gbo_bsr_plan: %s", hipGetErrorString(e));
+    }
+  }
+  const int rc = plan_fill(A, chunk, even, nch, scratch, A->plan, st);
   if (rc) gbo_bsr_plan_free(A);
   return rc;
 }
@@ -752,6 +931,7 @@ void gbo_bsr_plan_free(gbo_bsr* A) {
   A->plan = nullptr;
   A->plan_chunk = 0;
   A->plan_nchunks = 0;
+  A->plan_even = 0;
 }
 
 void gbo_bsr_free(gbo_bsr* A) {

@@ -58,7 +58,7 @@ class BsrStruct(ctypes.Structure):
         ("nblockrows", c_int32), ("nblockcols", c_int32), ("nblocks", c_int64),
         ("rowptr", c_void_p), ("colind", c_void_p), ("tiles", c_void_p),
         ("plan", c_void_p), ("plan_chunk", c_int32), ("plan_nchunks", c_int32),
-        ("plan_variant", c_int32),
+        ("plan_variant", c_int32), ("plan_even", c_int32),
     ]
 
 

@@ -67,9 +67,10 @@ typedef struct gbo_bsr {
   int32_t* colind;
   void* tiles;
   int32_t* plan;        /* device, plan_nchunks entries (first block row of each chunk) */
-  int32_t plan_chunk;   /* tiles per chunk */
+  int32_t plan_chunk;   /* tiles per chunk (the most of any, where the library chose) */
   int32_t plan_nchunks;
   int32_t plan_variant; /* kernel variant for bs 8/16 (0 = default; see gbo_bsr_plan_ex) */
+  int32_t plan_even;    /* 1: every chunk holds plan_chunk tiles (the last one the rest) */
 } gbo_bsr;
 
 const char* gbo_last_error(void);
@@ -209,8 +210,10 @@ int gbo_bsr_create_dev(int bs, int dir, const int32_t* d_rowptr, const int32_t* 
 int gbo_bsr_create(int bs, int dir, const int32_t* h_rowptr, const int32_t* h_colind,
                    int32_t nrows, int32_t ncols, gbo_bsr* out, gbo_stream_t stream);
 void gbo_bsr_free(gbo_bsr* A);
-/* Work decomposition: split the tiles into chunks of `chunk_tiles` (0 = the
- * default, 256 tiles) and record each chunk's first block row.
+/* Work decomposition: split the tiles into chunks of `chunk_tiles` and record
+ * each chunk's first block row.  0 lets the library choose: chunks of about
+ * equal work, at most 256 tiles each and shorter on small matrices and where
+ * tiles are dense (reads the tiles once and synchronizes the stream).
  * Allocates A->plan (released by gbo_bsr_free / gbo_bsr_plan_free). */
 int gbo_bsr_plan(gbo_bsr* A, int32_t chunk_tiles, gbo_stream_t stream);
 /* As gbo_bsr_plan, also selecting the bs 8/16 kernel variant of the COUNT
