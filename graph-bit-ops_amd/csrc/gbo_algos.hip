@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "gbo_device.hpp"
@@ -112,6 +113,241 @@ __global__ __launch_bounds__(256) void k_push(const word_t<BS>* __restrict__ f, 
   }
 }
 
+// ---- runs of levels with small frontiers in one launch.  One workgroup
+// pushes level after level, its frontier (block, word, tile range) in LDS, for
+// as long as the frontier stays below the limits: a level of the kernels above
+// is ten launches and a host read (50 us, a mesh has hundreds of levels), one
+// of these is bound by five dependent memory trips: a frontier block's tiles
+// and columns, the visited words, the atomic that adds a next word, then that
+// word and its visited word.  King grid 512 x 512 bs 8, 505 levels: 26 -> 3 ms.
+constexpr int kRunThreads = 1024;
+constexpr int kRunBlocks = 4096;   // most frontier blocks (LDS)
+constexpr int kRunTiles = 12288;   // most tiles of a frontier (LDS; past it many workgroups are faster)
+constexpr int kRunHeavy = 256;     // rows of more tiles are taken by the whole workgroup
+constexpr int kRunLevels = 1024;   // most levels of a launch
+
+enum { RUN_END = 0, RUN_STOP = 1, RUN_OVER = 2 };
+
+// What a launch leaves.  RUN_END: the frontier emptied.  RUN_STOP: level
+// `lvl` is complete and its frontier is in f (and, up to kRunBlocks, in
+// `queue`).  RUN_OVER: nx holds the words of level lvl + 1, which is not
+// entered into visited, level and f.
+struct RunState {
+  int32_t status, levels, lvl, qn;
+  int64_t sizes[kRunLevels];  // vertices of levels lvl0 + 1, ...
+};
+
+template <int BS>
+__global__ __launch_bounds__(256) void k_run_collect(const word_t<BS>* __restrict__ f, int32_t nbr,
+                                                     int32_t* __restrict__ queue, RunState* __restrict__ st) {
+  const int64_t J = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (J < nbr && f[J] != 0) {
+    const int at = atomicAdd(&st->qn, 1);
+    if (at < kRunBlocks) queue[at] = (int32_t)J;
+  }
+}
+
+// What a frontier word selects in a tile: at bs 8 the bytes of its rows, so
+// that a tile is one 8-byte load and a few operations; else the word.
+template <int BS>
+__device__ __forceinline__ uint64_t row_mask(uint64_t fw) {
+  if constexpr (BS != 8) return fw;
+  uint64_t m = 0;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) m |= (fw >> (7 - r)) & 1ull ? 0xFFull << (8 * r) : 0ull;
+  return m;
+}
+
+// OR of the rows of tile t that `sel` (row_mask) selects.
+template <int BS>
+__device__ __forceinline__ uint64_t tile_or(const word_t<BS>* __restrict__ tiles, int64_t t, uint64_t sel) {
+  if constexpr (BS == 8) {
+    uint64_t w = 0;
+    if (((uintptr_t)tiles & 7) == 0) w = ((const uint64_t*)tiles)[t];
+    else __builtin_memcpy(&w, tiles + t * 8, 8);
+    w &= sel;
+    uint32_t x = (uint32_t)w | (uint32_t)(w >> 32);
+    x |= x >> 16;
+    return (x | (x >> 8)) & 0xFFu;
+  }
+  uint64_t nb = 0;
+  while (sel) {  // two rows' loads in flight
+    const int p = __builtin_ctzll(sel);
+    sel &= sel - 1;
+    const int q = sel ? __builtin_ctzll(sel) : p;
+    sel &= sel - 1;
+    nb |= (uint64_t)tiles[t * BS + (BS - 1 - p)] | (uint64_t)tiles[t * BS + (BS - 1 - q)];
+  }
+  return nb;
+}
+
+// The words of `nx` and `vis` change during the launch, by this workgroup
+// alone: they are read and OR-ed at workgroup scope, which stays in the L2 of
+// the workgroup's die (agent scope goes to the memory side: 12.2 us a level).
+template <class W>
+__device__ __forceinline__ W ld_shared_word(const W* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <int BS>
+__global__ __launch_bounds__(kRunThreads) void k_push_run(word_t<BS>* __restrict__ f, word_t<BS>* nx, word_t<BS>* vis,
+                                                          int32_t* __restrict__ level, const int32_t* __restrict__ rowptr,
+                                                          const int32_t* __restrict__ colind,
+                                                          const word_t<BS>* __restrict__ tiles, int32_t n, int32_t lvl,
+                                                          int64_t most_vertices, int32_t* __restrict__ queue,
+                                                          RunState* __restrict__ st) {
+  using W = word_t<BS>;
+  using Sel = typename std::conditional<BS == 8, uint64_t, W>::type;
+  constexpr int kHeavyMost = kRunTiles / kRunHeavy;
+  __shared__ int32_t qj[kRunBlocks], next[kRunBlocks];  // frontier blocks; next frontier's blocks
+  __shared__ W qw[kRunBlocks];                          // frontier words
+  __shared__ Sel qm[BS == 8 ? kRunBlocks : 1];          // bs 8: their row masks
+  __shared__ int32_t it_tile[kRunTiles];                // the frontier's tiles: tile, frontier entry
+  __shared__ uint16_t it_entry[kRunTiles];
+  __shared__ int32_t heavy[kHeavyMost][4];              // entry, first item, first tile, tiles
+  __shared__ int32_t s_next, s_tiles, s_heavy;
+  __shared__ unsigned long long s_new;
+  const int tid = threadIdx.x, lane = lane_id();
+  int qn = st->qn;  // at most kRunBlocks: the host sees to it
+  if (tid == 0) s_next = s_tiles = s_heavy = 0, s_new = 0;
+  __syncthreads();
+  // Enters frontier entry e (block J, word w; `in`: the lane has one) and
+  // lists its tiles.  Every lane of the wave takes part.
+  auto enter = [&](bool in, int e, int32_t J, W w) {
+    int32_t s = 0, d = 0;
+    if (in) {
+      s = rowptr[J];
+      d = rowptr[J + 1] - s;
+      qj[e] = J;
+      qw[e] = w;
+      if constexpr (BS == 8) qm[e] = row_mask<BS>(w);
+    }
+    const int dd = min(d, kRunTiles + 1);  // a wave's sum stays far below 2^31
+    const int incl = wave_incl_scan(dd);
+    int at = 0;
+    if (lane == kWave - 1) at = atomicAdd(&s_tiles, min(incl, kRunTiles + 1));
+    at = __builtin_amdgcn_readlane(at, kWave - 1) + incl - dd;
+    if (at + dd > kRunTiles) return;  // the run ends before this frontier
+    if (d <= kRunHeavy) {
+      for (int k = 0; k < d; ++k) {
+        it_tile[at + k] = s + k;
+        it_entry[at + k] = (uint16_t)e;
+      }
+    } else {
+      const int h = atomicAdd(&s_heavy, 1);  // below kHeavyMost: their tiles fit
+      heavy[h][0] = e, heavy[h][1] = at, heavy[h][2] = s, heavy[h][3] = d;
+    }
+  };
+  for (int e0 = 0; e0 < qn; e0 += kRunThreads) {
+    const int e = e0 + tid;
+    const bool in = e < qn;
+    const int32_t J = in ? queue[e] : 0;
+    const W w = in ? f[J] : (W)0;
+    if (in) f[J] = (W)0;
+    enter(in, e, J, w);
+  }
+  int status = RUN_STOP, done = 0;
+  int64_t fsize = 0;  // not known at entry: the host has checked it
+  while (true) {
+    __syncthreads();
+    const int ntiles = s_tiles, nheavy = s_heavy;
+    if (ntiles > kRunTiles || fsize > most_vertices || done == kRunLevels) break;
+    if (nheavy) {  // rows of many tiles: listed by all threads
+      for (int h = 0; h < nheavy; ++h)
+        for (int k = tid; k < heavy[h][3]; k += kRunThreads) {
+          it_tile[heavy[h][1] + k] = heavy[h][2] + k;
+          it_entry[heavy[h][1] + k] = (uint16_t)heavy[h][0];
+        }
+      __syncthreads();
+    }
+    // U tiles per thread at a time: their columns and words together, then
+    // the visited words, then the atomics
+    constexpr int U = 4;
+    for (int i0 = tid; i0 < ntiles; i0 += U * kRunThreads) {
+      int32_t J2[U];
+      uint64_t nb[U];
+      W v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = min(i0 + u * kRunThreads, ntiles - 1);
+        const int32_t t = it_tile[i];
+        const int e = it_entry[i];
+        J2[u] = colind[t];
+        uint64_t sel;
+        if constexpr (BS == 8) sel = qm[e];
+        else sel = qw[e];
+        nb[u] = tile_or<BS>(tiles, t, i0 + u * kRunThreads < ntiles ? sel : 0ull);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = ld_shared_word(&vis[J2[u]]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint64_t w = nb[u] & ~(uint64_t)v[u] & low_mask<BS>();
+        if (w && atomic_or_word<BS, __HIP_MEMORY_SCOPE_WORKGROUP>(nx, J2[u], w) == 0) {
+          const int at = atomicAdd(&s_next, 1);
+          if (at < kRunBlocks) next[at] = J2[u];
+        }
+      }
+    }
+    __syncthreads();
+    const int nn = s_next;
+    if (nn > kRunBlocks) {
+      status = RUN_OVER;
+      break;
+    }
+    if (nn == 0) {
+      status = RUN_END;
+      qn = 0;
+      break;
+    }
+    __syncthreads();
+    if (tid == 0) s_next = s_tiles = s_heavy = 0, s_new = 0;
+    __syncthreads();
+    unsigned long long added = 0;
+    for (int e0 = 0; e0 < nn; e0 += kRunThreads) {
+      const int e = e0 + tid;
+      const bool in = e < nn;
+      const int32_t J = next[in ? e : 0];
+      const W w = in ? ld_shared_word(&nx[J]) : (W)0;
+      const W v = in ? ld_shared_word(&vis[J]) : (W)0;
+      enter(in, e, J, w);
+      if (!in) continue;
+      nx[J] = (W)0;
+      vis[J] = (W)(v | w);
+      added += popcw(w);
+      uint64_t m = (uint64_t)w;
+      while (m) {
+        const int p = __builtin_ctzll(m);
+        m &= m - 1;
+        const int64_t i = (int64_t)J * BS + (BS - 1 - p);
+        if (i < n) level[i] = lvl + 1;
+      }
+    }
+    // one LDS add per wave: 1024 threads adding to one word take turns
+    for (int off = 1; off < kWave; off <<= 1) added += __shfl_xor(added, off);
+    if (lane == 0 && added) atomicAdd(&s_new, added);
+    __syncthreads();
+    fsize = (int64_t)s_new;
+    if (tid == 0) st->sizes[done] = fsize;
+    qn = nn;
+    ++lvl;
+    ++done;
+  }
+  // the frontier goes back to memory (RUN_OVER: its next one is in nx)
+  if (status == RUN_STOP) {
+    for (int e = tid; e < qn; e += kRunThreads) {
+      f[qj[e]] = qw[e];
+      queue[e] = qj[e];
+    }
+  }
+  if (tid == 0) {
+    st->status = status;
+    st->levels = done;
+    st->lvl = lvl;
+    st->qn = qn;
+  }
+}
+
 // Set bits of the next-frontier words, summed per wave into the count slots
 // (folded by count_fold): one counter for every wave took 85 us on a pushed
 // level of 163K vertices (R-MAT s22), 8K waves queueing on one address.
@@ -156,8 +392,12 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
   }
   W* nx = f + std::max(nbr, 1);
   W* vis = nx + std::max(nbr, 1);
-  int32_t* segoff = nullptr;
-  if (Aout && (rc = mem.alloc(&segoff, sizeof(int32_t) * ((size_t)nbr + 1), "gbo_bfs_do"))) return rc;
+  int32_t *segoff = nullptr, *queue = nullptr;
+  RunState* run = nullptr;
+  if (Aout && ((rc = mem.alloc(&segoff, sizeof(int32_t) * ((size_t)nbr + 1), "gbo_bfs_do")) ||
+               (rc = mem.alloc(&queue, sizeof(int32_t) * kRunBlocks, "gbo_bfs_do")) ||
+               (rc = mem.alloc(&run, sizeof(RunState), "gbo_bfs_do"))))
+    return rc;
   PlanGuard g(st);
   if ((rc = acquire_plan(A, &g.pv, st))) return rc;
   PlanView pv = g.pv;
@@ -194,9 +434,37 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
   int32_t lvl = 0;
   int64_t fsize = 1;  // vertices in the current frontier
   if (sizes && max_levels > 0) sizes[0] = 1;
+  bool over = false;  // a run of levels left the next one in nx
   while (true) {
-    // both step forms end with count_fold, which writes d_cnt
-    if (Aout && fsize <= std::max<int64_t>(n / 64, 1)) {
+    if (Aout && fsize <= std::min<int64_t>(std::max<int64_t>(n / 64, 1), kRunBlocks)) {
+      // a run of small levels in one launch
+      GBO_HIP_CHECK(hipMemsetAsync(nx, 0, sizeof(W) * (size_t)std::max(nbr, 1), st));
+      GBO_HIP_CHECK(hipMemsetAsync(run, 0, offsetof(RunState, sizes), st));
+      k_run_collect<BS><<<(unsigned)((nbr + 255) / 256), 256, 0, st>>>(f, nbr, queue, run);
+      RunState h;
+      do {
+        k_push_run<BS><<<1, kRunThreads, 0, st>>>(f, nx, vis, d_level, Aout->rowptr, Aout->colind,
+                                                  (const W*)Aout->tiles, n, lvl, std::max<int64_t>(n / 64, 1), queue, run);
+        GBO_LAUNCH_CHECK();
+        GBO_HIP_CHECK(hipMemcpyAsync(&h, run, sizeof(h), hipMemcpyDeviceToHost, st));
+        GBO_HIP_CHECK(hipStreamSynchronize(st));
+        for (int k = 0; k < h.levels; ++k) {
+          ++lvl;
+          fsize = h.sizes[k];
+          visited += fsize;
+          if (sizes && lvl < max_levels) sizes[lvl] = fsize;
+        }
+      } while (h.status == RUN_STOP && h.levels == kRunLevels);
+      if (h.status == RUN_END) break;
+      over = h.status == RUN_OVER;
+    }
+    // every step form ends with count_fold, which writes d_cnt
+    if (over) {
+      over = false;
+      k_popc_words<BS><<<(unsigned)((nbr + 255) / 256), 256, 0, st>>>(nx, nbr, pv.slots);
+      GBO_LAUNCH_CHECK();
+      if ((rc = count_fold(pv.slots, d_cnt, st))) return rc;
+    } else if (Aout && fsize <= std::max<int64_t>(n / 64, 1)) {
       // push: only the frontier rows' tiles of A are read
       GBO_HIP_CHECK(hipMemsetAsync(nx, 0, sizeof(W) * (size_t)std::max(nbr, 1), st));
       k_push_segs<BS><<<(unsigned)(((int64_t)nbr + 1 + 255) / 256), 256, 0, st>>>(f, Aout->rowptr, nbr, segoff);

@@ -108,17 +108,15 @@ __device__ __forceinline__ uint64_t low_mask() {
 // Atomic OR of a BS-bit word into a word array (bytes and shorts go through
 // the aligned 32-bit word that contains them; little-endian).  Returns the
 // previous value of the BS-bit word.
-template <int BS>
+template <int BS, int SCOPE = __HIP_MEMORY_SCOPE_AGENT>
 __device__ __forceinline__ uint64_t atomic_or_word(word_t<BS>* base, int64_t idx, uint64_t v) {
-  if constexpr (BS == 64) {
-    return atomicOr((unsigned long long*)(base + idx), (unsigned long long)v);
-  } else if constexpr (BS == 32) {
-    return atomicOr((unsigned int*)(base + idx), (unsigned int)v);
+  if constexpr (BS >= 32) {
+    return __hip_atomic_fetch_or(base + idx, (word_t<BS>)v, __ATOMIC_RELAXED, SCOPE);
   } else {
     const uintptr_t addr = (uintptr_t)(base + idx);
     unsigned int* w32 = (unsigned int*)(addr & ~(uintptr_t)3);
     const int shift = (int)(addr & 3) * 8;
-    const unsigned int old = atomicOr(w32, (unsigned int)(v << shift));
+    const unsigned int old = __hip_atomic_fetch_or(w32, (unsigned int)(v << shift), __ATOMIC_RELAXED, SCOPE);
     return (old >> shift) & (unsigned int)low_mask<BS>();
   }
 }
