@@ -382,7 +382,7 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
                  int32_t max_levels, int32_t* nlevels, hipStream_t st, const BfsScratch* ext = nullptr) {
   using W = word_t<BS>;
   const int32_t nbr = A->nblockrows, n = A->nrows;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   W* f = nullptr;
   int rc;
   if (ext) {
@@ -446,8 +446,7 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
         k_push_run<BS><<<1, kRunThreads, 0, st>>>(f, nx, vis, d_level, Aout->rowptr, Aout->colind,
                                                   (const W*)Aout->tiles, n, lvl, std::max<int64_t>(n / 64, 1), queue, run);
         GBO_LAUNCH_CHECK();
-        GBO_HIP_CHECK(hipMemcpyAsync(&h, run, sizeof(h), hipMemcpyDeviceToHost, st));
-        GBO_HIP_CHECK(hipStreamSynchronize(st));
+        if ((rc = read_back(&h, run, sizeof(h), st))) return rc;
         for (int k = 0; k < h.levels; ++k) {
           ++lvl;
           fsize = h.sizes[k];
@@ -469,7 +468,7 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
       GBO_HIP_CHECK(hipMemsetAsync(nx, 0, sizeof(W) * (size_t)std::max(nbr, 1), st));
       k_push_segs<BS><<<(unsigned)(((int64_t)nbr + 1 + 255) / 256), 256, 0, st>>>(f, Aout->rowptr, nbr, segoff);
       GBO_LAUNCH_CHECK();
-      if ((rc = scan_exclusive<int32_t, int32_t>(segoff, segoff, (int64_t)nbr + 1, st))) return rc;
+      if ((rc = scan_exclusive<int32_t, int32_t>(segoff, segoff, (int64_t)nbr + 1, st, mem))) return rc;
       k_push<BS><<<2048, 256, 0, st>>>(f, vis, nx, Aout->rowptr, Aout->colind, (const W*)Aout->tiles, segoff, nbr);
       GBO_LAUNCH_CHECK();
       k_popc_words<BS><<<(unsigned)((nbr + 255) / 256), 256, 0, st>>>(nx, nbr, pv.slots);
@@ -493,8 +492,7 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
     k_bfs_update<BS><<<(unsigned)((nbr + 255) / 256), 256, 0, st>>>(nx, vis, d_level, nbr, n, lvl + 1);
     GBO_LAUNCH_CHECK();
     int64_t cnt = 0;
-    GBO_HIP_CHECK(hipMemcpyAsync(&cnt, d_cnt, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    GBO_HIP_CHECK(hipStreamSynchronize(st));
+    if ((rc = read_back(&cnt, d_cnt, sizeof(int64_t), st))) return rc;
     if (cnt == 0) break;
     ++lvl;
     fsize = cnt;
@@ -657,9 +655,7 @@ __global__ void k_iota(int32_t* a, int32_t* b, int32_t n) {
 }
 
 static int read_u64(unsigned long long* d, uint64_t* h, hipStream_t st) {
-  GBO_HIP_CHECK(hipMemcpyAsync(h, d, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
-  return GBO_OK;
+  return read_back(h, d, sizeof(uint64_t), st);
 }
 
 static int check_square(const gbo_bsr* A, const char* who) {
@@ -800,7 +796,7 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   hipStream_t st = stream;
   const int bs = AT->bs;
   const int64_t nact = ((int64_t)AT->nblockcols + 63) / 64;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   uint32_t* fr = nullptr;
   unsigned long long* active = nullptr;
   if ((rc = mem.alloc(&fr, sizeof(uint32_t) * (size_t)std::max(n, 1) * 2, "gbo_sssp"))) return rc;
@@ -864,7 +860,7 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   if (n == 0) return GBO_OK;
   hipStream_t st = stream;
   const int nparts = 1024;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   float* x = nullptr;
   double* dpart = nullptr;
   if ((rc = mem.alloc(&x, sizeof(float) * (size_t)n * 2, "gbo_pagerank"))) return rc;
@@ -906,8 +902,7 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
     k_pr_tail<<<lblocks, 256, 0, st>>>(q, p, d_outdeg, alpha, x, n, dpart);  // x for the next iteration
     k_sum_partials<<<1, 256, 0, st>>>(dpart, (int)lblocks, dpart + nparts);
     GBO_LAUNCH_CHECK();
-    GBO_HIP_CHECK(hipMemcpyAsync(&delta, dpart + nparts, sizeof(double), hipMemcpyDeviceToHost, st));
-    GBO_HIP_CHECK(hipStreamSynchronize(st));
+    if ((rc = read_back(&delta, dpart + nparts, sizeof(double), st))) return rc;
     ++it;
     std::swap(p, q);
     if (delta < tol) break;
@@ -930,7 +925,7 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   if (!d_label) return set_error(GBO_EINVAL, "gbo_cc: null label");
   if (n == 0) return GBO_OK;
   hipStream_t st = stream;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   int32_t* gf = nullptr;
   unsigned long long* changed = nullptr;
   if ((rc = mem.alloc(&gf, sizeof(int32_t) * (size_t)n * 2, "gbo_cc"))) return rc;

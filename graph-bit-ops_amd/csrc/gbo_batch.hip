@@ -314,7 +314,7 @@ static int msbfs_t(const gbo_bsr* A, const int32_t* h_src, int32_t nsrc, int32_t
   const int32_t n = A->nrows;
   const int64_t words = (int64_t)std::max(n, 1) * KW;
   const int64_t nact = ((int64_t)A->nblockcols + 63) / 64 + 1;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   uint64_t* buf = nullptr;
   int32_t* d_src = nullptr;
   int rc = mem.alloc(&buf, sizeof(uint64_t) * (3 * words + 2 * nact + 1), "gbo_bfs_multisource");
@@ -364,8 +364,7 @@ static int msbfs_t(const gbo_bsr* A, const int32_t* h_src, int32_t nsrc, int32_t
     k_ms_update<KW><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(Fn, V, d_level, n, nsrc, A->bs, lvl, act2, cnt);
     GBO_LAUNCH_CHECK();
     unsigned long long h = 0;
-    GBO_HIP_CHECK(hipMemcpyAsync(&h, cnt, sizeof(h), hipMemcpyDeviceToHost, st));
-    GBO_HIP_CHECK(hipStreamSynchronize(st));
+    if ((rc = read_back(&h, cnt, sizeof(h), st))) return rc;
     if (h == 0) {
       --lvl;
       break;

@@ -546,7 +546,7 @@ using namespace gbo;
 // radix sort of the tile indices by block column.  The tiles are stored in
 // block-row order, so every column's list comes out with ascending rows.
 // The three outputs are owned by `mem` (the caller's allocations).
-static int block_transpose(const gbo_bsr* B, AsyncAllocs& mem, int32_t** d_ptr, int32_t** d_row, int32_t** d_tile,
+static int block_transpose(const gbo_bsr* B, Workspace& mem, int32_t** d_ptr, int32_t** d_row, int32_t** d_tile,
                            hipStream_t st) {
   const int32_t nbr = B->nblockrows, nbc = B->nblockcols;
   const int64_t T = B->nblocks;
@@ -555,17 +555,16 @@ static int block_transpose(const gbo_bsr* B, AsyncAllocs& mem, int32_t** d_ptr, 
   if ((rc = mem.alloc(d_ptr, sizeof(int32_t) * ((size_t)nbc + 1), "block_transpose")) ||
       (rc = mem.alloc(d_row, tb, "block_transpose")) || (rc = mem.alloc(d_tile, tb, "block_transpose")))
     return rc;
-  AsyncAllocs tmpmem(st);
   int32_t *keys = nullptr, *idx = nullptr;
   void* tmp = nullptr;
   size_t tmp_bytes = 0;
   unsigned bits = 1;
   while (bits < 31 && (1ll << bits) <= nbc) ++bits;
-  if ((rc = tmpmem.alloc(&keys, tb, "block_transpose")) || (rc = tmpmem.alloc(&idx, tb, "block_transpose"))) return rc;
+  if ((rc = mem.alloc(&keys, tb, "block_transpose")) || (rc = mem.alloc(&idx, tb, "block_transpose"))) return rc;
   k_iota_i32<<<(unsigned)((T + 255) / 256), 256, 0, st>>>(idx, T);
   GBO_LAUNCH_CHECK();
   GBO_HIP_CHECK(rocprim::radix_sort_pairs(nullptr, tmp_bytes, B->colind, keys, idx, *d_tile, (size_t)T, 0, bits, st));
-  if ((rc = tmpmem.alloc(&tmp, std::max<size_t>(tmp_bytes, 1), "block_transpose"))) return rc;
+  if ((rc = mem.alloc(&tmp, std::max<size_t>(tmp_bytes, 1), "block_transpose"))) return rc;
   GBO_HIP_CHECK(rocprim::radix_sort_pairs(tmp, tmp_bytes, B->colind, keys, idx, *d_tile, (size_t)T, 0, bits, st));
   k_col_bounds<<<(unsigned)(((int64_t)nbc + 1 + 255) / 256), 256, 0, st>>>(keys, T, nbc, *d_ptr);
   GBO_LAUNCH_CHECK();
@@ -590,7 +589,7 @@ int gbo_bsrbmm_tc(const gbo_bsr* L, const gbo_bsr* LT, uint64_t* d_count, gbo_st
   hipStream_t st = stream;
   GBO_HIP_CHECK(hipMemsetAsync(d_count, 0, sizeof(uint64_t), st));
   if (L->nblocks == 0 || LT->nblocks == 0) return GBO_OK;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   int32_t *bt_ptr = nullptr, *bt_row = nullptr, *bt_tile = nullptr;
   if ((rc = block_transpose(LT, mem, &bt_ptr, &bt_row, &bt_tile, st))) return rc;
   // B's tiles in row form (same positions), for one popcount per set bit of A
@@ -643,7 +642,7 @@ int gbo_bsrbmm_tc(const gbo_bsr* L, const gbo_bsr* LT, uint64_t* d_count, gbo_st
     if (L->bs == 32) k_tile_bitcount<32><<<gb, 256, 0, st>>>((const uint32_t*)L->tiles, T, aoff);
     else k_tile_bitcount<64><<<gb, 256, 0, st>>>((const uint64_t*)L->tiles, T, aoff);
     GBO_LAUNCH_CHECK();
-    if ((rc = scan_exclusive<int32_t, int32_t>(aoff, aoff, T, st))) return rc;
+    if ((rc = scan_exclusive<int32_t, int32_t>(aoff, aoff, T, st, mem))) return rc;
     pending.armed = true;
     GBO_HIP_CHECK(hipMemcpyAsync(&nbits, aoff + T, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   }

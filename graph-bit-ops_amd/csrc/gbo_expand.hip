@@ -136,24 +136,23 @@ unsigned grid_of(int64_t items, int per_block) {
 }
 
 template <int BS>
-int expand_t(const gbo_bsr* A, AsyncAllocs& mem, CsrList* out, hipStream_t st) {
+int expand_t(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
   const int32_t nbr = A->nblockrows, n = A->nrows;
   const int64_t cap = (int64_t)nbr + A->nblocks / kItem<BS> + 1;  // items
-  AsyncAllocs tmp(st);
   int32_t *icnt = nullptr, *itemrow = nullptr, *cnt = nullptr;
   int64_t *itemptr = nullptr, *pos = nullptr, *rowptr = nullptr;
   const char* who = "expand";
   int rc;
-  if ((rc = tmp.alloc(&icnt, sizeof(int32_t) * (size_t)std::max(nbr, 1), who)) ||
-      (rc = tmp.alloc(&itemptr, sizeof(int64_t) * ((size_t)nbr + 1), who)) ||
-      (rc = tmp.alloc(&itemrow, sizeof(int32_t) * (size_t)cap, who)) ||
-      (rc = tmp.alloc(&cnt, sizeof(int32_t) * (size_t)cap * BS, who)) ||
-      (rc = tmp.alloc(&pos, sizeof(int64_t) * ((size_t)cap * BS + 1), who)) ||
+  if ((rc = mem.alloc(&icnt, sizeof(int32_t) * (size_t)std::max(nbr, 1), who)) ||
+      (rc = mem.alloc(&itemptr, sizeof(int64_t) * ((size_t)nbr + 1), who)) ||
+      (rc = mem.alloc(&itemrow, sizeof(int32_t) * (size_t)cap, who)) ||
+      (rc = mem.alloc(&cnt, sizeof(int32_t) * (size_t)cap * BS, who)) ||
+      (rc = mem.alloc(&pos, sizeof(int64_t) * ((size_t)cap * BS + 1), who)) ||
       (rc = mem.alloc(&rowptr, sizeof(int64_t) * ((size_t)n + 1), who)))
     return rc;
   k_item_count<<<grid_of(nbr, 256), 256, 0, st>>>(A->rowptr, nbr, kItem<BS>, icnt);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_exclusive<int32_t, int64_t>(icnt, itemptr, nbr, st))) return rc;
+  if ((rc = scan_exclusive<int32_t, int64_t>(icnt, itemptr, nbr, st, mem))) return rc;
   k_item_rows<<<grid_of(nbr, 256), 256, 0, st>>>(itemptr, nbr, itemrow);
   ItemArgs a{};
   a.rowptr = A->rowptr;
@@ -168,12 +167,11 @@ int expand_t(const gbo_bsr* A, AsyncAllocs& mem, CsrList* out, hipStream_t st) {
   GBO_LAUNCH_CHECK();
   // counts past the last item are never written; what they hold only moves
   // positions past the total, which nothing reads
-  if ((rc = scan_exclusive<int32_t, int64_t>(cnt, pos, cap * BS, st))) return rc;
+  if ((rc = scan_exclusive<int32_t, int64_t>(cnt, pos, cap * BS, st, mem))) return rc;
   k_item_rowptr<BS><<<grid_of((int64_t)n + 1, 256), 256, 0, st>>>(a, n, rowptr);
   GBO_LAUNCH_CHECK();
   int64_t nnz = 0;
-  GBO_HIP_CHECK(hipMemcpyAsync(&nnz, rowptr + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_back(&nnz, rowptr + n, sizeof(int64_t), st))) return rc;
   int32_t* col = nullptr;
   if ((rc = mem.alloc(&col, sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1), who))) return rc;
   a.col = col;
@@ -187,7 +185,7 @@ int expand_t(const gbo_bsr* A, AsyncAllocs& mem, CsrList* out, hipStream_t st) {
 
 }  // namespace
 
-int expand_csr(const gbo_bsr* A, AsyncAllocs& mem, CsrList* out, hipStream_t st) {
+int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
   switch (A->bs) {
     case 8: return expand_t<8>(A, mem, out, st);
     case 16: return expand_t<16>(A, mem, out, st);

@@ -65,8 +65,43 @@ struct PlanGuard {
   PlanGuard& operator=(const PlanGuard&) = delete;
 };
 
-// Stream-ordered device allocations of one call, released with hipFreeAsync
-// on every return path (success or error).
+// Device scratch of one call that waits for its stream before it returns:
+// blocks kept between calls (gbo_workspace.hip), given back on every return
+// path once the stream has been waited for.
+class Workspace {
+ public:
+  explicit Workspace(hipStream_t st) : st_(st) {}
+  ~Workspace();
+  Workspace(const Workspace&) = delete;
+  Workspace& operator=(const Workspace&) = delete;
+  template <class T>
+  int alloc(T** p, size_t bytes, const char* who) {
+    void* q = nullptr;
+    const int rc = take(&q, bytes, who);
+    *p = (T*)q;
+    return rc;
+  }
+
+ private:
+  int take(void** p, size_t bytes, const char* who);
+  static constexpr int kMax = 64;
+  hipStream_t st_;
+  int dev_ = -1;
+  void* ptrs_[kMax];
+  size_t bytes_[kMax];
+  int n_ = 0;
+};
+// hipMalloc that gives the kept blocks back before it reports that memory is
+// out; gives all kept blocks of a device (-1: of each) back; counts the
+// matrices and plans the library has allocated.
+hipError_t device_malloc(void** p, size_t bytes);
+void workspace_release(int dev);
+void workspace_live(int delta);
+// Copies a few bytes to the host and waits for the stream.
+int read_back(void* h, const void* d, size_t bytes, hipStream_t st);
+
+// Stream-ordered device allocations of a call that does not wait for its
+// stream, released with hipFreeAsync on every return path (success or error).
 class AsyncAllocs {
  public:
   explicit AsyncAllocs(hipStream_t st) : st_(st) {}
@@ -103,10 +138,13 @@ struct CsrList {
   const int32_t* col = nullptr;     // [nnz]
   int64_t nnz = 0;
 };
-int expand_csr(const gbo_bsr* A, AsyncAllocs& mem, CsrList* out, hipStream_t st);
+int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st);
 
 template <class TI, class TO>
 int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st);
+// The same with its block sums in a Workspace.
+template <class TI, class TO>
+int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st, Workspace& mem);
 
 constexpr uint32_t kInfU32 = 0xFFFFFFFFu;
 constexpr int kCountSlots = 1024;

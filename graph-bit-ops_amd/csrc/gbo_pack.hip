@@ -78,9 +78,10 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(const TI* in, int64
   }
 }
 
-// out[0..n] = exclusive prefix sums of in[0..n-1]; out[n] = total.
-template <class TI, class TO>
-int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st) {
+// The block sums' offsets of a scan of nb tiles (room for 2 nb + 1 int64 in
+// bsum), then the scan itself; nested through itself where nb needs it.
+template <class TI, class TO, class Alloc>
+static int scan_with(const TI* in, TO* out, int64_t n, hipStream_t st, Alloc alloc) {
   if (n <= 0) {
     GBO_HIP_CHECK(hipMemsetAsync(out, 0, sizeof(TO), st));
     return GBO_OK;
@@ -92,22 +93,35 @@ int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st) {
     return GBO_OK;
   }
   int64_t* bsum = nullptr;
-  GBO_HIP_CHECK(hipMallocAsync((void**)&bsum, sizeof(int64_t) * (2 * nb + 1), st));
+  int rc = alloc(&bsum, sizeof(int64_t) * (2 * nb + 1));
+  if (rc) return rc;
   int64_t* boff = bsum + nb;
   k_scan_reduce<TI><<<(unsigned)nb, kScanThreads, 0, st>>>(in, n, bsum);
   GBO_LAUNCH_CHECK();
-  int rc = scan_exclusive<int64_t, int64_t>(bsum, boff, nb, st);
-  if (rc == GBO_OK) {
-    k_scan_apply<TI, TO><<<(unsigned)nb, kScanThreads, 0, st>>>(in, n, boff, out);
-    GBO_LAUNCH_CHECK();
-  }
-  GBO_HIP_CHECK(hipFreeAsync(bsum, st));
-  return rc;
+  if ((rc = scan_with<int64_t, int64_t>(bsum, boff, nb, st, alloc))) return rc;
+  k_scan_apply<TI, TO><<<(unsigned)nb, kScanThreads, 0, st>>>(in, n, boff, out);
+  GBO_LAUNCH_CHECK();
+  return GBO_OK;
+}
+
+// out[0..n] = exclusive prefix sums of in[0..n-1]; out[n] = total.
+template <class TI, class TO>
+int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st) {
+  AsyncAllocs mem(st);
+  return scan_with(in, out, n, st, [&](int64_t** p, size_t bytes) { return mem.alloc(p, bytes, "scan"); });
+}
+
+template <class TI, class TO>
+int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st, Workspace& mem) {
+  return scan_with(in, out, n, st, [&](int64_t** p, size_t bytes) { return mem.alloc(p, bytes, "scan"); });
 }
 
 template int scan_exclusive<int32_t, int32_t>(const int32_t*, int32_t*, int64_t, hipStream_t);
+template int scan_exclusive<int32_t, int32_t>(const int32_t*, int32_t*, int64_t, hipStream_t, Workspace&);
 template int scan_exclusive<int32_t, int64_t>(const int32_t*, int64_t*, int64_t, hipStream_t);
+template int scan_exclusive<int32_t, int64_t>(const int32_t*, int64_t*, int64_t, hipStream_t, Workspace&);
 template int scan_exclusive<int64_t, int64_t>(const int64_t*, int64_t*, int64_t, hipStream_t);
+template int scan_exclusive<int64_t, int64_t>(const int64_t*, int64_t*, int64_t, hipStream_t, Workspace&);
 
 // ---------------------------------------------------------------- packing
 enum { PACK_COUNT = 0, PACK_ROW = 1, PACK_COL = 2, PACK_VALUES = 3 };
@@ -496,8 +510,8 @@ static int dispatch_pack(int bs, const int32_t* rp, const int32_t* ci, int32_t n
 
 static int check_err_flag(int* d_err, hipStream_t st, const char* who) {
   int h = 0;
-  GBO_HIP_CHECK(hipMemcpyAsync(&h, d_err, sizeof(int), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  const int rc = read_back(&h, d_err, sizeof(int), st);
+  if (rc) return rc;
   if (h & PACKERR_COLRANGE) return set_error(GBO_EINVAL, "%s: column index out of range", who);
   if (h & PACKERR_UNSORTED) return set_error(GBO_EINVAL, "%s: CSR rows must be sorted ascending", who);
   return GBO_OK;
@@ -515,7 +529,7 @@ struct PieceSet {
 };
 
 static int make_pieces(int bs, const int32_t* d_rp, const int32_t* d_ci, int32_t nrows, int32_t ncols, int32_t nbr,
-                       AsyncAllocs& mem, PieceSet* ps, const char* who, hipStream_t st) {
+                       Workspace& mem, PieceSet* ps, const char* who, hipStream_t st) {
   int rc;
   int32_t *poff = nullptr, *prow = nullptr, *plo = nullptr, *phi = nullptr, *pcnt = nullptr;
   int64_t* toff = nullptr;
@@ -527,10 +541,9 @@ static int make_pieces(int bs, const int32_t* d_rp, const int32_t* d_ci, int32_t
     k_piece_n<<<(unsigned)(((int64_t)nbr + 255) / 256), 256, 0, st>>>(d_rp, nrows, nbr, bs, poff);
     GBO_LAUNCH_CHECK();
   }
-  if ((rc = scan_exclusive<int32_t, int32_t>(poff, poff, nbr, st))) return rc;
+  if ((rc = scan_exclusive<int32_t, int32_t>(poff, poff, nbr, st, mem))) return rc;
   int32_t np = 0;
-  GBO_HIP_CHECK(hipMemcpyAsync(&np, poff + nbr, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_back(&np, poff + nbr, sizeof(int32_t), st))) return rc;
   if ((rc = mem.alloc(&prow, sizeof(int32_t) * std::max<int64_t>(np, 1), who)) ||
       (rc = mem.alloc(&plo, sizeof(int32_t) * std::max<int64_t>(np, 1), who)) ||
       (rc = mem.alloc(&phi, sizeof(int32_t) * std::max<int64_t>(np, 1), who)) ||
@@ -552,9 +565,8 @@ static int make_pieces(int bs, const int32_t* d_rp, const int32_t* d_ci, int32_t
                                       nullptr, nullptr, d_err, pc, st)))
     return rc;
   if ((rc = check_err_flag(d_err, st, who))) return rc;
-  if ((rc = scan_exclusive<int32_t, int64_t>(pcnt, toff, np, st))) return rc;
-  GBO_HIP_CHECK(hipMemcpyAsync(&ps->total, toff + np, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = scan_exclusive<int32_t, int64_t>(pcnt, toff, np, st, mem))) return rc;
+  if ((rc = read_back(&ps->total, toff + np, sizeof(int64_t), st))) return rc;
   if (ps->total >= ((int64_t)1 << 31))
     return set_error(GBO_ERANGE, "tile count %lld exceeds int32", (long long)ps->total);
   pc.cnt = nullptr;
@@ -627,7 +639,7 @@ struct WorkCut {
 };
 
 template <int BS>
-static int work_cut(const gbo_bsr* A, int32_t chunk, AsyncAllocs& mem, WorkCut* w, hipStream_t st) {
+static int work_cut(const gbo_bsr* A, int32_t chunk, Workspace& mem, WorkCut* w, hipStream_t st) {
   constexpr int UT = kUnitTiles<BS>, G = BS == 8 ? 8 : BS == 16 ? 2 : 1;  // units per wave
   w->unit = UT;
   w->nunits = (A->nblocks + UT - 1) / UT;
@@ -642,14 +654,12 @@ static int work_cut(const gbo_bsr* A, int32_t chunk, AsyncAllocs& mem, WorkCut* 
   k_unit_work<BS><<<(unsigned)((w->nunits + 4 * G - 1) / (4 * G)), 256, 0, st>>>((const uint4*)A->tiles, A->nblocks,
                                                                                   w->nunits, work);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_exclusive<int32_t, int64_t>(work, w->pre, w->nunits, st))) return rc;
+  if ((rc = scan_exclusive<int32_t, int64_t>(work, w->pre, w->nunits, st, mem))) return rc;
   k_unit_heads<<<blocks, 256, 0, st>>>(w->pre, w->nunits, w->target, work);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_exclusive<int32_t, int64_t>(work, w->rank, w->nunits, st))) return rc;
-  GBO_HIP_CHECK(hipMemcpyAsync(&w->total, w->pre + w->nunits, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipMemcpyAsync(&w->nch, w->rank + w->nunits, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
-  return GBO_OK;
+  if ((rc = scan_exclusive<int32_t, int64_t>(work, w->rank, w->nunits, st, mem))) return rc;
+  if ((rc = read_back(&w->total, w->pre + w->nunits, sizeof(int64_t), st))) return rc;
+  return read_back(&w->nch, w->rank + w->nunits, sizeof(int64_t), st);
 }
 
 // Plan for a matrix: uses A->plan (made by gbo_bsr_plan, with its scratch)
@@ -686,7 +696,7 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, 
   // from it need the same alignment
   bool even = chunk_tiles > 0 || A->nblocks == 0 || A->nblocks >= kEvenTiles || !A->tiles || ((uintptr_t)A->tiles & 15);
   int64_t nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   WorkCut w;
   if (!even) {
     int rc = GBO_OK;
@@ -703,7 +713,11 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, 
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "gbo_bsr_plan: too many chunks");
   gbo_bsr_plan_free(A);
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, scratch);
-  GBO_HIP_CHECK(hipMalloc((void**)&A->plan, L.bytes));
+  if (device_malloc((void**)&A->plan, L.bytes) != hipSuccess) {
+    A->plan = nullptr;
+    return set_error(GBO_ENOMEM, "gbo_bsr_plan: allocation of %zu bytes failed", L.bytes);
+  }
+  workspace_live(1);
   A->plan_chunk = chunk;
   A->plan_nchunks = (int32_t)nch;
   A->plan_variant = variant;
@@ -759,7 +773,7 @@ int gbo_csr2bsr_nnzb_dev(int bs, const int32_t* d_rp, const int32_t* d_ci, int32
     return set_error(GBO_EINVAL, "gbo_csr2bsr_nnzb_dev: bad argument");
   hipStream_t st = stream;
   const int32_t nbr = (nrows + bs - 1) / bs;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   PieceSet ps;
   int rc = make_pieces(bs, d_rp, d_ci, nrows, ncols, nbr, mem, &ps, "gbo_csr2bsr_nnzb_dev", st);
   if (rc != GBO_OK) return rc;
@@ -782,14 +796,13 @@ int gbo_csr2bsr_fill_dev(int bs, int dir, const int32_t* d_rp, const int32_t* d_
   const int32_t nbr = (nrows + bs - 1) / bs;
   // the tile offsets come from the pieces' counts (the same as d_bsrRowPtr
   // at block-row starts); the rows are checked again on the way
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   PieceSet ps;
   int rc = make_pieces(bs, d_rp, d_ci, nrows, ncols, nbr, mem, &ps, "gbo_csr2bsr_fill_dev", st);
   if (rc != GBO_OK) return rc;
   if (ps.total > 0 && (!d_bsrColInd || !d_tiles)) return set_error(GBO_EINVAL, "gbo_csr2bsr_fill_dev: null output");
   int32_t given = 0;  // the caller sized colind and tiles by rowptr[nbr]
-  GBO_HIP_CHECK(hipMemcpyAsync(&given, d_bsrRowPtr + nbr, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_back(&given, d_bsrRowPtr + nbr, sizeof(int32_t), st))) return rc;
   if (given != ps.total)
     return set_error(GBO_EINVAL, "gbo_csr2bsr_fill_dev: rowptr[nblockrows] = %d, the CSR has %lld tiles", given,
                      (long long)ps.total);
@@ -817,15 +830,17 @@ int gbo_bsr_create_dev(int bs, int dir, const int32_t* d_rp, const int32_t* d_ci
   A.ncols = ncols;
   A.nblockrows = nbr;
   A.nblockcols = (ncols + bs - 1) / bs;
-  GBO_HIP_CHECK(hipMalloc((void**)&A.rowptr, sizeof(int32_t) * ((size_t)nbr + 1)));
+  if (device_malloc((void**)&A.rowptr, sizeof(int32_t) * ((size_t)nbr + 1)) != hipSuccess)
+    return set_error(GBO_ENOMEM, "gbo_bsr_create_dev: cannot allocate %d row pointers", nbr + 1);
+  workspace_live(1);
   int rc = gbo_csr2bsr_nnzb_dev(bs, d_rp, d_ci, nrows, ncols, A.rowptr, &A.nblocks, stream);
   if (rc != GBO_OK) {
-    (void)hipFree(A.rowptr);
+    gbo_bsr_free(&A);
     return rc;
   }
   const size_t tile_bytes = (size_t)A.nblocks * bs * (bs / 8);
-  hipError_t e1 = hipMalloc((void**)&A.colind, sizeof(int32_t) * std::max<int64_t>(A.nblocks, 1));
-  hipError_t e2 = hipMalloc(&A.tiles, std::max<size_t>(tile_bytes, 8));
+  hipError_t e1 = device_malloc((void**)&A.colind, sizeof(int32_t) * std::max<int64_t>(A.nblocks, 1));
+  hipError_t e2 = device_malloc(&A.tiles, std::max<size_t>(tile_bytes, 8));
   if (e1 != hipSuccess || e2 != hipSuccess) {
     gbo_bsr_free(&A);
     return set_error(GBO_ENOMEM, "gbo_bsr_create: cannot allocate %zu tile bytes", tile_bytes);
@@ -927,7 +942,10 @@ int gbo_bsr_create(int bs, int dir, const int32_t* h_rp, const int32_t* h_ci, in
 
 void gbo_bsr_plan_free(gbo_bsr* A) {
   if (!A) return;
-  if (A->plan) (void)hipFree(A->plan);
+  if (A->plan) {
+    (void)hipFree(A->plan);
+    workspace_live(-1);
+  }
   A->plan = nullptr;
   A->plan_chunk = 0;
   A->plan_nchunks = 0;
@@ -937,7 +955,10 @@ void gbo_bsr_plan_free(gbo_bsr* A) {
 void gbo_bsr_free(gbo_bsr* A) {
   if (!A) return;
   gbo_bsr_plan_free(A);
-  if (A->rowptr) (void)hipFree(A->rowptr);
+  if (A->rowptr) {
+    (void)hipFree(A->rowptr);
+    workspace_live(-1);
+  }
   if (A->colind) (void)hipFree(A->colind);
   if (A->tiles) (void)hipFree(A->tiles);
   A->rowptr = nullptr;
@@ -965,8 +986,9 @@ int gbo_csr2bsr_values_u32(const gbo_bsr* A, const int32_t* d_rp, const int32_t*
   if (!d_rp || !d_val || !d_tval || !d_woff) return set_error(GBO_EINVAL, "gbo_csr2bsr_values_u32: null argument");
   hipStream_t st = stream;
   const int64_t T = A->nblocks;
+  Workspace mem(st);
   int64_t* cnt = nullptr;
-  GBO_HIP_CHECK(hipMallocAsync((void**)&cnt, sizeof(int64_t) * std::max<int64_t>(T, 1), st));
+  if ((rc = mem.alloc(&cnt, sizeof(int64_t) * (size_t)std::max<int64_t>(T, 1), "gbo_csr2bsr_values_u32"))) return rc;
   if (T > 0) {
     const unsigned blocks = (unsigned)((T + 255) / 256);
     switch (A->bs) {
@@ -977,10 +999,7 @@ int gbo_csr2bsr_values_u32(const gbo_bsr* A, const int32_t* d_rp, const int32_t*
     }
     GBO_LAUNCH_CHECK();
   }
-  rc = scan_exclusive<int64_t, int64_t>(cnt, d_woff, T, st);
-  (void)hipFreeAsync(cnt, st);
-  if (rc) return rc;
-  AsyncAllocs mem(st);
+  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, d_woff, T, st, mem))) return rc;
   PieceSet ps;
   if ((rc = make_pieces(A->bs, d_rp, d_ci, A->nrows, A->ncols, A->nblockrows, mem, &ps, "gbo_csr2bsr_values_u32", st)))
     return rc;

@@ -458,27 +458,25 @@ struct Operand {
   int64_t nseg = 0, nslot = 0, nmulti = 0;
 };
 
-int make_operand(const gbo_bsr* M, AsyncAllocs& mem, Operand* o, hipStream_t st) {
+int make_operand(const gbo_bsr* M, Workspace& mem, Operand* o, hipStream_t st) {
   const char* who = "gbo_ppr";
   const int32_t n = M->nrows;
   int rc = expand_csr(M, mem, &o->csr, st);
   if (rc) return rc;
-  AsyncAllocs tmp(st);
   int64_t *cnt = nullptr, *moff = nullptr, *off = nullptr;
   int32_t *multi = nullptr, *mrow = nullptr;
-  if ((rc = tmp.alloc(&cnt, sizeof(int64_t) * (size_t)std::max(n, 1), who)) ||
-      (rc = tmp.alloc(&multi, sizeof(int32_t) * (size_t)std::max(n, 1), who)) ||
-      (rc = tmp.alloc(&moff, sizeof(int64_t) * ((size_t)n + 1), who)) ||
+  if ((rc = mem.alloc(&cnt, sizeof(int64_t) * (size_t)std::max(n, 1), who)) ||
+      (rc = mem.alloc(&multi, sizeof(int32_t) * (size_t)std::max(n, 1), who)) ||
+      (rc = mem.alloc(&moff, sizeof(int64_t) * ((size_t)n + 1), who)) ||
       (rc = mem.alloc(&off, sizeof(int64_t) * ((size_t)n + 1), who)))
     return rc;
   k_seg_count<<<grid_of(n, 256), 256, 0, st>>>(o->csr.rowptr, n, cnt, multi);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, off, n, st))) return rc;
-  if ((rc = scan_exclusive<int32_t, int64_t>(multi, moff, n, st))) return rc;
+  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, off, n, st, mem))) return rc;
+  if ((rc = scan_exclusive<int32_t, int64_t>(multi, moff, n, st, mem))) return rc;
   int64_t tot = 0;
-  GBO_HIP_CHECK(hipMemcpyAsync(&tot, off + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipMemcpyAsync(&o->nmulti, moff + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_back(&tot, off + n, sizeof(int64_t), st)) || (rc = read_back(&o->nmulti, moff + n, sizeof(int64_t), st)))
+    return rc;
   o->nseg = tot & 0xFFFFFFFF;
   o->nslot = tot >> 32;
   Seg* segs = nullptr;
@@ -532,7 +530,7 @@ struct Scratch {
   Ctl* ctl = nullptr;
 };
 
-int make_scratch(const int32_t* d_outdeg, int32_t n, int32_t ld, int64_t nslot, AsyncAllocs& mem, Scratch* s,
+int make_scratch(const int32_t* d_outdeg, int32_t n, int32_t ld, int64_t nslot, Workspace& mem, Scratch* s,
                  hipStream_t st) {
   const char* who = "gbo_ppr";
   int rc;
@@ -567,8 +565,8 @@ int iterate(int32_t max_iter, const Scratch& s, int32_t* iters, double* dmax, hi
       const int rc = step(it);
       if (rc) return rc;
     }
-    GBO_HIP_CHECK(hipMemcpyAsync(&h, s.ctl, offsetof(Ctl, val), hipMemcpyDeviceToHost, st));
-    GBO_HIP_CHECK(hipStreamSynchronize(st));
+    const int rc = read_back(&h, s.ctl, offsetof(Ctl, val), st);
+    if (rc) return rc;
   }
   *iters = (int32_t)h.iters;
   *dmax = h.dmax;
@@ -596,7 +594,7 @@ int gbo_ppr_forward(const gbo_bsr* AT, const int32_t* d_outdeg, int32_t K, float
   hipStream_t st = stream;
   const int32_t n = AT->nrows, ld = (K + 3) / 4 * 4;
   const size_t bytes = sizeof(float) * (size_t)std::max<int64_t>((int64_t)n * ld, 1);
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   Operand o;
   Scratch s;
   if ((rc = make_operand(AT, mem, &o, st)) || (rc = make_scratch(d_outdeg, n, ld, o.nslot, mem, &s, st))) return rc;
@@ -662,12 +660,12 @@ int gbo_ppr_adjoint(const gbo_bsr* A, const gbo_bsr* AT, const int32_t* d_outdeg
   const size_t bytes = sizeof(float) * (size_t)std::max<int64_t>((int64_t)n * ld, 1);
   const bool same = A->rowptr == AT->rowptr && A->colind == AT->colind && A->tiles == AT->tiles && A->bs == AT->bs &&
                     A->nblocks == AT->nblocks;
-  AsyncAllocs mem(st), memT(st);
+  Workspace mem(st);
   Operand o, oT;
   Scratch s;
   if ((rc = make_operand(A, mem, &o, st))) return rc;
   if (same) oT = o;
-  else if ((rc = make_operand(AT, memT, &oT, st))) return rc;
+  else if ((rc = make_operand(AT, mem, &oT, st))) return rc;
   if ((rc = make_scratch(d_outdeg, n, ld, std::max(o.nslot, oT.nslot), mem, &s, st))) return rc;
   float* lam[2] = {nullptr, nullptr};
   if ((rc = mem.alloc(&lam[0], bytes, "gbo_ppr_adjoint")) || (rc = mem.alloc(&lam[1], bytes, "gbo_ppr_adjoint")))
@@ -715,8 +713,7 @@ int gbo_ppr_adjoint(const gbo_bsr* A, const gbo_bsr* AT, const int32_t* d_outdeg
   T.ctl = s.ctl;
   if ((rc = spmm(oT, T, 0.0, st))) return rc;
   double ga[64];
-  GBO_HIP_CHECK(hipMemcpyAsync(ga, s.ctl->val, sizeof(double) * K, hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_back(ga, s.ctl->val, sizeof(double) * K, st))) return rc;
   if (h_grad_alpha) {
     double g = 0.0;
     for (int32_t k = 0; k < K; ++k) g += ga[k];

@@ -3,6 +3,7 @@
 #include <algorithm>
 
 #include "gbo_device.hpp"
+#include "gbo_ops.hpp"
 
 namespace {
 
@@ -154,7 +155,7 @@ int gbo_malloc(void** p, size_t bytes) {
   if (!p) return gbo::set_error(GBO_EINVAL, "gbo_malloc: null");
   *p = nullptr;
   if (bytes == 0) bytes = 256;
-  hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = gbo::device_malloc(p, bytes);
   if (e != hipSuccess)
     return gbo::set_error(GBO_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   return GBO_OK;

@@ -317,21 +317,20 @@ struct Pairs {
 };
 
 template <int BS>
-int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, AsyncAllocs& mem, Pairs* out, hipStream_t st) {
+int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, Workspace& mem, Pairs* out, hipStream_t st) {
   using W = word_t<BS>;
   const int64_t T = A->nblocks;
   out->jbits = (int)bits_for(std::max<int32_t>(B->nblockcols, 1) - 1);
   if (T == 0 || B->nblocks == 0) return GBO_OK;
-  AsyncAllocs tmp(st);
   W *amask = nullptr, *bmask = nullptr;
   int32_t* trow = nullptr;
   int64_t *cnt = nullptr, *coff = nullptr;
   int rc;
-  if ((rc = tmp.alloc(&amask, sizeof(W) * (size_t)T, "gbo_bsrbmm")) ||
-      (rc = tmp.alloc(&bmask, sizeof(W) * (size_t)B->nblocks, "gbo_bsrbmm")) ||
-      (rc = tmp.alloc(&trow, sizeof(int32_t) * (size_t)T, "gbo_bsrbmm")) ||
-      (rc = tmp.alloc(&cnt, sizeof(int64_t) * (size_t)T, "gbo_bsrbmm")) ||
-      (rc = tmp.alloc(&coff, sizeof(int64_t) * ((size_t)T + 1), "gbo_bsrbmm")))
+  if ((rc = mem.alloc(&amask, sizeof(W) * (size_t)T, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&bmask, sizeof(W) * (size_t)B->nblocks, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&trow, sizeof(int32_t) * (size_t)T, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&cnt, sizeof(int64_t) * (size_t)T, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&coff, sizeof(int64_t) * ((size_t)T + 1), "gbo_bsrbmm")))
     return rc;
   constexpr int G = kWave / BS;
   k_masks<BS><<<grid_for((T + G - 1) / G, 4), 256, 0, st>>>((const W*)A->tiles, T, false, amask);
@@ -339,15 +338,14 @@ int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, AsyncAllocs
   k_tile_rows_of<<<grid_for(T, 256), 256, 0, st>>>(A->rowptr, A->nblockrows, T, trow);
   k_cand_count<<<grid_for(T, 256), 256, 0, st>>>(A->colind, T, B->rowptr, cnt);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, coff, T, st))) return rc;
+  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, coff, T, st, mem))) return rc;
   int64_t Pc = 0;
-  GBO_HIP_CHECK(hipMemcpyAsync(&Pc, coff + T, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_back(&Pc, coff + T, sizeof(int64_t), st))) return rc;
   if (Pc == 0) return GBO_OK;
   const int64_t nw = (Pc + kPerWave - 1) / kPerWave;
   int64_t *wcount = nullptr, *woff = nullptr;
-  if ((rc = tmp.alloc(&wcount, sizeof(int64_t) * (size_t)nw, "gbo_bsrbmm")) ||
-      (rc = tmp.alloc(&woff, sizeof(int64_t) * ((size_t)nw + 1), "gbo_bsrbmm")))
+  if ((rc = mem.alloc(&wcount, sizeof(int64_t) * (size_t)nw, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&woff, sizeof(int64_t) * ((size_t)nw + 1), "gbo_bsrbmm")))
     return rc;
   PairArgs pa{};
   pa.a_colind = A->colind;
@@ -363,16 +361,15 @@ int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, AsyncAllocs
   pa.wcount = wcount;
   k_pairs<BS, 0><<<grid_for(nw, 4), 256, 0, st>>>(pa);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_exclusive<int64_t, int64_t>(wcount, woff, nw, st))) return rc;
+  if ((rc = scan_exclusive<int64_t, int64_t>(wcount, woff, nw, st, mem))) return rc;
   int64_t P = 0;
-  GBO_HIP_CHECK(hipMemcpyAsync(&P, woff + nw, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_back(&P, woff + nw, sizeof(int64_t), st))) return rc;
   if (P == 0) return GBO_OK;
   uint64_t *k0 = nullptr, *v0 = nullptr;
-  if ((rc = tmp.alloc(&k0, sizeof(uint64_t) * (size_t)P, "gbo_bsrbmm")) ||
+  if ((rc = mem.alloc(&k0, sizeof(uint64_t) * (size_t)P, "gbo_bsrbmm")) ||
       (rc = mem.alloc(&out->keys, sizeof(uint64_t) * (size_t)P, "gbo_bsrbmm")))
     return rc;
-  if (with_vals && ((rc = tmp.alloc(&v0, sizeof(uint64_t) * (size_t)P, "gbo_bsrbmm")) ||
+  if (with_vals && ((rc = mem.alloc(&v0, sizeof(uint64_t) * (size_t)P, "gbo_bsrbmm")) ||
                     (rc = mem.alloc(&out->vals, sizeof(uint64_t) * (size_t)P, "gbo_bsrbmm"))))
     return rc;
   pa.woff = woff;
@@ -388,7 +385,7 @@ int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, AsyncAllocs
   } else {
     GBO_HIP_CHECK(rocprim::radix_sort_keys(nullptr, tb, k0, out->keys, (size_t)P, 0, end_bit, st));
   }
-  if ((rc = tmp.alloc(&sort_tmp, std::max<size_t>(tb, 8), "gbo_bsrbmm"))) return rc;
+  if ((rc = mem.alloc(&sort_tmp, std::max<size_t>(tb, 8), "gbo_bsrbmm"))) return rc;
   if (with_vals) {
     GBO_HIP_CHECK(rocprim::radix_sort_pairs(sort_tmp, tb, k0, out->keys, v0, out->vals, (size_t)P, 0, end_bit, st));
   } else {
@@ -400,20 +397,18 @@ int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, AsyncAllocs
 
 // Runs of the sorted keys: C's block rows (and columns, segment starts) per
 // C tile; *nc = number of C tiles.
-int key_runs(const Pairs& pr, AsyncAllocs& mem, int32_t** crow, int32_t* ccol, int64_t** seg, int64_t* nc,
+int key_runs(const Pairs& pr, Workspace& mem, int32_t** crow, int32_t* ccol, int64_t** seg, int64_t* nc,
              hipStream_t st) {
-  AsyncAllocs tmp(st);
   int32_t* head = nullptr;
   int64_t* rank = nullptr;
   int rc;
-  if ((rc = tmp.alloc(&head, sizeof(int32_t) * (size_t)pr.P, "gbo_bsrbmm")) ||
-      (rc = tmp.alloc(&rank, sizeof(int64_t) * ((size_t)pr.P + 1), "gbo_bsrbmm")))
+  if ((rc = mem.alloc(&head, sizeof(int32_t) * (size_t)pr.P, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&rank, sizeof(int64_t) * ((size_t)pr.P + 1), "gbo_bsrbmm")))
     return rc;
   k_heads<<<grid_for(pr.P, 256), 256, 0, st>>>(pr.keys, pr.P, head);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_exclusive<int32_t, int64_t>(head, rank, pr.P, st))) return rc;
-  GBO_HIP_CHECK(hipMemcpyAsync(nc, rank + pr.P, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  GBO_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = scan_exclusive<int32_t, int64_t>(head, rank, pr.P, st, mem))) return rc;
+  if ((rc = read_back(nc, rank + pr.P, sizeof(int64_t), st))) return rc;
   if ((rc = mem.alloc(crow, sizeof(int32_t) * (size_t)std::max<int64_t>(*nc, 1), "gbo_bsrbmm"))) return rc;
   if (seg) {
     if ((rc = mem.alloc(seg, sizeof(int64_t) * ((size_t)*nc + 1), "gbo_bsrbmm"))) return rc;
@@ -428,7 +423,7 @@ int key_runs(const Pairs& pr, AsyncAllocs& mem, int32_t** crow, int32_t* ccol, i
 
 template <int BS>
 int symbolic_t(const gbo_bsr* A, const gbo_bsr* B, int32_t* d_rowptr, int64_t* nblocks, hipStream_t st) {
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   Pairs pr;
   int rc = sorted_pairs<BS>(A, B, false, mem, &pr, st);
   if (rc) return rc;
@@ -449,7 +444,7 @@ template <int BS>
 int numeric_t(const gbo_bsr* A, const gbo_bsr* B, int64_t nc_expect, int32_t* d_colind, word_t<BS>* d_tiles,
               const int64_t* d_valoff, int32_t* d_counts, hipStream_t st) {
   using W = word_t<BS>;
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   Pairs pr;
   int rc = sorted_pairs<BS>(A, B, true, mem, &pr, st);
   if (rc) return rc;
@@ -481,7 +476,7 @@ int numeric_t(const gbo_bsr* A, const gbo_bsr* B, int64_t nc_expect, int32_t* d_
 
 template <int BS>
 int valoff_t(const word_t<BS>* tiles, int64_t nc, int64_t* d_valoff, int64_t* nnz, hipStream_t st) {
-  AsyncAllocs mem(st);
+  Workspace mem(st);
   int64_t* cnt = nullptr;
   int rc = mem.alloc(&cnt, sizeof(int64_t) * (size_t)std::max<int64_t>(nc, 1), "gbo_bsrbmm_numeric");
   if (rc) return rc;
@@ -489,10 +484,9 @@ int valoff_t(const word_t<BS>* tiles, int64_t nc, int64_t* d_valoff, int64_t* nn
     k_tile_popc64<BS><<<grid_for(nc, 256), 256, 0, st>>>(tiles, nc, cnt);
     GBO_LAUNCH_CHECK();
   }
-  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, d_valoff, nc, st))) return rc;
+  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, d_valoff, nc, st, mem))) return rc;
   if (nnz) {
-    GBO_HIP_CHECK(hipMemcpyAsync(nnz, d_valoff + nc, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    GBO_HIP_CHECK(hipStreamSynchronize(st));
+    if ((rc = read_back(nnz, d_valoff + nc, sizeof(int64_t), st))) return rc;
   }
   return GBO_OK;
 }
@@ -588,12 +582,14 @@ int gbo_bsrbmm(const gbo_bsr* A, const gbo_bsr* B, gbo_bsr* C, gbo_stream_t stre
   R.ncols = B->ncols;
   R.nblockrows = A->nblockrows;
   R.nblockcols = B->nblockcols;
-  GBO_HIP_CHECK(hipMalloc((void**)&R.rowptr, sizeof(int32_t) * ((size_t)R.nblockrows + 1)));
+  if (device_malloc((void**)&R.rowptr, sizeof(int32_t) * ((size_t)R.nblockrows + 1)) != hipSuccess)
+    return set_error(GBO_ENOMEM, "gbo_bsrbmm: cannot allocate %d row pointers", R.nblockrows + 1);
+  workspace_live(1);
   rc = gbo_bsrbmm_symbolic(A, B, R.rowptr, &R.nblocks, stream);
   if (rc == GBO_OK) {
     const size_t tile_bytes = (size_t)R.nblocks * R.bs * (R.bs / 8);
-    hipError_t e1 = hipMalloc((void**)&R.colind, sizeof(int32_t) * std::max<int64_t>(R.nblocks, 1));
-    hipError_t e2 = hipMalloc(&R.tiles, std::max<size_t>(tile_bytes, 8));
+    hipError_t e1 = device_malloc((void**)&R.colind, sizeof(int32_t) * std::max<int64_t>(R.nblocks, 1));
+    hipError_t e2 = device_malloc(&R.tiles, std::max<size_t>(tile_bytes, 8));
     if (e1 != hipSuccess || e2 != hipSuccess)
       rc = set_error(GBO_ENOMEM, "gbo_bsrbmm: cannot allocate %zu tile bytes", tile_bytes);
   }

@@ -1,0 +1,211 @@
+// Device scratch of synchronous calls, kept between calls.
+//
+// Every driver and two-phase operation needs a few buffers and waits for its
+// stream before it returns.  From the runtime's stream-ordered pool they cost
+// 10 to 100 us each (an allocation of 64 MB 30 us, its release 9, and the next
+// synchronization gives the memory back: 31 us for 4 x 1 MB, 0.8 ms for 4 x
+// 64 MB), several times the kernels of a small call.  Here a block goes back
+// to a list when its call is over and is handed out again:
+//   - a block enters the list only after the stream that used it has been
+//     waited for, so whichever thread or stream takes it next finds it idle;
+//   - the list holds at most kKeepBytes and kKeepBlocks per device, the
+//     longest unused go first; all of it goes back to the runtime when an
+//     allocation fails and when the last matrix that the library allocated or
+//     planned is freed.
+#include <algorithm>
+#include <cstring>
+#include <mutex>
+#include <vector>
+
+#include "gbo_device.hpp"
+#include "gbo_ops.hpp"
+
+namespace gbo {
+namespace {
+
+constexpr size_t kKeepBytes = (size_t)1 << 30;
+constexpr size_t kKeepBlocks = 128;
+constexpr int kDevices = 64;
+
+struct Block {
+  void* p;
+  size_t bytes;
+};
+
+struct Pool {
+  std::mutex mu;
+  std::vector<Block> idle[kDevices];  // the longest unused first
+  size_t bytes[kDevices] = {};
+  int64_t live = 0;  // matrices and plans the library allocated
+};
+
+// Never destroyed: at exit the runtime may be gone before it.
+Pool& pool() {
+  static Pool* p = new Pool;
+  return *p;
+}
+
+// Sizes in steps of an eighth of a power of two (512 bytes at least), so that
+// calls of about the same size find each other's blocks.
+size_t rounded(size_t bytes) {
+  size_t step = 512;
+  while (step * 16 < bytes) step *= 2;
+  return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+}
+
+void give_back(const std::vector<Block>& blocks) {
+  for (const Block& b : blocks) (void)hipFree(b.p);
+}
+
+}  // namespace
+
+void workspace_release(int dev) {
+  std::vector<Block> out;
+  {
+    Pool& P = pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    for (int d = dev < 0 ? 0 : dev; d < (dev < 0 ? kDevices : std::min(dev + 1, kDevices)); ++d) {
+      out.insert(out.end(), P.idle[d].begin(), P.idle[d].end());
+      P.idle[d].clear();
+      P.bytes[d] = 0;
+    }
+  }
+  give_back(out);
+}
+
+void workspace_live(int delta) {
+  bool last = false;
+  {
+    Pool& P = pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    P.live += delta;
+    last = delta < 0 && P.live <= 0;
+  }
+  if (last) workspace_release(-1);
+}
+
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    workspace_release(dev);
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
+Workspace::~Workspace() {
+  if (n_ == 0) return;
+  const bool idle = hipStreamSynchronize(st_) == hipSuccess;
+  std::vector<Block> out;
+  {
+    Pool& P = pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    for (int i = 0; i < n_; ++i) {
+      if (!idle || dev_ < 0 || dev_ >= kDevices) {
+        out.push_back({ptrs_[i], bytes_[i]});
+        continue;
+      }
+      P.idle[dev_].push_back({ptrs_[i], bytes_[i]});
+      P.bytes[dev_] += bytes_[i];
+    }
+    if (dev_ >= 0 && dev_ < kDevices) {
+      auto& v = P.idle[dev_];
+      size_t drop = 0;
+      while (drop < v.size() && (P.bytes[dev_] > kKeepBytes || v.size() - drop > kKeepBlocks)) {
+        P.bytes[dev_] -= v[drop].bytes;
+        out.push_back(v[drop++]);
+      }
+      v.erase(v.begin(), v.begin() + (ptrdiff_t)drop);
+    }
+  }
+  give_back(out);
+}
+
+int Workspace::take(void** p, size_t bytes, const char* who) {
+  *p = nullptr;
+  if (n_ == kMax) return set_error(GBO_EINVAL, "%s: too many scratch allocations", who);
+  if (n_ == 0) GBO_HIP_CHECK(hipGetDevice(&dev_));
+  const size_t want = rounded(bytes);
+  void* q = nullptr;
+  size_t got = want;
+  if (dev_ >= 0 && dev_ < kDevices) {
+    Pool& P = pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    auto& v = P.idle[dev_];
+    size_t best = v.size();
+    for (size_t i = 0; i < v.size(); ++i)  // the smallest that fits and is not twice too large
+      if (v[i].bytes >= want && v[i].bytes <= 2 * want && (best == v.size() || v[i].bytes < v[best].bytes)) best = i;
+    if (best < v.size()) {
+      q = v[best].p;
+      got = v[best].bytes;
+      P.bytes[dev_] -= got;
+      v.erase(v.begin() + (ptrdiff_t)best);
+    }
+  }
+  if (!q) {
+    const hipError_t e = device_malloc(&q, want);
+    if (e != hipSuccess)
+      return set_error(GBO_ENOMEM, "%s: device allocation of %zu bytes failed: %s", who, bytes, hipGetErrorString(e));
+  }
+  ptrs_[n_] = q;
+  bytes_[n_++] = got;
+  *p = q;
+  return GBO_OK;
+}
+
+// ---- small host reads.  A copy into ordinary host memory is staged by the
+// runtime (20 us with the wait); into one of these pinned slots it is not
+// (12 us).  With every slot taken the ordinary copy serves.
+namespace {
+
+constexpr size_t kSlotBytes = 16384;
+constexpr int kSlots = 16;
+
+struct Slots {
+  std::mutex mu;
+  char* base = nullptr;
+  bool tried = false;
+  uint32_t taken = 0;
+};
+Slots& slots() {
+  static Slots* s = new Slots;
+  return *s;
+}
+
+}  // namespace
+
+int read_back(void* h, const void* d, size_t bytes, hipStream_t st) {
+  Slots& S = slots();
+  int k = -1;
+  if (bytes <= kSlotBytes) {
+    std::lock_guard<std::mutex> lk(S.mu);
+    if (!S.tried) {
+      S.tried = true;
+      void* p = nullptr;
+      if (hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocPortable) == hipSuccess) S.base = (char*)p;
+      else (void)hipGetLastError();
+    }
+    if (S.base)
+      for (int i = 0; i < kSlots && k < 0; ++i)
+        if (!(S.taken >> i & 1u)) k = i;
+    if (k >= 0) S.taken |= 1u << k;
+  }
+  void* to = k >= 0 ? S.base + (size_t)k * kSlotBytes : h;
+  hipError_t e = hipMemcpyAsync(to, d, bytes, hipMemcpyDeviceToHost, st);
+  // waited for in any case: the slot must not be written once it is free again
+  const hipError_t s = hipStreamSynchronize(st);
+  if (e == hipSuccess) e = s;
+  if (k >= 0) {
+    if (e == hipSuccess) std::memcpy(h, to, bytes);
+    std::lock_guard<std::mutex> lk(S.mu);
+    S.taken &= ~(1u << k);
+  }
+  if (e != hipSuccess) return set_error(GBO_EDEVICE, "device to host copy: %s", hipGetErrorString(e));
+  return GBO_OK;
+}
+
+}  // namespace gbo
