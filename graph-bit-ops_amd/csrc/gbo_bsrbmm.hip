@@ -6,22 +6,17 @@
 // The reference walks, per mask tile (I,K), every tile (I,J) of block row I
 // and binary-searches B's block row J for K -- O(deg^2 log) per block row.
 // Here the block-column structure of B is transposed once (a stable radix
-// sort of the tiles by block column on the device: csr2csc on blocks) so
-// that the J's that contribute to mask tile (I,K) are the intersection of
-// two sorted lists: block row I of A and block column K of B.  Each wave
-// takes a fixed chunk of mask tiles; its 64 lanes look up 64 entries of the
-// shorter list at a time in the longer one (a binary search, or one load
-// from the bitmap of a heavy row's block columns), or, when both lists have
-// bitmaps, AND the two maps 64 words at a time.  Each match J adds
-// sum_{a,k} M[a][k] (A_IJ B_JK)[a][k] = sum over the set bits (a,j) of A_IJ
-// of popc(M[a] & B_JK row j) -- one popcount per set bit of A_IJ, with B's
-// tiles turned into row form once per call.
+// sort of the tiles by block column on the device: csr2csc on blocks), and
+// the count is, over the set bits (i, k) of A, |A_i and C_k|: row i of A
+// against column k of B.  Sparse tiles are listed once as rows and columns of
+// ids (k_tc_light, k_tc_heavy), dense ones are intersected word by word
+// (k_tc_tiles).
 //
 // Plain product sum (bmm{N}_sparse, bsrbmm/bsrbmm.cu:296-555):
 //   sum_{i,k} (A B)_ik = sum_j colsum_A(j) * rowsum_B(j),
 // two linear passes over the tiles instead of the reference's tile-pair loop.
 #include <algorithm>
-#include <vector>
+#include <type_traits>
 
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -29,50 +24,6 @@
 #include "gbo_ops.hpp"
 
 namespace gbo {
-
-struct TcArgs {
-  const int32_t* a_rowptr;
-  const int32_t* a_colind;
-  const void* a_tiles;
-  int32_t nbr;
-  int64_t T;
-  const int32_t* plan;
-  int32_t chunk, nchunks;
-  const int32_t* bt_ptr;   // block-CSC of B: column K lists [bt_ptr[K], bt_ptr[K+1])
-  const int32_t* bt_row;   //   block row J of each entry (ascending inside a column)
-  const int32_t* bt_tile;  //   tile index in B of each entry
-  const void* b_tiles;
-  unsigned long long* count;
-  // heavy block rows of A (many tiles): a bitmap of the row's block columns
-  // and the rank of each 64-bit word, so membership of J in the row and
-  // J's tile index are two loads instead of a binary search
-  const int32_t* hslot;    // per block row: slot of its bitmap, or -1 (nullable)
-  const uint4* hmap;       // [slots][hwords]: x, y = the word's 64 bits (low,
-                           // high), z = set bits in the words before it
-  int64_t hwords;
-  // per block column K of B: the slot whose bitmap holds B's column K list
-  // (B = L^T, so column K of B is row K of L), or -1 (nullable)
-  const int32_t* hcol;
-  // bs 32/64 (nullable): the set bits of every A tile, row-major (entry =
-  // row * BS + column), from aoff[t]; a match whose A tile has at most
-  // kLaneMatchBits of them is counted by its own lane
-  const int32_t* aoff;
-  const uint16_t* abits;
-  int vec16;  // bs 16: the tiles of A and B are 16-byte aligned (vector loads)
-};
-
-// A match (I,J,K) at bs 32/64 whose A tile (I,J) has at most this many set
-// bits is counted by one lane (a popcount per bit from the tile's bit list)
-// instead of by a group of bs lanes, one per tile row: R-MAT tiles hold 2-3
-// bits, so the group form left all but a few of its lanes idle.
-constexpr int32_t kLaneMatchBits = 16;
-
-// A mask tile (I,K) whose row I and column K both have bitmaps intersects
-// them by an AND of the two maps over the words both lists span when that
-// takes at most 1/kAndRatio of the passes of the key lookups (64 words or 64
-// keys a pass).  R-MAT s20: 5-13 % faster than the lookups alone with 1 or 2,
-// the key lookups' gathers being dearer than the AND's coalesced loads.
-constexpr int64_t kAndRatio = 2;
 
 // First index in [lo, hi) of sorted arr whose value is >= key.
 __device__ __forceinline__ int64_t lower_bound_i32(const int32_t* __restrict__ arr, int64_t lo, int64_t hi, int32_t key) {
@@ -82,385 +33,6 @@ __device__ __forceinline__ int64_t lower_bound_i32(const int32_t* __restrict__ a
     else hi = mid;
   }
   return lo;
-}
-
-// Row-packed copy of column-packed tiles (same positions): word j of the
-// output holds row j of the tile, bit BS-1-k = column k.  One wave takes
-// 64/BS tiles; lane l holds column word l % BS of tile l / BS, and one
-// ballot per row j collects that row over the columns of every tile.
-template <int BS>
-__global__ __launch_bounds__(256) void k_tile_rows(const word_t<BS>* __restrict__ in, int64_t T,
-                                                   word_t<BS>* __restrict__ out) {
-  constexpr int G = kWave / BS;
-  const int lane = lane_id();
-  const int64_t t = (int64_t)wave_index() * G + lane / BS;  // tile of this lane
-  const int k = lane % BS;                                  // its column word
-  const uint64_t w = t < T ? (uint64_t)in[t * BS + k] : 0ull;
-  const int g = lane / BS;
-#pragma unroll 8
-  for (int j = 0; j < BS; ++j) {
-    const uint64_t b = __ballot((w >> (BS - 1 - j)) & 1ull);  // bit l: column l % BS of tile l / BS has row j
-    const uint64_t mine = (b >> (g * BS)) & low_mask<BS>();
-    if (k == j && t < T) out[t * BS + j] = (word_t<BS>)brev_low<BS>(mine);
-  }
-}
-
-// Triangles contributed by one matching (I,J,K): with A = tile (I,J) of L,
-// M = mask tile (I,K) and R = B's tile (J,K) in row form,
-//   sum_{a,k} M[a][k] sum_j A[a][j] R[j][k] = sum_{(a,j) in A} popc(M[a] & R[j]),
-// one popcount per set bit of A.
-template <int BS>
-__device__ __forceinline__ uint64_t tc_hit(const word_t<BS>* __restrict__ A, const word_t<BS>* __restrict__ M,
-                                           const word_t<BS>* __restrict__ R, bool vec16) {
-  uint64_t s = 0;
-  if constexpr (BS == 16) {
-    if (vec16) {
-    // A and M as four 64-bit words each (word q = rows 4q..4q+3, row 4q+i
-    // in bits 16i..16i+15), all loaded together, instead of a chain of
-    // row loads; R rows are gathered per set bit of A
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    const u32x4 a0 = *(const u32x4*)A, a1 = *((const u32x4*)A + 1);
-    const u32x4 m0 = *(const u32x4*)M, m1 = *((const u32x4*)M + 1);
-    const uint64_t aw[4] = {a0.x | ((uint64_t)a0.y << 32), a0.z | ((uint64_t)a0.w << 32),
-                            a1.x | ((uint64_t)a1.y << 32), a1.z | ((uint64_t)a1.w << 32)};
-    const uint64_t mw[4] = {m0.x | ((uint64_t)m0.y << 32), m0.z | ((uint64_t)m0.w << 32),
-                            m1.x | ((uint64_t)m1.y << 32), m1.z | ((uint64_t)m1.w << 32)};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      uint64_t wa = aw[q];
-      while (wa) {
-        const int p = __builtin_ctzll(wa);
-        wa &= wa - 1;
-        const int i = p >> 4, col = 15 - (p & 15);  // row 4q+i, column col
-        s += __popc((uint32_t)((mw[q] >> (16 * i)) & 0xFFFFu) & (uint32_t)R[col]);
-      }
-    }
-    return s;
-    }
-  }
-  if constexpr (BS == 8) {
-    uint64_t a = *(const uint64_t*)A;  // byte r = row r, bit 7 - c = column c
-    const uint64_t m = *(const uint64_t*)M, r = *(const uint64_t*)R;
-    while (a) {
-      const int p = __builtin_ctzll(a);
-      a &= a - 1;
-      const int row = p >> 3, col = 7 - (p & 7);
-      s += __popc((uint32_t)((m >> (8 * row)) & (r >> (8 * col)) & 0xFFu));
-    }
-  } else {
-    for (int row = 0; row < BS; ++row) {
-      uint64_t wa = (uint64_t)A[row];
-      if (!wa) continue;
-      const uint64_t ma = (uint64_t)M[row];
-      if (!ma) continue;
-      while (wa) {
-        const int p = __builtin_ctzll(wa);
-        wa &= wa - 1;
-        s += (uint64_t)popcw((word_t<BS>)(ma & (uint64_t)R[BS - 1 - p]));
-      }
-    }
-  }
-  return s;
-}
-
-// Eight waves per SIMD: the kernel is a chain of dependent loads, and
-// without the bound its scalar registers (TcArgs) cost one wave per SIMD
-// (a few of them move to vector-register lanes instead).
-template <int BS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_tc(const TcArgs a) {
-  using W = word_t<BS>;
-  const int lane = lane_id();
-  const int c = wave_index();
-  if (c >= a.nchunks) return;
-  const int64_t cb = (int64_t)c * a.chunk;
-  const int64_t ce = min(cb + (int64_t)a.chunk, a.T);
-  const W* __restrict__ At = (const W*)a.a_tiles;
-  const W* __restrict__ Rt = (const W*)a.b_tiles;  // B's tiles in row form
-  uint64_t total = 0;
-
-  for (int32_t R0 = a.plan[c]; R0 < a.nbr;) {
-    const int32_t Rl = R0 + lane;
-    int32_t rsl = 0, rel = 0;
-    if (Rl < a.nbr) {
-      rsl = a.a_rowptr[Rl];
-      rel = a.a_rowptr[Rl + 1];
-    }
-    const bool belong = (Rl < a.nbr) && ((int64_t)rsl < ce);
-    const uint64_t bmask = __ballot(belong);
-    uint64_t work = __ballot(belong && rel > rsl);
-    while (work) {
-      const int j = __builtin_ctzll(work);
-      work &= work - 1;
-      const int64_t rs = __builtin_amdgcn_readlane(rsl, j), re = __builtin_amdgcn_readlane(rel, j);
-      const int64_t s = rs > cb ? rs : cb;
-      const int64_t te = re < ce ? re : ce;
-      const int32_t hs = a.hslot ? a.hslot[R0 + j] : -1;  // wave-uniform
-      const uint4* __restrict__ hm = hs >= 0 ? a.hmap + (int64_t)hs * a.hwords : nullptr;
-      for (int64_t tm = s; tm < te; ++tm) {  // mask tile (I, K)
-        const int32_t K = a.a_colind[tm];
-        // Intersect block row I of A (J ascending) with block column K of B;
-        // every lane that finds a match adds that (I,J,K) term itself.
-        const int64_t la0 = rs, la1 = re;
-        const int64_t lb0 = a.bt_ptr[K], lb1 = a.bt_ptr[K + 1];
-        // a heavy row walks B's column and looks each J up in its bitmap; a
-        // short row facing a heavy column walks its own tiles and looks them
-        // up in the column's bitmap
-        const bool use_map = hs >= 0 && (lb1 - lb0) <= (la1 - la0);
-        const bool a_short = !use_map && (la1 - la0) <= (lb1 - lb0);
-        const int32_t hk = (a_short && a.hcol) ? a.hcol[K] : -1;
-        const uint4* __restrict__ cm = hk >= 0 ? a.hmap + (int64_t)hk * a.hwords : nullptr;
-        const int64_t s0 = a_short ? la0 : lb0, s1 = a_short ? la1 : lb1;
-        const int64_t l0 = a_short ? lb0 : la0, l1 = a_short ? lb1 : la1;
-        const int32_t* skeys = a_short ? a.a_colind : a.bt_row;
-        const int32_t* lkeys = a_short ? a.bt_row : a.a_colind;
-        // bs 32/64: one lane per tile row; mask row r stays in a register
-        const uint64_t mrow = (BS >= 32 && lane < (kWave / BS) * BS) ? (uint64_t)At[tm * BS + lane % BS] : 0ull;
-        // adds the matches (tA, tB) of the lanes that have one (tA >= 0); every
-        // lane of the wave calls it together
-        auto process = [&](int64_t tA, int64_t tB) {
-          if constexpr (BS <= 16) {
-            // each lane adds its own match
-            if (tA >= 0) total += tc_hit<BS>(At + tA * BS, At + tm * BS, Rt + tB * BS, a.vec16 != 0);
-          } else {
-            // 64/BS matches at a time, one per group of BS lanes (lane = row)
-            constexpr int G = kWave / BS;
-            const int grp = lane / BS, r = lane % BS;
-            // a sparse A tile: this lane counts the match alone, from the
-            // tile's bit list (mask row a, B row j per set bit (a, j))
-            if (tA >= 0 && a.abits) {
-              const int32_t o0 = a.aoff[tA], o1 = a.aoff[tA + 1];
-              if (o1 - o0 <= kLaneMatchBits) {
-                for (int32_t k = o0; k < o1; ++k) {
-                  const uint32_t e = a.abits[k];
-                  total += (uint64_t)popcw((W)((uint64_t)At[tm * BS + e / BS] & (uint64_t)Rt[tB * BS + e % BS]));
-                }
-                tA = -1;
-              }
-            }
-            // the other matches: 64/BS at a time, one per group of BS lanes
-            uint64_t hits = __ballot(tA >= 0);
-            while (hits) {
-              int hsel = -1;
-#pragma unroll
-              for (int g2 = 0; g2 < G; ++g2) {
-                if (hits) {
-                  const int h = __builtin_ctzll(hits);
-                  hits &= hits - 1;
-                  if (g2 == grp) hsel = h;
-                }
-              }
-              const int src = hsel >= 0 ? hsel : 0;
-              const int64_t hA = __shfl(tA, src), hB = __shfl(tB, src);
-              if (hsel >= 0) {
-                uint64_t wa = (uint64_t)At[hA * BS + r];
-                if (mrow) {
-                  while (wa) {
-                    const int p = __builtin_ctzll(wa);
-                    wa &= wa - 1;
-                    total += (uint64_t)popcw((W)(mrow & (uint64_t)Rt[hB * BS + (BS - 1 - p)]));
-                  }
-                }
-              }
-            }
-          }
-        };
-        // both rows have bitmaps: the common J are the set bits of the AND of
-        // the two maps over the words both lists span
-        const int32_t hK = (hs >= 0 && a.hcol) ? a.hcol[K] : -1;
-        if (hK >= 0 && la1 > la0 && lb1 > lb0) {
-          const int32_t jlo = max(a.a_colind[la0], a.bt_row[lb0]);
-          const int32_t jhi = min(a.a_colind[la1 - 1], a.bt_row[lb1 - 1]);
-          const int64_t len = min(la1 - la0, lb1 - lb0);
-          const int64_t wpass = jhi >= jlo ? ((jhi >> 6) - (jlo >> 6) + kWave) / kWave : 0;
-          if (wpass * kAndRatio <= (len + kWave - 1) / kWave) {
-            const uint4* __restrict__ km = a.hmap + (int64_t)hK * a.hwords;
-            for (int32_t w0 = jlo >> 6; jhi >= jlo && w0 <= (jhi >> 6); w0 += kWave) {
-              const int32_t w = w0 + lane;
-              uint64_t x = 0, wi = 0, wk = 0;
-              uint32_t ri = 0, rk = 0;
-              if (w <= (jhi >> 6)) {
-                const uint4 ei = hm[w], ek = km[w];
-                wi = (uint64_t)ei.x | ((uint64_t)ei.y << 32);
-                wk = (uint64_t)ek.x | ((uint64_t)ek.y << 32);
-                ri = ei.z;
-                rk = ek.z;
-                x = wi & wk;
-              }
-              // the chunk's matches spread over the lanes: match p is set bit
-              // k of the word of lane o (prefix sums of the words' popcounts)
-              const int cnt = __popcll(x);
-              const int incl = wave_incl_scan(cnt);
-              const int tot = __builtin_amdgcn_readlane(incl, kWave - 1);
-              for (int mb = 0; mb < tot; mb += kWave) {
-                const int p = mb + lane;
-                int o = 0;
-#pragma unroll
-                for (int step = kWave / 2; step >= 1; step >>= 1)
-                  if (__shfl(incl, o + step - 1) <= p) o += step;
-                o = o < kWave ? o : kWave - 1;
-                const int k = p - (__shfl(incl, o) - __shfl(cnt, o));
-                uint64_t xo = __shfl(x, o);
-                const uint64_t wio = __shfl(wi, o), wko = __shfl(wk, o);
-                const uint32_t rio = __shfl(ri, o), rko = __shfl(rk, o);
-                int64_t tA = -1, tB = -1;
-                if (p < tot) {
-                  // bit position of the k-th set bit of xo (k < popc(xo))
-                  int b = 0;
-#pragma unroll
-                  for (int step = 32; step >= 1; step >>= 1) {
-                    if (__popcll(xo & ((1ull << (b + step)) - 1ull)) <= k) b += step;  // b + step <= 63
-                  }
-                  const uint64_t below = (1ull << b) - 1ull;
-                  tA = la0 + (int64_t)rio + __popcll(wio & below);
-                  tB = a.bt_tile[lb0 + (int64_t)rko + __popcll(wko & below)];
-                }
-                process(tA, tB);
-              }
-            }
-            continue;
-          }
-        }
-        for (int64_t base = s0; base < s1; base += kWave) {
-          const int64_t q = base + lane;
-          int64_t tA = -1, tB = -1;
-          if (q < s1) {
-            const int32_t J = skeys[q];
-            if (use_map) {
-              const uint4 e = hm[J >> 6];  // word and rank in one load
-              const uint64_t wd = (uint64_t)e.x | ((uint64_t)e.y << 32);
-              if ((wd >> (J & 63)) & 1ull) {
-                tA = la0 + (int64_t)e.z + __popcll(wd & ((1ull << (J & 63)) - 1ull));
-                tB = a.bt_tile[q];
-              }
-            } else if (hk >= 0) {
-              const uint4 e = cm[J >> 6];
-              const uint64_t wd = (uint64_t)e.x | ((uint64_t)e.y << 32);
-              if ((wd >> (J & 63)) & 1ull) {
-                tA = q;
-                tB = a.bt_tile[lb0 + (int64_t)e.z + __popcll(wd & ((1ull << (J & 63)) - 1ull))];
-              }
-            } else {
-              const int64_t pos = lower_bound_i32(lkeys, l0, l1, J);
-              if (pos < l1 && lkeys[pos] == J) {
-                tA = a_short ? q : pos;
-                tB = a_short ? a.bt_tile[pos] : a.bt_tile[q];
-              }
-            }
-          }
-          process(tA, tB);
-        }
-      }
-    }
-    if (__popcll(bmask) < kWave) break;
-    R0 += kWave;
-  }
-  for (int off = 1; off < kWave; off <<= 1) total += __shfl_xor(total, off);
-  if (lane == 0 && total) atomicAdd(a.count, (unsigned long long)total);
-}
-
-// Set bits per tile (a group of BS lanes per tile, lane = word).
-template <int BS>
-__global__ __launch_bounds__(256) void k_tile_bitcount(const word_t<BS>* __restrict__ tiles, int64_t T,
-                                                       int32_t* __restrict__ cnt) {
-  constexpr int G = kWave / BS;
-  const int lane = lane_id();
-  const int64_t t = (int64_t)wave_index() * G + lane / BS;
-  int c = t < T ? popcw(tiles[t * BS + lane % BS]) : 0;
-  for (int off = 1; off < BS; off <<= 1) c += __shfl_xor(c, off);
-  if (lane % BS == 0 && t < T) cnt[t] = c;
-}
-
-// Set-bit list of every tile from off[t]: entries row * BS + column, rows in
-// order, columns ascending.
-template <int BS>
-__global__ __launch_bounds__(256) void k_tile_bitlist(const word_t<BS>* __restrict__ tiles, int64_t T,
-                                                      const int32_t* __restrict__ off, uint16_t* __restrict__ list) {
-  constexpr int G = kWave / BS;
-  const int lane = lane_id();
-  const int64_t t = (int64_t)wave_index() * G + lane / BS;
-  const int r = lane % BS;
-  const uint64_t w = t < T ? (uint64_t)tiles[t * BS + r] : 0ull;
-  const int pc = __popcll(w);
-  int before = pc;  // set bits of this tile's rows before r
-  for (int o = 1; o < BS; o <<= 1) {
-    const int v = __shfl_up(before, o, BS);
-    if (r >= o) before += v;
-  }
-  before -= pc;
-  if (t >= T) return;
-  int32_t at = off[t] + before;
-  uint64_t m = w;
-  while (m) {
-    const int p = 63 - __builtin_clzll(m);  // highest set bit: column BS-1-p
-    m &= ~(1ull << p);
-    list[at++] = (uint16_t)(r * BS + (BS - 1 - p));
-  }
-}
-
-// Bitmaps of the heavy rows: block column J of row rows[h] sets bit J of
-// slot h (one workgroup per heavy row, its tiles taken strided).  Each
-// 16-byte map entry holds a 64-bit word (x, y) and, after k_heavy_rank, the
-// set bits of the words before it (z).
-__global__ __launch_bounds__(256) void k_heavy_bits(const int32_t* __restrict__ rowptr,
-                                                    const int32_t* __restrict__ colind,
-                                                    const int32_t* __restrict__ rows, int64_t hwords,
-                                                    uint4* __restrict__ map) {
-  const int32_t I = rows[blockIdx.x];
-  uint4* m = map + (int64_t)blockIdx.x * hwords;
-  for (int64_t t = rowptr[I] + threadIdx.x; t < rowptr[I + 1]; t += blockDim.x) {
-    const int32_t J = colind[t];
-    atomicOr((unsigned long long*)&m[J >> 6], 1ull << (J & 63));
-  }
-}
-
-// hcol[K] = h when B's column K list (bt_row over [bt_ptr[K], bt_ptr[K+1]))
-// equals row K = rows[h] of A, so that slot h's bitmap and ranks also
-// locate J inside B's column K (one workgroup per slot).
-__global__ __launch_bounds__(256) void k_heavy_colcheck(const int32_t* __restrict__ rowptr,
-                                                        const int32_t* __restrict__ colind,
-                                                        const int32_t* __restrict__ bt_ptr,
-                                                        const int32_t* __restrict__ bt_row,
-                                                        const int32_t* __restrict__ rows, int32_t* __restrict__ hcol) {
-  __shared__ int same;
-  const int32_t K = rows[blockIdx.x];
-  const int32_t a0 = rowptr[K], n = rowptr[K + 1] - a0, b0 = bt_ptr[K];
-  if (threadIdx.x == 0) same = (bt_ptr[K + 1] - b0 == n);
-  __syncthreads();
-  if (same) {
-    for (int32_t i = threadIdx.x; i < n; i += blockDim.x)
-      if (colind[a0 + i] != bt_row[b0 + i]) same = 0;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0 && same) hcol[K] = (int32_t)blockIdx.x;
-}
-
-// rank (z) of every word = set bits of the slot's words before it (one
-// workgroup per slot: each thread sums a contiguous run of words, a block
-// scan of the 256 run totals, then the runs are written out).
-__global__ __launch_bounds__(256) void k_heavy_rank(int64_t hwords, uint4* __restrict__ map) {
-  __shared__ int32_t part[256];
-  uint4* m = map + (int64_t)blockIdx.x * hwords;
-  const int64_t per = (hwords + 255) / 256;
-  const int64_t w0 = min((int64_t)threadIdx.x * per, hwords), w1 = min(w0 + per, hwords);
-  int32_t s = 0;
-  for (int64_t w = w0; w < w1; ++w) s += __popc(m[w].x) + __popc(m[w].y);
-  part[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t acc = 0;
-    for (int k = 0; k < 256; ++k) {
-      const int32_t v = part[k];
-      part[k] = acc;
-      acc += v;
-    }
-  }
-  __syncthreads();
-  int32_t acc = part[threadIdx.x];
-  for (int64_t w = w0; w < w1; ++w) {
-    const int32_t c = __popc(m[w].x) + __popc(m[w].y);
-    m[w].z = (uint32_t)acc;
-    acc += c;
-  }
 }
 
 // colsum (rows=false): S[J*BS + c] += #rows of tile (I,J) with column c set.
@@ -573,6 +145,419 @@ static int block_transpose(const gbo_bsr* B, Workspace& mem, int32_t** d_ptr, in
   return GBO_OK;
 }
 
+// ------------------------------------------ triangle counting on lists
+// A_i goes into a set in LDS and the C_k are streamed past it: coalesced reads
+// and one LDS probe per element.  (The form before worked on tiles: for a mask
+// tile it looked the block columns of its row up in the rows of its column and
+// gathered both tiles of every match, a chain of dependent loads for two or
+// three bits: R-MAT 2^18 bs 32 13.0 ms against 2.0.)  Where C_k is much longer
+// than A_i (a hub column under a short row) the elements of A_i are searched in
+// C_k instead, so an edge costs about the shorter list.
+//
+// Rows of at most kTinyRow columns: eight to a wave.  Up to kLightRow: a wave
+// each.  Their sets are hash tables of the wave's own, a quarter full at most.
+// Longer rows: items of kHeavyKeys columns k, a workgroup takes one after
+// another from a counter, the set a bitmap of up to 2^20 ids (more: window by
+// window).  A bitmap probe is a load and a shift, a hash probe a loop, so the
+// line is low: R-MAT 2^18 2.2 / 3.1 / 3.7 ms at 32 / 64 / 128 columns.
+constexpr int kTinyRow = 8;
+constexpr int kTinyRows = kWave / kTinyRow;  // tiny rows per wave
+constexpr int kTinySlots = 32;
+constexpr int kLightRow = 32;
+constexpr int kLightSlots = 128;
+constexpr int kHeavyKeys = 512;
+constexpr int kHeavyThreads = 1024;
+constexpr int64_t kWindow = (int64_t)1 << 20;  // ids of a bitmap: 128 KB of LDS
+
+struct ListTcArgs {
+  const int64_t* arp;   // A_i
+  const int32_t* acol;
+  const int64_t* crp;   // C_k
+  const int32_t* ccol;
+  int32_t nrows;        // rows of A
+  int32_t nids;         // columns of A = rows of B: the ids in the sets
+  const int64_t* hoff;  // heavy items before row i (scan), [nrows + 1]
+  const int2* items;    // heavy items: row, first key
+  unsigned long long* next;  // heavy items taken
+  unsigned long long* count;
+};
+
+// C_k is searched rather than streamed: a search is a chain of log2(dk)
+// loads per 64 elements of A_i, a stream dk / 256 rounds.
+__device__ __forceinline__ bool search_pays(int64_t dk, int64_t di) { return dk > 2048 * ((di + 63) / 64); }
+
+// Elements of A_i (`di` from a) that are in c[0 .. dk), searched 64 at a time.
+__device__ __forceinline__ int64_t count_searched(const int32_t* __restrict__ a, int64_t di,
+                                                  const int32_t* __restrict__ c, int64_t dk) {
+  int64_t hits = 0;
+  for (int64_t e = lane_id(); e < di; e += kWave) {
+    const int32_t v = a[e];
+    int64_t lo = 0, hi = dk;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (c[mid] < v) lo = mid + 1;
+      else hi = mid;
+    }
+    hits += lo < dk && c[lo] == v;
+  }
+  return hits;
+}
+
+// The keys of the wave's lanes (k, where `in`), each of the row of di columns
+// from a0: the elements of their C_k that has(element, lane) holds, this
+// lane's share.  Lists of 64 or more are streamed one after another by the
+// whole wave; the shorter ones are laid end to end, 64 elements a round
+// whatever lists they come from.
+template <class Has>
+__device__ __forceinline__ int64_t count_keys(const ListTcArgs& A, bool in, int32_t k, int64_t a0, int64_t di,
+                                              bool searches, const Has& has) {
+  const int lane = lane_id();
+  const int64_t c0 = in ? A.crp[k] : 0;
+  const int64_t dk = in ? A.crp[k + 1] - c0 : 0;
+  int64_t hits = 0;
+  const bool far = search_pays(dk, di);
+  for (uint64_t m = __ballot(far && searches); m; m &= m - 1) {
+    const int j = __builtin_ctzll(m);
+    hits += count_searched(A.acol + __shfl((long long)a0, j), __shfl((long long)di, j),
+                           A.ccol + __shfl((long long)c0, j), __shfl((long long)dk, j));
+  }
+  for (uint64_t m = __ballot(!far && dk >= kWave); m; m &= m - 1) {
+    const int j = __builtin_ctzll(m);
+    const int32_t* __restrict__ c = A.ccol + __shfl((long long)c0, j);
+    const int d = __shfl((int)dk, j);
+    constexpr int U = 4;
+    for (int e = lane; e < d; e += U * kWave) {
+      int32_t v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = c[min(e + u * kWave, d - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) hits += e + u * kWave < d && has(v[u], j);
+    }
+  }
+  const int w = dk < kWave ? (int)dk : 0;
+  const int incl = wave_incl_scan(w);
+  const int tot = __builtin_amdgcn_readlane(incl, kWave - 1);
+  for (int p0 = 0; p0 < tot; p0 += kWave) {  // wave-uniform
+    const int p = p0 + lane;
+    int j = 0;  // the list of element p: how many lists end at or before p
+#pragma unroll
+    for (int step = kWave / 2; step >= 1; step >>= 1)
+      if (__shfl(incl, j + step - 1) <= p) j += step;
+    j = min(j, kWave - 1);
+    const int e = p - (__shfl(incl, j) - __shfl(w, j));
+    const int64_t b = __shfl((long long)c0, j);
+    if (p < tot) hits += has(A.ccol[b + e], j);
+  }
+  return hits;
+}
+
+// One atomic per workgroup: thousands of waves queue on the address.
+__device__ __forceinline__ void add_count(int64_t hits, unsigned long long* count) {
+  __shared__ unsigned long long s_hits;
+  if (threadIdx.x == 0) s_hits = 0;
+  __syncthreads();
+  for (int off = 1; off < kWave; off <<= 1) hits += __shfl_xor(hits, off);
+  if (lane_id() == 0 && hits) atomicAdd(&s_hits, (unsigned long long)hits);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_hits) atomicAdd(count, s_hits);
+}
+
+// Open addressing in N slots (a power of two), -1 = free; ids are not
+// negative and at most a quarter of the slots are taken, so the loops end.
+template <int N>
+struct HashSet {
+  static __device__ __forceinline__ uint32_t slot(int32_t v) {
+    return (uint32_t)v * 2654435761u >> (32 - __builtin_ctz(N));
+  }
+  static __device__ __forceinline__ void insert(int32_t* t, int32_t v) {
+    for (uint32_t s = slot(v);; s = (s + 1) % N) {
+      const int32_t was = atomicCAS(&t[s], -1, v);
+      if (was == -1 || was == v) return;
+    }
+  }
+  static __device__ __forceinline__ int has(const int32_t* t, int32_t v) {
+    for (uint32_t s = slot(v);; s = (s + 1) % N) {
+      const int32_t x = t[s];
+      if (x == v) return 1;
+      if (x < 0) return 0;
+    }
+  }
+};
+
+// A wave takes kTinyRows rows at a time: lane l looks at row l / kTinyRow.
+__global__ __launch_bounds__(256) void k_tc_light(const ListTcArgs A) {
+  constexpr int kSlots = kTinyRows * kTinySlots;
+  static_assert(kSlots >= kLightSlots, "the tiny rows' tables hold a light row's");
+  __shared__ int32_t tables[256 / kWave][kSlots];
+  int32_t* __restrict__ table = tables[threadIdx.x / kWave];
+  const int lane = lane_id(), g = lane / kTinyRow, e = lane % kTinyRow;
+  const int64_t nw = (int64_t)gridDim.x * (256 / kWave);
+  const int64_t groups = ((int64_t)A.nrows + kTinyRows - 1) / kTinyRows;
+  int64_t hits = 0;
+  for (int64_t w = wave_index(); w < groups; w += nw) {  // wave-uniform
+    const int64_t i = w * kTinyRows + g;
+    const int64_t a0 = i < A.nrows ? A.arp[i] : 0;
+    const int64_t d = i < A.nrows ? A.arp[i + 1] - a0 : 0;
+    const bool tiny = d > 0 && d <= kTinyRow;
+    if (__ballot(tiny)) {
+      const bool in = tiny && e < d;
+      const int32_t k = in ? A.acol[a0 + e] : -1;
+      for (int s = lane; s < kSlots; s += kWave) table[s] = -1;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      if (in) HashSet<kTinySlots>::insert(table + g * kTinySlots, k);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      hits += count_keys(A, in, k, a0, d, true, [&](int32_t v, int j) {
+        return HashSet<kTinySlots>::has(table + j / kTinyRow * kTinySlots, v);
+      });
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+    for (uint64_t m = __ballot(e == 0 && d > kTinyRow && d <= kLightRow); m; m &= m - 1) {
+      const int j = __builtin_ctzll(m);
+      const int64_t b0 = __shfl((long long)a0, j);
+      const int db = __shfl((int)d, j);
+      const int32_t k = lane < db ? A.acol[b0 + lane] : -1;
+      for (int s = lane; s < kLightSlots; s += kWave) table[s] = -1;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      if (lane < db) HashSet<kLightSlots>::insert(table, k);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      hits += count_keys(A, lane < db, k, b0, db, true,
+                         [&](int32_t v, int) { return HashSet<kLightSlots>::has(table, v); });
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+  }
+  add_count(hits, A.count);
+}
+
+__global__ __launch_bounds__(256) void k_tc_items_count(const int64_t* __restrict__ arp, int32_t n,
+                                                        int32_t* __restrict__ cnt) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t d = arp[i + 1] - arp[i];
+  cnt[i] = d > kLightRow ? (int32_t)((d + kHeavyKeys - 1) / kHeavyKeys) : 0;
+}
+
+__global__ __launch_bounds__(256) void k_tc_items_fill(const int64_t* __restrict__ hoff, int32_t n,
+                                                       int2* __restrict__ items) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int64_t k = hoff[i]; k < hoff[i + 1]; ++k) items[k] = make_int2((int)i, (int)(k - hoff[i]) * kHeavyKeys);
+}
+
+// `bits`: LDS, a bit per id of a window.
+__global__ __launch_bounds__(kHeavyThreads) void k_tc_heavy(const ListTcArgs A) {
+  extern __shared__ uint32_t bits[];
+  __shared__ unsigned long long s_item;
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int64_t total = A.hoff[A.nrows];
+  const int window = (int)min(kWindow, (int64_t)A.nids);
+  for (int s = tid; s < (window + 31) / 32; s += nt) bits[s] = 0;
+  int64_t hits = 0;
+  while (true) {
+    __syncthreads();
+    if (tid == 0) s_item = atomicAdd(A.next, 1ull);
+    __syncthreads();
+    const int64_t it = (int64_t)s_item;
+    if (it >= total) break;  // each workgroup ends here: the counter only grows
+    const int32_t i = A.items[it].x;
+    const int64_t a0 = A.arp[i], d = A.arp[i + 1] - a0;
+    const int32_t* __restrict__ ai = A.acol + a0;
+    const int64_t k0 = A.items[it].y, k1 = min(k0 + kHeavyKeys, d);
+    for (int64_t base = 0; base < A.nids; base += window) {
+      for (int64_t e = tid; e < d; e += nt) {
+        const uint32_t v = (uint32_t)((int64_t)ai[e] - base);
+        if (v < (uint32_t)window) atomicOr(&bits[v >> 5], 1u << (v & 31));
+      }
+      __syncthreads();
+      auto has = [&](int32_t id, int) -> int {
+        const uint32_t v = (uint32_t)((int64_t)id - base);
+        return v < (uint32_t)window ? (bits[v >> 5] >> (v & 31)) & 1u : 0;
+      };
+      // 16 keys per wave and turn, so that the waves of a workgroup share the
+      // keys of a short item
+      constexpr int KW = 16;
+      for (int64_t k = k0 + (tid / kWave) * KW; k < k1; k += (nt / kWave) * KW) {
+        const int64_t kk = k + lane_id();
+        const bool in = lane_id() < KW && kk < k1;
+        hits += count_keys(A, in, in ? ai[kk] : 0, a0, d, base == 0, has);
+      }
+      __syncthreads();
+      for (int64_t e = tid; e < d; e += nt) {
+        const uint32_t v = (uint32_t)((int64_t)ai[e] - base);
+        if (v < (uint32_t)window) bits[v >> 5] = 0;
+      }
+      __syncthreads();
+    }
+  }
+  add_count(hits, A.count);
+}
+
+// ------------------------------------------- triangle counting on tiles
+// Dense tiles: row i of A as a vector of bs-bit words in LDS (word J = row i of
+// tile (I,J)), against which the words of B's block column K are counted for
+// every mask tile (I,K) that has bits in row i: lane r holds column k = r of
+// the 64 / bs tiles of a step, one AND and popcount per bs ids.  At bs 8 the
+// vector holds the whole tiles of block row I, and one 64-bit AND and popcount
+// takes a column word against the rows of the mask's column.  A workgroup takes
+// one row (block row) after another from a counter; a matrix wider than the
+// vector window by window.
+struct TileTcArgs {
+  const int32_t *a_rowptr, *a_colind;
+  const void* a_tiles;
+  const int32_t *bt_ptr, *bt_row, *bt_tile;  // block columns of B: rows J, tiles
+  const void* b_tiles;
+  int32_t nrows, nblocks;  // rows (bs 8: block rows); block columns of A = block rows of B
+  unsigned long long *next, *count;
+};
+
+template <int BS>
+__global__ __launch_bounds__(kHeavyThreads) void k_tc_tiles(const TileTcArgs A) {
+  using W = word_t<BS>;
+  using X = typename std::conditional<BS == 8, uint64_t, W>::type;  // an element of the vector
+  constexpr int G = kWave / BS;
+  extern __shared__ uint64_t xs64[];
+  X* __restrict__ xs = (X*)xs64;
+  __shared__ unsigned long long s_row;
+  const int tid = threadIdx.x, nt = blockDim.x, lane = lane_id(), g = lane / BS, r = lane % BS;
+  const W* __restrict__ at = (const W*)A.a_tiles;
+  const W* __restrict__ bt = (const W*)A.b_tiles;
+  const int window = (int)min(kWindow / (8 * (int64_t)sizeof(X)), (int64_t)A.nblocks);
+  for (int s = tid; s < window; s += nt) xs[s] = (X)0;
+  int64_t hits = 0;
+  while (true) {
+    __syncthreads();
+    if (tid == 0) s_row = atomicAdd(A.next, 1ull);
+    __syncthreads();
+    // the last rows first: those of a lower triangle are the longest
+    const int64_t i = A.nrows - 1 - (int64_t)s_row;
+    if (i < 0) break;  // each workgroup ends here: the counter only grows
+    const int64_t I = BS == 8 ? i : i / BS;
+    const int64_t t0 = A.a_rowptr[I], t1 = A.a_rowptr[I + 1];
+    auto own = [&](int64_t t) -> X {  // row i of tile t; bs 8: the tile
+      if constexpr (BS == 8) {
+        uint64_t w;
+        __builtin_memcpy(&w, at + t * 8, 8);
+        return w;
+      } else {
+        return at[t * BS + i % BS];
+      }
+    };
+    for (int64_t base = 0; base < A.nblocks; base += window) {
+      for (int64_t t = t0 + tid; t < t1; t += nt) {
+        const int64_t J = A.a_colind[t] - base;
+        if (J >= 0 && J < window) xs[J] = own(t);
+      }
+      __syncthreads();
+      for (int64_t t = t0 + tid / kWave; t < t1; t += nt / kWave) {  // wave-uniform
+        uint64_t m = (uint64_t)own(t);
+        if constexpr (BS == 8) {
+          // the bytes of the rows that have column r
+          m = ((m >> (7 - r)) & 0x0101010101010101ull) * 0xFFull;
+        } else {
+          if (m == 0) continue;
+          m = (m >> (BS - 1 - r)) & 1ull;
+        }
+        const int32_t K = A.a_colind[t];
+        const int64_t e1 = A.bt_ptr[K + 1];
+        int acc = 0;
+#pragma unroll 4
+        for (int64_t e = A.bt_ptr[K] + g; e < e1; e += G) {
+          const int64_t J = A.bt_row[e] - base;
+          if (J >= 0 && J < window) {
+            const W w = bt[(int64_t)A.bt_tile[e] * BS + r];
+            if constexpr (BS == 8) acc += __popcll(xs[J] & (w * 0x0101010101010101ull) & m);
+            else acc += popcw((W)(w & xs[J]));
+          }
+        }
+        if (m) hits += acc;
+      }
+      __syncthreads();
+      for (int64_t t = t0 + tid; t < t1; t += nt) {
+        const int64_t J = A.a_colind[t] - base;
+        if (J >= 0 && J < window) xs[J] = (X)0;
+      }
+      __syncthreads();
+    }
+  }
+  add_count(hits, A.count);
+}
+
+// Workgroups and threads of a kernel whose workgroups hold `lds` bytes each:
+// as many as fit a CU's 160 KB of LDS and 32 waves (`wide`: of 16 waves each).
+static void lds_grid(size_t lds, bool wide, int* threads, int* blocks) {
+  *threads = wide || lds > ((size_t)40 << 10) ? kHeavyThreads : 256;
+  *blocks = 256 * std::max(1, (int)std::min<size_t>(2048 / *threads, ((size_t)158 << 10) / (lds + 1024)));
+}
+
+// The list form: A's rows are in `a`, B's block lists by column in `cl`.
+static int tc_lists(const gbo_bsr* A, const CsrList& a, const TileLists& cl, unsigned long long* count,
+                    Workspace& mem, hipStream_t st) {
+  const char* who = "gbo_bsrbmm_tc";
+  const int32_t n = A->nrows;
+  CsrList c;
+  int rc = expand_lists(cl, mem, &c, st);
+  if (rc) return rc;
+  int32_t* cnt = nullptr;
+  int64_t* hoff = nullptr;
+  int2* items = nullptr;
+  unsigned long long* next = nullptr;
+  // an item has at least kLightRow + 1 nonzeros of a row or kHeavyKeys of one
+  const int64_t cap = a.nnz / (kLightRow + 1) + a.nnz / kHeavyKeys + 1;
+  if ((rc = mem.alloc(&cnt, sizeof(int32_t) * (size_t)n, who)) ||
+      (rc = mem.alloc(&hoff, sizeof(int64_t) * ((size_t)n + 1), who)) ||
+      (rc = mem.alloc(&items, sizeof(int2) * (size_t)cap, who)) || (rc = mem.alloc(&next, sizeof(*next), who)))
+    return rc;
+  const unsigned nb = (unsigned)(((int64_t)n + 255) / 256);
+  k_tc_items_count<<<nb, 256, 0, st>>>(a.rowptr, n, cnt);
+  GBO_LAUNCH_CHECK();
+  if ((rc = scan_exclusive<int32_t, int64_t>(cnt, hoff, n, st, mem))) return rc;
+  k_tc_items_fill<<<nb, 256, 0, st>>>(hoff, n, items);
+  GBO_HIP_CHECK(hipMemsetAsync(next, 0, sizeof(*next), st));
+  ListTcArgs t{};
+  t.arp = a.rowptr;
+  t.acol = a.col;
+  t.crp = c.rowptr;
+  t.ccol = c.col;
+  t.nrows = n;
+  t.nids = A->ncols;
+  t.hoff = hoff;
+  t.items = items;
+  t.next = next;
+  t.count = count;
+  const size_t lds = (size_t)(std::min<int64_t>(kWindow, A->ncols) + 31) / 32 * 4;
+  int threads = 0, blocks = 0;
+  lds_grid(lds, false, &threads, &blocks);
+  GBO_HIP_CHECK(hipFuncSetAttribute((const void*)k_tc_heavy, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  k_tc_heavy<<<blocks, threads, lds, st>>>(t);
+  GBO_LAUNCH_CHECK();
+  k_tc_light<<<(unsigned)std::min<int64_t>(2048, ((int64_t)n + 4 * kTinyRows - 1) / (4 * kTinyRows)), 256, 0, st>>>(t);
+  GBO_LAUNCH_CHECK();
+  return GBO_OK;
+}
+
+template <int BS>
+static int tc_tiles(const TileTcArgs& t, hipStream_t st) {
+  constexpr size_t X = BS == 8 ? 8 : BS / 8;  // bytes of an element of the vector
+  const size_t lds = ((size_t)std::min<int64_t>(kWindow / 8 / (int64_t)X, t.nblocks) * X + 7) / 8 * 8;
+  int threads = 0, blocks = 0;
+  lds_grid(lds, t.nrows < 2048, &threads, &blocks);  // few rows: more waves on each
+  GBO_HIP_CHECK(hipFuncSetAttribute((const void*)k_tc_tiles<BS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  k_tc_tiles<BS><<<blocks, threads, lds, st>>>(t);
+  GBO_LAUNCH_CHECK();
+  return GBO_OK;
+}
+
+// Whether the tiles are dense enough for the word form.  The lists' work falls
+// with the third power of the density, the words' hardly: G(4096, p), lists /
+// words: bs 8 p 0.1 (6 bits a tile) 496 / 648 us, 0.2 (13) 723 / 647; bs 16 0.2
+// (51) 693 / 861, 0.3 (77) 1049 / 858; bs 32 0.1 (102) 480 / 528, 0.2 (203) 708
+// / 551; bs 64 0.05 (202) 373 / 395, 0.1 (403) 514 / 427; p 1 6.1-7.2 ms / 0.8-
+// 1.3 (the tile-pair form before 1.6-6.1).  King grids, 0.8 bits a tile row,
+// belong to the lists.
+static bool tc_dense(int bs, int64_t nnz, int64_t tiles) {
+  const int64_t bits = bs == 8 ? 12 : bs == 16 ? 64 : bs == 32 ? 128 : 320;
+  return nnz > bits * tiles;
+}
+
 extern "C" {
 
 int gbo_bsrbmm_tc(const gbo_bsr* L, const gbo_bsr* LT, uint64_t* d_count, gbo_stream_t stream) {
@@ -591,150 +576,42 @@ int gbo_bsrbmm_tc(const gbo_bsr* L, const gbo_bsr* LT, uint64_t* d_count, gbo_st
   if (L->nblocks == 0 || LT->nblocks == 0) return GBO_OK;
   Workspace mem(st);
   int32_t *bt_ptr = nullptr, *bt_row = nullptr, *bt_tile = nullptr;
-  if ((rc = block_transpose(LT, mem, &bt_ptr, &bt_row, &bt_tile, st))) return rc;
-  // B's tiles in row form (same positions), for one popcount per set bit of A
-  void* rows = nullptr;
-  const size_t tbytes = (size_t)LT->nblocks * LT->bs * LT->bs / 8;
-  if ((rc = mem.alloc(&rows, std::max<size_t>(tbytes, 8), "gbo_bsrbmm_tc"))) return rc;
-  {
-    const int64_t waves = (LT->nblocks * LT->bs + kWave - 1) / kWave;
-    const unsigned tb = (unsigned)((waves + 3) / 4);
-    switch (LT->bs) {
-      case 8: k_tile_rows<8><<<tb, 256, 0, st>>>((const uint8_t*)LT->tiles, LT->nblocks, (uint8_t*)rows); break;
-      case 16: k_tile_rows<16><<<tb, 256, 0, st>>>((const uint16_t*)LT->tiles, LT->nblocks, (uint16_t*)rows); break;
-      case 32: k_tile_rows<32><<<tb, 256, 0, st>>>((const uint32_t*)LT->tiles, LT->nblocks, (uint32_t*)rows); break;
-      case 64: k_tile_rows<64><<<tb, 256, 0, st>>>((const uint64_t*)LT->tiles, LT->nblocks, (uint64_t*)rows); break;
+  unsigned long long* count = (unsigned long long*)d_count;
+  CsrList a;
+  if ((rc = block_transpose(LT, mem, &bt_ptr, &bt_row, &bt_tile, st)) || (rc = expand_csr(L, mem, &a, st))) return rc;
+  if (tc_dense(L->bs, a.nnz, L->nblocks)) {
+    TileTcArgs t{};
+    t.a_rowptr = L->rowptr;
+    t.a_colind = L->colind;
+    t.a_tiles = L->tiles;
+    t.bt_ptr = bt_ptr;
+    t.bt_row = bt_row;
+    t.bt_tile = bt_tile;
+    t.b_tiles = LT->tiles;
+    t.nrows = L->bs == 8 ? L->nblockrows : L->nrows;
+    t.nblocks = L->nblockcols;
+    t.count = count;
+    if ((rc = mem.alloc(&t.next, sizeof(*t.next), "gbo_bsrbmm_tc"))) return rc;
+    GBO_HIP_CHECK(hipMemsetAsync(t.next, 0, sizeof(*t.next), st));
+    switch (L->bs) {
+      case 8: rc = tc_tiles<8>(t, st); break;
+      case 16: rc = tc_tiles<16>(t, st); break;
+      case 32: rc = tc_tiles<32>(t, st); break;
+      case 64: rc = tc_tiles<64>(t, st); break;
     }
-    GBO_LAUNCH_CHECK();
+  } else {
+    TileLists cl;
+    cl.bs = LT->bs;
+    cl.nbr = LT->nblockcols;
+    cl.n = LT->ncols;
+    cl.T = LT->nblocks;
+    cl.ptr = bt_ptr;
+    cl.ind = bt_row;
+    cl.tiles = LT->tiles;
+    cl.perm = bt_tile;
+    rc = tc_lists(L, a, cl, count, mem, st);
   }
-  TcArgs a{};
-  a.a_rowptr = L->rowptr;
-  a.a_colind = L->colind;
-  a.a_tiles = L->tiles;
-  a.nbr = L->nblockrows;
-  a.T = L->nblocks;
-  a.bt_ptr = bt_ptr;
-  a.bt_row = bt_row;
-  a.bt_tile = bt_tile;
-  a.b_tiles = rows;
-  a.count = (unsigned long long*)d_count;
-  a.vec16 = (((uintptr_t)L->tiles) & 15) == 0;
-  // bs 32/64: set bits per A tile and their scan; the total is read at the
-  // synchronization below, and the bit lists are built when the tiles are
-  // sparse (at most 8 set bits per tile on average)
-  int32_t* aoff = nullptr;
-  int32_t nbits = 0;
-  // copies into host memory (nbits, hrp) are waited for on every return
-  // until the explicit synchronization below
-  struct SyncOnExit {
-    hipStream_t st;
-    bool armed = false;
-    ~SyncOnExit() {
-      if (armed) (void)hipStreamSynchronize(st);
-    }
-  } pending{st};
-  std::vector<int32_t> hrp((size_t)L->nblockrows + 1);
-  if (L->bs >= 32) {
-    const int64_t T = L->nblocks;
-    if ((rc = mem.alloc(&aoff, sizeof(int32_t) * ((size_t)T + 1), "gbo_bsrbmm_tc"))) return rc;
-    const int64_t waves = (T * L->bs + kWave - 1) / kWave;
-    const unsigned gb = (unsigned)((waves + 3) / 4);
-    if (L->bs == 32) k_tile_bitcount<32><<<gb, 256, 0, st>>>((const uint32_t*)L->tiles, T, aoff);
-    else k_tile_bitcount<64><<<gb, 256, 0, st>>>((const uint64_t*)L->tiles, T, aoff);
-    GBO_LAUNCH_CHECK();
-    if ((rc = scan_exclusive<int32_t, int32_t>(aoff, aoff, T, st, mem))) return rc;
-    pending.armed = true;
-    GBO_HIP_CHECK(hipMemcpyAsync(&nbits, aoff + T, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  }
-  // heavy rows (more than kHeavyTiles tiles) get a block-column bitmap, the
-  // largest rows first, within a budget of device memory
-  {
-    constexpr int32_t kHeavyTiles = 64;
-    constexpr int64_t kHeavyBudget = (int64_t)1 << 30;
-    const int32_t nbr = L->nblockrows;
-    const int64_t hwords = ((int64_t)L->nblockcols + 63) / 64;
-    pending.armed = true;
-    GBO_HIP_CHECK(hipMemcpyAsync(hrp.data(), L->rowptr, sizeof(int32_t) * hrp.size(), hipMemcpyDeviceToHost, st));
-    GBO_HIP_CHECK(hipStreamSynchronize(st));
-    pending.armed = false;
-    if (aoff && (double)nbits <= 8.0 * (double)L->nblocks) {
-      const int64_t T = L->nblocks;
-      uint16_t* abits = nullptr;
-      if ((rc = mem.alloc(&abits, sizeof(uint16_t) * (size_t)std::max<int32_t>(nbits, 1), "gbo_bsrbmm_tc")))
-        return rc;
-      const int64_t waves = (T * L->bs + kWave - 1) / kWave;
-      const unsigned gb = (unsigned)((waves + 3) / 4);
-      if (L->bs == 32) k_tile_bitlist<32><<<gb, 256, 0, st>>>((const uint32_t*)L->tiles, T, aoff, abits);
-      else k_tile_bitlist<64><<<gb, 256, 0, st>>>((const uint64_t*)L->tiles, T, aoff, abits);
-      GBO_LAUNCH_CHECK();
-      a.aoff = aoff;
-      a.abits = abits;
-    }
-    std::vector<int32_t> heavy;
-    for (int32_t I = 0; I < nbr; ++I)
-      if (hrp[(size_t)I + 1] - hrp[(size_t)I] > kHeavyTiles) heavy.push_back(I);
-    std::sort(heavy.begin(), heavy.end(), [&](int32_t x, int32_t y) {
-      return hrp[(size_t)x + 1] - hrp[(size_t)x] > hrp[(size_t)y + 1] - hrp[(size_t)y];
-    });
-    const int64_t per_row = hwords * (int64_t)sizeof(uint4);
-    const size_t nh = (size_t)std::min<int64_t>((int64_t)heavy.size(), kHeavyBudget / std::max<int64_t>(per_row, 1));
-    heavy.resize(nh);
-    if (nh > 0) {
-      std::vector<int32_t> slot((size_t)nbr, -1);
-      for (size_t h = 0; h < nh; ++h) slot[(size_t)heavy[h]] = (int32_t)h;
-      SyncOnExit sources{st};  // slot and heavy are sources of the copies below
-      int32_t *d_slot = nullptr, *d_rows = nullptr;
-      uint4* d_map = nullptr;
-      if ((rc = mem.alloc(&d_slot, sizeof(int32_t) * (size_t)nbr, "gbo_bsrbmm_tc")) ||
-          (rc = mem.alloc(&d_rows, sizeof(int32_t) * nh, "gbo_bsrbmm_tc")) ||
-          (rc = mem.alloc(&d_map, sizeof(uint4) * nh * (size_t)hwords, "gbo_bsrbmm_tc")))
-        return rc;
-      sources.armed = true;
-      GBO_HIP_CHECK(hipMemcpyAsync(d_slot, slot.data(), sizeof(int32_t) * (size_t)nbr, hipMemcpyHostToDevice, st));
-      GBO_HIP_CHECK(hipMemcpyAsync(d_rows, heavy.data(), sizeof(int32_t) * nh, hipMemcpyHostToDevice, st));
-      GBO_HIP_CHECK(hipMemsetAsync(d_map, 0, sizeof(uint4) * nh * (size_t)hwords, st));
-      k_heavy_bits<<<(unsigned)nh, 256, 0, st>>>(L->rowptr, L->colind, d_rows, hwords, d_map);
-      GBO_LAUNCH_CHECK();
-      k_heavy_rank<<<(unsigned)nh, 256, 0, st>>>(hwords, d_map);
-      GBO_LAUNCH_CHECK();
-      // L is square, so block column K of B = L^T is block row K of L: the
-      // row bitmaps serve B's heavy columns once the lists are checked equal
-      int32_t* d_hcol = nullptr;
-      if ((rc = mem.alloc(&d_hcol, sizeof(int32_t) * (size_t)nbr, "gbo_bsrbmm_tc"))) return rc;
-      GBO_HIP_CHECK(hipMemsetAsync(d_hcol, 0xFF, sizeof(int32_t) * (size_t)nbr, st));
-      k_heavy_colcheck<<<(unsigned)nh, 256, 0, st>>>(L->rowptr, L->colind, bt_ptr, bt_row, d_rows, d_hcol);
-      GBO_LAUNCH_CHECK();
-      a.hcol = d_hcol;
-      // the host vectors above are sources of asynchronous copies
-      GBO_HIP_CHECK(hipStreamSynchronize(st));
-      sources.armed = false;
-      a.hslot = d_slot;
-      a.hmap = d_map;
-      a.hwords = hwords;
-    }
-  }
-  // TC work per mask tile is far larger than a bsrbmv tile: small chunks
-  // (a plan without the bsrbmv scratch), made last so that no early return
-  // above leaves it allocated
-  gbo_bsr tmp = *L;
-  tmp.plan = nullptr;
-  tmp.plan_chunk = 0;
-  if ((rc = plan_create(&tmp, 16, 0, false, st))) return rc;
-  a.plan = tmp.plan;
-  a.chunk = tmp.plan_chunk;
-  a.nchunks = tmp.plan_nchunks;
-  const unsigned blocks = (unsigned)(((int64_t)a.nchunks + 3) / 4);
-  switch (L->bs) {
-    case 8: k_tc<8><<<blocks, 256, 0, st>>>(a); break;
-    case 16: k_tc<16><<<blocks, 256, 0, st>>>(a); break;
-    case 32: k_tc<32><<<blocks, 256, 0, st>>>(a); break;
-    case 64: k_tc<64><<<blocks, 256, 0, st>>>(a); break;
-  }
-  if (hipGetLastError() != hipSuccess) rc = set_error(GBO_EDEVICE, "k_tc launch failed");
-  // the plan is a plain allocation: wait for the kernel before freeing it
-  (void)hipStreamSynchronize(st);
-  gbo_bsr_plan_free(&tmp);
-  return rc;
+  return rc;  // the scratch waits for the stream
   GBO_TRY_END
 }
 

@@ -40,6 +40,7 @@ struct ItemArgs {
   const int32_t* rowptr;
   const void* tiles;
   const int32_t* colind;
+  const int32_t* perm;     // nullable: where tile t lies in `tiles`
   const int64_t* itemptr;  // [nbr + 1]
   const int32_t* itemrow;  // [items]
   int32_t nbr;
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(256) void k_item_bits(const ItemArgs a) {
   const word_t<BS>* __restrict__ tiles = (const word_t<BS>*)a.tiles;
   int c = 0;
 #pragma unroll 8
-  for (int64_t t = t0 + g; t < t1; t += G) c += popcw(tiles[t * BS + r]);
+  for (int64_t t = t0 + g; t < t1; t += G) c += popcw(tiles[(a.perm ? (int64_t)a.perm[t] : t) * BS + r]);
   for (int off = BS; off < kWave; off <<= 1) c += __shfl_xor(c, off);
   if (g == 0) a.cnt[item_slot<BS>(i0, m, r, k)] = c;
 }
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256) void k_item_fill(const ItemArgs a) {
     for (int u = 0; u < U; ++u) {
       const int64_t t = b + u * G + g;
       const int64_t tc = t < t1 ? t : t0;
-      const uint64_t wv = (uint64_t)tiles[tc * BS + r];
+      const uint64_t wv = (uint64_t)tiles[(a.perm ? (int64_t)a.perm[tc] : tc) * BS + r];
       c[u] = a.colind[tc];
       w[u] = t < t1 ? wv : 0ull;
     }
@@ -136,9 +137,9 @@ unsigned grid_of(int64_t items, int per_block) {
 }
 
 template <int BS>
-int expand_t(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
-  const int32_t nbr = A->nblockrows, n = A->nrows;
-  const int64_t cap = (int64_t)nbr + A->nblocks / kItem<BS> + 1;  // items
+int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
+  const int32_t nbr = A.nbr, n = A.n;
+  const int64_t cap = (int64_t)nbr + A.T / kItem<BS> + 1;  // items
   int32_t *icnt = nullptr, *itemrow = nullptr, *cnt = nullptr;
   int64_t *itemptr = nullptr, *pos = nullptr, *rowptr = nullptr;
   const char* who = "expand";
@@ -150,14 +151,15 @@ int expand_t(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
       (rc = mem.alloc(&pos, sizeof(int64_t) * ((size_t)cap * BS + 1), who)) ||
       (rc = mem.alloc(&rowptr, sizeof(int64_t) * ((size_t)n + 1), who)))
     return rc;
-  k_item_count<<<grid_of(nbr, 256), 256, 0, st>>>(A->rowptr, nbr, kItem<BS>, icnt);
+  k_item_count<<<grid_of(nbr, 256), 256, 0, st>>>(A.ptr, nbr, kItem<BS>, icnt);
   GBO_LAUNCH_CHECK();
   if ((rc = scan_exclusive<int32_t, int64_t>(icnt, itemptr, nbr, st, mem))) return rc;
   k_item_rows<<<grid_of(nbr, 256), 256, 0, st>>>(itemptr, nbr, itemrow);
   ItemArgs a{};
-  a.rowptr = A->rowptr;
-  a.tiles = A->tiles;
-  a.colind = A->colind;
+  a.rowptr = A.ptr;
+  a.tiles = A.tiles;
+  a.colind = A.ind;
+  a.perm = A.perm;
   a.itemptr = itemptr;
   a.itemrow = itemrow;
   a.nbr = nbr;
@@ -185,14 +187,26 @@ int expand_t(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
 
 }  // namespace
 
-int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
-  switch (A->bs) {
+int expand_lists(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
+  switch (A.bs) {
     case 8: return expand_t<8>(A, mem, out, st);
     case 16: return expand_t<16>(A, mem, out, st);
     case 32: return expand_t<32>(A, mem, out, st);
     case 64: return expand_t<64>(A, mem, out, st);
   }
-  return set_error(GBO_EUNSUPPORTED, "block size %d not supported", A->bs);
+  return set_error(GBO_EUNSUPPORTED, "block size %d not supported", A.bs);
+}
+
+int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
+  TileLists l;
+  l.bs = A->bs;
+  l.nbr = A->nblockrows;
+  l.n = A->nrows;
+  l.T = A->nblocks;
+  l.ptr = A->rowptr;
+  l.ind = A->colind;
+  l.tiles = A->tiles;
+  return expand_lists(l, mem, out, st);
 }
 
 }  // namespace gbo

@@ -30,7 +30,7 @@ namespace gbo {
 struct PlanLayout {
   size_t start = 0, tail = 0, slots = 0, count = 0, partial = 0, bfs_counts = 0, bytes = 0;
 };
-PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr, bool scratch);
+PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr);
 
 struct PlanView {
   const int32_t* plan = nullptr;
@@ -50,10 +50,9 @@ struct PlanView {
 int default_chunk(int bs, int64_t tiles);
 int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st);
 int release_plan(PlanView* pv, hipStream_t st);
-// Allocates A->plan (chunk tiles per chunk, 0 = the library's own plan); with
-// `scratch` the allocation also holds the scratch parts above.  The library's
-// own plan reads the tiles once and synchronizes the stream.
-int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, hipStream_t st);
+// Allocates A->plan with its scratch (chunk tiles per chunk, 0 = the library's
+// own plan, which reads the tiles once and synchronizes the stream).
+int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st);
 
 // A plan acquired for the length of one call, released on every return path.
 struct PlanGuard {
@@ -139,6 +138,17 @@ struct CsrList {
   int64_t nnz = 0;
 };
 int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st);
+// The same for any block lists: list R (of nbr) holds the blocks ind[t], t in
+// [ptr[R], ptr[R+1]); word k of tile t (or perm[t]) holds list R * bs + k's
+// bits in block ind[t], top bit first.
+struct TileLists {
+  int32_t bs = 0, nbr = 0, n = 0;  // n: lists of words (at most nbr * bs)
+  int64_t T = 0;
+  const int32_t *ptr = nullptr, *ind = nullptr;
+  const void* tiles = nullptr;
+  const int32_t* perm = nullptr;
+};
+int expand_lists(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st);
 
 template <class TI, class TO>
 int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st);

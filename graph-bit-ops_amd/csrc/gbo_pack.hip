@@ -579,30 +579,28 @@ static int make_pieces(int bs, const int32_t* d_rp, const int32_t* d_ci, int32_t
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr, bool scratch) {
+PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr) {
   PlanLayout L;
   size_t off = align256(sizeof(int32_t) * (size_t)nchunks);
   L.start = off;
   off += align256(sizeof(int64_t) * ((size_t)nchunks + 1));
   L.tail = off;
   off += align256(sizeof(int32_t) * (size_t)nchunks);
-  if (scratch) {
-    L.slots = off;
-    off += align256(sizeof(unsigned long long) * kCountSlots);
-    L.count = off;
-    off += 256;
-    L.partial = off;
-    off += align256(sizeof(double) * 2 * (size_t)nchunks * bs);
-    L.bfs_counts = off;
-    off += align256(sizeof(int32_t) * (size_t)bs * ((size_t)nbr + 1));
-  }
+  L.slots = off;
+  off += align256(sizeof(unsigned long long) * kCountSlots);
+  L.count = off;
+  off += 256;
+  L.partial = off;
+  off += align256(sizeof(double) * 2 * (size_t)nchunks * bs);
+  L.bfs_counts = off;
+  off += align256(sizeof(int32_t) * (size_t)bs * ((size_t)nbr + 1));
   L.bytes = off;
   return L;
 }
 
 // Points the view's scratch pointers into a plan allocation made with scratch.
 static void view_scratch(PlanView* pv, int bs, int32_t nbr, bool even) {
-  const PlanLayout L = plan_layout(bs, pv->nchunks, nbr, true);
+  const PlanLayout L = plan_layout(bs, pv->nchunks, nbr);
   char* base = (char*)const_cast<int32_t*>(pv->plan);
   if (!even) pv->start = (const int64_t*)(base + L.start);
   pv->tail = (const int32_t*)(base + L.tail);
@@ -613,20 +611,17 @@ static void view_scratch(PlanView* pv, int bs, int32_t nbr, bool even) {
 }
 
 // Plan entries (of the chunks whose starts are in place, or of even chunks of
-// `chunk` tiles) plus (optionally) zeroed count slots in one allocation.
-static int plan_fill(const gbo_bsr* A, int32_t chunk, bool even, int64_t nch, bool scratch, int32_t* plan,
-                     hipStream_t st) {
-  const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, scratch);
+// `chunk` tiles) and zeroed count slots.
+static int plan_fill(const gbo_bsr* A, int32_t chunk, bool even, int64_t nch, int32_t* plan, hipStream_t st) {
+  const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
   int64_t* start = (int64_t*)((char*)plan + L.start);
   if (even) k_even_starts<<<(unsigned)((nch + 256) / 256), 256, 0, st>>>(A->nblocks, chunk, (int32_t)nch, start);
   k_plan<<<(unsigned)((nch + 255) / 256), 256, 0, st>>>(A->rowptr, A->nblockrows, start, (int32_t)nch, plan,
                                                        (int32_t*)((char*)plan + L.tail));
   GBO_LAUNCH_CHECK();
-  if (scratch) {
-    unsigned long long* slots = (unsigned long long*)((char*)plan + L.slots);
-    k_fill_u64<<<kCountSlots / 256, 256, 0, st>>>(slots, kCountSlots, 0ull);
-    GBO_LAUNCH_CHECK();
-  }
+  unsigned long long* slots = (unsigned long long*)((char*)plan + L.slots);
+  k_fill_u64<<<kCountSlots / 256, 256, 0, st>>>(slots, kCountSlots, 0ull);
+  GBO_LAUNCH_CHECK();
   return GBO_OK;
 }
 
@@ -678,7 +673,7 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
   const int32_t chunk = default_chunk(A->bs, A->nblocks);
   const int64_t nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "too many chunks");
-  const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, true);
+  const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
   int32_t* plan = nullptr;
   GBO_HIP_CHECK(hipMallocAsync((void**)&plan, L.bytes, st));
   pv->plan = plan;
@@ -687,10 +682,10 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
   pv->variant = A->plan_variant;
   pv->owned = true;
   view_scratch(pv, A->bs, A->nblockrows, true);
-  return plan_fill(A, chunk, true, nch, true, plan, st);
+  return plan_fill(A, chunk, true, nch, plan, st);
 }
 
-int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, hipStream_t st) {
+int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st) {
   const int32_t chunk = chunk_tiles > 0 ? chunk_tiles : default_chunk(A->bs, A->nblocks);
   // equal work needs the tiles' bits in 16-byte reads; the kernels that gain
   // from it need the same alignment
@@ -712,7 +707,7 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, 
   }
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "gbo_bsr_plan: too many chunks");
   gbo_bsr_plan_free(A);
-  const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows, scratch);
+  const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
   if (device_malloc((void**)&A->plan, L.bytes) != hipSuccess) {
     A->plan = nullptr;
     return set_error(GBO_ENOMEM, "gbo_bsr_plan: allocation of %zu bytes failed", L.bytes);
@@ -731,7 +726,7 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool scratch, 
       return set_error(GBO_EDEVICE, "gbo_bsr_plan: %s", hipGetErrorString(e));
     }
   }
-  const int rc = plan_fill(A, chunk, even, nch, scratch, A->plan, st);
+  const int rc = plan_fill(A, chunk, even, nch, A->plan, st);
   if (rc) gbo_bsr_plan_free(A);
   return rc;
 }
@@ -976,7 +971,7 @@ int gbo_bsr_plan_ex(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, gbo_stream
   if (rc) return rc;
   if (chunk_tiles < 0) return set_error(GBO_EINVAL, "gbo_bsr_plan: negative chunk");
   if (variant < 0 || variant > 3) return set_error(GBO_EINVAL, "gbo_bsr_plan: variant must be 0, 1, 2 or 3");
-  return plan_create(A, chunk_tiles, variant, true, stream);
+  return plan_create(A, chunk_tiles, variant, stream);
 }
 
 int gbo_csr2bsr_values_u32(const gbo_bsr* A, const int32_t* d_rp, const int32_t* d_ci, const uint32_t* d_val,
