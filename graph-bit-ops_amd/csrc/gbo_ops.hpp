@@ -156,6 +156,25 @@ int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st);
 template <class TI, class TO>
 int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st, Workspace& mem);
 
+// Packing of the heavy block rows (gbo_pack_fill.hip), those of more than
+// `above` nonzeros: heavy_list finds them, heavy_count writes their tile counts
+// and raises PACKERR flags, heavy_fill writes their block columns and tiles
+// (from off, the first tile of each block row), for rows that raised none.
+enum { PACKERR_COLRANGE = 1, PACKERR_UNSORTED = 2 };
+struct PackCsr {
+  const int32_t *rp, *ci;
+  int32_t nrows, ncols, nbr;
+};
+struct HeavyRows {
+  int32_t* list = nullptr;
+  int32_t* n = nullptr;  // device
+  int32_t above = 0;
+};
+int heavy_list(int bs, const PackCsr& A, Workspace& mem, HeavyRows* h, const char* who, hipStream_t st);
+int heavy_count(int bs, const PackCsr& A, const HeavyRows& h, int32_t* cnt, int* err, hipStream_t st);
+int heavy_fill(int bs, int dir, const PackCsr& A, const HeavyRows& h, int32_t nheavy, const int64_t* off, int64_t T,
+               int32_t* colind, void* tiles, Workspace& mem, hipStream_t st);
+
 constexpr uint32_t kInfU32 = 0xFFFFFFFFu;
 constexpr int kCountSlots = 1024;
 

@@ -9,10 +9,9 @@
 // block row, the group takes the minimum pending block column (a k-way merge
 // of the bs sorted rows), and every lane ORs its entries of that block
 // column into its own row word -- which is directly word r of the tile in
-// the reference layout (MSB = column 0).  A block row of more than 2048
-// nonzeros is split into pieces (block-column ranges) merged by groups of
-// their own.  Two passes: count tiles per piece, scan, then fill
-// colind/tiles.  No dense staging.
+// the reference layout (MSB = column 0).  Two passes: count tiles, scan, then
+// fill colind/tiles.  No dense staging.  Block rows of many nonzeros are not
+// merged (gbo_pack_fill.hip).
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -126,14 +125,12 @@ template int scan_exclusive<int64_t, int64_t>(const int64_t*, int64_t*, int64_t,
 // ---------------------------------------------------------------- packing
 enum { PACK_COUNT = 0, PACK_ROW = 1, PACK_COL = 2, PACK_VALUES = 3 };
 
-// Error flags raised by the packer (device int, OR-ed).
-enum { PACKERR_COLRANGE = 1, PACKERR_UNSORTED = 2 };
-
-// A block row with more than kPieceNnz nonzeros is packed in pieces: ranges
-// of block columns [lo, hi), one group each, cut at evenly spaced entries of
-// the block row's longest CSR row.  A single group's merge over the hub
-// block row of R-MAT s22 (129,447 tiles at bs 8, one dependent step per
-// tile) had set the time of each whole packing pass (~75 ms).
+// Where values follow the tiles' bits, a block row with more than kPieceNnz
+// nonzeros is merged in pieces: ranges of block columns [lo, hi), one group
+// each, cut at evenly spaced entries of the block row's longest CSR row.  A
+// single group's merge over the hub block row of R-MAT s22 (129,447 tiles at
+// bs 8, one dependent step per tile) had set the time of each whole pass
+// (~75 ms).
 constexpr int32_t kPieceNnz = 2048;
 
 // The pieces: piece p is block row row[p] over block columns [lo[p], hi[p])
@@ -146,7 +143,13 @@ struct PackPieces {
   const int64_t* base = nullptr;  // fill: first tile of each piece
   int32_t* cnt = nullptr;         // count: tiles of each piece
   int32_t n = 0;
+  int32_t above = INT_MAX;        // without a table: block rows of more nonzeros are left out
 };
+
+// Column indices a wave stages in LDS (4 KB): a merge step waits for LDS and
+// not for memory (12 nonzeros a row, 2^20 rows at bs 8, count and fill:
+// 690 -> 500 us).
+constexpr int kStage = 1024;
 
 // First index q in [q0, q1) with ci[q] / BS >= J (q1 if none).  On rows that
 // are not sorted the result is still monotone in J, so the pieces of a row
@@ -181,9 +184,10 @@ __global__ __launch_bounds__(256) void k_pack(const int32_t* __restrict__ rp,
   const int64_t npc = pc.row ? (int64_t)pc.n : (int64_t)nbr;
   const int64_t pi = wave * G + g;  // piece of this group
   if (wave * G >= npc) return;      // wave-uniform
-  const bool blk_ok = pi < npc;
+  bool blk_ok = pi < npc;
   const int64_t I = pc.row ? (blk_ok ? (int64_t)pc.row[pi] : 0) : pi;
   const int64_t row = I * BS + r;
+  if (blk_ok && pc.above != INT_MAX) blk_ok = rp[min((I + 1) * BS, (int64_t)nrows)] - rp[I * BS] <= pc.above;
   int32_t p = 0, pe = 0;
   if (blk_ok && row < nrows) {
     const int32_t r0 = rp[row], r1 = rp[row + 1];
@@ -198,8 +202,23 @@ __global__ __launch_bounds__(256) void k_pack(const int32_t* __restrict__ rp,
       if (MODE == PACK_COUNT && p > r0 && p < r1 && ci[p - 1] / BS > ci[p] / BS) atomicOr(err, PACKERR_UNSORTED);
     }
   }
+  // the wave's rows are one run of the CSR: a short one is staged
+  __shared__ int32_t stage[256 / kWave][kStage];
+  int32_t* sci = stage[threadIdx.x / kWave];
+  int32_t s0 = 0;
+  bool staged = false;
+  if (!pc.row) {
+    const int64_t w0 = wave * G * BS;
+    s0 = rp[w0];
+    const int32_t s1 = rp[min(w0 + kWave, (int64_t)nrows)];
+    staged = (int64_t)s1 - s0 <= kStage && __all(p == pe || (p >= s0 && pe <= s1));
+    if (staged)
+      for (int32_t q = lane; q < s1 - s0; q += kWave) sci[q] = ci[s0 + q];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+  auto entry = [&](int32_t q) -> int32_t { return staged ? sci[q - s0] : ci[q]; };
   auto blockcol = [&](int32_t q) -> int32_t {
-    const int32_t c = ci[q];
+    const int32_t c = entry(q);
     if (MODE == PACK_COUNT && (c < 0 || c >= ncols)) {
       atomicOr(err, PACKERR_COLRANGE);
       return INT_MAX - 1;  // poison: still terminates
@@ -217,7 +236,7 @@ __global__ __launch_bounds__(256) void k_pack(const int32_t* __restrict__ rp,
     int32_t p0 = p;
     if (m != INT_MAX) {
       while (cur == m) {
-        w |= 1ull << (BS - 1 - (ci[p] % BS));
+        w |= 1ull << (BS - 1 - (entry(p) % BS));
         ++p;
         const int32_t nxt = (p < pe) ? blockcol(p) : INT_MAX;
         if (MODE == PACK_COUNT && nxt < cur) atomicOr(err, PACKERR_UNSORTED);
@@ -309,11 +328,24 @@ __global__ __launch_bounds__(256) void k_piece_fill(const int32_t* __restrict__ 
   }
 }
 
-// rowptr[I] = first tile of block row I's first piece (rowptr[nbr] = total).
-__global__ __launch_bounds__(256) void k_piece_rowptr(const int32_t* __restrict__ poff, const int64_t* __restrict__ toff,
-                                                      int32_t nbr, int32_t* __restrict__ rowptr) {
+// rowptr[I] = first tile of block row I (rowptr[nbr] = total).
+__global__ __launch_bounds__(256) void k_pack_rowptr(const int64_t* __restrict__ off, int32_t nbr,
+                                                     int32_t* __restrict__ rowptr) {
   const int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (I <= nbr) rowptr[I] = (int32_t)toff[poff[I]];
+  if (I <= nbr) rowptr[I] = (int32_t)off[I];
+}
+
+struct PackSummary {
+  int64_t total;
+  int32_t err, heavy, given;
+};
+__global__ void k_pack_summary(const int64_t* __restrict__ total, const int* __restrict__ err,
+                               const int32_t* __restrict__ heavy, const int32_t* __restrict__ given,
+                               PackSummary* __restrict__ out) {
+  out->total = *total;
+  out->err = *err;
+  out->heavy = *heavy;
+  out->given = given ? *given : 0;
 }
 
 template <int BS>
@@ -508,10 +540,7 @@ static int dispatch_pack(int bs, const int32_t* rp, const int32_t* ci, int32_t n
   return set_error(GBO_EUNSUPPORTED, "block size %d not supported (8, 16, 32, 64)", bs);
 }
 
-static int check_err_flag(int* d_err, hipStream_t st, const char* who) {
-  int h = 0;
-  const int rc = read_back(&h, d_err, sizeof(int), st);
-  if (rc) return rc;
+static int check_err_flag(int h, const char* who) {
   if (h & PACKERR_COLRANGE) return set_error(GBO_EINVAL, "%s: column index out of range", who);
   if (h & PACKERR_UNSORTED) return set_error(GBO_EINVAL, "%s: CSR rows must be sorted ascending", who);
   return GBO_OK;
@@ -520,11 +549,9 @@ static int check_err_flag(int* d_err, hipStream_t st, const char* who) {
 // The pieces of every block row, their tile counts (a count pass that also
 // checks the rows: columns in range, block columns ascending) and the first
 // tile of each (toff, npieces + 1 entries); *total = tiles.  Buffers are
-// owned by `mem`; poff (nbr + 1) is each block row's first piece.
+// owned by `mem`.
 struct PieceSet {
   PackPieces pc;
-  int32_t* poff = nullptr;
-  int64_t* toff = nullptr;
   int64_t total = 0;
 };
 
@@ -564,7 +591,8 @@ static int make_pieces(int bs, const int32_t* d_rp, const int32_t* d_ci, int32_t
   if ((rc = dispatch_pack<PACK_COUNT>(bs, d_rp, d_ci, nrows, ncols, nbr, nullptr, nullptr, nullptr, nullptr,
                                       nullptr, nullptr, d_err, pc, st)))
     return rc;
-  if ((rc = check_err_flag(d_err, st, who))) return rc;
+  int err = 0;
+  if ((rc = read_back(&err, d_err, sizeof(int), st)) || (rc = check_err_flag(err, who))) return rc;
   if ((rc = scan_exclusive<int32_t, int64_t>(pcnt, toff, np, st, mem))) return rc;
   if ((rc = read_back(&ps->total, toff + np, sizeof(int64_t), st))) return rc;
   if (ps->total >= ((int64_t)1 << 31))
@@ -572,9 +600,63 @@ static int make_pieces(int bs, const int32_t* d_rp, const int32_t* d_ci, int32_t
   pc.cnt = nullptr;
   pc.base = toff;
   ps->pc = pc;
-  ps->poff = poff;
-  ps->toff = toff;
   return GBO_OK;
+}
+
+// The tiles of every block row: off (nbr + 1 first tiles, owned by `mem`), the
+// heavy block rows and one read of what the host needs.  Checks the rows.
+struct PackCount {
+  int64_t* off = nullptr;
+  HeavyRows heavy;
+  PackSummary sum{};
+};
+
+static int pack_count(int bs, const PackCsr& A, const int32_t* d_given, Workspace& mem, PackCount* pk, const char* who,
+                      hipStream_t st) {
+  int rc;
+  int32_t* cnt = nullptr;
+  int* d_err = nullptr;
+  PackSummary* d_sum = nullptr;
+  if ((rc = mem.alloc(&cnt, sizeof(int32_t) * (size_t)std::max(A.nbr, 1), who)) ||
+      (rc = mem.alloc(&pk->off, sizeof(int64_t) * ((size_t)A.nbr + 1), who)) ||
+      (rc = mem.alloc(&d_err, sizeof(int), who)) || (rc = mem.alloc(&d_sum, sizeof(PackSummary), who)))
+    return rc;
+  GBO_HIP_CHECK(hipMemsetAsync(d_err, 0, sizeof(int), st));
+  if ((rc = heavy_list(bs, A, mem, &pk->heavy, who, st))) return rc;
+  PackPieces pc;
+  pc.above = pk->heavy.above;
+  if ((rc = dispatch_pack<PACK_COUNT>(bs, A.rp, A.ci, A.nrows, A.ncols, A.nbr, cnt, nullptr, nullptr, nullptr, nullptr,
+                                      nullptr, d_err, pc, st)) ||
+      (rc = heavy_count(bs, A, pk->heavy, cnt, d_err, st)) ||
+      (rc = scan_exclusive<int32_t, int64_t>(cnt, pk->off, A.nbr, st, mem)))
+    return rc;
+  k_pack_summary<<<1, 1, 0, st>>>(pk->off + A.nbr, d_err, pk->heavy.n, d_given, d_sum);
+  GBO_LAUNCH_CHECK();
+  if ((rc = read_back(&pk->sum, d_sum, sizeof(PackSummary), st)) || (rc = check_err_flag(pk->sum.err, who))) return rc;
+  if (pk->sum.total >= ((int64_t)1 << 31))
+    return set_error(GBO_ERANGE, "tile count %lld exceeds int32", (long long)pk->sum.total);
+  return GBO_OK;
+}
+
+static int pack_rowptr(const PackCount& pk, int32_t nbr, int32_t* d_rowptr, hipStream_t st) {
+  k_pack_rowptr<<<(unsigned)(((int64_t)nbr + 1 + 255) / 256), 256, 0, st>>>(pk.off, nbr, d_rowptr);
+  GBO_LAUNCH_CHECK();
+  return GBO_OK;
+}
+
+// Block columns and tiles of counted rows.
+static int pack_fill(int bs, int dir, const PackCsr& A, const PackCount& pk, int32_t* d_col, void* d_tiles,
+                     Workspace& mem, hipStream_t st) {
+  if (pk.sum.total == 0) return GBO_OK;
+  PackPieces pc;
+  pc.above = pk.heavy.above;
+  pc.base = pk.off;
+  const int rc = dir == 0 ? dispatch_pack<PACK_ROW>(bs, A.rp, A.ci, A.nrows, A.ncols, A.nbr, nullptr, d_col, d_tiles,
+                                                    nullptr, nullptr, nullptr, nullptr, pc, st)
+                          : dispatch_pack<PACK_COL>(bs, A.rp, A.ci, A.nrows, A.ncols, A.nbr, nullptr, d_col, d_tiles,
+                                                    nullptr, nullptr, nullptr, nullptr, pc, st);
+  if (rc) return rc;
+  return heavy_fill(bs, dir, A, pk.heavy, pk.sum.heavy, pk.off, pk.sum.total, d_col, d_tiles, mem, st);
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -769,13 +851,11 @@ int gbo_csr2bsr_nnzb_dev(int bs, const int32_t* d_rp, const int32_t* d_ci, int32
   hipStream_t st = stream;
   const int32_t nbr = (nrows + bs - 1) / bs;
   Workspace mem(st);
-  PieceSet ps;
-  int rc = make_pieces(bs, d_rp, d_ci, nrows, ncols, nbr, mem, &ps, "gbo_csr2bsr_nnzb_dev", st);
-  if (rc != GBO_OK) return rc;
-  k_piece_rowptr<<<(unsigned)(((int64_t)nbr + 1 + 255) / 256), 256, 0, st>>>(ps.poff, ps.toff, nbr, d_bsrRowPtr);
-  GBO_LAUNCH_CHECK();
+  PackCount pk;
+  int rc = pack_count(bs, {d_rp, d_ci, nrows, ncols, nbr}, nullptr, mem, &pk, "gbo_csr2bsr_nnzb_dev", st);
+  if (rc != GBO_OK || (rc = pack_rowptr(pk, nbr, d_bsrRowPtr, st))) return rc;
   GBO_HIP_CHECK(hipStreamSynchronize(st));
-  *nblocks = ps.total;
+  *nblocks = pk.sum.total;
   return GBO_OK;
   GBO_TRY_END
 }
@@ -789,24 +869,18 @@ int gbo_csr2bsr_fill_dev(int bs, int dir, const int32_t* d_rp, const int32_t* d_
   if (nrows < 0 || ncols < 0 || !d_rp || !d_bsrRowPtr) return set_error(GBO_EINVAL, "gbo_csr2bsr_fill_dev: bad argument");
   hipStream_t st = stream;
   const int32_t nbr = (nrows + bs - 1) / bs;
-  // the tile offsets come from the pieces' counts (the same as d_bsrRowPtr
-  // at block-row starts); the rows are checked again on the way
+  // the rows are counted and checked again: the tile offsets are that count's
+  // (the same as d_bsrRowPtr at block-row starts)
   Workspace mem(st);
-  PieceSet ps;
-  int rc = make_pieces(bs, d_rp, d_ci, nrows, ncols, nbr, mem, &ps, "gbo_csr2bsr_fill_dev", st);
+  const PackCsr A{d_rp, d_ci, nrows, ncols, nbr};
+  PackCount pk;
+  int rc = pack_count(bs, A, d_bsrRowPtr + nbr, mem, &pk, "gbo_csr2bsr_fill_dev", st);
   if (rc != GBO_OK) return rc;
-  if (ps.total > 0 && (!d_bsrColInd || !d_tiles)) return set_error(GBO_EINVAL, "gbo_csr2bsr_fill_dev: null output");
-  int32_t given = 0;  // the caller sized colind and tiles by rowptr[nbr]
-  if ((rc = read_back(&given, d_bsrRowPtr + nbr, sizeof(int32_t), st))) return rc;
-  if (given != ps.total)
-    return set_error(GBO_EINVAL, "gbo_csr2bsr_fill_dev: rowptr[nblockrows] = %d, the CSR has %lld tiles", given,
-                     (long long)ps.total);
-  if (dir == 0)
-    rc = dispatch_pack<PACK_ROW>(bs, d_rp, d_ci, nrows, ncols, nbr, const_cast<int32_t*>(d_bsrRowPtr), d_bsrColInd,
-                                 d_tiles, nullptr, nullptr, nullptr, nullptr, ps.pc, st);
-  else
-    rc = dispatch_pack<PACK_COL>(bs, d_rp, d_ci, nrows, ncols, nbr, const_cast<int32_t*>(d_bsrRowPtr), d_bsrColInd,
-                                 d_tiles, nullptr, nullptr, nullptr, nullptr, ps.pc, st);
+  if (pk.sum.total > 0 && (!d_bsrColInd || !d_tiles)) return set_error(GBO_EINVAL, "gbo_csr2bsr_fill_dev: null output");
+  if (pk.sum.given != pk.sum.total)  // the caller sized colind and tiles by rowptr[nbr]
+    return set_error(GBO_EINVAL, "gbo_csr2bsr_fill_dev: rowptr[nblockrows] = %d, the CSR has %lld tiles", pk.sum.given,
+                     (long long)pk.sum.total);
+  rc = pack_fill(bs, dir, A, pk, d_bsrColInd, d_tiles, mem, st);
   return rc;
   GBO_TRY_END
 }
@@ -817,6 +891,7 @@ int gbo_bsr_create_dev(int bs, int dir, const int32_t* d_rp, const int32_t* d_ci
   std::memset(out, 0, sizeof(*out));
   if (!bs_ok(bs)) return set_error(GBO_EUNSUPPORTED, "block size %d not supported (8, 16, 32, 64)", bs);
   if (dir != 0 && dir != 1) return set_error(GBO_EINVAL, "dir must be 0 (row) or 1 (col)");
+  if (nrows < 0 || ncols < 0 || !d_rp) return set_error(GBO_EINVAL, "gbo_bsr_create_dev: bad argument");
   const int32_t nbr = (nrows + bs - 1) / bs;
   gbo_bsr A{};
   A.bs = bs;
@@ -828,11 +903,15 @@ int gbo_bsr_create_dev(int bs, int dir, const int32_t* d_rp, const int32_t* d_ci
   if (device_malloc((void**)&A.rowptr, sizeof(int32_t) * ((size_t)nbr + 1)) != hipSuccess)
     return set_error(GBO_ENOMEM, "gbo_bsr_create_dev: cannot allocate %d row pointers", nbr + 1);
   workspace_live(1);
-  int rc = gbo_csr2bsr_nnzb_dev(bs, d_rp, d_ci, nrows, ncols, A.rowptr, &A.nblocks, stream);
-  if (rc != GBO_OK) {
+  Workspace mem(stream);
+  const PackCsr csr{d_rp, d_ci, nrows, ncols, nbr};
+  PackCount pk;
+  int rc = pack_count(bs, csr, nullptr, mem, &pk, "gbo_bsr_create_dev", stream);
+  if (rc != GBO_OK || (rc = pack_rowptr(pk, nbr, A.rowptr, stream))) {
     gbo_bsr_free(&A);
     return rc;
   }
+  A.nblocks = pk.sum.total;
   const size_t tile_bytes = (size_t)A.nblocks * bs * (bs / 8);
   hipError_t e1 = device_malloc((void**)&A.colind, sizeof(int32_t) * std::max<int64_t>(A.nblocks, 1));
   hipError_t e2 = device_malloc(&A.tiles, std::max<size_t>(tile_bytes, 8));
@@ -840,7 +919,7 @@ int gbo_bsr_create_dev(int bs, int dir, const int32_t* d_rp, const int32_t* d_ci
     gbo_bsr_free(&A);
     return set_error(GBO_ENOMEM, "gbo_bsr_create: cannot allocate %zu tile bytes", tile_bytes);
   }
-  rc = gbo_csr2bsr_fill_dev(bs, dir, d_rp, d_ci, nrows, ncols, A.rowptr, A.colind, A.tiles, stream);
+  rc = pack_fill(bs, dir, csr, pk, A.colind, A.tiles, mem, stream);
   if (rc != GBO_OK) {
     gbo_bsr_free(&A);
     return rc;
