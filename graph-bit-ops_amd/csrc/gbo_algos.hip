@@ -658,6 +658,12 @@ static int read_u64(unsigned long long* d, uint64_t* h, hipStream_t st) {
   return read_back(h, d, sizeof(uint64_t), st);
 }
 
+// One product of a driver, over the edge lists where it has them.
+static int sweep(int bs, int op, const SpmvArgs& a, const ListView& lists, hipStream_t st) {
+  if (!lists.on) return spmv_launch(bs, op, a, st);
+  return lists_sweep(op, lists, {a.xval, a.out, a.w, a.woff, a.scale, a.bias}, st);
+}
+
 static int check_square(const gbo_bsr* A, const char* who) {
   int rc = validate_bsr(A, 0, who);
   if (rc) return rc;
@@ -827,13 +833,15 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   a.variant = pv.variant;
   a.w = d_w;
   a.woff = d_woff;
+  ListView lists;
+  lists_build(AT, true, mem, &lists, st);
   int32_t it = 0;
   unsigned long long *act_cur = active, *act_next = active2;
   while (true) {
     a.xval = fr;
     a.out = cand;
     a.active = (const uint64_t*)act_cur;
-    if ((rc = spmv_launch(bs, OP_MINPLUS, a, st))) return rc;
+    if ((rc = sweep(bs, OP_MINPLUS, a, lists, st))) return rc;
     GBO_HIP_CHECK(hipMemsetAsync(act_next, 0, sizeof(unsigned long long) * nact, st));
     GBO_HIP_CHECK(hipMemsetAsync(changed, 0, sizeof(unsigned long long), st));
     k_sssp_update<<<blocks_n, 256, 0, st>>>(cand, d_dist, fr, act_next, n, bs, changed);
@@ -889,6 +897,8 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   a.bias = (1.0f - alpha) / (float)n;
   const unsigned blocks_n = (unsigned)((n + 255) / 256);
   const unsigned lblocks = (unsigned)std::min<int64_t>(nparts, (n + 255) / 256);
+  ListView lists;
+  lists_build(AT, true, mem, &lists, st);
   int32_t it = 0;
   double delta = 0.0;
   float* p = d_p;
@@ -898,7 +908,7 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   while (it < max_iter) {
     a.xval = x;
     a.out = q;
-    if ((rc = spmv_launch(AT->bs, OP_SUM, a, st))) return rc;
+    if ((rc = sweep(AT->bs, OP_SUM, a, lists, st))) return rc;
     k_pr_tail<<<lblocks, 256, 0, st>>>(q, p, d_outdeg, alpha, x, n, dpart);  // x for the next iteration
     k_sum_partials<<<1, 256, 0, st>>>(dpart, (int)lblocks, dpart + nparts);
     GBO_LAUNCH_CHECK();
@@ -952,11 +962,13 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
+  ListView lists;
+  lists_build(A, false, mem, &lists, st);
   int32_t it = 0;
   while (true) {
     a.xval = gf;
     a.out = mngf;
-    if ((rc = spmv_launch(A->bs, OP_MIN, a, st))) return rc;
+    if ((rc = sweep(A->bs, OP_MIN, a, lists, st))) return rc;
     k_cc_hook<<<blocks_n, 256, 0, st>>>(mngf, gf, f, n);
     GBO_HIP_CHECK(hipMemsetAsync(changed, 0, sizeof(unsigned long long), st));
     k_cc_grand<<<blocks_n, 256, 0, st>>>(f, gf, n, changed);

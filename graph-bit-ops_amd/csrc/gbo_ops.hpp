@@ -176,6 +176,47 @@ int heavy_fill(int bs, int dir, const PackCsr& A, const HeavyRows& h, int32_t nh
                int32_t* colind, void* tiles, Workspace& mem, hipStream_t st);
 
 constexpr uint32_t kInfU32 = 0xFFFFFFFFu;
+
+// Edge lists for drivers that sweep one matrix many times (gbo_lists.hip).
+// lists_build leaves `on` false where sweeps over the tiles are to be used:
+// few tiles, mostly dense ones, more than 2^26 rows, no memory.
+struct ListPart {
+  const uint32_t* at;  // entries
+  int32_t n;
+  int32_t win;   // window of 64 rows
+  int32_t tile;  // first tile of its item
+  int32_t skip;  // entries of the item before it
+};
+struct ListView {
+  bool on = false;
+  int bs;
+  int32_t n, nbr, nwin, per, nmulti;
+  int64_t nparts;
+  const int32_t *rowptr, *colind;
+  const void* tiles;
+  const int64_t* first;   // building: items, then parts before each window
+  const int32_t* win;     // window of each item
+  const int32_t* multi;   // windows of several parts
+  const ListPart* parts;
+  double* partial;
+};
+constexpr int kListSlots = 64;
+struct ListInfo {
+  int64_t items, parts, over;
+  unsigned long long sample[kListSlots];
+  int32_t multi;
+};
+struct ListSweep {
+  const void* x;
+  void* out;
+  const uint32_t* w;
+  const int64_t* woff;
+  float scale, bias;  // sum: scale * (A x) + bias
+};
+void lists_build(const gbo_bsr* A, bool many, Workspace& mem, ListView* out, hipStream_t st);
+// OP_SUM, OP_MIN, or OP_MINPLUS without the vertex's own value.
+int lists_sweep(int op, const ListView& l, const ListSweep& s, hipStream_t st);
+
 constexpr int kCountSlots = 1024;
 
 // bsrbmv operation codes.
