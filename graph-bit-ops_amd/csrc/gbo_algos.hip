@@ -508,13 +508,19 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
 // dist = min(dist, cand); the improved vertices form the next frontier: their
 // distance goes to `fr` (INF elsewhere) and their block column is marked
 // active so the next min-plus product only reads tiles of active columns.
-__global__ __launch_bounds__(256) void k_sssp_update(const uint32_t* __restrict__ cand, uint32_t* __restrict__ dist,
-                                                     uint32_t* __restrict__ fr, unsigned long long* __restrict__ active,
-                                                     int32_t n, int bs, unsigned long long* __restrict__ changed) {
+constexpr int kSsspThreads = 512;  // vertices of whole bytes of `active` at every block size
+__global__ __launch_bounds__(kSsspThreads) void k_sssp_update(uint32_t* __restrict__ cand,
+                                                              uint32_t* __restrict__ dist, uint32_t* __restrict__ fr,
+                                                              unsigned char* __restrict__ active, int32_t n, int bs,
+                                                              const unsigned long long* __restrict__ go,
+                                                              unsigned long long* __restrict__ changed) {
+  __shared__ int sh[kSsspThreads / kWave];
+  if (over(go)) return;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int improved = 0;
   if (i < n) {
     const uint32_t c = cand[i], d = dist[i];
+    cand[i] = kInfU32;  // where the next product's split rows start from
     if (c < d) {
       dist[i] = c;
       fr[i] = c;
@@ -523,19 +529,29 @@ __global__ __launch_bounds__(256) void k_sssp_update(const uint32_t* __restrict_
       fr[i] = kInfU32;
     }
   }
-  // block columns of the improved vertices: the 64 vertices of a wave (64-
-  // aligned) cover 64/bs consecutive block columns inside one 64-bit word
-  const int64_t J = i / bs;
-  const uint64_t m = wave_or64(improved ? 1ull << (J & 63) : 0ull);
-  if (lane_id() == 0 && m) atomicOr(&active[((i - lane_id()) / bs) >> 6], m);
+  // block columns of the improved vertices: 64 / bs bits of each wave
+  const int lane = lane_id(), per = kWave / bs;
+  const unsigned long long m = __ballot(improved);
+  if (lane == 0) {
+    int bits = 0;
+    for (int k = 0; k < per; ++k) bits |= (m >> (k * bs) & (~0ull >> (kWave - bs))) ? 1 << k : 0;
+    sh[threadIdx.x / kWave] = bits;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < per) {  // 512 / bs bits: `per` bytes
+    int byte = 0;
+    for (int k = 0; k < 8 / per; ++k) byte |= sh[threadIdx.x * (8 / per) + k] << (k * per);
+    active[(int64_t)blockIdx.x * per + threadIdx.x] = (unsigned char)byte;
+  }
   wave_flag(improved, changed);
 }
 
-__global__ void k_sssp_init(uint32_t* dist, uint32_t* fr, unsigned long long* active, int32_t n, int bs, int32_t s) {
+__global__ void k_sssp_init(uint32_t* dist, uint32_t* fr, uint32_t* cand, unsigned long long* active, int32_t n, int bs, int32_t s) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {
     dist[i] = (i == s) ? 0u : kInfU32;
     fr[i] = (i == s) ? 0u : kInfU32;
+    cand[i] = kInfU32;
   }
   if (i == 0) {
     const int64_t J = s / bs;
@@ -559,11 +575,18 @@ __global__ __launch_bounds__(256) void k_pr_scale(const float* __restrict__ p, c
 // Per-block partial sums of |q-p| in double, and the next iteration's
 // x[j] = alpha * q[j] / outdeg[j] (as k_pr_scale) from the same read of q.
 // The partials are added in a fixed order by k_sum_partials, so the L1
-// change is reproducible.
-__global__ __launch_bounds__(256) void k_pr_tail(const float* __restrict__ q, const float* __restrict__ p,
-                                                 const int32_t* __restrict__ outdeg, float alpha,
-                                                 float* __restrict__ x, int32_t n, double* __restrict__ part) {
-  __shared__ double sh[256];
+// change is reproducible.  Up to kOneBlock vertices one block takes them all and
+// writes the sum and the flag itself: a launch costs the host 5 us.
+constexpr int kOneBlock = 1 << 14;
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_pr_tail(const float* __restrict__ q, const float* __restrict__ p,
+                                                     const int32_t* __restrict__ outdeg, float alpha,
+                                                     float* __restrict__ x, int32_t n, double tol,
+                                                     double* __restrict__ part,
+                                                     const unsigned long long* __restrict__ go,
+                                                     unsigned long long* __restrict__ again) {
+  __shared__ double sh[THREADS];
+  if (over(go)) return;
   double s = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const float qi = q[i];
@@ -573,18 +596,24 @@ __global__ __launch_bounds__(256) void k_pr_tail(const float* __restrict__ q, co
   }
   sh[threadIdx.x] = s;
   __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
+  for (int off = THREADS / 2; off > 0; off >>= 1) {
     if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = sh[0];
+    if (gridDim.x == 1) *again = sh[0] < tol ? 0 : 1;
+  }
 }
 
 // *out = the sum of part[0..np) in a fixed order: thread t adds entries
 // t, t+256, ... in turn, then a fixed tree over the threads (one block of
-// 256 threads).
-__global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__ part, int np, double* out) {
+// 256 threads); *again = 0 where it is below tol.
+__global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__ part, int np, double tol, double* out,
+                                                      const unsigned long long* __restrict__ go,
+                                                      unsigned long long* __restrict__ again) {
   __shared__ double sh[256];
+  if (over(go)) return;
   double s = 0.0;
   for (int i = threadIdx.x; i < np; i += 256) s += part[i];
   sh[threadIdx.x] = s;
@@ -593,7 +622,10 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__
     if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = sh[0];
+  if (threadIdx.x == 0) {
+    *out = sh[0];
+    *again = sh[0] < tol ? 0 : 1;
+  }
 }
 
 // ------------------------------------------------------------------ CC
@@ -605,11 +637,14 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__
 // would change nothing and is not issued: millions of vertices share a few
 // roots, and their atomics on the root's label serialised (0.26 ms a call
 // at R-MAT s22).
-__global__ __launch_bounds__(256) void k_cc_hook(const int32_t* __restrict__ mngf, const int32_t* __restrict__ gf,
-                                                 int32_t* __restrict__ f, int32_t n) {
+__global__ __launch_bounds__(256) void k_cc_hook(int32_t* __restrict__ mngf, const int32_t* __restrict__ gf,
+                                                 int32_t* __restrict__ f, int32_t n,
+                                                 const unsigned long long* __restrict__ go) {
+  if (over(go)) return;
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= n) return;
   const int32_t m = mngf[u];
+  mngf[u] = INT32_MAX;  // where the next product's split rows start from
   const int32_t fu = f[u];
   if (m < fu && m < f[fu]) atomicMin(&f[fu], m);
   const int32_t g = gf[u];
@@ -619,7 +654,9 @@ __global__ __launch_bounds__(256) void k_cc_hook(const int32_t* __restrict__ mng
 
 // gf[u] = f[f[u]]; *changed = 1 if any vertex's grandparent changed.
 __global__ __launch_bounds__(256) void k_cc_grand(const int32_t* __restrict__ f, int32_t* __restrict__ gf, int32_t n,
+                                                  const unsigned long long* __restrict__ go,
                                                   unsigned long long* __restrict__ changed) {
+  if (over(go)) return;
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int ch = 0;
   if (u < n) {
@@ -633,7 +670,9 @@ __global__ __launch_bounds__(256) void k_cc_grand(const int32_t* __restrict__ f,
 }
 
 // f[u] = f[f[u]] until every vertex points at a root (final star shape).
-__global__ __launch_bounds__(256) void k_cc_jump(int32_t* __restrict__ f, int32_t n, unsigned long long* changed) {
+__global__ __launch_bounds__(256) void k_cc_jump(int32_t* __restrict__ f, int32_t n, const unsigned long long* go,
+                                                 unsigned long long* changed) {
+  if (over(go)) return;
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int ch = 0;
   if (u < n) {
@@ -646,22 +685,59 @@ __global__ __launch_bounds__(256) void k_cc_jump(int32_t* __restrict__ f, int32_
   wave_flag(ch, changed);
 }
 
-__global__ void k_iota(int32_t* a, int32_t* b, int32_t n) {
+__global__ void k_cc_init(int32_t* a, int32_t* b, int32_t* m, int32_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {
     a[i] = (int32_t)i;
     b[i] = (int32_t)i;
+    m[i] = INT32_MAX;
   }
 }
 
-static int read_u64(unsigned long long* d, uint64_t* h, hipStream_t st) {
-  return read_back(h, d, sizeof(uint64_t), st);
-}
+// The flags of the iterations queued between two looks at them: iteration k
+// runs only if flag k - 1 of its batch is set, and sets flag k if another is to
+// follow.  A look costs about 12 us with the stream's gap; an iteration past the
+// end a few launches that do nothing, so that batches grow with the iterations
+// there have been: by half of them.
+struct Rounds {
+  static constexpr int kMax = 32, kFlags = 1024;
+  struct Flag {
+    unsigned long long again;
+    double value;
+  };
+  Flag* flags = nullptr;
+  int at = kFlags;  // first flag of the batch
+  Flag h[kMax];
+
+  int alloc(Workspace& mem, const char* who) { return mem.alloc(&flags, sizeof(Flag) * kFlags, who); }
+  // iterations to queue after `done`; their flags are clear
+  int batch(int done, int* n, hipStream_t st) {
+    *n = done == 0 ? 3 : std::min(std::max(2, done / 2), kMax);
+    if (at + *n > kFlags) {
+      GBO_HIP_CHECK(hipMemsetAsync(flags, 0, sizeof(Flag) * kFlags, st));
+      at = 0;
+    }
+    return GBO_OK;
+  }
+  const unsigned long long* go(int k) const { return k ? &flags[at + k - 1].again : nullptr; }
+  unsigned long long* again(int k) const { return &flags[at + k].again; }
+  double* value(int k) const { return &flags[at + k].value; }
+  // iterations of the batch of n that ran; *more: the last of them asks for another
+  int look(int n, int* ran, bool* more, hipStream_t st) {
+    const int rc = read_back(h, flags + at, sizeof(Flag) * n, st);
+    if (rc) return rc;
+    at += n;
+    *ran = 1;
+    while (*ran < n && h[*ran - 1].again) ++*ran;
+    *more = h[*ran - 1].again != 0;
+    return GBO_OK;
+  }
+};
 
 // One product of a driver, over the edge lists where it has them.
 static int sweep(int bs, int op, const SpmvArgs& a, const ListView& lists, hipStream_t st) {
   if (!lists.on) return spmv_launch(bs, op, a, st);
-  return lists_sweep(op, lists, {a.xval, a.out, a.w, a.woff, a.scale, a.bias}, st);
+  return lists_sweep(op, lists, {a.xval, a.out, a.w, a.woff, a.scale, a.bias, a.go}, st);
 }
 
 static int check_square(const gbo_bsr* A, const char* who) {
@@ -806,16 +882,17 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   uint32_t* fr = nullptr;
   unsigned long long* active = nullptr;
   if ((rc = mem.alloc(&fr, sizeof(uint32_t) * (size_t)std::max(n, 1) * 2, "gbo_sssp"))) return rc;
-  if ((rc = mem.alloc(&active, sizeof(unsigned long long) * (size_t)(nact + 1) * 2, "gbo_sssp"))) return rc;
+  if ((rc = mem.alloc(&active, sizeof(unsigned long long) * (size_t)nact * 2, "gbo_sssp"))) return rc;
+  Rounds rounds;
+  if ((rc = rounds.alloc(mem, "gbo_sssp"))) return rc;
   uint32_t* cand = fr + std::max(n, 1);
-  unsigned long long* changed = active + 2 * nact + 1;
   unsigned long long* active2 = active + nact;
   PlanGuard g(st);
   if ((rc = acquire_plan(AT, &g.pv, st))) return rc;
   const PlanView& pv = g.pv;
-  GBO_HIP_CHECK(hipMemsetAsync(active, 0, sizeof(unsigned long long) * nact, st));
+  GBO_HIP_CHECK(hipMemsetAsync(active, 0, sizeof(unsigned long long) * nact * 2, st));
   const unsigned blocks_n = (unsigned)((n + 255) / 256);
-  k_sssp_init<<<blocks_n, 256, 0, st>>>(d_dist, fr, active, n, bs, source);
+  k_sssp_init<<<blocks_n, 256, 0, st>>>(d_dist, fr, cand, active, n, bs, source);
   GBO_LAUNCH_CHECK();
   SpmvArgs a{};
   a.rowptr = AT->rowptr;
@@ -837,22 +914,27 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   lists_build(AT, true, mem, &lists, st);
   int32_t it = 0;
   unsigned long long *act_cur = active, *act_next = active2;
-  while (true) {
-    a.xval = fr;
-    a.out = cand;
-    a.active = (const uint64_t*)act_cur;
-    if ((rc = sweep(bs, OP_MINPLUS, a, lists, st))) return rc;
-    GBO_HIP_CHECK(hipMemsetAsync(act_next, 0, sizeof(unsigned long long) * nact, st));
-    GBO_HIP_CHECK(hipMemsetAsync(changed, 0, sizeof(unsigned long long), st));
-    k_sssp_update<<<blocks_n, 256, 0, st>>>(cand, d_dist, fr, act_next, n, bs, changed);
-    GBO_LAUNCH_CHECK();
-    ++it;
-    uint64_t h = 0;
-    if ((rc = read_u64(changed, &h, st))) return rc;
-    if (h == 0) break;
-    if (it > n + 1)  // distances only decrease: cannot happen
+  const unsigned blocks_u = (unsigned)(((int64_t)n + kSsspThreads - 1) / kSsspThreads);
+  a.prefilled = 1;
+  for (bool more = true; more;) {
+    int nb = 0;
+    if ((rc = rounds.batch(it, &nb, st))) return rc;
+    for (int k = 0; k < nb; ++k) {
+      a.xval = fr;
+      a.out = cand;
+      a.active = (const uint64_t*)act_cur;
+      a.go = rounds.go(k);
+      if ((rc = sweep(bs, OP_MINPLUS, a, lists, st))) return rc;
+      k_sssp_update<<<blocks_u, kSsspThreads, 0, st>>>(cand, d_dist, fr, (unsigned char*)act_next, n, bs, a.go,
+                                                       rounds.again(k));
+      GBO_LAUNCH_CHECK();
+      std::swap(act_cur, act_next);
+    }
+    int ran = 0;
+    if ((rc = rounds.look(nb, &ran, &more, st))) return rc;
+    it += ran;
+    if (more && it > n + 1)  // distances only decrease: cannot happen
       return set_error(GBO_ENOCONV, "gbo_sssp: no convergence after %d iterations", it);
-    std::swap(act_cur, act_next);
   }
   if (h_iters) *h_iters = it;
   return GBO_OK;
@@ -872,7 +954,9 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   float* x = nullptr;
   double* dpart = nullptr;
   if ((rc = mem.alloc(&x, sizeof(float) * (size_t)n * 2, "gbo_pagerank"))) return rc;
-  if ((rc = mem.alloc(&dpart, sizeof(double) * (nparts + 1), "gbo_pagerank"))) return rc;
+  if ((rc = mem.alloc(&dpart, sizeof(double) * nparts, "gbo_pagerank"))) return rc;
+  Rounds rounds;
+  if ((rc = rounds.alloc(mem, "gbo_pagerank"))) return rc;
   float* y = x + n;
   PlanGuard g(st);
   if ((rc = acquire_plan(AT, &g.pv, st))) return rc;
@@ -901,22 +985,35 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   lists_build(AT, true, mem, &lists, st);
   int32_t it = 0;
   double delta = 0.0;
-  float* p = d_p;
-  float* q = y;  // next iterate
-  k_pr_scale<<<blocks_n, 256, 0, st>>>(p, d_outdeg, alpha, x, n);
+  k_pr_scale<<<blocks_n, 256, 0, st>>>(d_p, d_outdeg, alpha, x, n);
   GBO_LAUNCH_CHECK();
-  while (it < max_iter) {
-    a.xval = x;
-    a.out = q;
-    if ((rc = sweep(AT->bs, OP_SUM, a, lists, st))) return rc;
-    k_pr_tail<<<lblocks, 256, 0, st>>>(q, p, d_outdeg, alpha, x, n, dpart);  // x for the next iteration
-    k_sum_partials<<<1, 256, 0, st>>>(dpart, (int)lblocks, dpart + nparts);
-    GBO_LAUNCH_CHECK();
-    if ((rc = read_back(&delta, dpart + nparts, sizeof(double), st))) return rc;
-    ++it;
-    std::swap(p, q);
-    if (delta < tol) break;
+  for (bool more = true; more && it < max_iter;) {
+    int nb = 0;
+    if ((rc = rounds.batch(it, &nb, st))) return rc;
+    nb = std::min(nb, max_iter - it);
+    for (int k = 0; k < nb; ++k) {
+      // iterate it + k is in d_p where that is even, else in y
+      const float* from = (it + k) % 2 ? y : d_p;
+      float* to = (it + k) % 2 ? d_p : y;
+      a.xval = x;
+      a.out = to;
+      a.go = rounds.go(k);
+      if ((rc = sweep(AT->bs, OP_SUM, a, lists, st))) return rc;
+      // x for the next iteration, the change of this one
+      if (n <= kOneBlock) {
+        k_pr_tail<1024><<<1, 1024, 0, st>>>(to, from, d_outdeg, alpha, x, n, tol, rounds.value(k), a.go, rounds.again(k));
+      } else {
+        k_pr_tail<256><<<lblocks, 256, 0, st>>>(to, from, d_outdeg, alpha, x, n, tol, dpart, a.go, nullptr);
+        k_sum_partials<<<1, 256, 0, st>>>(dpart, (int)lblocks, tol, rounds.value(k), a.go, rounds.again(k));
+      }
+      GBO_LAUNCH_CHECK();
+    }
+    int ran = 0;
+    if ((rc = rounds.look(nb, &ran, &more, st))) return rc;
+    it += ran;
+    delta = rounds.h[ran - 1].value;
   }
+  const float* p = it % 2 ? y : d_p;
   if (p != d_p) {
     GBO_HIP_CHECK(hipMemcpyAsync(d_p, p, sizeof(float) * n, hipMemcpyDeviceToDevice, st));
     GBO_HIP_CHECK(hipStreamSynchronize(st));
@@ -937,13 +1034,13 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   hipStream_t st = stream;
   Workspace mem(st);
   int32_t* gf = nullptr;
-  unsigned long long* changed = nullptr;
+  Rounds rounds;
   if ((rc = mem.alloc(&gf, sizeof(int32_t) * (size_t)n * 2, "gbo_cc"))) return rc;
-  if ((rc = mem.alloc(&changed, sizeof(unsigned long long), "gbo_cc"))) return rc;
+  if ((rc = rounds.alloc(mem, "gbo_cc"))) return rc;
   int32_t* mngf = gf + n;
   int32_t* f = d_label;
   const unsigned blocks_n = (unsigned)((n + 255) / 256);
-  k_iota<<<blocks_n, 256, 0, st>>>(f, gf, n);
+  k_cc_init<<<blocks_n, 256, 0, st>>>(f, gf, mngf, n);
   GBO_LAUNCH_CHECK();
   PlanGuard g(st);
   if ((rc = acquire_plan(A, &g.pv, st))) return rc;
@@ -965,27 +1062,31 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   ListView lists;
   lists_build(A, false, mem, &lists, st);
   int32_t it = 0;
-  while (true) {
-    a.xval = gf;
-    a.out = mngf;
-    if ((rc = sweep(A->bs, OP_MIN, a, lists, st))) return rc;
-    k_cc_hook<<<blocks_n, 256, 0, st>>>(mngf, gf, f, n);
-    GBO_HIP_CHECK(hipMemsetAsync(changed, 0, sizeof(unsigned long long), st));
-    k_cc_grand<<<blocks_n, 256, 0, st>>>(f, gf, n, changed);
-    GBO_LAUNCH_CHECK();
-    ++it;
-    uint64_t h = 0;
-    if ((rc = read_u64(changed, &h, st))) return rc;
-    if (h == 0) break;
-    if (it > n + 2) return set_error(GBO_ENOCONV, "gbo_cc: no convergence");
+  a.prefilled = 1;
+  for (bool more = true; more;) {
+    int nb = 0;
+    if ((rc = rounds.batch(it, &nb, st))) return rc;
+    for (int k = 0; k < nb; ++k) {
+      a.xval = gf;
+      a.out = mngf;
+      a.go = rounds.go(k);
+      if ((rc = sweep(A->bs, OP_MIN, a, lists, st))) return rc;
+      k_cc_hook<<<blocks_n, 256, 0, st>>>(mngf, gf, f, n, a.go);
+      k_cc_grand<<<blocks_n, 256, 0, st>>>(f, gf, n, a.go, rounds.again(k));
+      GBO_LAUNCH_CHECK();
+    }
+    int ran = 0;
+    if ((rc = rounds.look(nb, &ran, &more, st))) return rc;
+    it += ran;
+    if (more && it > n + 2) return set_error(GBO_ENOCONV, "gbo_cc: no convergence");
   }
-  while (true) {  // make every tree a star
-    GBO_HIP_CHECK(hipMemsetAsync(changed, 0, sizeof(unsigned long long), st));
-    k_cc_jump<<<blocks_n, 256, 0, st>>>(f, n, changed);
+  for (bool more = true; more;) {  // make every tree a star
+    int nb = 0;
+    if ((rc = rounds.batch(0, &nb, st))) return rc;
+    for (int k = 0; k < nb; ++k) k_cc_jump<<<blocks_n, 256, 0, st>>>(f, n, rounds.go(k), rounds.again(k));
     GBO_LAUNCH_CHECK();
-    uint64_t h = 0;
-    if ((rc = read_u64(changed, &h, st))) return rc;
-    if (h == 0) break;
+    int ran = 0;
+    if ((rc = rounds.look(nb, &ran, &more, st))) return rc;
   }
   if (h_iters) *h_iters = it;
   return GBO_OK;

@@ -78,7 +78,7 @@ __device__ __forceinline__ T ld_tile_meta(const T* p, int64_t i) {
   else return p[i];
 }
 
-template <int BS, int OP>
+template <int BS, int OP, bool GO = false>
 __global__ __launch_bounds__(256) void k_spmv(const SpmvArgs a) {
   using W = word_t<BS>;
   constexpr int G = kWave / BS;
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) void k_spmv(const SpmvArgs a) {
   // wave-uniform for the scalar loads below
   const int g = BS == 64 ? 0 : lane / BS, r = lane % BS;
   const int c = wave_index();
-  if (c >= a.nchunks) return;  // wave-uniform
+  if (c >= a.nchunks || (GO && over(a.go))) return;  // wave-uniform
   const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const W* __restrict__ tiles = (const W*)a.tiles;
@@ -1309,7 +1309,7 @@ __global__ __launch_bounds__(256) void k_count32q(const SpmvArgs a) {
 // only the weighted min-plus gains (6.77 -> 5.60 ms); min, the sum and the
 // unit-weight min-plus are faster on the row-group kernel, whose per-tile
 // reads are scalar there.
-template <int BS, int OP>
+template <int BS, int OP, bool GO>
 __global__ __launch_bounds__(256) void k_value_q(const SpmvArgs a) {
   static_assert(BS == 16 || BS == 32 || BS == 64, "four rows per lane");
   using RW = typename std::conditional<BS == 64, uint64_t, uint32_t>::type;  // row word
@@ -1323,7 +1323,7 @@ __global__ __launch_bounds__(256) void k_value_q(const SpmvArgs a) {
   const int lane = lane_id();
   const int slot = lane / LPT, p = lane % LPT;
   const int c = wave_index();
-  if (c >= a.nchunks) return;  // wave-uniform
+  if (c >= a.nchunks || (GO && over(a.go))) return;  // wave-uniform
   const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const int32_t* __restrict__ colind = a.colind;
@@ -1527,7 +1527,7 @@ __device__ __forceinline__ uint32_t flip_rows(uint32_t v) {
   return BS == 8 ? __builtin_bswap32(v) : (v << 16) | (v >> 16);
 }
 
-template <int BS, int OP>
+template <int BS, int OP, bool GO>
 __global__ __launch_bounds__(256) void k_value_lpt(const SpmvArgs a) {
   static_assert(BS == 8 || BS == 16, "lane-per-tile tiles of 8 or 32 bytes");
   static_assert(OP == OP_MIN || OP == OP_MINPLUS || OP == OP_SUM, "min / min-plus / sum only");
@@ -1549,7 +1549,7 @@ __global__ __launch_bounds__(256) void k_value_lpt(const SpmvArgs a) {
   const int lane = lane_id();
   const int wv = threadIdx.x / kWave;
   const int c = wave_index();
-  if (c >= a.nchunks) return;  // wave-uniform; no workgroup barriers below
+  if (c >= a.nchunks || (GO && over(a.go))) return;  // wave-uniform; no workgroup barriers below
   const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const int32_t* __restrict__ colind = a.colind;
@@ -1761,8 +1761,9 @@ __global__ __launch_bounds__(256) void k_prefill_split(const SpmvArgs a) {
 // shuffles need every lane.
 constexpr int kOwnTail = 5;
 
-template <int BS>
+template <int BS, bool GO>
 __global__ __launch_bounds__(256) void k_sum_fixup(const SpmvArgs a) {
+  if (GO && over(a.go)) return;
   constexpr int G = kWave / BS, U = 8;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t c = min(idx / BS, (int64_t)a.nchunks - 2);  // nchunks >= 2
@@ -1832,6 +1833,18 @@ __global__ __launch_bounds__(256) void k_bfs_pack(const int32_t* __restrict__ cn
   if (lane_id() == 0 && added) atomicAdd(&slots[(R / kWave) & (kCountSlots - 1)], (unsigned long long)added);
 }
 
+// Min, min-plus and sum: the set-bit list kernel at bs 8/16 (variant 3, their
+// default), four rows a lane at bs 32 and where weights are read at bs 64.
+template <int BS, int OP, bool GO>
+static void launch_value(const SpmvArgs& a, bool aligned, unsigned blocks, hipStream_t st) {
+  if constexpr (BS <= 16) {
+    if (a.variant == 3 && aligned) return k_value_lpt<BS, OP, GO><<<blocks, 256, 0, st>>>(a);
+  } else if constexpr (BS == 32 || OP == OP_MINPLUS) {
+    if (aligned && (BS == 32 || a.w)) return k_value_q<BS, OP, GO><<<blocks, 256, 0, st>>>(a);
+  }
+  k_spmv<BS, OP, GO><<<blocks, 256, 0, st>>>(a);
+}
+
 template <int BS, int OP>
 static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
   // the streamed and multi-row-per-lane kernels (variants 2 and 3, the bs
@@ -1864,7 +1877,8 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
       return GBO_OK;
     }
   }
-  const bool need_prefill = OP == OP_BFS || OP == OP_MINPLUS || OP == OP_MIN || (OP == OP_COUNT && !a.accumulate);
+  const bool need_prefill = OP == OP_BFS || ((OP == OP_MINPLUS || OP == OP_MIN) && !a.prefilled) ||
+                            (OP == OP_COUNT && !a.accumulate);
   if (need_prefill && a.nchunks > 1) {
     const int64_t n = (int64_t)(a.nchunks - 1) * BS;
     k_prefill_split<BS, OP><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
@@ -1890,16 +1904,9 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
   } else if constexpr (BS <= 16 && OP == OP_BFS) {
     if (lpt) k_spmv_lpt<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
     else k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
-  } else if constexpr (BS <= 16 && (OP == OP_MIN || OP == OP_MINPLUS || OP == OP_SUM)) {
-    // variant 3 (the bs 8/16 default): the set-bit list kernel
-    if (a.variant == 3 && aligned) k_value_lpt<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
-    else k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
-  } else if constexpr (BS == 32 && (OP == OP_MIN || OP == OP_MINPLUS || OP == OP_SUM)) {
-    if (aligned) k_value_q<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
-    else k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
-  } else if constexpr (BS == 64 && OP == OP_MINPLUS) {
-    if (aligned && a.w) k_value_q<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
-    else k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
+  } else if constexpr (OP == OP_MIN || OP == OP_MINPLUS || OP == OP_SUM) {
+    if (a.go) launch_value<BS, OP, true>(a, aligned, (unsigned)blocks, st);
+    else launch_value<BS, OP, false>(a, aligned, (unsigned)blocks, st);
   } else if constexpr (BS == 32 && OP == OP_COUNT) {
     if (aligned) k_count32q<<<(unsigned)blocks, 256, 0, st>>>(a);
     else k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
@@ -1909,7 +1916,8 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
   GBO_LAUNCH_CHECK();
   if (OP == OP_SUM && a.nchunks > 1) {
     const int64_t n = (int64_t)(a.nchunks - 1) * BS;
-    k_sum_fixup<BS><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
+    if (a.go) k_sum_fixup<BS, true><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
+    else k_sum_fixup<BS, false><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
     GBO_LAUNCH_CHECK();
   }
   return GBO_OK;

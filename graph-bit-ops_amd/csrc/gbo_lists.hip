@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256) void k_list_sweep(const ListView l, const List
   T* acc = sh[threadIdx.x / kWave];
   const int lane = lane_id();
   const int64_t k = wave_index();
-  if (k >= l.nparts) return;
+  if (k >= l.nparts || over(s.go)) return;
   const ListPart P = l.parts[k];
   acc[lane] = A::none();
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -358,6 +358,7 @@ __global__ __launch_bounds__(kFoldThreads) void k_list_fold(const ListView l, co
   using T = typename A::T;
   constexpr int G = kFoldThreads / kWin, U = 4;
   __shared__ T sh[G][kWin];
+  if (over(s.go)) return;
   const int64_t w = l.multi[blockIdx.x];
   const int g = threadIdx.x / kWin, r = threadIdx.x % kWin;
   const int64_t i0 = l.first[w], i1 = l.first[w + 1];

@@ -212,6 +212,7 @@ struct ListSweep {
   const uint32_t* w;
   const int64_t* woff;
   float scale, bias;  // sum: scale * (A x) + bias
+  const unsigned long long* go;
 };
 void lists_build(const gbo_bsr* A, bool many, Workspace& mem, ListView* out, hipStream_t st);
 // OP_SUM, OP_MIN, or OP_MINPLUS without the vertex's own value.
@@ -253,7 +254,14 @@ struct SpmvArgs {
                         // block column's frontier word is nonzero (row-group kernel)
   int accumulate;       // COUNT: add into y
   float scale, bias;    // SUM: y = scale * (A x) + bias  (scale 1, bias 0 for the plain op)
+  const unsigned long long* go;  // MINPLUS / SUM / MIN: nothing is done where *go is 0 (nullable; kernels of their
+                                 // own, the look costs a plain product 0.2 us a launch)
+  int prefilled;        // MINPLUS / MIN: `out` holds the identity where rows are split
 };
+
+// The iteration before this one was the last: a driver queues a few iterations
+// between two looks at their flags, and those past the end do nothing.
+__device__ __forceinline__ bool over(const unsigned long long* go) { return go && *go == 0; }
 
 // First tile of chunk c, for c up to nchunks.  The even form is kept apart
 // because it needs no load before the chunk's tiles can be asked for.
