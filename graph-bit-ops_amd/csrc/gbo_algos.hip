@@ -694,46 +694,6 @@ __global__ void k_cc_init(int32_t* a, int32_t* b, int32_t* m, int32_t n) {
   }
 }
 
-// The flags of the iterations queued between two looks at them: iteration k
-// runs only if flag k - 1 of its batch is set, and sets flag k if another is to
-// follow.  A look costs about 12 us with the stream's gap; an iteration past the
-// end a few launches that do nothing, so that batches grow with the iterations
-// there have been: by half of them.
-struct Rounds {
-  static constexpr int kMax = 32, kFlags = 1024;
-  struct Flag {
-    unsigned long long again;
-    double value;
-  };
-  Flag* flags = nullptr;
-  int at = kFlags;  // first flag of the batch
-  Flag h[kMax];
-
-  int alloc(Workspace& mem, const char* who) { return mem.alloc(&flags, sizeof(Flag) * kFlags, who); }
-  // iterations to queue after `done`; their flags are clear
-  int batch(int done, int* n, hipStream_t st) {
-    *n = done == 0 ? 3 : std::min(std::max(2, done / 2), kMax);
-    if (at + *n > kFlags) {
-      GBO_HIP_CHECK(hipMemsetAsync(flags, 0, sizeof(Flag) * kFlags, st));
-      at = 0;
-    }
-    return GBO_OK;
-  }
-  const unsigned long long* go(int k) const { return k ? &flags[at + k - 1].again : nullptr; }
-  unsigned long long* again(int k) const { return &flags[at + k].again; }
-  double* value(int k) const { return &flags[at + k].value; }
-  // iterations of the batch of n that ran; *more: the last of them asks for another
-  int look(int n, int* ran, bool* more, hipStream_t st) {
-    const int rc = read_back(h, flags + at, sizeof(Flag) * n, st);
-    if (rc) return rc;
-    at += n;
-    *ran = 1;
-    while (*ran < n && h[*ran - 1].again) ++*ran;
-    *more = h[*ran - 1].again != 0;
-    return GBO_OK;
-  }
-};
-
 // One product of a driver, over the edge lists where it has them.
 static int sweep(int bs, int op, const SpmvArgs& a, const ListView& lists, hipStream_t st) {
   if (!lists.on) return spmv_launch(bs, op, a, st);
@@ -911,7 +871,7 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   a.w = d_w;
   a.woff = d_woff;
   ListView lists;
-  lists_build(AT, true, mem, &lists, st);
+  lists_build(AT, ListUse::kMany, mem, &lists, st);
   int32_t it = 0;
   unsigned long long *act_cur = active, *act_next = active2;
   const unsigned blocks_u = (unsigned)(((int64_t)n + kSsspThreads - 1) / kSsspThreads);
@@ -982,7 +942,7 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   const unsigned blocks_n = (unsigned)((n + 255) / 256);
   const unsigned lblocks = (unsigned)std::min<int64_t>(nparts, (n + 255) / 256);
   ListView lists;
-  lists_build(AT, true, mem, &lists, st);
+  lists_build(AT, ListUse::kMany, mem, &lists, st);
   int32_t it = 0;
   double delta = 0.0;
   k_pr_scale<<<blocks_n, 256, 0, st>>>(d_p, d_outdeg, alpha, x, n);
@@ -1060,7 +1020,7 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
   ListView lists;
-  lists_build(A, false, mem, &lists, st);
+  lists_build(A, ListUse::kFew, mem, &lists, st);
   int32_t it = 0;
   a.prefilled = 1;
   for (bool more = true; more;) {

@@ -34,7 +34,15 @@ struct MsArgs {
   const uint64_t* V;       // n * KW
   uint64_t* Fn;            // n * KW (next frontier, masked by ~V)
   const uint64_t* active;  // per block column bit
+  const uint64_t* live;    // KW: the sources that have a frontier
+  const unsigned long long* go;  // as in SpmvArgs
 };
+
+// A row that every source with a frontier has visited gains nothing from its
+// neighbours: its bits are left out (and with all rows of a block row its
+// tiles).  256 sources on R-MAT 2^18, half of them isolated vertices, sweeps
+// over the tiles: bs 8 1.76 -> 1.46 ms a call, bs 64 3.01 -> 2.92.
+
 
 template <int BS, int KW>
 __global__ __launch_bounds__(256) void k_msbfs(const MsArgs a) {
@@ -43,10 +51,13 @@ __global__ __launch_bounds__(256) void k_msbfs(const MsArgs a) {
   const int lane = lane_id();
   const int g = lane / BS, r = lane % BS;
   const int c = wave_index();
-  if (c >= a.nchunks) return;
+  if (c >= a.nchunks || over(a.go)) return;
   const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const W* __restrict__ tiles = (const W*)a.tiles;
+  uint64_t live[KW];
+#pragma unroll
+  for (int w = 0; w < KW; ++w) live[w] = a.live[w];
 
   for (int32_t R0 = a.plan[c]; R0 < a.nbr;) {
     const int32_t Rl = R0 + lane;
@@ -73,16 +84,22 @@ __global__ __launch_bounds__(256) void k_msbfs(const MsArgs a) {
       const int64_t s = rs > cb ? rs : cb;
       const int64_t te = re < ce ? re : ce;
       const bool full = (rs >= cb) && (re <= ce);
-      uint64_t acc[KW];
+      const int64_t i = (int64_t)R * BS + r;
+      uint64_t acc[KW], open[KW], any = 0;
 #pragma unroll
-      for (int w = 0; w < KW; ++w) acc[w] = 0;
+      for (int w = 0; w < KW; ++w) {
+        acc[w] = 0;
+        open[w] = i < a.nrows ? live[w] & ~a.V[i * KW + w] : 0;
+        any |= open[w];
+      }
+      const int64_t tend = __any(any != 0) ? te : s;  // none of the block row's rows: no tiles
       // Four tiles per group and round: their column indices, then their
       // activity bits, then the words of the active ones (inactive block
       // columns hold no frontier bit: their tiles are not read), then one
       // set bit of each tile per pass with its KW frontier words, so the
       // loads of a stage are in flight together.
       constexpr int U = 4;
-      for (int64_t t = s + g; t < te; t += U * G) {
+      for (int64_t t = s + g; t < tend; t += U * G) {
         int32_t cc[U];
         uint64_t wd[U];
 #pragma unroll
@@ -91,7 +108,7 @@ __global__ __launch_bounds__(256) void k_msbfs(const MsArgs a) {
         for (int u = 0; u < U; ++u) {
           wd[u] = 0;
           if (cc[u] >= 0 && ((a.active[cc[u] >> 6] >> (cc[u] & 63)) & 1ull))  // group-uniform
-            wd[u] = (uint64_t)tiles[(t + u * G) * BS + r];
+            wd[u] = any ? (uint64_t)tiles[(t + u * G) * BS + r] : 0;
         }
         while (wd[0] | wd[1] | wd[2] | wd[3]) {
           uint64_t f[U][KW];
@@ -116,11 +133,10 @@ __global__ __launch_bounds__(256) void k_msbfs(const MsArgs a) {
 #pragma unroll
       for (int w = 0; w < KW; ++w)
         for (int off = BS; off < kWave; off <<= 1) acc[w] |= (uint64_t)__shfl_xor((long long)acc[w], off);
-      const int64_t i = (int64_t)R * BS + r;
       if (g == 0 && i < a.nrows) {
 #pragma unroll
         for (int w = 0; w < KW; ++w) {
-          const uint64_t m = acc[w] & ~a.V[i * KW + w];
+          const uint64_t m = acc[w] & open[w];
           if (full) a.Fn[i * KW + w] = m;
           else if (m) atomicOr((unsigned long long*)&a.Fn[i * KW + w], (unsigned long long)m);
         }
@@ -148,10 +164,11 @@ __global__ __launch_bounds__(256) void k_msbfs8r(const MsArgs a) {
   const bool wok = wi < KW;
   uint32_t* __restrict__ list = lists[threadIdx.x / kWave];
   const int c = wave_index();
-  if (c >= a.nchunks) return;
+  if (c >= a.nchunks || over(a.go)) return;
   const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const uint64_t* __restrict__ tw = (const uint64_t*)a.tiles;
+  const uint64_t live = wok ? a.live[wi] : 0;
 
   for (int32_t R0 = a.plan[c]; R0 < a.nbr;) {
     const int32_t Rl = R0 + lane;
@@ -179,12 +196,21 @@ __global__ __launch_bounds__(256) void k_msbfs8r(const MsArgs a) {
       const int64_t te = re < ce ? re : ce;
       const bool full = (rs >= cb) && (re <= ce);
       uint64_t acc = 0;
-      for (int64_t b = s; b < te; b += kWave) {
+      const int64_t i = (int64_t)R * BS + row;
+      const uint64_t open = wok && i < a.nrows ? live & ~a.V[i * KW + wi] : 0;
+      uint64_t need = __ballot(open != 0);  // bits 8 r .. 8 r + 7 are tile row r's lanes
+      need |= need >> 4;
+      need |= need >> 2;
+      need |= need >> 1;
+      need = (need & 0x0101010101010101ull) * 0xFF;
+      const int64_t tend = need ? te : s;
+      for (int64_t b = s; b < tend; b += kWave) {
         const int64_t nt = min((int64_t)kWave, te - b);
         const int32_t col = lane < nt ? a.colind[b + lane] : -1;
         const bool act = col >= 0 && ((a.active[col >> 6] >> (col & 63)) & 1ull);
-        const uint64_t word = act ? tw[b + lane] : 0ull;
+        const uint64_t word = act ? tw[b + lane] & need : 0ull;
         const uint32_t vb = act ? (uint32_t)col * BS + (BS - 1) : 0u;
+        if (!__any(word != 0)) continue;
         int maxlen = 0, mylen = 0;
         {
           uint32_t tot[4];
@@ -235,9 +261,8 @@ __global__ __launch_bounds__(256) void k_msbfs8r(const MsArgs a) {
         }
       }
       acc |= (uint64_t)__shfl_xor((long long)acc, 4);  // the two parities
-      const int64_t i = (int64_t)R * BS + row;
       if (par == 0 && wok && i < a.nrows) {
-        const uint64_t m = acc & ~a.V[i * KW + wi];
+        const uint64_t m = acc & open;
         if (full) a.Fn[i * KW + wi] = m;
         else if (m) atomicOr((unsigned long long*)&a.Fn[i * KW + wi], (unsigned long long)m);
       }
@@ -247,63 +272,80 @@ __global__ __launch_bounds__(256) void k_msbfs8r(const MsArgs a) {
   }
 }
 
-// Zero the next-frontier words of rows cut by chunk boundaries (they are
-// OR-ed atomically by several waves).
-template <int BS, int KW>
-__global__ __launch_bounds__(256) void k_ms_prefill(const MsArgs a) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t c = idx / BS;
-  const int r = (int)(idx % BS);
-  if (c + 1 >= a.nchunks) return;
-  const int32_t R = a.plan[c + 1];
-  if (a.tail[c] == 0) return;
-  const int64_t i = (int64_t)R * BS + r;
-  if (i < a.nrows)
-    for (int w = 0; w < KW; ++w) a.Fn[i * KW + w] = 0;
-}
-
-// V |= Fn; level[s][v] = lvl for every new (s, v); next activity mask;
-// *count = 1 if any (s, v) is new.
+// V |= Fn; level[s][v] = lvl for every new (s, v); next activity mask; the
+// sources with a new vertex; *again = 1 if there is any.  The old frontier's words are
+// zeroed: the next sweep ORs the rows that chunk boundaries cut into them.
+constexpr int kMsThreads = 512;  // vertices of whole bytes of the activity mask
 template <int KW>
-__global__ __launch_bounds__(256) void k_ms_update(const uint64_t* __restrict__ Fn, uint64_t* __restrict__ V,
-                                                   int32_t* __restrict__ level, int32_t n, int32_t nsrc, int bs,
-                                                   int32_t lvl, unsigned long long* __restrict__ active,
-                                                   unsigned long long* __restrict__ count) {
+__global__ __launch_bounds__(kMsThreads) void k_ms_update(const uint64_t* __restrict__ Fn, uint64_t* __restrict__ F,
+                                                          uint64_t* __restrict__ V, int32_t* __restrict__ level,
+                                                          int32_t n, int bs, int32_t lvl,
+                                                          unsigned char* __restrict__ active,
+                                                          unsigned long long* __restrict__ live,  // 3 of KW, in turn
+                                                          const unsigned long long* __restrict__ go,
+                                                          unsigned long long* __restrict__ again) {
+  __shared__ int sh[kMsThreads / kWave];
+  __shared__ unsigned long long found[KW];
+  if (over(go)) return;
+  if (threadIdx.x < KW) found[threadIdx.x] = 0;
+  __syncthreads();
   const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint64_t cnt = 0, act = 0;
-  if (v < n) {
-    bool any = false;
+  uint64_t m[KW];
 #pragma unroll
-    for (int w = 0; w < KW; ++w) {
-      uint64_t m = Fn[v * KW + w];
-      if (!m) continue;
-      any = true;
-      V[v * KW + w] |= m;
-      cnt += __popcll(m);
-      while (m) {
-        const int b = __builtin_ctzll(m);
-        m &= m - 1;
-        level[(int64_t)(w * 64 + b) * n + v] = lvl;
-      }
-    }
-    if (any) act = 1ull << ((v / bs) & 63);
+  for (int w = 0; w < KW; ++w) {
+    m[w] = v < n ? Fn[v * KW + w] : 0;
+    if (v < n) F[v * KW + w] = 0;
   }
-  // the 64 vertices of a wave (64-aligned) fall in one word of the block
-  // column mask
-  const uint64_t m = wave_or64(act);
-  if (lane_id() == 0 && m) atomicOr(&active[((v - lane_id()) / bs) >> 6], m);
-  wave_flag(cnt != 0, count);
+  bool any = false;
+#pragma unroll
+  for (int w = 0; w < KW; ++w) {
+    if (!__any(m[w] != 0)) continue;
+    uint64_t all = wave_or64(m[w]);
+    if (lane_id() == 0) atomicOr(&found[w], (unsigned long long)all);
+    if (m[w]) {
+      any = true;
+      V[v * KW + w] |= m[w];
+    }
+    // one source at a time: its new vertices' levels are neighbours
+    while (all) {
+      const int b = __builtin_ctzll(all);
+      all &= all - 1;
+      if ((m[w] >> b) & 1) level[(int64_t)(w * 64 + b) * n + v] = lvl;
+    }
+  }
+  // as in the shortest paths' update: 64 / bs bits of each wave
+  const int per = kWave / bs;
+  const unsigned long long act = __ballot(any);
+  if (lane_id() == 0) {
+    int bits = 0;
+    for (int k = 0; k < per; ++k) bits |= (act >> (k * bs) & (~0ull >> (kWave - bs))) ? 1 << k : 0;
+    sh[threadIdx.x / kWave] = bits;
+  }
+  wave_flag(any, again);
+  __syncthreads();
+  if ((int)threadIdx.x < per) {
+    int byte = 0;
+    for (int k = 0; k < 8 / per; ++k) byte |= sh[threadIdx.x * (8 / per) + k] << (k * per);
+    active[(int64_t)blockIdx.x * per + threadIdx.x] = (unsigned char)byte;
+  }
+  if (threadIdx.x < KW) {
+    unsigned long long* next = live + (lvl % 3) * KW + threadIdx.x;
+    const unsigned long long add = found[threadIdx.x] & ~*next;  // mostly there already
+    if (add) atomicOr(next, add);
+    if (blockIdx.x == 0) live[(lvl + 1) % 3 * KW + threadIdx.x] = 0;
+  }
 }
 
 template <int KW>
 __global__ void k_ms_init(const int32_t* __restrict__ src, int32_t nsrc, uint64_t* F, uint64_t* V, int32_t* level,
-                          int32_t n, int bs, unsigned long long* active) {
+                          int32_t n, int bs, unsigned long long* active, unsigned long long* live) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nsrc) return;
   const int64_t v = src[s];
   atomicOr((unsigned long long*)&F[v * KW + s / 64], 1ull << (s % 64));
   atomicOr((unsigned long long*)&V[v * KW + s / 64], 1ull << (s % 64));
   level[(int64_t)s * n + v] = 0;
+  atomicOr(&live[s / 64], 1ull << (s % 64));
   const int64_t J = v / bs;
   atomicOr(&active[J >> 6], 1ull << (J & 63));
 }
@@ -317,16 +359,18 @@ static int msbfs_t(const gbo_bsr* A, const int32_t* h_src, int32_t nsrc, int32_t
   Workspace mem(st);
   uint64_t* buf = nullptr;
   int32_t* d_src = nullptr;
-  int rc = mem.alloc(&buf, sizeof(uint64_t) * (3 * words + 2 * nact + 1), "gbo_bfs_multisource");
+  int rc = mem.alloc(&buf, sizeof(uint64_t) * (3 * words + 2 * nact + 3 * KW), "gbo_bfs_multisource");
   if (rc || (rc = mem.alloc(&d_src, sizeof(int32_t) * nsrc, "gbo_bfs_multisource"))) return rc;
+  Rounds rounds;
+  if ((rc = rounds.alloc(mem, "gbo_bfs_multisource"))) return rc;
   uint64_t *F = buf, *Fn = buf + words, *V = buf + 2 * words;
   unsigned long long* act = (unsigned long long*)(buf + 3 * words);
   unsigned long long* act2 = act + nact;
-  unsigned long long* cnt = (unsigned long long*)(buf + 3 * words + 2 * nact);
+  unsigned long long* live = act + 2 * nact;  // level l's at (l - 1) % 3
   GBO_HIP_CHECK(hipMemcpyAsync(d_src, h_src, sizeof(int32_t) * nsrc, hipMemcpyHostToDevice, st));
-  GBO_HIP_CHECK(hipMemsetAsync(buf, 0, sizeof(uint64_t) * (3 * words + 2 * nact + 1), st));
+  GBO_HIP_CHECK(hipMemsetAsync(buf, 0, sizeof(uint64_t) * (3 * words + 2 * nact + 3 * KW), st));
   GBO_HIP_CHECK(hipMemsetAsync(d_level, 0xFF, sizeof(int32_t) * (size_t)nsrc * n, st));
-  k_ms_init<KW><<<(nsrc + 255) / 256, 256, 0, st>>>(d_src, nsrc, F, V, d_level, n, A->bs, act);
+  k_ms_init<KW><<<(nsrc + 255) / 256, 256, 0, st>>>(d_src, nsrc, F, V, d_level, n, A->bs, act, live);
   GBO_LAUNCH_CHECK();
   PlanGuard g(st);
   if ((rc = acquire_plan(A, &g.pv, st))) return rc;
@@ -343,35 +387,36 @@ static int msbfs_t(const gbo_bsr* A, const int32_t* h_src, int32_t nsrc, int32_t
   a.tail = pv.tail;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
-  int32_t lvl = 0;
-  while (true) {
-    a.F = F;
-    a.V = V;
-    a.Fn = Fn;
-    a.active = (const uint64_t*)act;
-    if (a.nchunks > 1) {
-      const int64_t np = (int64_t)(a.nchunks - 1) * BS;
-      k_ms_prefill<BS, KW><<<(unsigned)((np + 255) / 256), 256, 0, st>>>(a);
+  ListView lists;
+  lists_build(A, ListUse::kFrontiers, mem, &lists, st);
+  int32_t lvl = 0;  // levels done, the last of them empty at the end
+  for (bool more = true; more;) {
+    int nb = 0;
+    if ((rc = rounds.batch(lvl, &nb, st))) return rc;
+    for (int k = 0; k < nb; ++k) {
+      a.F = F;
+      a.V = V;
+      a.Fn = Fn;
+      a.active = (const uint64_t*)act;
+      a.live = (const uint64_t*)live + (lvl + k) % 3 * KW;
+      a.go = rounds.go(k);
+      if (lists.on) {
+        if ((rc = lists_ms(KW, lists, {F, V, Fn, a.active, a.live, a.go}, st))) return rc;
+      } else if (BS == 8)
+        k_msbfs8r<KW><<<(unsigned)(((int64_t)a.nchunks + 3) / 4), 256, 0, st>>>(a);
+      else
+        k_msbfs<BS, KW><<<(unsigned)(((int64_t)a.nchunks + 3) / 4), 256, 0, st>>>(a);
+      k_ms_update<KW><<<(unsigned)(((int64_t)n + kMsThreads - 1) / kMsThreads), kMsThreads, 0, st>>>(
+          Fn, F, V, d_level, n, A->bs, lvl + k + 1, (unsigned char*)act2, live, a.go, rounds.again(k));
+      GBO_LAUNCH_CHECK();
+      std::swap(F, Fn);
+      std::swap(act, act2);
     }
-    if (BS == 8)
-      k_msbfs8r<KW><<<(unsigned)(((int64_t)a.nchunks + 3) / 4), 256, 0, st>>>(a);
-    else
-      k_msbfs<BS, KW><<<(unsigned)(((int64_t)a.nchunks + 3) / 4), 256, 0, st>>>(a);
-    GBO_LAUNCH_CHECK();
-    GBO_HIP_CHECK(hipMemsetAsync(act2, 0, sizeof(unsigned long long) * nact, st));
-    GBO_HIP_CHECK(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), st));
-    ++lvl;
-    k_ms_update<KW><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(Fn, V, d_level, n, nsrc, A->bs, lvl, act2, cnt);
-    GBO_LAUNCH_CHECK();
-    unsigned long long h = 0;
-    if ((rc = read_back(&h, cnt, sizeof(h), st))) return rc;
-    if (h == 0) {
-      --lvl;
-      break;
-    }
-    std::swap(F, Fn);
-    std::swap(act, act2);
+    int ran = 0;
+    if ((rc = rounds.look(nb, &ran, &more, st))) return rc;
+    lvl += ran;
   }
+  --lvl;
   if (h_nlevels) *h_nlevels = lvl + 1;
   return GBO_OK;
 }

@@ -382,6 +382,82 @@ __global__ __launch_bounds__(kFoldThreads) void k_list_fold(const ListView l, co
   }
 }
 
+// ---- frontiers of KW words a vertex (multi-source BFS).  The entries of open
+// rows and active block columns are listed in LDS, kMsStage looked at a time; KW
+// lanes (4 for 3) then gather an entry's words.
+constexpr int kMsStage = 4 * kWave;
+
+template <int KW>
+__global__ __launch_bounds__(256) void k_list_ms(const ListView l, const ListMs s) {
+  constexpr int LPE = KW == 3 ? 4 : KW, EPI = kWave / LPE, U = 4, Q = kMsStage / kWave;
+  __shared__ unsigned long long sacc[4][kWin * KW];
+  __shared__ uint64_t sopen[4][kWin * KW];
+  __shared__ uint32_t sstage[4][kMsStage];
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  unsigned long long* acc = sacc[wave];
+  uint64_t* open = sopen[wave];
+  uint32_t* stage = sstage[wave];
+  const int64_t k = wave_index();
+  if (k >= l.nparts || over(s.go)) return;
+  const ListPart P = l.parts[k];
+  const int64_t i = (int64_t)P.win * kWin + lane;
+  uint64_t any = 0;
+#pragma unroll
+  for (int w = 0; w < KW; ++w) {
+    const uint64_t o = i < l.n ? s.live[w] & ~s.V[i * KW + w] : 0;
+    any |= o;
+    open[lane * KW + w] = o;
+    acc[lane * KW + w] = 0;
+  }
+  const uint64_t rows = __ballot(any != 0);
+  constexpr uint32_t kMask = (1u << kColBits) - 1;
+  const int lgbs = 31 - __builtin_clz(l.bs), wi = lane % LPE;
+  const int n = rows ? P.n : 0;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  for (int p = 0; p < n; p += kMsStage) {
+    uint32_t e[Q];
+    uint64_t act[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) e[q] = P.at[min(p + q * kWave + lane, n - 1)];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const uint32_t J = (e[q] & kMask) >> lgbs;
+      act[q] = s.active[J >> 6] >> (J & 63);
+    }
+    int m = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const bool ok = p + q * kWave + lane < n && (act[q] & (rows >> (e[q] >> kColBits)) & 1);
+      const unsigned long long b = __ballot(ok);
+      if (ok) stage[m + __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0))] = e[q];
+      m += __popcll(b);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    for (int j = lane / LPE; j - lane / LPE < m; j += U * EPI) {
+      uint32_t x[U];
+      uint64_t f[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = stage[min(j + u * EPI, m - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) f[u] = s.F[(int64_t)(x[u] & kMask) * KW + (wi < KW ? wi : 0)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {  // the last entry again past the end: OR
+        const int at = (int)(x[u] >> kColBits) * KW + wi;
+        if (wi < KW && (f[u] & open[at])) atomicOr(&acc[at], (unsigned long long)f[u]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+  if (i >= l.n) return;
+  const bool shared = l.first[P.win + 1] - l.first[P.win] > 1;
+#pragma unroll
+  for (int w = 0; w < KW; ++w) {
+    const unsigned long long m = acc[lane * KW + w] & open[lane * KW + w];
+    if (!shared) s.Fn[i * KW + w] = m;
+    else if (m) atomicOr((unsigned long long*)&s.Fn[i * KW + w], m);
+  }
+}
+
 unsigned grid_of(int64_t items, int per_block) {
   return (unsigned)std::max<int64_t>(1, (items + per_block - 1) / per_block);
 }
@@ -481,11 +557,18 @@ int sweep_t(const ListView& l, const ListSweep& s, hipStream_t st) {
 //   3 to 5 sweeps (components), bs 16: 700 MB 0.80 -> 0.82; bs 32: 207 MB
 //   0.45 -> 0.49, 367 MB 0.62 -> 0.47, 1.9 GB 1.88 -> 1.13; bs 64: 350 MB
 //   0.38 -> 0.39, 761 MB 0.99 -> 0.58, 5.2 GB 2.78 -> 1.77
-void lists_build(const gbo_bsr* A, bool many, Workspace& mem, ListView* out, hipStream_t st) {
+//   256 sources, bs 8: 4 MB 0.36 -> 0.35 ms, 62 MB 1.42 -> 0.75; bs 64, 370 MB
+//   2.24 -> 0.54, 890 MB 2.92 -> 1.07; 128 at bs 8, 19 MB 0.33 -> 0.31; 100 at
+//   bs 16, 3 MB 0.16 -> 0.21
+void lists_build(const gbo_bsr* A, ListUse use, Workspace& mem, ListView* out, hipStream_t st) {
   *out = ListView{};
   const int64_t bytes = A->nblocks * (A->bs * A->bs / 8 + 4), mb = 1 << 20;
-  const int64_t least = many ? (A->bs == 8 ? 192 * mb : A->bs == 16 ? 96 * mb : 48 * mb)
-                             : (A->bs <= 16 ? INT64_MAX : A->bs == 32 ? 256 * mb : 512 * mb);
+  int64_t least = 0;
+  switch (use) {
+    case ListUse::kMany: least = A->bs == 8 ? 192 * mb : A->bs == 16 ? 96 * mb : 48 * mb; break;
+    case ListUse::kFew: least = A->bs <= 16 ? INT64_MAX : A->bs == 32 ? 256 * mb : 512 * mb; break;
+    case ListUse::kFrontiers: least = 16 * mb; break;
+  }
   if (bytes < least || A->nrows > (1 << kColBits) || A->ncols > (1 << kColBits) || ((uintptr_t)A->tiles & 7)) return;
   switch (A->bs) {
     case 8: (void)build_t<8>(A, mem, out, st); break;
@@ -502,6 +585,19 @@ int lists_sweep(int op, const ListView& l, const ListSweep& s, hipStream_t st) {
     case OP_MINPLUS: return sweep_t<OP_MINPLUS>(l, s, st);
   }
   return set_error(GBO_EUNSUPPORTED, "op %d not supported", op);
+}
+
+int lists_ms(int kw, const ListView& l, const ListMs& s, hipStream_t st) {
+  const unsigned blocks = grid_of(l.nparts, 4);
+  switch (kw) {
+    case 1: k_list_ms<1><<<blocks, 256, 0, st>>>(l, s); break;
+    case 2: k_list_ms<2><<<blocks, 256, 0, st>>>(l, s); break;
+    case 3: k_list_ms<3><<<blocks, 256, 0, st>>>(l, s); break;
+    case 4: k_list_ms<4><<<blocks, 256, 0, st>>>(l, s); break;
+    default: return set_error(GBO_EUNSUPPORTED, "%d frontier words not supported", kw);
+  }
+  GBO_LAUNCH_CHECK();
+  return GBO_OK;
 }
 
 }  // namespace gbo

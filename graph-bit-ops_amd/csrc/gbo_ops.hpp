@@ -1,6 +1,7 @@
 // Shared declarations between the packer, the bsrbmv/bsrbmm operations and
 // the drivers (device-side translation units).
 #pragma once
+#include <algorithm>
 
 #include <hip/hip_runtime.h>
 
@@ -177,6 +178,46 @@ int heavy_fill(int bs, int dir, const PackCsr& A, const HeavyRows& h, int32_t nh
 
 constexpr uint32_t kInfU32 = 0xFFFFFFFFu;
 
+// The flags of the iterations queued between two looks at them: iteration k
+// runs only if flag k - 1 of its batch is set, and sets flag k if another is to
+// follow.  A look costs about 12 us with the stream's gap; an iteration past the
+// end a few launches that do nothing, so that batches grow with the iterations
+// there have been: by half of them.
+struct Rounds {
+  static constexpr int kMax = 32, kFlags = 1024;
+  struct Flag {
+    unsigned long long again;
+    double value;
+  };
+  Flag* flags = nullptr;
+  int at = kFlags;  // first flag of the batch
+  Flag h[kMax];
+
+  int alloc(Workspace& mem, const char* who) { return mem.alloc(&flags, sizeof(Flag) * kFlags, who); }
+  // iterations to queue after `done`; their flags are clear
+  int batch(int done, int* n, hipStream_t st) {
+    *n = done == 0 ? 3 : std::min(std::max(2, done / 2), kMax);
+    if (at + *n > kFlags) {
+      GBO_HIP_CHECK(hipMemsetAsync(flags, 0, sizeof(Flag) * kFlags, st));
+      at = 0;
+    }
+    return GBO_OK;
+  }
+  const unsigned long long* go(int k) const { return k ? &flags[at + k - 1].again : nullptr; }
+  unsigned long long* again(int k) const { return &flags[at + k].again; }
+  double* value(int k) const { return &flags[at + k].value; }
+  // iterations of the batch of n that ran; *more: the last of them asks for another
+  int look(int n, int* ran, bool* more, hipStream_t st) {
+    const int rc = read_back(h, flags + at, sizeof(Flag) * n, st);
+    if (rc) return rc;
+    at += n;
+    *ran = 1;
+    while (*ran < n && h[*ran - 1].again) ++*ran;
+    *more = h[*ran - 1].again != 0;
+    return GBO_OK;
+  }
+};
+
 // Edge lists for drivers that sweep one matrix many times (gbo_lists.hip).
 // lists_build leaves `on` false where sweeps over the tiles are to be used:
 // few tiles, mostly dense ones, more than 2^26 rows, no memory.
@@ -214,9 +255,18 @@ struct ListSweep {
   float scale, bias;  // sum: scale * (A x) + bias
   const unsigned long long* go;
 };
-void lists_build(const gbo_bsr* A, bool many, Workspace& mem, ListView* out, hipStream_t st);
+struct ListMs {
+  const uint64_t *F, *V;
+  uint64_t* Fn;  // zero on entry
+  const uint64_t *active, *live;
+  const unsigned long long* go;
+};
+enum class ListUse { kMany, kFew, kFrontiers };  // sweeps of a call: ten and more, a few; multi-source BFS
+void lists_build(const gbo_bsr* A, ListUse use, Workspace& mem, ListView* out, hipStream_t st);
 // OP_SUM, OP_MIN, or OP_MINPLUS without the vertex's own value.
 int lists_sweep(int op, const ListView& l, const ListSweep& s, hipStream_t st);
+// Next frontiers: the unvisited (of the live sources) in-neighbours' words.
+int lists_ms(int kw, const ListView& l, const ListMs& s, hipStream_t st);
 
 constexpr int kCountSlots = 1024;
 
