@@ -426,9 +426,8 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
   a.count_slots = pv.slots;
-  // bs 8/16 variant 3 and bs 32/64: levels while fewer than half the
-  // vertices are visited take the dense step (count kernel + pack); later
-  // ones skip visited rows
+  // bs 8 variant 3: levels while fewer than half the vertices are visited take
+  // the dense step (count kernel + pack); later ones skip visited rows
   int32_t* dense_counts = dense_bfs_step(BS, pv.variant) ? pv.bfs_counts : nullptr;
   int64_t visited = 1;
   int32_t lvl = 0;
@@ -479,11 +478,6 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
       a.visited = vis;
       a.out = nx;
       a.bfs_counts = (dense_counts && visited < (int64_t)n / 2) ? dense_counts : nullptr;
-      // a frontier of f vertices leaves at most f*BS/n of the frontier words
-      // nonzero: below a quarter, tiles are read only under nonzero words
-      // (bs 16-64: R-MAT s22 pull BFS bs 64 23.6 -> 17.6 ms; at bs 8 the dense
-      // count step stays faster than the gated row-group kernel)
-      a.sparse_frontier = BS >= 16 && fsize * BS <= (int64_t)n / 4;
       if ((rc = spmv_launch(BS, OP_BFS, a, st))) return rc;
       if ((rc = count_fold(pv.slots, d_cnt, st))) return rc;
     }

@@ -179,6 +179,7 @@ __global__ __launch_bounds__(256) void k_spmv(const SpmvArgs a) {
           }
         }
       } else if constexpr (OP == OP_BFS) {
+        static_assert(OP != OP_BFS || BS == 8, "k_bfs_scan at the larger block sizes");
         const W* __restrict__ fb = (const W*)a.xbits;
         W* nx = (W*)a.out;
         const W vword = ((const W*)a.visited)[R];
@@ -190,45 +191,20 @@ __global__ __launch_bounds__(256) void k_spmv(const SpmvArgs a) {
         }
         // Tile words and column indices of eight tiles are loaded together,
         // then their frontier words: two dependent loads per eight tiles.
-        // With a sparse frontier the column indices go first, then the
-        // frontier words, and only the tiles whose frontier word is nonzero
-        // are read (group-uniform).
-        // At bs 64 the column indices and frontier words are wave-uniform
-        // and are read with scalar loads (as in the count).
-        auto col_at = [&](int64_t k) -> int32_t { return ld_tile_meta<BS>(colind, k); };
-        auto front_at = [&](int32_t cx) -> W { return ld_tile_meta<BS>(fb, cx); };
         int hit = 0;
         int64_t t = s + g;
-        if (a.sparse_frontier) {
-          for (; t < te; t += 8 * G) {
-            int32_t cc[8];
-            W fw[8];
-            // column and frontier-word loads unconditional (slots past the
-            // row read tile s's) so each stage's loads are in flight together
-#pragma unroll
-            for (int u = 0; u < 8; ++u) cc[u] = col_at(t + u * G < te ? t + u * G : s);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-              const W f = front_at(cc[u]);
-              fw[u] = t + u * G < te ? f : (W)0;
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-              if (fw[u]) hit |= (W)(tiles[(t + u * G) * BS + r] & fw[u]) != 0;
-          }
-        }
         for (; t + 7 * G < te; t += 8 * G) {
           int32_t cc[8];
           W ww[8];
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
-            cc[u] = col_at(t + u * G);
+            cc[u] = colind[t + u * G];
             ww[u] = tiles[(t + u * G) * BS + r];
           }
 #pragma unroll
-          for (int u = 0; u < 8; ++u) hit |= (W)(ww[u] & front_at(cc[u])) != 0;
+          for (int u = 0; u < 8; ++u) hit |= (W)(ww[u] & fb[cc[u]]) != 0;
         }
-        for (; t < te; t += G) hit |= (W)(tiles[t * BS + r] & front_at(col_at(t))) != 0;
+        for (; t < te; t += G) hit |= (W)(tiles[t * BS + r] & fb[colind[t]]) != 0;
         const uint64_t bal = fold_groups<BS>(__ballot(hit));  // row r: any of its lane groups hit
         const uint64_t word = brev_low<BS>(bal) & ~(uint64_t)vword & low_mask<BS>();
         if (lane == 0) {
@@ -490,6 +466,115 @@ __device__ __forceinline__ void load_tile(const void* tiles, int64_t t, uint64_t
     w[2] = ((uint64_t)q1.y << 32) | q1.x;
     w[3] = ((uint64_t)q1.w << 32) | q1.z;
   }
+}
+
+// BFS step at bs 16 to 64: a wave looks at the columns of kScan tiles at a
+// time, a tile a lane, lists those whose frontier word has a bit in LDS, and
+// only these tiles' rows are read, 64 / BS tiles an instruction and four in
+// flight.  A block row is left as soon as its unvisited rows are all found.
+// Levels of one source on R-MAT 2^20 at bs 32 (1.9 GB of tiles), a group of BS
+// lanes per tile before: 211, 411, 330 (every tile, by the count kernel), 190,
+// 118, 106 us; now 68, 174, 323, 144, 60, 56: scanning 59 MB of columns, then
+// the tiles under the frontier.  bs 64 3.0 -> 1.9 ms a call, bs 16 1.20 -> 0.84.
+constexpr int kScan = 4 * kWave;
+template <int BS>
+__global__ __launch_bounds__(256) void k_bfs_scan(const SpmvArgs a) {
+  using W = word_t<BS>;
+  constexpr int G = kWave / BS, Q = kScan / kWave, U = 4;
+  __shared__ int s_tile[4][kScan];
+  __shared__ W s_word[4][kScan];
+  const int lane = lane_id(), g = lane / BS, r = lane % BS;
+  int* stile = s_tile[threadIdx.x / kWave];
+  W* sword = s_word[threadIdx.x / kWave];
+  const int c = wave_index();
+  if (c >= a.nchunks) return;
+  const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
+  const bool last = (c == a.nchunks - 1);
+  const W* __restrict__ tiles = (const W*)a.tiles;
+  const W* __restrict__ fb = (const W*)a.xbits;
+  const W* __restrict__ vis = (const W*)a.visited;
+  const int32_t* __restrict__ colind = a.colind;
+  W* nx = (W*)a.out;
+  int64_t added = 0;
+  for (int32_t R0 = a.plan[c]; R0 < a.nbr;) {
+    const int32_t Rl = R0 + lane;
+    int32_t rsl = 0, rel = 0;
+    uint64_t openl = 0;  // unvisited rows, as in the words
+    if (Rl < a.nbr) {
+      rsl = a.rowptr[Rl];
+      rel = a.rowptr[Rl + 1];
+      const int64_t valid = (int64_t)a.nrows - (int64_t)Rl * BS;
+      openl = ~(uint64_t)vis[Rl] & low_mask<BS>() & ~(valid >= BS ? 0ull : (low_mask<BS>() >> valid));
+    }
+    const bool belong = (Rl < a.nbr) && (last || (int64_t)rsl < ce);
+    const uint64_t bmask = __ballot(belong);
+    // nothing to find: written here unless the row is cut (zero already)
+    if (belong && (rel == rsl || (!openl && rsl >= cb && rel <= ce))) nx[Rl] = (W)0;
+    uint64_t work = __ballot(belong && rel > rsl && openl);
+    while (work) {
+      const int j = __builtin_ctzll(work);
+      work &= work - 1;
+      const int32_t R = R0 + j;
+      const int64_t rs = __builtin_amdgcn_readlane(rsl, j), re = __builtin_amdgcn_readlane(rel, j);
+      const uint64_t open = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)openl, j) |
+                            ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(openl >> 32), j) << 32);
+      const int64_t s = rs > cb ? rs : cb;
+      const int64_t te = re < ce ? re : ce;
+      const bool full = (rs >= cb) && (re <= ce);
+      int hit = 0;
+      uint64_t word = 0;
+      for (int64_t b = s; b < te && word != open; b += kScan) {
+        int32_t cc[Q];
+        W fw[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) cc[q] = colind[min(b + q * kWave + lane, te - 1)];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) fw[q] = fb[cc[q]];
+        int m = 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const bool in = b + q * kWave + lane < te && fw[q] != 0;
+          const unsigned long long any = __ballot(in);
+          if (in) {
+            const int at = m + __builtin_amdgcn_mbcnt_hi((uint32_t)(any >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)any, 0));
+            stile[at] = q * kWave + lane;
+            sword[at] = fw[q];
+          }
+          m += __popcll(any);
+        }
+        if (m == 0) continue;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        for (int k = g; k - g < m; k += U * G) {
+          int64_t t[U];
+          W f[U], w[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int at = min(k + u * G, m - 1);
+            t[u] = b + stile[at];
+            f[u] = sword[at];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) w[u] = tiles[t[u] * BS + r];
+#pragma unroll
+          for (int u = 0; u < U; ++u) hit |= (W)(w[u] & f[u]) != 0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        word = brev_low<BS>(fold_groups<BS>(__ballot(hit))) & open;
+      }
+      if (lane == 0) {
+        if (full) {
+          nx[R] = (W)word;
+          added += popcw((W)word);
+        } else if (word) {
+          const uint64_t old = atomic_or_word<BS>(nx, R, word);
+          added += popcw((W)(word & ~old));
+        }
+      }
+    }
+    if (__popcll(bmask) < kWave) break;
+    R0 += kWave;
+  }
+  if (lane == 0 && added) atomicAdd(&a.count_slots[c & (kCountSlots - 1)], (unsigned long long)added);
 }
 
 template <int BS, int OP>
@@ -1858,14 +1943,12 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
   const bool stream = (BS <= 16 && OP == OP_COUNT && a.variant == 2 && aligned);
   // variant 3 at bs 8 is the lean count kernel; its BFS step is the
   // lane-per-tile kernel (faster than the row-group one at bs 8)
-  const bool lpt = ((BS <= 16 && (OP == OP_COUNT || OP == OP_BFS) && a.variant == 1) ||
-                    (BS == 8 && OP == OP_BFS && a.variant == 3)) &&
-                   !(OP == OP_BFS && a.sparse_frontier);
-  if constexpr (OP == OP_BFS) {
-    if (dense_bfs_step(BS, a.variant) && a.bfs_counts && aligned && !a.sparse_frontier) {
-      // dense step: the count kernel (k_count8 / k_count16q / k_count32q /
-      // k_spmv<64>) gives each row's number of frontier neighbours (every
-      // tile is read; no visited-row skip)
+  const bool lpt = (BS <= 16 && OP == OP_COUNT && a.variant == 1) ||
+                   (BS == 8 && OP == OP_BFS && (a.variant == 1 || a.variant == 3));
+  if constexpr (BS == 8 && OP == OP_BFS) {
+    if (dense_bfs_step(BS, a.variant) && a.bfs_counts && aligned) {
+      // dense step: the count kernel gives each row's number of frontier
+      // neighbours (every tile is read; no visited-row skip)
       SpmvArgs c = a;
       c.out = a.bfs_counts;
       c.accumulate = 0;
@@ -1901,7 +1984,9 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
     } else {
       k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
     }
-  } else if constexpr (BS <= 16 && OP == OP_BFS) {
+  } else if constexpr (OP == OP_BFS && BS >= 16) {
+    k_bfs_scan<BS><<<(unsigned)blocks, 256, 0, st>>>(a);
+  } else if constexpr (OP == OP_BFS) {
     if (lpt) k_spmv_lpt<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
     else k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
   } else if constexpr (OP == OP_MIN || OP == OP_MINPLUS || OP == OP_SUM) {

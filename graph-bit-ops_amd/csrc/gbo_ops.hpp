@@ -25,7 +25,7 @@ namespace gbo {
 //   slots       kCountSlots x u64   BFS frontier-size slots (zero between calls)
 //   count       1 x int64           the folded frontier size
 //   partial     nchunks*2*bs x f64  split-row partials of the FP32 sum
-//   bfs_counts  bs*(nbr+1) x int32  per-row counts of the dense BFS step
+//   bfs_counts  bs*(nbr+1) x int32  per-row counts of the dense BFS step (bs 8)
 // Calls on one matrix therefore share that scratch: they must be ordered
 // (one stream, or synchronised); separately created matrices do not share.
 struct PlanLayout {
@@ -274,9 +274,8 @@ constexpr int kCountSlots = 1024;
 enum SpmvOp { OP_COUNT = 0, OP_BFS = 1, OP_MINPLUS = 2, OP_SUM = 3, OP_MIN = 4 };
 
 // Whether a BFS step at this block size and plan variant may take the dense
-// form (count kernel into per-row counts, then a pack of the nonzero rows):
-// bs 8/16 under variant 3, bs 32/64 under every variant.
-inline bool dense_bfs_step(int bs, int variant) { return (bs <= 16 && variant == 3) || bs >= 32; }
+// form (count kernel into per-row counts, then a pack of the nonzero rows).
+inline bool dense_bfs_step(int bs, int variant) { return bs == 8 && variant == 3; }
 
 struct SpmvArgs {
   const int32_t* rowptr;
@@ -300,8 +299,6 @@ struct SpmvArgs {
                         // the count kernel into it and packs the rows with a nonzero count (dense step)
   double* partial;      // SUM: split-row partials [nchunks][2][bs]
   const uint64_t* active;  // MINPLUS: optional per-block-column activity bits (nullable)
-  int sparse_frontier;  // BFS: most frontier words are zero, so a tile is read only where its
-                        // block column's frontier word is nonzero (row-group kernel)
   int accumulate;       // COUNT: add into y
   float scale, bias;    // SUM: y = scale * (A x) + bias  (scale 1, bias 0 for the plain op)
   const unsigned long long* go;  // MINPLUS / SUM / MIN: nothing is done where *go is 0 (nullable; kernels of their
