@@ -36,12 +36,13 @@ static int fill(T* p, int64_t n, T v, hipStream_t st) {
 
 // ------------------------------------------------------------------ BFS
 template <int BS>
-__global__ __launch_bounds__(256) void k_bfs_init(word_t<BS>* f, word_t<BS>* vis, int32_t* level, int32_t nbr,
+__global__ __launch_bounds__(256) void k_bfs_init(word_t<BS>* f, word_t<BS>* nx, word_t<BS>* vis, int32_t* level, int32_t nbr,
                                                   int32_t n, int32_t source) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nbr) {
     const word_t<BS> w = (i == source / BS) ? (word_t<BS>)(1ull << (BS - 1 - (source % BS))) : (word_t<BS>)0;
     f[i] = w;
+    nx[i] = 0;
     vis[i] = w;
   }
   if (i < n) level[i] = (i == source) ? 0 : -1;
@@ -61,6 +62,41 @@ __global__ __launch_bounds__(256) void k_bfs_update(const word_t<BS>* __restrict
     w &= w - 1;
     const int64_t v = J * BS + (BS - 1 - p);
     if (v < n) level[v] = lvl;
+  }
+}
+
+// The same, counting the new vertices; the old frontier is cleared: the next
+// step ORs the rows that chunk boundaries cut into its words.
+template <int BS>
+__global__ __launch_bounds__(256) void k_bfs_level(const word_t<BS>* __restrict__ next, word_t<BS>* __restrict__ f,
+                                                   word_t<BS>* __restrict__ vis, int32_t* __restrict__ level,
+                                                   int32_t nbr, int32_t n, int32_t lvl,
+                                                   const unsigned long long* __restrict__ go,
+                                                   unsigned long long* __restrict__ count) {
+  __shared__ int sh[256 / kWave];
+  if (over(go)) return;
+  const int64_t J = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  uint64_t w = 0;
+  if (J < nbr) {
+    w = (uint64_t)next[J];
+    f[J] = (word_t<BS>)0;
+  }
+  int added = __popcll(w);
+  if (w) {
+    vis[J] = (word_t<BS>)((uint64_t)vis[J] | w);
+    while (w) {
+      const int p = __builtin_ctzll(w);
+      w &= w - 1;
+      const int64_t v = J * BS + (BS - 1 - p);
+      if (v < n) level[v] = lvl;
+    }
+  }
+  for (int off = 1; off < kWave; off <<= 1) added += __shfl_xor(added, off);
+  if (lane_id() == 0) sh[threadIdx.x / kWave] = added;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int all = sh[0] + sh[1] + sh[2] + sh[3];
+    if (all) atomicAdd(count, (unsigned long long)all);
   }
 }
 
@@ -361,63 +397,24 @@ __global__ __launch_bounds__(256) void k_popc_words(const word_t<BS>* __restrict
 }
 
 // Scratch of a BFS call supplied by the caller of bfs_t instead of being
-// allocated: frontier / next / visited words (3 x nbr words), the frontier-
-// size slots (kCountSlots, cleared on entry) and count, and (where
-// dense_bfs_step holds and they fit) the dense step's row counts (bs x
-// (nbr + 1) int32, else null).
+// allocated: frontier / next / visited words (3 x nbr words), the levels' flags
+// (kBfsFlagBytes) and (where dense_bfs_step holds and they fit) the dense
+// step's row counts (bs x (nbr + 1) int32, else null).
+constexpr size_t kBfsFlagBytes = 8192;
 struct BfsScratch {
   void* words;
-  unsigned long long* slots;
-  int64_t* count;
+  void* flags;
   int32_t* dense_counts;
 };
 
-// Pull BFS over AT; with A (the out-edge matrix, AT itself for an undirected
-// graph) levels whose frontier holds at most n/64 vertices are pushed.  The
-// frontier-size slots and the dense step's row counts come from the plan's
-// scratch; the frontier, next and visited words are this call's -- or, with
-// `ext` (pull only), all of them come from there.
-template <int BS>
-static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t* d_level, int64_t* sizes,
-                 int32_t max_levels, int32_t* nlevels, hipStream_t st, const BfsScratch* ext = nullptr) {
-  using W = word_t<BS>;
-  const int32_t nbr = A->nblockrows, n = A->nrows;
-  Workspace mem(st);
-  W* f = nullptr;
-  int rc;
-  if (ext) {
-    f = (W*)ext->words;
-  } else if ((rc = mem.alloc(&f, sizeof(W) * (size_t)std::max(nbr, 1) * 3 + 64, "gbo_bfs"))) {
-    return rc;
-  }
-  W* nx = f + std::max(nbr, 1);
-  W* vis = nx + std::max(nbr, 1);
-  int32_t *segoff = nullptr, *queue = nullptr;
-  RunState* run = nullptr;
-  if (Aout && ((rc = mem.alloc(&segoff, sizeof(int32_t) * ((size_t)nbr + 1), "gbo_bfs_do")) ||
-               (rc = mem.alloc(&queue, sizeof(int32_t) * kRunBlocks, "gbo_bfs_do")) ||
-               (rc = mem.alloc(&run, sizeof(RunState), "gbo_bfs_do"))))
-    return rc;
-  PlanGuard g(st);
-  if ((rc = acquire_plan(A, &g.pv, st))) return rc;
-  PlanView pv = g.pv;
-  if (ext) {
-    pv.slots = ext->slots;
-    pv.count = ext->count;
-    pv.bfs_counts = ext->dense_counts;
-    GBO_HIP_CHECK(hipMemsetAsync(pv.slots, 0, sizeof(unsigned long long) * kCountSlots, st));
-  }
-  int64_t* d_cnt = pv.count;
-  const unsigned blocks_n = (unsigned)((std::max<int64_t>(n, nbr) + 255) / 256);
-  k_bfs_init<BS><<<blocks_n, 256, 0, st>>>(f, vis, d_level, nbr, n, source);
-  GBO_LAUNCH_CHECK();
+static SpmvArgs bfs_args(const gbo_bsr* A, const PlanView& pv) {
   SpmvArgs a{};
   a.rowptr = A->rowptr;
   a.colind = A->colind;
   a.tiles = A->tiles;
   a.nrows = A->nrows;
   a.ncols = A->ncols;
-  a.nbr = nbr;
+  a.nbr = A->nblockrows;
   a.T = A->nblocks;
   a.plan = pv.plan;
   a.start = pv.start;
@@ -425,6 +422,110 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
+  return a;
+}
+
+// From how many tiles on bs 8 takes the dense step: its kernels have no look at
+// the flags, so its levels are not queued.  Queued, dense: 1.6M tiles (200,000
+// vertices of 8) 216 and 269 us, 1.1M (R-MAT 2^16) 247 and 241, 5.2M (R-MAT
+// 2^18) 490 and 447, 24M 1045 and 958.
+constexpr int64_t kDenseTiles = 2 << 20;
+
+// Pull BFS over AT, several levels between two looks at their sizes: one level
+// of a king grid of 65,536 takes 11 us instead of 26 (bs 16 6.5 -> 2.7 ms).
+// The dense step's row counts come from the plan's scratch; the frontier, next
+// and visited words and the sizes are this call's -- or, with `ext`, all of them
+// come from there.
+template <int BS>
+static int bfs_t(const gbo_bsr* A, int32_t source, int32_t* d_level, int64_t* sizes, int32_t max_levels,
+                 int32_t* nlevels, hipStream_t st, const BfsScratch* ext = nullptr) {
+  using W = word_t<BS>;
+  const int32_t nbr = A->nblockrows, n = A->nrows;
+  Workspace mem(st);
+  W* f = nullptr;
+  Rounds rounds;
+  int rc;
+  if (ext) {
+    f = (W*)ext->words;
+    rounds.place(ext->flags, kBfsFlagBytes);
+  } else if ((rc = mem.alloc(&f, sizeof(W) * (size_t)std::max(nbr, 1) * 3 + 64, "gbo_bfs")) ||
+             (rc = rounds.alloc(mem, "gbo_bfs"))) {
+    return rc;
+  }
+  W* nx = f + std::max(nbr, 1);
+  W* vis = nx + std::max(nbr, 1);
+  PlanGuard g(st);
+  if ((rc = acquire_plan(A, &g.pv, st))) return rc;
+  const unsigned blocks_n = (unsigned)((std::max<int64_t>(n, nbr) + 255) / 256);
+  k_bfs_init<BS><<<blocks_n, 256, 0, st>>>(f, nx, vis, d_level, nbr, n, source);
+  GBO_LAUNCH_CHECK();
+  SpmvArgs a = bfs_args(A, g.pv);
+  a.prefilled = 1;
+  // bs 8 variant 3, large matrices: levels while fewer than half the vertices
+  // are visited take the dense step (count kernel + pack); later ones skip
+  // visited rows
+  int32_t* dense_counts = !dense_bfs_step(BS, g.pv.variant) ? nullptr : ext ? ext->dense_counts : g.pv.bfs_counts;
+  int64_t visited = 1;
+  int32_t lvl = 0;
+  if (sizes && max_levels > 0) sizes[0] = 1;
+  for (bool more = true; more;) {
+    int nb = 0;
+    if ((rc = rounds.batch(lvl, &nb, st))) return rc;
+    const bool dense = dense_counts && A->nblocks >= kDenseTiles && visited < (int64_t)n / 2;
+    if (dense || (BS == 8 && g.pv.variant != 1 && g.pv.variant != 3)) nb = 1;
+    for (int k = 0; k < nb; ++k) {
+      a.xbits = f;
+      a.visited = vis;
+      a.out = nx;
+      a.bfs_counts = dense ? dense_counts : nullptr;
+      a.go = rounds.go(k);
+      if ((rc = spmv_launch(BS, OP_BFS, a, st))) return rc;
+      k_bfs_level<BS><<<(unsigned)((nbr + 255) / 256), 256, 0, st>>>(nx, f, vis, d_level, nbr, n, lvl + k + 1, a.go,
+                                                                     rounds.again(k));
+      GBO_LAUNCH_CHECK();
+      std::swap(f, nx);
+    }
+    int ran = 0;
+    if ((rc = rounds.look(nb, &ran, &more, st))) return rc;
+    for (int k = 0; k < ran && rounds.h[k].again; ++k) {
+      ++lvl;
+      visited += (int64_t)rounds.h[k].again;
+      if (sizes && lvl < max_levels) sizes[lvl] = (int64_t)rounds.h[k].again;
+    }
+  }
+  if (nlevels) *nlevels = lvl + 1;
+  return GBO_OK;
+}
+
+// Direction-optimizing BFS: levels whose frontier holds at most n/64 vertices
+// are pushed over A (the out-edge matrix, AT itself for an undirected graph),
+// the others pulled over AT.  The frontier-size slots and the dense step's row
+// counts come from the plan's scratch.
+template <int BS>
+static int bfs_do_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t* d_level, int64_t* sizes,
+                    int32_t max_levels, int32_t* nlevels, hipStream_t st) {
+  using W = word_t<BS>;
+  const int32_t nbr = A->nblockrows, n = A->nrows;
+  Workspace mem(st);
+  W* f = nullptr;
+  int rc;
+  if ((rc = mem.alloc(&f, sizeof(W) * (size_t)std::max(nbr, 1) * 3 + 64, "gbo_bfs_do"))) return rc;
+  W* nx = f + std::max(nbr, 1);
+  W* vis = nx + std::max(nbr, 1);
+  int32_t *segoff = nullptr, *queue = nullptr;
+  RunState* run = nullptr;
+  if (((rc = mem.alloc(&segoff, sizeof(int32_t) * ((size_t)nbr + 1), "gbo_bfs_do")) ||
+               (rc = mem.alloc(&queue, sizeof(int32_t) * kRunBlocks, "gbo_bfs_do")) ||
+               (rc = mem.alloc(&run, sizeof(RunState), "gbo_bfs_do"))))
+    return rc;
+  PlanGuard g(st);
+  if ((rc = acquire_plan(A, &g.pv, st))) return rc;
+  const PlanView& pv = g.pv;
+  int64_t* d_cnt = pv.count;
+  const unsigned blocks_n = (unsigned)((std::max<int64_t>(n, nbr) + 255) / 256);
+  k_bfs_init<BS><<<blocks_n, 256, 0, st>>>(f, nx, vis, d_level, nbr, n, source);
+  GBO_LAUNCH_CHECK();
+  SpmvArgs a = bfs_args(A, pv);
   a.count_slots = pv.slots;
   // bs 8 variant 3: levels while fewer than half the vertices are visited take
   // the dense step (count kernel + pack); later ones skip visited rows
@@ -435,7 +536,7 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
   if (sizes && max_levels > 0) sizes[0] = 1;
   bool over = false;  // a run of levels left the next one in nx
   while (true) {
-    if (Aout && fsize <= std::min<int64_t>(std::max<int64_t>(n / 64, 1), kRunBlocks)) {
+    if (fsize <= std::min<int64_t>(std::max<int64_t>(n / 64, 1), kRunBlocks)) {
       // a run of small levels in one launch
       GBO_HIP_CHECK(hipMemsetAsync(nx, 0, sizeof(W) * (size_t)std::max(nbr, 1), st));
       GBO_HIP_CHECK(hipMemsetAsync(run, 0, offsetof(RunState, sizes), st));
@@ -462,7 +563,7 @@ static int bfs_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32_t*
       k_popc_words<BS><<<(unsigned)((nbr + 255) / 256), 256, 0, st>>>(nx, nbr, pv.slots);
       GBO_LAUNCH_CHECK();
       if ((rc = count_fold(pv.slots, d_cnt, st))) return rc;
-    } else if (Aout && fsize <= std::max<int64_t>(n / 64, 1)) {
+    } else if (fsize <= std::max<int64_t>(n / 64, 1)) {
       // push: only the frontier rows' tiles of A are read
       GBO_HIP_CHECK(hipMemsetAsync(nx, 0, sizeof(W) * (size_t)std::max(nbr, 1), st));
       k_push_segs<BS><<<(unsigned)(((int64_t)nbr + 1 + 255) / 256), 256, 0, st>>>(f, Aout->rowptr, nbr, segoff);
@@ -735,8 +836,7 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // does not fit.
 static int noalloc_layout(const gbo_bsr* AT, unsigned char* base, BfsScratch* s) {
   const size_t wbytes = (size_t)(AT->bs / 8) * (size_t)std::max(AT->nblockrows, 1) * 3 + 64;
-  const size_t o_count = align256(sizeof(unsigned long long) * kCountSlots);
-  const size_t o_words = o_count + 256;
+  const size_t o_words = kBfsFlagBytes + 256;
   const size_t o_dense = o_words + align256(wbytes);
   // the dense step's row counts (4 bytes a vertex) when they fit as well;
   // without them every level takes the step that skips visited rows (same
@@ -749,8 +849,7 @@ static int noalloc_layout(const gbo_bsr* AT, unsigned char* base, BfsScratch* s)
     return set_error(GBO_ERANGE,
                      "gbo_bfs_noalloc: %d vertices at bs %d need %zu bytes of scratch, the static array holds %zu",
                      AT->nrows, AT->bs, need, kNoAllocScratchBytes);
-  s->slots = (unsigned long long*)base;
-  s->count = (int64_t*)(base + o_count);
+  s->flags = base;
   s->words = base + o_words;
   s->dense_counts = dense ? (int32_t*)(base + o_dense) : nullptr;
   return GBO_OK;
@@ -769,10 +868,10 @@ int gbo_bfs(const gbo_bsr* AT, int32_t source, int32_t* d_level, int64_t* h_leve
   if (source < 0 || source >= AT->nrows) return set_error(GBO_EINVAL, "gbo_bfs: source %d out of range", source);
   if (!d_level) return set_error(GBO_EINVAL, "gbo_bfs: null level");
   switch (AT->bs) {
-    case 8: return bfs_t<8>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
-    case 16: return bfs_t<16>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
-    case 32: return bfs_t<32>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
-    case 64: return bfs_t<64>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 8: return bfs_t<8>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 16: return bfs_t<16>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 32: return bfs_t<32>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 64: return bfs_t<64>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
   }
   return set_error(GBO_EUNSUPPORTED, "gbo_bfs: block size");
 }
@@ -792,10 +891,10 @@ int gbo_bfs_noalloc(const gbo_bsr* AT, int32_t source, int32_t* d_level, int64_t
   BfsScratch s{};
   if ((rc = noalloc_layout(AT, base, &s))) return rc;
   switch (AT->bs) {
-    case 8: return bfs_t<8>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
-    case 16: return bfs_t<16>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
-    case 32: return bfs_t<32>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
-    case 64: return bfs_t<64>(AT, nullptr, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
+    case 8: return bfs_t<8>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
+    case 16: return bfs_t<16>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
+    case 32: return bfs_t<32>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
+    case 64: return bfs_t<64>(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream, &s);
   }
   return set_error(GBO_EUNSUPPORTED, "gbo_bfs_noalloc: block size");
   GBO_TRY_END
@@ -812,11 +911,12 @@ int gbo_bfs_do(const gbo_bsr* AT, const gbo_bsr* A, int32_t source, int32_t* d_l
   }
   if (source < 0 || source >= AT->nrows) return set_error(GBO_EINVAL, "gbo_bfs_do: source %d out of range", source);
   if (!d_level) return set_error(GBO_EINVAL, "gbo_bfs_do: null level");
+  if (!A) return gbo_bfs(AT, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
   switch (AT->bs) {
-    case 8: return bfs_t<8>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
-    case 16: return bfs_t<16>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
-    case 32: return bfs_t<32>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
-    case 64: return bfs_t<64>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 8: return bfs_do_t<8>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 16: return bfs_do_t<16>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 32: return bfs_do_t<32>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
+    case 64: return bfs_do_t<64>(AT, A, source, d_level, h_level_sizes, max_levels, h_nlevels, stream);
   }
   return set_error(GBO_EUNSUPPORTED, "gbo_bfs_do: block size");
 }

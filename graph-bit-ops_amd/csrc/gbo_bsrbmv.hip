@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) void k_spmv(const SpmvArgs a) {
     R0 += kWave;
   }
   if constexpr (OP == OP_BFS) {
-    if (lane == 0 && added) atomicAdd(&a.count_slots[c & (kCountSlots - 1)], (unsigned long long)added);
+    if (lane == 0 && added && a.count_slots) atomicAdd(&a.count_slots[c & (kCountSlots - 1)], (unsigned long long)added);
   }
 }
 
@@ -487,7 +487,7 @@ __global__ __launch_bounds__(256) void k_bfs_scan(const SpmvArgs a) {
   int* stile = s_tile[threadIdx.x / kWave];
   W* sword = s_word[threadIdx.x / kWave];
   const int c = wave_index();
-  if (c >= a.nchunks) return;
+  if (c >= a.nchunks || over(a.go)) return;
   const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const W* __restrict__ tiles = (const W*)a.tiles;
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(256) void k_bfs_scan(const SpmvArgs a) {
     if (__popcll(bmask) < kWave) break;
     R0 += kWave;
   }
-  if (lane == 0 && added) atomicAdd(&a.count_slots[c & (kCountSlots - 1)], (unsigned long long)added);
+  if (lane == 0 && added && a.count_slots) atomicAdd(&a.count_slots[c & (kCountSlots - 1)], (unsigned long long)added);
 }
 
 template <int BS, int OP>
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(256) void k_spmv_lpt(const SpmvArgs a) {
   constexpr int LPR = kWave / BS;        // lanes per row after the reduce-scatter
   const int lane = lane_id();
   const int c = wave_index();
-  if (c >= a.nchunks) return;
+  if (c >= a.nchunks || (OP == OP_BFS && over(a.go))) return;
   const int64_t cb = chunk_start(a, c), ce = chunk_start(a, c + 1);
   const bool last = (c == a.nchunks - 1);
   const int32_t* __restrict__ colind = a.colind;
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(256) void k_spmv_lpt(const SpmvArgs a) {
     R0 += kWave;
   }
   if constexpr (OP == OP_BFS) {
-    if (lane == 0 && added) atomicAdd(&a.count_slots[c & (kCountSlots - 1)], (unsigned long long)added);
+    if (lane == 0 && added && a.count_slots) atomicAdd(&a.count_slots[c & (kCountSlots - 1)], (unsigned long long)added);
   }
 }
 
@@ -1915,7 +1915,7 @@ __global__ __launch_bounds__(256) void k_bfs_pack(const int32_t* __restrict__ cn
   }
   uint64_t added = (uint64_t)__popcll(word);
   for (int off = 1; off < kWave; off <<= 1) added += __shfl_xor(added, off);
-  if (lane_id() == 0 && added) atomicAdd(&slots[(R / kWave) & (kCountSlots - 1)], (unsigned long long)added);
+  if (lane_id() == 0 && added && slots) atomicAdd(&slots[(R / kWave) & (kCountSlots - 1)], (unsigned long long)added);
 }
 
 // Min, min-plus and sum: the set-bit list kernel at bs 8/16 (variant 3, their
@@ -1960,7 +1960,7 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
       return GBO_OK;
     }
   }
-  const bool need_prefill = OP == OP_BFS || ((OP == OP_MINPLUS || OP == OP_MIN) && !a.prefilled) ||
+  const bool need_prefill = ((OP == OP_BFS || OP == OP_MINPLUS || OP == OP_MIN) && !a.prefilled) ||
                             (OP == OP_COUNT && !a.accumulate);
   if (need_prefill && a.nchunks > 1) {
     const int64_t n = (int64_t)(a.nchunks - 1) * BS;

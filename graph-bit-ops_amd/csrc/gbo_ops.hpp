@@ -190,15 +190,20 @@ struct Rounds {
     double value;
   };
   Flag* flags = nullptr;
+  int cap = kFlags;
   int at = kFlags;  // first flag of the batch
   Flag h[kMax];
 
   int alloc(Workspace& mem, const char* who) { return mem.alloc(&flags, sizeof(Flag) * kFlags, who); }
+  void place(void* p, size_t bytes) {
+    flags = (Flag*)p;
+    cap = at = (int)std::min<size_t>(bytes / sizeof(Flag), kFlags);
+  }
   // iterations to queue after `done`; their flags are clear
   int batch(int done, int* n, hipStream_t st) {
     *n = done == 0 ? 3 : std::min(std::max(2, done / 2), kMax);
-    if (at + *n > kFlags) {
-      GBO_HIP_CHECK(hipMemsetAsync(flags, 0, sizeof(Flag) * kFlags, st));
+    if (at + *n > cap) {
+      GBO_HIP_CHECK(hipMemsetAsync(flags, 0, sizeof(Flag) * cap, st));
       at = 0;
     }
     return GBO_OK;
@@ -294,16 +299,16 @@ struct SpmvArgs {
   const uint32_t* w;    // MINPLUS weights in tile bit order (nullable)
   const int64_t* woff;  // MINPLUS per-tile weight offsets
   const void* xval;     // MINPLUS dist / SUM x / MIN x
-  unsigned long long* count_slots;  // BFS: newly set bits, summed per slot (kCountSlots, zero on entry)
+  unsigned long long* count_slots;  // BFS: newly set bits, summed per slot (kCountSlots, zero on entry; nullable)
   int32_t* bfs_counts;  // BFS where dense_bfs_step holds (nullable): int32 scratch of nbr*bs; when set the step runs
                         // the count kernel into it and packs the rows with a nonzero count (dense step)
   double* partial;      // SUM: split-row partials [nchunks][2][bs]
   const uint64_t* active;  // MINPLUS: optional per-block-column activity bits (nullable)
   int accumulate;       // COUNT: add into y
   float scale, bias;    // SUM: y = scale * (A x) + bias  (scale 1, bias 0 for the plain op)
-  const unsigned long long* go;  // MINPLUS / SUM / MIN: nothing is done where *go is 0 (nullable; kernels of their
+  const unsigned long long* go;  // MINPLUS / SUM / MIN, BFS at bs 16 to 64: nothing is done where *go is 0 (nullable; kernels of their
                                  // own, the look costs a plain product 0.2 us a launch)
-  int prefilled;        // MINPLUS / MIN: `out` holds the identity where rows are split
+  int prefilled;        // BFS / MINPLUS / MIN: `out` holds the identity where rows are split
 };
 
 // The iteration before this one was the last: a driver queues a few iterations

@@ -1,5 +1,7 @@
 """Drivers that queue several iterations between two looks at their flags: runs
 that end at, before and after each look, and more iterations than flags."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -20,6 +22,21 @@ def test_shortest_paths_on_paths(gbo, bs):
     for n in list(range(1, 26)) + [513, 3001]:
         d, it = gbo.sssp(gbo.BsrMatrix.from_csr(_path(gbo, n), bs), 0)
         assert np.array_equal(d, np.arange(n)) and it == n, n
+
+
+@pytest.mark.parametrize("variant", (0, 1, 3))
+@pytest.mark.parametrize("bs", (8, 16, 32, 64))
+def test_bfs_on_paths(gbo, bs, variant):
+    for n in list(range(1, 26)) + [513, 3001]:
+        A = gbo.BsrMatrix.from_csr(_path(gbo, n), bs).plan(0, variant)
+        for source in {0, n // 2}:
+            d = np.abs(np.arange(n) - source)
+            want = np.bincount(d)
+            level, sizes = gbo.bfs(A, source)
+            assert np.array_equal(level, d) and np.array_equal(sizes, want), (n, source)
+            out, got, nl = gbo.DeviceBuffer(4 * n), np.zeros(4096, np.int64), ctypes.c_int32()
+            gbo._check(gbo.lib().gbo_bfs_noalloc(A.ref, source, out.ptr, got.ctypes.data, 4096, ctypes.byref(nl), None))
+            assert np.array_equal(out.to_numpy(np.int32, n), d) and np.array_equal(got[:nl.value], want), (n, source)
 
 
 @pytest.mark.parametrize("bs", (8, 16, 32, 64))
