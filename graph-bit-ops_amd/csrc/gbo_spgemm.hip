@@ -31,6 +31,8 @@
 //      segment of popc(A(I,K) row r & column j of B(K,J)), columns of B
 //      coming from a transposed copy of B's tiles.
 //
+// Where no block row has many candidates all of it stays in LDS (k_rows).
+//
 // The symbolic phase runs steps 1-4 on the keys alone; the numeric phase
 // and the count phase redo the expansion with the pair indices attached.
 #include <algorithm>
@@ -46,25 +48,32 @@ namespace {
 
 constexpr int kPerWave = 1024;  // candidate pairs per wave
 
-// colmask[t] = OR of A tile t's words; rowmask[u] = bit BS-1-r set iff row r
-// of B tile u is nonzero.  Group of BS lanes per tile.
+// amask[t] = OR of A tile t's words (its columns in use); bmask[u] = bit BS-1-r
+// set iff row r of B tile u is nonzero.  Group of BS lanes per tile, the first
+// `ablocks` blocks A's; clears *flag.
 template <int BS>
-__global__ __launch_bounds__(256) void k_masks(const word_t<BS>* __restrict__ tiles, int64_t T, bool rows,
-                                               word_t<BS>* __restrict__ mask) {
+__global__ __launch_bounds__(256) void k_masks(const word_t<BS>* __restrict__ at, int64_t Ta, int64_t ablocks,
+                                               word_t<BS>* __restrict__ amask, const word_t<BS>* __restrict__ bt,
+                                               int64_t Tb, word_t<BS>* __restrict__ bmask, int64_t* __restrict__ flag) {
   constexpr int G = kWave / BS;
-  const int lane = lane_id();
-  const int64_t t = (int64_t)wave_index() * G + lane / BS;
-  const int r = lane % BS;
-  const uint64_t w = t < T ? (uint64_t)tiles[t * BS + r] : 0ull;
-  uint64_t m;
-  if (rows) {
-    const uint64_t b = __ballot(w != 0);
-    m = brev_low<BS>((b >> ((lane / BS) * BS)) & low_mask<BS>());
-  } else {
-    m = w;
-    for (int off = 1; off < BS; off <<= 1) m |= __shfl_xor(m, off);
+  const int lane = lane_id(), r = lane % BS;
+  const bool rows = blockIdx.x >= ablocks;
+  const int64_t T = rows ? Tb : Ta, blocks = rows ? gridDim.x - ablocks : ablocks;
+  const word_t<BS>* tiles = rows ? bt : at;
+  if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+  for (int64_t b = blockIdx.x - (rows ? ablocks : 0); b * 4 * G < T; b += blocks) {
+    const int64_t t = (b * 4 + threadIdx.x / kWave) * G + lane / BS;
+    const uint64_t w = t < T ? (uint64_t)tiles[t * BS + r] : 0ull;
+    uint64_t m;
+    if (rows) {
+      const uint64_t bits = __ballot(w != 0);
+      m = brev_low<BS>((bits >> ((lane / BS) * BS)) & low_mask<BS>());
+    } else {
+      m = w;
+      for (int off = 1; off < BS; off <<= 1) m |= __shfl_xor(m, off);
+    }
+    if (r == 0 && t < T) (rows ? bmask : amask)[t] = (word_t<BS>)m;
   }
-  if (r == 0 && t < T) mask[t] = (word_t<BS>)m;
 }
 
 // Block row of every tile: the first I with rowptr[I + 1] > t (a binary
@@ -285,6 +294,170 @@ __global__ __launch_bounds__(256) void k_transpose_tiles(const word_t<BS>* __res
   }
 }
 
+// ---- Products whose block rows have at most kRowPairs candidate pairs each
+// (grids, bands): a wave per block row of C lists its productive pairs in LDS,
+// sorts them by block column there, and the runs of one column are C's tiles.
+// No pair goes through memory, and a phase is 6 to 8 launches instead of about
+// 40 (at 5 us of host time each): three phases on a king grid of a million
+// vertices at bs 32 1.20 -> 0.46 ms, on one of 10,000 at bs 16 0.70 -> 0.17.
+constexpr int kRowPairs = 256;
+
+struct RowArgs {
+  const int32_t *a_rowptr, *a_colind, *b_rowptr, *b_colind;
+  const void *a_mask, *b_mask;  // column masks, row masks
+  const void *a_tiles, *b_tiles;
+  int32_t nbr;
+  int32_t* cnt;         // ROW_COUNT: C tiles of each block row
+  int64_t* heavy;       // ROW_COUNT: set where a block row has more candidates
+  const int64_t* off;   // first C tile of each block row
+  int32_t* colind;      // ROW_TILES
+  void* tiles;          // C: ROW_TILES written, ROW_VALUES read
+  const int64_t* valoff;
+  int32_t* values;
+};
+
+enum { ROW_COUNT = 0, ROW_TILES = 1, ROW_VALUES = 2 };
+
+// ROW_VALUES takes B's tiles in column form.
+template <int BS, int MODE>
+__global__ __launch_bounds__(256) void k_rows(const RowArgs a) {
+  using W = word_t<BS>;
+  constexpr int G = kWave / BS;
+  __shared__ uint64_t s_key[4][kRowPairs];
+  __shared__ int32_t s_t[4][kRowPairs], s_u[4][kRowPairs];
+  __shared__ int32_t s_end[4][kWave], s_head[4][kRowPairs + 1];
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  uint64_t* key = s_key[wave];
+  int32_t *pt = s_t[wave], *pu = s_u[wave], *cend = s_end[wave], *head = s_head[wave];
+  const int64_t I = wave_index();
+  if (I >= a.nbr) return;
+  const W* am = (const W*)a.a_mask;
+  const W* bm = (const W*)a.b_mask;
+  const int32_t ra = a.a_rowptr[I], rb = a.a_rowptr[I + 1];
+  int n = 0, cands = 0;
+  for (int32_t t0 = ra; t0 < rb; t0 += kWave) {
+    const int32_t t = t0 + lane;
+    int32_t u0 = 0, len = 0;
+    if (t < rb) {
+      const int32_t K = a.a_colind[t];
+      u0 = a.b_rowptr[K];
+      len = a.b_rowptr[K + 1] - u0;
+    }
+    // a long row of B makes the block row heavy by itself
+    const int incl = wave_incl_scan(min(len, kRowPairs + 1)), all = __shfl(incl, kWave - 1);
+    cands += all;
+    if (cands > kRowPairs) {
+      if (MODE == ROW_COUNT && lane == 0) {
+        *a.heavy = 1;
+        a.cnt[I] = 0;
+      }
+      return;
+    }
+    cend[lane] = incl;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    for (int p0 = 0; p0 < all; p0 += kWave) {
+      const int p = p0 + lane;
+      int lo = 0, hi = kWave - 1;  // the A tile: the first whose end is past p
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (cend[mid] <= p) lo = mid + 1;
+        else hi = mid;
+      }
+      const int32_t first = __shfl(u0, lo), before = lo ? cend[lo - 1] : 0;
+      const int32_t u = first + (p - before);
+      const bool prod = p < all && ((uint64_t)am[t0 + (p < all ? lo : 0)] & (uint64_t)bm[p < all ? u : 0]) != 0;
+      const unsigned long long b = __ballot(prod);
+      if (prod) {
+        const int at = n + __popcll(b & ((1ull << lane) - 1));
+        key[at] = ((uint64_t)(uint32_t)a.b_colind[u] << 32) | (uint32_t)at;
+        pt[at] = t0 + lo;
+        pu[at] = u;
+      }
+      n += __popcll(b);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+  // bitonic sort of the next power of two
+  int size = 2;
+  while (size < n) size *= 2;
+  for (int i = n + lane; i < size; i += kWave) key[i] = ~0ull;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  for (int k = 2; k <= size; k *= 2) {
+    for (int j = k / 2; j > 0; j /= 2) {
+      for (int x = lane; x < size / 2; x += kWave) {
+        const int i = 2 * x - (x & (j - 1));
+        const uint64_t lo = key[i], hi = key[i + j];
+        if ((lo > hi) == ((i & k) == 0)) {
+          key[i] = hi;
+          key[i + j] = lo;
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+  }
+  int nc = 0;
+  for (int i0 = 0; i0 < n; i0 += kWave) {
+    const int i = i0 + lane;
+    const bool first = i < n && (i == 0 || (key[i] >> 32) != (key[i - 1] >> 32));
+    const unsigned long long b = __ballot(first);
+    if (MODE != ROW_COUNT && first) {
+      const int c = nc + __popcll(b & ((1ull << lane) - 1));
+      head[c] = i;
+      if (MODE == ROW_TILES) a.colind[a.off[I] + c] = (int32_t)(key[i] >> 32);
+    }
+    nc += __popcll(b);
+  }
+  if constexpr (MODE == ROW_COUNT) {
+    if (lane == 0) a.cnt[I] = nc;
+  } else {
+    if (lane == 0) head[nc] = n;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const W* __restrict__ at = (const W*)a.a_tiles;
+    const W* __restrict__ bt = (const W*)a.b_tiles;
+    W* ct = (W*)a.tiles;
+    const int g = lane / BS, r = lane % BS;
+    const int64_t base = a.off[I];
+    for (int c0 = 0; c0 < nc; c0 += G) {
+      const int c = c0 + g;
+      const bool in = c < nc;
+      const int q0 = in ? head[c] : 0, q1 = in ? head[c + 1] : 0;
+      if constexpr (MODE == ROW_TILES) {
+        uint64_t acc = 0;
+        for (int q = q0; q < q1; ++q) {
+          const int e = (int)(uint32_t)key[q];
+          const int64_t t = pt[e], u = pu[e];
+          uint64_t w = (uint64_t)at[t * BS + r];
+          while (w) {
+            const int p = 63 - __builtin_clzll(w);  // highest set bit: column BS-1-p
+            w &= ~(1ull << p);
+            acc |= (uint64_t)bt[u * BS + (BS - 1 - p)];
+          }
+        }
+        if (in) ct[(base + c) * BS + r] = (W)acc;
+      } else {
+        const uint64_t crow = in ? (uint64_t)ct[(base + c) * BS + r] : 0ull;
+        int before = popcw(crow);  // bits of the rows above inside the tile
+        for (int off = 1; off < BS; off <<= 1) {
+          const int o = __shfl_up(before, off, BS);
+          if (r >= off) before += o;
+        }
+        int64_t pos = in ? a.valoff[base + c] + before - popcw(crow) : 0;
+        uint64_t m = crow;
+        while (m) {
+          const int p = 63 - __builtin_clzll(m);
+          m &= ~(1ull << p);
+          int32_t s = 0;
+          for (int q = q0; q < q1; ++q) {
+            const int e = (int)(uint32_t)key[q];
+            s += popcw((W)((uint64_t)at[(int64_t)pt[e] * BS + r] & (uint64_t)bt[(int64_t)pu[e] * BS + (BS - 1 - p)]));
+          }
+          a.values[pos++] = s;
+        }
+      }
+    }
+  }
+}
+
 unsigned bits_for(int64_t n) {  // smallest b with 2^b > n (at least 1)
   unsigned b = 1;
   while (b < 63 && (1ll << b) <= n) ++b;
@@ -317,24 +490,84 @@ struct Pairs {
 };
 
 template <int BS>
-int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, Workspace& mem, Pairs* out, hipStream_t st) {
+int tile_masks(const gbo_bsr* A, const gbo_bsr* B, Workspace& mem, void** am, void** bm, int64_t* flag, hipStream_t st) {
   using W = word_t<BS>;
+  constexpr int per = 4 * kWave / BS;  // tiles of a block
+  W *amask = nullptr, *bmask = nullptr;
+  int rc;
+  if ((rc = mem.alloc(&amask, sizeof(W) * (size_t)A->nblocks, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&bmask, sizeof(W) * (size_t)B->nblocks, "gbo_bsrbmm")))
+    return rc;
+  const int64_t most = 1 << 21;
+  const int64_t ab = std::min((A->nblocks + per - 1) / per, most), bb = std::min((B->nblocks + per - 1) / per, most);
+  k_masks<BS><<<(unsigned)(ab + bb), 256, 0, st>>>((const W*)A->tiles, A->nblocks, ab, amask, (const W*)B->tiles,
+                                                  B->nblocks, bmask, flag);
+  GBO_LAUNCH_CHECK();
+  *am = amask;
+  *bm = bmask;
+  return GBO_OK;
+}
+
+// The product by rows, counted: its arguments with `off`, and the number of C
+// tiles; *ok = false where a block row has too many candidates.
+template <int BS>
+int count_rows(const gbo_bsr* A, const gbo_bsr* B, Workspace& mem, RowArgs* out, int64_t* nc, bool* ok, hipStream_t st) {
+  *ok = false;
+  // half of that on average: some block row has more (20,011 rows of 4 at random, bs 8,
+  // 256 on average: 0.82 ms, with the count here in vain 0.85)
+  const double mean = (double)A->nblocks / std::max(A->nblockrows, 1) * ((double)B->nblocks / std::max(B->nblockrows, 1));
+  if (A->nblocks == 0 || B->nblocks == 0 || A->nblockrows > (1 << 25) || mean > kRowPairs / 2) return GBO_OK;
+  RowArgs a{};
+  a.a_rowptr = A->rowptr;
+  a.a_colind = A->colind;
+  a.b_rowptr = B->rowptr;
+  a.b_colind = B->colind;
+  a.a_tiles = A->tiles;
+  a.b_tiles = B->tiles;
+  a.nbr = A->nblockrows;
+  int64_t* off = nullptr;
+  void *am = nullptr, *bm = nullptr;
+  int rc;
+  if ((rc = mem.alloc(&a.cnt, sizeof(int32_t) * (size_t)a.nbr, "gbo_bsrbmm")) ||
+      (rc = mem.alloc(&off, sizeof(int64_t) * ((size_t)a.nbr + 2), "gbo_bsrbmm")))
+    return rc;
+  a.heavy = off + a.nbr + 1;
+  if ((rc = tile_masks<BS>(A, B, mem, &am, &bm, a.heavy, st))) return rc;
+  a.a_mask = am;
+  a.b_mask = bm;
+  k_rows<BS, ROW_COUNT><<<grid_for(a.nbr, 4), 256, 0, st>>>(a);
+  GBO_LAUNCH_CHECK();
+  if ((rc = scan_exclusive<int32_t, int64_t>(a.cnt, off, a.nbr, st, mem))) return rc;
+  int64_t h[2] = {0, 0};
+  if ((rc = read_back(h, off + a.nbr, sizeof(h), st))) return rc;
+  if (h[1]) return GBO_OK;
+  a.off = off;
+  *out = a;
+  *nc = h[0];
+  *ok = true;
+  return GBO_OK;
+}
+
+__global__ __launch_bounds__(256) void k_row_ptr(const int64_t* __restrict__ off, int32_t nbr,
+                                                 int32_t* __restrict__ rowptr) {
+  const int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (I <= nbr) rowptr[I] = (int32_t)off[I];
+}
+
+template <int BS>
+int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, Workspace& mem, Pairs* out, hipStream_t st) {
   const int64_t T = A->nblocks;
   out->jbits = (int)bits_for(std::max<int32_t>(B->nblockcols, 1) - 1);
   if (T == 0 || B->nblocks == 0) return GBO_OK;
-  W *amask = nullptr, *bmask = nullptr;
+  void *amask = nullptr, *bmask = nullptr;
   int32_t* trow = nullptr;
   int64_t *cnt = nullptr, *coff = nullptr;
   int rc;
-  if ((rc = mem.alloc(&amask, sizeof(W) * (size_t)T, "gbo_bsrbmm")) ||
-      (rc = mem.alloc(&bmask, sizeof(W) * (size_t)B->nblocks, "gbo_bsrbmm")) ||
+  if ((rc = tile_masks<BS>(A, B, mem, &amask, &bmask, nullptr, st)) ||
       (rc = mem.alloc(&trow, sizeof(int32_t) * (size_t)T, "gbo_bsrbmm")) ||
       (rc = mem.alloc(&cnt, sizeof(int64_t) * (size_t)T, "gbo_bsrbmm")) ||
       (rc = mem.alloc(&coff, sizeof(int64_t) * ((size_t)T + 1), "gbo_bsrbmm")))
     return rc;
-  constexpr int G = kWave / BS;
-  k_masks<BS><<<grid_for((T + G - 1) / G, 4), 256, 0, st>>>((const W*)A->tiles, T, false, amask);
-  k_masks<BS><<<grid_for((B->nblocks + G - 1) / G, 4), 256, 0, st>>>((const W*)B->tiles, B->nblocks, true, bmask);
   k_tile_rows_of<<<grid_for(T, 256), 256, 0, st>>>(A->rowptr, A->nblockrows, T, trow);
   k_cand_count<<<grid_for(T, 256), 256, 0, st>>>(A->colind, T, B->rowptr, cnt);
   GBO_LAUNCH_CHECK();
@@ -424,10 +657,22 @@ int key_runs(const Pairs& pr, Workspace& mem, int32_t** crow, int32_t* ccol, int
 template <int BS>
 int symbolic_t(const gbo_bsr* A, const gbo_bsr* B, int32_t* d_rowptr, int64_t* nblocks, hipStream_t st) {
   Workspace mem(st);
-  Pairs pr;
-  int rc = sorted_pairs<BS>(A, B, false, mem, &pr, st);
-  if (rc) return rc;
+  RowArgs rows;
   int64_t nc = 0;
+  bool by_rows = false;
+  int rc = count_rows<BS>(A, B, mem, &rows, &nc, &by_rows, st);
+  if (rc) return rc;
+  if (by_rows) {
+    if (nc >= ((int64_t)1 << 31))
+      return set_error(GBO_ERANGE, "gbo_bsrbmm_symbolic: %lld tiles exceed int32", (long long)nc);
+    k_row_ptr<<<grid_for((int64_t)A->nblockrows + 1, 256), 256, 0, st>>>(rows.off, A->nblockrows, d_rowptr);
+    GBO_LAUNCH_CHECK();
+    GBO_HIP_CHECK(hipStreamSynchronize(st));
+    *nblocks = nc;
+    return GBO_OK;
+  }
+  Pairs pr;
+  if ((rc = sorted_pairs<BS>(A, B, false, mem, &pr, st))) return rc;
   int32_t* crow = nullptr;
   if (pr.P > 0 && (rc = key_runs(pr, mem, &crow, nullptr, nullptr, &nc, st))) return rc;
   if (nc >= ((int64_t)1 << 31)) return set_error(GBO_ERANGE, "gbo_bsrbmm_symbolic: %lld tiles exceed int32", (long long)nc);
@@ -444,11 +689,14 @@ template <int BS>
 int numeric_t(const gbo_bsr* A, const gbo_bsr* B, int64_t nc_expect, int32_t* d_colind, word_t<BS>* d_tiles,
               const int64_t* d_valoff, int32_t* d_counts, hipStream_t st) {
   using W = word_t<BS>;
+  constexpr int G = kWave / BS;
   Workspace mem(st);
   Pairs pr;
-  int rc = sorted_pairs<BS>(A, B, true, mem, &pr, st);
-  if (rc) return rc;
+  RowArgs rows;
   int64_t nc = 0;
+  bool by_rows = false;
+  int rc = count_rows<BS>(A, B, mem, &rows, &nc, &by_rows, st);
+  if (rc || (!by_rows && (rc = sorted_pairs<BS>(A, B, true, mem, &pr, st)))) return rc;
   int32_t* crow = nullptr;
   int64_t* seg = nullptr;
   if (pr.P > 0 && (rc = key_runs(pr, mem, &crow, d_counts ? nullptr : d_colind, &seg, &nc, st))) return rc;
@@ -456,16 +704,26 @@ int numeric_t(const gbo_bsr* A, const gbo_bsr* B, int64_t nc_expect, int32_t* d_
     return set_error(GBO_EINVAL, "gbo_bsrbmm: C has %lld tiles, the given structure %lld", (long long)nc,
                      (long long)nc_expect);
   if (nc == 0) return GBO_OK;
-  constexpr int G = kWave / BS;
-  if (!d_counts) {
+  W* btc = nullptr;  // B's tiles in column form
+  if (d_counts) {
+    if ((rc = mem.alloc(&btc, sizeof(W) * (size_t)B->nblocks * BS, "gbo_bsrbmm_values"))) return rc;
+    k_transpose_tiles<BS><<<grid_for((B->nblocks + G - 1) / G, 4), 256, 0, st>>>((const W*)B->tiles, B->nblocks, btc);
+    GBO_LAUNCH_CHECK();
+  }
+  if (by_rows) {
+    rows.colind = d_colind;
+    rows.tiles = d_tiles;
+    rows.valoff = d_valoff;
+    rows.values = d_counts;
+    if (btc) rows.b_tiles = btc;
+    if (d_counts) k_rows<BS, ROW_VALUES><<<grid_for(rows.nbr, 4), 256, 0, st>>>(rows);
+    else k_rows<BS, ROW_TILES><<<grid_for(rows.nbr, 4), 256, 0, st>>>(rows);
+    GBO_LAUNCH_CHECK();
+  } else if (!d_counts) {
     k_numeric<BS><<<grid_for((nc + G - 1) / G, 4), 256, 0, st>>>(pr.vals, seg, nc, (const W*)A->tiles,
                                                                  (const W*)B->tiles, d_tiles);
     GBO_LAUNCH_CHECK();
   } else {
-    W* btc = nullptr;
-    if ((rc = mem.alloc(&btc, sizeof(W) * (size_t)B->nblocks * BS, "gbo_bsrbmm_values"))) return rc;
-    k_transpose_tiles<BS><<<grid_for((B->nblocks + G - 1) / G, 4), 256, 0, st>>>((const W*)B->tiles, B->nblocks, btc);
-    GBO_LAUNCH_CHECK();
     k_counts<BS><<<grid_for((nc + G - 1) / G, 4), 256, 0, st>>>(pr.vals, seg, nc, (const W*)A->tiles, btc,
                                                                 (const W*)d_tiles, d_valoff, d_counts);
     GBO_LAUNCH_CHECK();
