@@ -419,6 +419,7 @@ static SpmvArgs bfs_args(const gbo_bsr* A, const PlanView& pv) {
   a.plan = pv.plan;
   a.start = pv.start;
   a.tail = pv.tail;
+  a.whole = pv.whole;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -959,6 +960,7 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   a.plan = pv.plan;
   a.start = pv.start;
   a.tail = pv.tail;
+  a.whole = pv.whole;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -1027,6 +1029,7 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   a.plan = pv.plan;
   a.start = pv.start;
   a.tail = pv.tail;
+  a.whole = pv.whole;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -1110,6 +1113,7 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   a.plan = pv.plan;
   a.start = pv.start;
   a.tail = pv.tail;
+  a.whole = pv.whole;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

@@ -1962,7 +1962,7 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
   }
   const bool need_prefill = ((OP == OP_BFS || OP == OP_MINPLUS || OP == OP_MIN) && !a.prefilled) ||
                             (OP == OP_COUNT && !a.accumulate);
-  if (need_prefill && a.nchunks > 1) {
+  if (need_prefill && a.nchunks > 1 && !a.whole) {
     const int64_t n = (int64_t)(a.nchunks - 1) * BS;
     k_prefill_split<BS, OP><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
     GBO_LAUNCH_CHECK();
@@ -1999,7 +1999,7 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
     k_spmv<BS, OP><<<(unsigned)blocks, 256, 0, st>>>(a);
   }
   GBO_LAUNCH_CHECK();
-  if (OP == OP_SUM && a.nchunks > 1) {
+  if (OP == OP_SUM && a.nchunks > 1 && !a.whole) {
     const int64_t n = (int64_t)(a.nchunks - 1) * BS;
     if (a.go) k_sum_fixup<BS, true><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
     else k_sum_fixup<BS, false><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
@@ -2042,6 +2042,7 @@ static SpmvArgs base_args(const gbo_bsr* A, const PlanView& pv) {
   a.plan = pv.plan;
   a.start = pv.start;
   a.tail = pv.tail;
+  a.whole = pv.whole;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

@@ -45,6 +45,7 @@ struct PlanView {
   int64_t* count = nullptr;
   double* partial = nullptr;
   int32_t* bfs_counts = nullptr;  // the dense BFS step's row counts
+  bool whole = false;             // no block row is cut
 };
 
 // Most tiles per chunk of the library's own plans.
@@ -308,6 +309,7 @@ struct SpmvArgs {
   float scale, bias;    // SUM: y = scale * (A x) + bias  (scale 1, bias 0 for the plain op)
   const unsigned long long* go;  // MINPLUS / SUM / MIN, BFS at bs 16 to 64: nothing is done where *go is 0 (nullable; kernels of their
                                  // own, the look costs a plain product 0.2 us a launch)
+  int whole;            // no block row is cut by a chunk's end
   int prefilled;        // BFS / MINPLUS / MIN: `out` holds the identity where rows are split
 };
 

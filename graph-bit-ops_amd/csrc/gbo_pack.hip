@@ -509,6 +509,17 @@ int default_chunk(int bs, int64_t tiles) {
 // with equal work, min 757 against 774).
 constexpr int64_t kEvenTiles = 32ll << 20;
 
+// The longest block row, in tiles, of a matrix whose chunks end at block rows:
+// no product then has rows to zero or partial sums to add in a launch of its own
+// (G(1024) of degree 20 at bs 32 count 7.7 -> 4.4 us, G(5003) of 16 at bs 8 sum 9.2
+// -> 5.6, king grid of 62,500 at bs 64 min 10.0 -> 6.2).  Longer rows leave too
+// few waves: min-plus at bs 32 with rows of 63 tiles 10.5 -> 13.2 us.  On larger
+// matrices the rows have to be short against a chunk.
+static int32_t whole_row(int bs, int64_t tiles, int32_t chunk) {
+  const int32_t small = bs == 8 ? 256 : bs == 16 ? 128 : bs == 32 ? 32 : 16;
+  return tiles <= (128 << 10) ? small : chunk / 8;
+}
+
 static bool bs_ok(int bs) { return bs == 8 || bs == 16 || bs == 32 || bs == 64; }
 
 template <int BS, int MODE>
@@ -692,12 +703,39 @@ static void view_scratch(PlanView* pv, int bs, int32_t nbr, bool even) {
   pv->bfs_counts = (int32_t*)(base + L.bfs_counts);
 }
 
+// *most = tiles of the longest block row (zero before).
+__global__ __launch_bounds__(256) void k_row_most(const int32_t* __restrict__ rowptr, int32_t nbr,
+                                                  int32_t* __restrict__ most) {
+  const int64_t R = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int t = R < nbr ? rowptr[R + 1] - rowptr[R] : 0;
+  for (int off = 1; off < kWave; off <<= 1) t = max(t, __shfl_xor(t, off));
+  if (lane_id() == 0 && t) atomicMax(most, t);
+}
+
+// Chunk starts moved back to the start of the block row they lie in.
+__global__ __launch_bounds__(256) void k_whole_starts(const int32_t* __restrict__ rowptr, int32_t nbr, int32_t nchunks,
+                                                      int64_t* __restrict__ start) {
+  const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= nchunks) return;
+  const int64_t b = start[c];
+  int32_t lo = 0, hi = nbr - 1;  // the first row that ends past b
+  while (lo < hi) {
+    const int32_t mid = lo + (hi - lo) / 2;
+    if ((int64_t)rowptr[mid + 1] <= b) lo = mid + 1;
+    else hi = mid;
+  }
+  start[c] = rowptr[lo];
+}
+
 // Plan entries (of the chunks whose starts are in place, or of even chunks of
 // `chunk` tiles) and zeroed count slots.
-static int plan_fill(const gbo_bsr* A, int32_t chunk, bool even, int64_t nch, int32_t* plan, hipStream_t st) {
+static int plan_fill(const gbo_bsr* A, int32_t chunk, bool even, bool whole, int64_t nch, int32_t* plan,
+                     hipStream_t st) {
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
   int64_t* start = (int64_t*)((char*)plan + L.start);
   if (even) k_even_starts<<<(unsigned)((nch + 256) / 256), 256, 0, st>>>(A->nblocks, chunk, (int32_t)nch, start);
+  if (whole)
+    k_whole_starts<<<(unsigned)((nch + 255) / 256), 256, 0, st>>>(A->rowptr, A->nblockrows, (int32_t)nch, start);
   k_plan<<<(unsigned)((nch + 255) / 256), 256, 0, st>>>(A->rowptr, A->nblockrows, start, (int32_t)nch, plan,
                                                        (int32_t*)((char*)plan + L.tail));
   GBO_LAUNCH_CHECK();
@@ -749,6 +787,7 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
     pv->nchunks = A->plan_nchunks;
     pv->variant = A->plan_variant;
     pv->owned = false;
+    pv->whole = A->plan_even == 2;
     view_scratch(pv, A->bs, A->nblockrows, A->plan_even == 1);
     return GBO_OK;
   }
@@ -764,7 +803,7 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
   pv->variant = A->plan_variant;
   pv->owned = true;
   view_scratch(pv, A->bs, A->nblockrows, true);
-  return plan_fill(A, chunk, true, nch, plan, st);
+  return plan_fill(A, chunk, true, false, nch, plan, st);
 }
 
 int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st) {
@@ -788,6 +827,18 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st
     if (!even) nch = w.nch;
   }
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "gbo_bsr_plan: too many chunks");
+  bool whole = false;
+  const int32_t longest = whole_row(A->bs, A->nblocks, chunk);
+  if (chunk_tiles <= 0 && A->nblocks > 0 && A->nblocks < kEvenTiles && A->nblocks <= (int64_t)A->nblockrows * longest) {
+    int32_t most = 0, *d_most = nullptr;
+    int rc = mem.alloc(&d_most, sizeof(int32_t), "gbo_bsr_plan");
+    if (rc) return rc;
+    GBO_HIP_CHECK(hipMemsetAsync(d_most, 0, sizeof(int32_t), st));
+    k_row_most<<<(unsigned)(((int64_t)A->nblockrows + 255) / 256), 256, 0, st>>>(A->rowptr, A->nblockrows, d_most);
+    GBO_LAUNCH_CHECK();
+    if ((rc = read_back(&most, d_most, sizeof(int32_t), st))) return rc;
+    whole = most <= longest;
+  }
   gbo_bsr_plan_free(A);
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
   if (device_malloc((void**)&A->plan, L.bytes) != hipSuccess) {
@@ -798,7 +849,7 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st
   A->plan_chunk = chunk;
   A->plan_nchunks = (int32_t)nch;
   A->plan_variant = variant;
-  A->plan_even = even ? 1 : 0;
+  A->plan_even = whole ? 2 : even ? 1 : 0;
   if (!even) {
     k_unit_chunks<<<(unsigned)((w.nunits + 255) / 256), 256, 0, st>>>(w.pre, w.rank, w.nunits, w.target, w.unit,
                                                                       A->nblocks, (int64_t*)((char*)A->plan + L.start));
@@ -808,7 +859,7 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st
       return set_error(GBO_EDEVICE, "gbo_bsr_plan: %s", hipGetErrorString(e));
     }
   }
-  const int rc = plan_fill(A, chunk, even, nch, A->plan, st);
+  const int rc = plan_fill(A, chunk, even, whole, nch, A->plan, st);
   if (rc) gbo_bsr_plan_free(A);
   return rc;
 }

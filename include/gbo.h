@@ -67,10 +67,10 @@ typedef struct gbo_bsr {
   int32_t* colind;
   void* tiles;
   int32_t* plan;        /* device, plan_nchunks entries (first block row of each chunk) */
-  int32_t plan_chunk;   /* tiles per chunk (the most of any, where the library chose) */
+  int32_t plan_chunk;   /* tiles per chunk (about the most of any, where the library chose) */
   int32_t plan_nchunks;
   int32_t plan_variant; /* kernel variant for bs 8/16 (0 = default; see gbo_bsr_plan_ex) */
-  int32_t plan_even;    /* 1: every chunk holds plan_chunk tiles (the last one the rest) */
+  int32_t plan_even;    /* 1: every chunk holds plan_chunk tiles (the last one the rest); 2: chunks end at block rows */
 } gbo_bsr;
 
 const char* gbo_last_error(void);
