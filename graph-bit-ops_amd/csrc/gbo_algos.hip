@@ -398,7 +398,7 @@ __global__ __launch_bounds__(256) void k_popc_words(const word_t<BS>* __restrict
 
 // Scratch of a BFS call supplied by the caller of bfs_t instead of being
 // allocated: frontier / next / visited words (3 x nbr words), the levels' flags
-// (kBfsFlagBytes) and (where dense_bfs_step holds and they fit) the dense
+// (kBfsFlagBytes) and (bs 8, where dense_bfs_step holds and they fit) the dense
 // step's row counts (bs x (nbr + 1) int32, else null).
 constexpr size_t kBfsFlagBytes = 8192;
 struct BfsScratch {
@@ -429,7 +429,10 @@ static SpmvArgs bfs_args(const gbo_bsr* A, const PlanView& pv) {
 // From how many tiles on bs 8 takes the dense step: its kernels have no look at
 // the flags, so its levels are not queued.  Queued, dense: 1.6M tiles (200,000
 // vertices of 8) 216 and 269 us, 1.1M (R-MAT 2^16) 247 and 241, 5.2M (R-MAT
-// 2^18) 490 and 447, 24M 1045 and 958.
+// 2^18) 490 and 447, 24M 1045 and 958.  At bs 16 to 64 k_bfs_scan leaves block
+// rows early and is the better one at every size (R-MAT 2^22, dense where a
+// quarter of the frontier words may have bits: bs 16 2.68 against 3.02 ms, bs 32
+// 3.25 against 4.19).
 constexpr int64_t kDenseTiles = 2 << 20;
 
 // Pull BFS over AT, several levels between two looks at their sizes: one level
@@ -465,7 +468,9 @@ static int bfs_t(const gbo_bsr* A, int32_t source, int32_t* d_level, int64_t* si
   // bs 8 variant 3, large matrices: levels while fewer than half the vertices
   // are visited take the dense step (count kernel + pack); later ones skip
   // visited rows
-  int32_t* dense_counts = !dense_bfs_step(BS, g.pv.variant) ? nullptr : ext ? ext->dense_counts : g.pv.bfs_counts;
+  int32_t* dense_counts = BS != 8 || !dense_bfs_step(BS, g.pv.variant) ? nullptr
+                          : ext                                        ? ext->dense_counts
+                                                                       : g.pv.bfs_counts;
   int64_t visited = 1;
   int32_t lvl = 0;
   if (sizes && max_levels > 0) sizes[0] = 1;
@@ -530,7 +535,7 @@ static int bfs_do_t(const gbo_bsr* A, const gbo_bsr* Aout, int32_t source, int32
   a.count_slots = pv.slots;
   // bs 8 variant 3: levels while fewer than half the vertices are visited take
   // the dense step (count kernel + pack); later ones skip visited rows
-  int32_t* dense_counts = dense_bfs_step(BS, pv.variant) ? pv.bfs_counts : nullptr;
+  int32_t* dense_counts = BS == 8 && dense_bfs_step(BS, pv.variant) ? pv.bfs_counts : nullptr;
   int64_t visited = 1;
   int32_t lvl = 0;
   int64_t fsize = 1;  // vertices in the current frontier
@@ -844,7 +849,7 @@ static int noalloc_layout(const gbo_bsr* AT, unsigned char* base, BfsScratch* s)
   // levels)
   const size_t dbytes = sizeof(int32_t) * (size_t)AT->bs * ((size_t)AT->nblockrows + 1);
   const bool dense =
-      dense_bfs_step(AT->bs, AT->plan_variant) && o_dense + align256(dbytes) <= kNoAllocScratchBytes;
+      AT->bs == 8 && dense_bfs_step(AT->bs, AT->plan_variant) && o_dense + align256(dbytes) <= kNoAllocScratchBytes;
   const size_t need = o_dense + (dense ? align256(dbytes) : 0);
   if (need > kNoAllocScratchBytes)
     return set_error(GBO_ERANGE,
@@ -967,7 +972,7 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   a.w = d_w;
   a.woff = d_woff;
   ListView lists;
-  lists_build(AT, ListUse::kMany, mem, &lists, st);
+  lists_build(AT, ListUse::kPaths, mem, &lists, st);
   int32_t it = 0;
   unsigned long long *act_cur = active, *act_next = active2;
   const unsigned blocks_u = (unsigned)(((int64_t)n + kSsspThreads - 1) / kSsspThreads);

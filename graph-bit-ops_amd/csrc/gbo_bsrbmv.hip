@@ -476,6 +476,9 @@ __device__ __forceinline__ void load_tile(const void* tiles, int64_t t, uint64_t
 // lanes per tile before: 211, 411, 330 (every tile, by the count kernel), 190,
 // 118, 106 us; now 68, 174, 323, 144, 60, 56: scanning 59 MB of columns, then
 // the tiles under the frontier.  bs 64 3.0 -> 1.9 ms a call, bs 16 1.20 -> 0.84.
+// Where every vertex is in the frontier and none visited the count kernel is the
+// faster one (R-MAT 2^22 bs 16 0.81 against 1.34 ms, bs 32 1.51 against 1.82):
+// a single step, which knows neither, takes it where it has room for the counts.
 constexpr int kScan = 4 * kWave;
 template <int BS>
 __global__ __launch_bounds__(256) void k_bfs_scan(const SpmvArgs a) {
@@ -1945,10 +1948,11 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
   // lane-per-tile kernel (faster than the row-group one at bs 8)
   const bool lpt = (BS <= 16 && OP == OP_COUNT && a.variant == 1) ||
                    (BS == 8 && OP == OP_BFS && (a.variant == 1 || a.variant == 3));
-  if constexpr (BS == 8 && OP == OP_BFS) {
+  if constexpr (OP == OP_BFS) {
     if (dense_bfs_step(BS, a.variant) && a.bfs_counts && aligned) {
-      // dense step: the count kernel gives each row's number of frontier
-      // neighbours (every tile is read; no visited-row skip)
+      // dense step: the count kernel (k_count8 / k_count16q / k_count32q /
+      // k_spmv<64>) gives each row's number of frontier neighbours (every
+      // tile is read; no visited-row skip)
       SpmvArgs c = a;
       c.out = a.bfs_counts;
       c.accumulate = 0;

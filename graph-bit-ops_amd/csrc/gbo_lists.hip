@@ -553,7 +553,9 @@ int sweep_t(const ListView& l, const ListSweep& s, hipStream_t st) {
 //   15 to 20 sweeps (PageRank), bs 8: R-MAT 2^18, 62 MB, 1.01 -> 1.05 ms,
 //   285 MB 3.18 -> 2.30; bs 16: 57 MB 0.79 -> 0.80, 143 MB 1.38 -> 1.02; bs 32,
 //   63 MB 1.61 -> 0.73; bs 64, 41 MB 0.65 -> 0.56, 151 MB 1.04 -> 0.64, 5.2 GB
-//   15.5 -> 3.1 (weighted shortest paths 8.4 -> 2.7)
+//   15.5 -> 3.1
+//   weighted shortest paths, which skip the tiles of inactive block columns,
+//   bs 8: 285 MB 1.94 -> 1.63, 1.26 GB 7.53 -> 7.72; bs 64 5.2 GB 8.4 -> 2.7
 //   3 to 5 sweeps (components), bs 16: 700 MB 0.80 -> 0.82; bs 32: 207 MB
 //   0.45 -> 0.49, 367 MB 0.62 -> 0.47, 1.9 GB 1.88 -> 1.13; bs 64: 350 MB
 //   0.38 -> 0.39, 761 MB 0.99 -> 0.58, 5.2 GB 2.78 -> 1.77
@@ -565,6 +567,9 @@ void lists_build(const gbo_bsr* A, ListUse use, Workspace& mem, ListView* out, h
   const int64_t bytes = A->nblocks * (A->bs * A->bs / 8 + 4), mb = 1 << 20;
   int64_t least = 0;
   switch (use) {
+    case ListUse::kPaths:
+      if (A->bs == 8 && bytes > 1024 * mb) return;
+      [[fallthrough]];
     case ListUse::kMany: least = A->bs == 8 ? 192 * mb : A->bs == 16 ? 96 * mb : 48 * mb; break;
     case ListUse::kFew: least = A->bs <= 16 ? INT64_MAX : A->bs == 32 ? 256 * mb : 512 * mb; break;
     case ListUse::kFrontiers: least = 16 * mb; break;

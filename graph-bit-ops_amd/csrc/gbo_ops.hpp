@@ -25,7 +25,7 @@ namespace gbo {
 //   slots       kCountSlots x u64   BFS frontier-size slots (zero between calls)
 //   count       1 x int64           the folded frontier size
 //   partial     nchunks*2*bs x f64  split-row partials of the FP32 sum
-//   bfs_counts  bs*(nbr+1) x int32  per-row counts of the dense BFS step (bs 8)
+//   bfs_counts  bs*(nbr+1) x int32  per-row counts of the dense BFS step
 // Calls on one matrix therefore share that scratch: they must be ordered
 // (one stream, or synchronised); separately created matrices do not share.
 struct PlanLayout {
@@ -267,7 +267,7 @@ struct ListMs {
   const uint64_t *active, *live;
   const unsigned long long* go;
 };
-enum class ListUse { kMany, kFew, kFrontiers };  // sweeps of a call: ten and more, a few; multi-source BFS
+enum class ListUse { kMany, kPaths, kFew, kFrontiers };  // sweeps of a call: PageRank's, shortest paths', a few; multi-source BFS
 void lists_build(const gbo_bsr* A, ListUse use, Workspace& mem, ListView* out, hipStream_t st);
 // OP_SUM, OP_MIN, or OP_MINPLUS without the vertex's own value.
 int lists_sweep(int op, const ListView& l, const ListSweep& s, hipStream_t st);
@@ -280,8 +280,9 @@ constexpr int kCountSlots = 1024;
 enum SpmvOp { OP_COUNT = 0, OP_BFS = 1, OP_MINPLUS = 2, OP_SUM = 3, OP_MIN = 4 };
 
 // Whether a BFS step at this block size and plan variant may take the dense
-// form (count kernel into per-row counts, then a pack of the nonzero rows).
-inline bool dense_bfs_step(int bs, int variant) { return bs == 8 && variant == 3; }
+// form (count kernel into per-row counts, then a pack of the nonzero rows):
+// bs 8/16 under variant 3, bs 32/64 under every variant.
+inline bool dense_bfs_step(int bs, int variant) { return (bs <= 16 && variant == 3) || bs >= 32; }
 
 struct SpmvArgs {
   const int32_t* rowptr;

@@ -686,7 +686,7 @@ PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr) {
   L.partial = off;
   off += align256(sizeof(double) * 2 * (size_t)nchunks * bs);
   L.bfs_counts = off;
-  if (bs == 8) off += align256(sizeof(int32_t) * (size_t)bs * ((size_t)nbr + 1));
+  off += align256(sizeof(int32_t) * (size_t)bs * ((size_t)nbr + 1));
   L.bytes = off;
   return L;
 }

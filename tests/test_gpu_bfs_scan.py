@@ -8,9 +8,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("chunk", (0, 7, 300))  # rows whole and cut
-@pytest.mark.parametrize("bs", (16, 32, 64))
-def test_steps(gbo, po, bs, chunk):
+def _graph(gbo, bs):
     rng = np.random.default_rng(bs)
     n = 1030 * bs + 5
     counts = np.zeros(n, np.int64)
@@ -25,10 +23,43 @@ def test_steps(gbo, po, bs, chunk):
         blocks = rng.choice(1030, k, replace=False) if k <= 1030 else np.arange(k)
         rows.append(np.sort(blocks * bs + rng.integers(0, bs, k)))
     ci = np.concatenate(rows).astype(np.int32)
-    g = gbo.Csr(n, n, rp, ci)
+    return gbo.Csr(n, n, rp, ci)
+
+
+@pytest.mark.parametrize("chunk", (0, 7, 300))  # rows whole and cut
+@pytest.mark.parametrize("bs", (16, 32, 64))
+def test_searches(gbo, bs, chunk):
+    g = _graph(gbo, bs)
+    n, ci = g.nrows, g.colind
     A = gbo.BsrMatrix.from_csr(g, bs)
     if chunk:
         A.plan(chunk)
+    edge = np.repeat(np.arange(n), np.diff(g.rowptr))
+    rng = np.random.default_rng(1)
+    into = np.bincount(ci, minlength=n)
+    for source in [int(np.argmax(into)), int(ci[0])] + list(rng.integers(0, n, 4)):
+        level = np.full(n, -1, np.int32)
+        front, depth = np.array([source]), 0
+        while len(front):
+            level[front] = depth
+            depth += 1
+            hit = np.unique(edge[np.isin(ci, front)])
+            front = hit[level[hit] < 0]
+        got, sizes = gbo.bfs(A, int(source))
+        assert np.array_equal(got, level) and len(sizes) == depth
+
+
+@pytest.mark.parametrize("chunk", (0, 7, 300))
+@pytest.mark.parametrize("bs", (16, 32, 64))
+def test_steps(gbo, po, bs, chunk):
+    g = _graph(gbo, bs)
+    n, rp, ci = g.nrows, g.rowptr, g.colind
+    counts = np.diff(rp)
+    rng = np.random.default_rng(2)
+    A = gbo.BsrMatrix.from_csr(g, bs)
+    A.plan(0, 0)  # at bs 16 the variant without the count kernel's form
+    if chunk:
+        A.plan(chunk, 0)
     edge = np.repeat(np.arange(n), counts)
     cnt = gbo.DeviceBuffer(8)
     for share in (0.0, 0.002, 0.3, 1.0):
