@@ -4,10 +4,10 @@
 //
 // The reference drivers launch five to nine kernels per iteration, fill
 // vectors with single-thread <<<1,1>>> kernels inside the timed loop and
-// copy a convergence scalar to the host each iteration.  Here every
-// iteration is one bsrbmv launch plus one fused element-wise kernel (update
-// of frontier/visited/levels, distances, scores or labels together with the
-// convergence reduction); the host reads one 8-byte scalar per iteration.
+// copy a convergence scalar to the host each iteration.  Here an iteration is
+// one product and one or two fused element-wise kernels (update of frontier/
+// visited/levels, distances, scores or labels together with the convergence
+// reduction), and the host looks at the flags of several iterations together.
 #include <algorithm>
 #include <cmath>
 #include <mutex>

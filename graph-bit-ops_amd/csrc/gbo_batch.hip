@@ -11,7 +11,8 @@
 // tile row, four lanes per entry); rows are masked with ~V and stored (or
 // OR-ed atomically for rows cut by a chunk boundary).  A per
 // block-column activity mask (any frontier bit among the block's vertices)
-// lets the sweep skip tiles whose columns hold no frontier vertex.
+// lets the sweep skip tiles whose columns hold no frontier vertex.  Larger
+// matrices are swept as edge lists (gbo_lists.hip) instead.
 #include <algorithm>
 #include <vector>
 

@@ -4,8 +4,8 @@
 // masked_v4 (BFS), bmv32_sparse_full_minplus (SSSP), bmv32_sparse_full (PR),
 // bmv32_sparse_full_cc_new (CC) in algorithm/bsrbmv.cu.  The reference maps
 // one warp to one block row (lane = tile row) and so idles on power-law
-// rows; here every wavefront takes a fixed-size CHUNK of consecutive tiles
-// (a tile-balanced split, independent of the row structure) and walks the
+// rows; here every wavefront takes a CHUNK of consecutive tiles (about equal
+// work, mostly independent of the row structure) and walks the
 // block rows that chunk touches.  Lane l of the wave is row (l % bs) of tile
 // group (l / bs): a bs=64 tile is one coalesced 512-B load per wave, a bs=32
 // step loads two tiles, bs=16 four, bs=8 eight.  Rows that a chunk boundary

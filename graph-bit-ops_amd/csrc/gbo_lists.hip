@@ -172,17 +172,22 @@ __global__ __launch_bounds__(256) void k_list(const ListView l, uint32_t* __rest
   if (lane_id() == 0) cnt[it] = n;
 }
 
-// An item's entries past its room (0: it is listed) and its parts.
+// An item's entries past its room (0: it is listed) and its parts; the items
+// past their room, in any order.
 template <int BS>
 __global__ __launch_bounds__(256) void k_item_parts(const ListView l, const int32_t* __restrict__ cnt, int64_t cap,
-                                                    int32_t* __restrict__ over, int32_t* __restrict__ parts) {
+                                                    int32_t* __restrict__ over, int32_t* __restrict__ parts,
+                                                    int32_t* __restrict__ overs, ListInfo* __restrict__ info) {
   const int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (it >= cap) return;
   int32_t o = 0, p = 0;
   if (it < l.first[l.nwin]) {
     const Item I = item_of<BS>(l, it);
     const int32_t n = cnt[it];
-    if (n > (I.t1 - I.t0) * kRoom<BS>) o = n;
+    if (n > (I.t1 - I.t0) * kRoom<BS>) {
+      o = n;
+      overs[atomicAdd(&info->overs, 1)] = (int32_t)it;  // one item in a hundred
+    }
     p = max((n + kPart - 1) / kPart, 1);
   }
   over[it] = o;
@@ -227,41 +232,40 @@ __global__ __launch_bounds__(256) void k_win_parts(const ListView l, const int64
 
 // The items past their room, kOverSplit workgroups each: the waves of all of
 // them take consecutive shares of the tiles and write one after another; a
-// workgroup counts the shares up to its own.
+// workgroup counts the shares up to its own.  (Workgroups for every item, most
+// of which leave at once, took 212 us on R-MAT 2^20 at bs 64.)
 constexpr int kOverThreads = 1024, kOverSplit = 4;
 template <int BS>
 __global__ __launch_bounds__(kOverThreads) void k_list_over(const ListView l, const int64_t* __restrict__ opos,
-                                                            int64_t items, uint32_t* __restrict__ edges) {
+                                                            const int32_t* __restrict__ overs,
+                                                            uint32_t* __restrict__ edges) {
   using Wk = Walk<BS>;
   constexpr int W = kOverThreads / kWave;
   __shared__ int sh[W * kOverSplit];
   const int wave = threadIdx.x / kWave, q = blockIdx.y;
-  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
-    if (opos[it + 1] == opos[it]) continue;
-    const Item I = item_of<BS>(l, it);
-    const Wk walk(l, l.win[it]);
-    const int64_t share = ((I.t1 - I.t0 + W * kOverSplit - 1) / (W * kOverSplit) + Wk::TS - 1) / Wk::TS * Wk::TS;
-    __syncthreads();
-    for (int k = wave; k < (q + 1) * W; k += W) {
-      const int64_t b0 = min(I.t0 + k * share, I.t1), b1 = min(b0 + share, I.t1);
-      int own = 0;
-      for (int64_t x = b0 * Wk::WPT + lane_id(); x < b1 * Wk::WPT; x += kWave) own += __popcll(((const uint64_t*)l.tiles)[x]);
-      own = __shfl(wave_incl_scan(own), kWave - 1);
-      if (lane_id() == 0) sh[k] = own;
-    }
-    __syncthreads();
-    const int mine = q * W + wave;
-    int at = 0;
-    for (int k = 0; k < mine; ++k) at += sh[k];
-    const int64_t b0 = min(I.t0 + mine * share, I.t1), b1 = min(b0 + share, I.t1);
-    uint32_t* out = edges + opos[it];
-    for (int64_t b = b0; b < b1; b += Wk::U * Wk::TS) {
-      uint64_t v[Wk::U];
-      uint32_t e[Wk::U];
-      walk.load(l, b, b1, v, e);
+  const int64_t it = overs[blockIdx.x];
+  const Item I = item_of<BS>(l, it);
+  const Wk walk(l, l.win[it]);
+  const int64_t share = ((I.t1 - I.t0 + W * kOverSplit - 1) / (W * kOverSplit) + Wk::TS - 1) / Wk::TS * Wk::TS;
+  for (int k = wave; k < (q + 1) * W; k += W) {
+    const int64_t b0 = min(I.t0 + k * share, I.t1), b1 = min(b0 + share, I.t1);
+    int own = 0;
+    for (int64_t x = b0 * Wk::WPT + lane_id(); x < b1 * Wk::WPT; x += kWave) own += __popcll(((const uint64_t*)l.tiles)[x]);
+    own = __shfl(wave_incl_scan(own), kWave - 1);
+    if (lane_id() == 0) sh[k] = own;
+  }
+  __syncthreads();
+  const int mine = q * W + wave;
+  int at = 0;
+  for (int k = 0; k < mine; ++k) at += sh[k];
+  const int64_t b0 = min(I.t0 + mine * share, I.t1), b1 = min(b0 + share, I.t1);
+  uint32_t* out = edges + opos[it];
+  for (int64_t b = b0; b < b1; b += Wk::U * Wk::TS) {
+    uint64_t v[Wk::U];
+    uint32_t e[Wk::U];
+    walk.load(l, b, b1, v, e);
 #pragma unroll
-      for (int u = 0; u < Wk::U; ++u) at += put_bits<BS>(out, at, v[u], e[u]);
-    }
+    for (int u = 0; u < Wk::U; ++u) at += put_bits<BS>(out, at, v[u], e[u]);
   }
 }
 
@@ -496,13 +500,14 @@ int build_t(const gbo_bsr* A, Workspace& mem, ListView* out, hipStream_t st) {
       (rc = mem.alloc(&first, sizeof(int64_t) * ((size_t)l.nwin + 1), who)) ||
       (rc = mem.alloc(&wfirst, sizeof(int64_t) * ((size_t)l.nwin + 1), who)) ||
       (rc = mem.alloc(&multi, sizeof(int32_t) * (size_t)l.nwin, who)) ||
-      (rc = mem.alloc(&win, sizeof(int32_t) * (size_t)cap * 4, who)) ||
+      (rc = mem.alloc(&win, sizeof(int32_t) * (size_t)cap * 5, who)) ||
       (rc = mem.alloc(&opos, sizeof(int64_t) * ((size_t)cap + 1), who)) ||
       (rc = mem.alloc(&ppos, sizeof(int64_t) * ((size_t)cap + 1), who)))
     return rc;
   cnt = win + cap;
   over = cnt + cap;
   np = over + cap;
+  int32_t* overs = np + cap;
   l.first = first;
   l.win = win;
   k_win_items<BS><<<grid_of(l.nwin, 256), 256, 0, st>>>(l, icnt);
@@ -510,7 +515,7 @@ int build_t(const gbo_bsr* A, Workspace& mem, ListView* out, hipStream_t st) {
   if ((rc = scan_exclusive<int32_t, int64_t>(icnt, first, l.nwin, st, mem))) return rc;
   k_item_wins<<<grid_of(l.nwin, 256), 256, 0, st>>>(l, win);
   k_list<BS><<<grid_of(cap, 4), 256, 0, st>>>(l, edges, cnt);
-  k_item_parts<BS><<<grid_of(cap, 256), 256, 0, st>>>(l, cnt, cap, over, np);
+  k_item_parts<BS><<<grid_of(cap, 256), 256, 0, st>>>(l, cnt, cap, over, np, overs, info);
   GBO_LAUNCH_CHECK();
   if ((rc = scan_exclusive<int32_t, int64_t>(over, opos, cap, st, mem)) ||
       (rc = scan_exclusive<int32_t, int64_t>(np, ppos, cap, st, mem)))
@@ -525,7 +530,7 @@ int build_t(const gbo_bsr* A, Workspace& mem, ListView* out, hipStream_t st) {
   uint32_t* rest = nullptr;
   if (h.over && (rc = mem.alloc(&rest, sizeof(uint32_t) * (size_t)h.over, who))) return rc;
   k_parts_fill<BS><<<grid_of(h.items, 256), 256, 0, st>>>(l, cnt, opos, ppos, edges, rest, parts);
-  if (h.over) k_list_over<BS><<<dim3((unsigned)std::min<int64_t>(h.items, 4096), kOverSplit), kOverThreads, 0, st>>>(l, opos, h.items, rest);
+  if (h.over) k_list_over<BS><<<dim3((unsigned)h.overs, kOverSplit), kOverThreads, 0, st>>>(l, opos, overs, rest);
   GBO_LAUNCH_CHECK();
   l.first = wfirst;
   l.multi = multi;

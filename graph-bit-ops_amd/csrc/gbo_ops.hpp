@@ -251,7 +251,7 @@ constexpr int kListSlots = 64;
 struct ListInfo {
   int64_t items, parts, over;
   unsigned long long sample[kListSlots];
-  int32_t multi;
+  int32_t multi, overs;
 };
 struct ListSweep {
   const void* x;
