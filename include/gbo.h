@@ -212,8 +212,9 @@ int gbo_bsr_create(int bs, int dir, const int32_t* h_rowptr, const int32_t* h_co
 void gbo_bsr_free(gbo_bsr* A);
 /* Work decomposition: split the tiles into chunks of `chunk_tiles` and record
  * each chunk's first block row.  0 lets the library choose: chunks of about
- * equal work, at most 256 tiles each and shorter on small matrices and where
- * tiles are dense (reads the tiles once and synchronizes the stream).
+ * equal work, about 256 tiles each and shorter on small matrices and where
+ * tiles are dense, ending at block rows where these are short (reads the tiles
+ * once and synchronizes the stream).
  * Allocates A->plan (released by gbo_bsr_free / gbo_bsr_plan_free). */
 int gbo_bsr_plan(gbo_bsr* A, int32_t chunk_tiles, gbo_stream_t stream);
 /* As gbo_bsr_plan, also selecting the bs 8/16 kernel variant of the COUNT
@@ -224,16 +225,17 @@ int gbo_bsr_plan(gbo_bsr* A, int32_t chunk_tiles, gbo_stream_t stream);
  * variant 0; needs 16-byte-aligned tiles/colind, else variant 0 runs),
  * 3 = bs 8 COUNT with 32-bit chunk-relative indexing and byte-transposed
  * popcounts (4 tiles per v_bcnt) and a permlane/DPP row reduction, bs 16
- * COUNT with four lanes per tile (8 bytes each); the BFS step of both is
- * dense (that count kernel gives each row's number of frontier neighbours, a
- * pack kernel keeps the nonzero unvisited rows; every tile is read, so
- * gbo_bfs takes it while fewer than half the vertices are visited and the
- * visited-row-skipping step after); at bs 8 and 16, min / min-plus / FP32 sum
+ * COUNT with four lanes per tile (8 bytes each); gbo_bsrbmv_bfs_step of both
+ * is dense (that count kernel gives each row's number of frontier neighbours,
+ * a pack kernel keeps the nonzero unvisited rows; every tile is read, so at
+ * bs 8 gbo_bfs takes it on large matrices while fewer than half the vertices
+ * are visited and the visited-row-skipping step after); at bs 8 and 16, min / min-plus / FP32 sum
  * list the tiles' set bits in LDS so the value gathers spread over all lanes
  * (the sum folds them into FP64 accumulators private to one wavefront).
- * bs 32 and 64 have one kernel set whatever the variant; their BFS step is
- * dense too (bs 32 COUNT with eight lanes per tile, bs 64 COUNT with scalar
- * per-tile reads).
+ * bs 32 and 64 have one kernel set whatever the variant; their
+ * gbo_bsrbmv_bfs_step is dense too (bs 32 COUNT with eight lanes per tile, bs
+ * 64 COUNT with scalar per-tile reads).  Searches at bs 16 to 64 read the column
+ * indices and then only the tiles under the frontier.
  * Integer results are identical; only speed differs (the autotuner picks).
  * The FP32 sum's order of additions depends on the chunk size and variant,
  * each fixed by the plan, so its last bits may differ between plans.
@@ -374,6 +376,10 @@ int gbo_bfs_do(const gbo_bsr* AT, const gbo_bsr* A, int32_t source, int32_t* d_l
                int64_t* h_level_sizes, int32_t max_levels, int32_t* h_nlevels,
                gbo_stream_t stream);
 
+/* The drivers below and gbo_bfs_multisource list the nonzeros of large sparse
+ * matrices once per call and sweep the list: 12 (bs 8) to 64 (bs 64) bytes of
+ * scratch per tile, kept between calls up to 1 GiB; without that memory they
+ * sweep the tiles, with the same results. */
 /* SSSP (algorithm/sssp.cu:420-488) generalised to uint32 weights:
  * frontier Bellman-Ford on the min-plus semiring; dist = INF (0xFFFFFFFF)
  * when unreachable.  d_w/d_woff as for gbo_bsrbmv_minplus (NULL = unit). */
