@@ -49,7 +49,7 @@ struct PlanView {
 };
 
 // Most tiles per chunk of the library's own plans.
-int default_chunk(int bs, int64_t tiles);
+int default_chunk(int bs, int64_t tiles, bool uniform);
 int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st);
 int release_plan(PlanView* pv, hipStream_t st);
 // Allocates A->plan with its scratch (chunk tiles per chunk, 0 = the library's

@@ -491,17 +491,40 @@ __global__ __launch_bounds__(256) void k_unit_chunks(const int64_t* __restrict__
 
 // Most tiles per chunk of the library's own plans: 256 on large matrices, and
 // less where that leaves a sweep short of waves (8192 are resident), down to
-// 16.  At bs 16 to 64 256 tiles make two to four rounds of waves and an
-// uneven last one up to some 12M tiles: R-MAT 2^18 bs 16 (4M) count 67 / 88 us
-// at 128 / 256 tiles, G(n, m) with 3.2M tiles 31 / 31 us, with 16.6M tiles bs
-// 32 sum 512 / 487 us.  At bs 8 a step of the count takes 256 tiles (G(n, m)
-// with 3.2M tiles 20 / 17 us).  Small ones: G(n, m) with 0.5M tiles bs 8 12.6 /
-// 8.3 / 8.1 us at 32 / 128 / 256; G(1024) bs 32 (1024 tiles) sum 9 / 18 / 59 us
-// at 16 / 64 / 256.
-int default_chunk(int bs, int64_t tiles) {
-  if (tiles >= (bs == 8 ? 2ll << 20 : 12ll << 20)) return 256;
+// 16.  `uniform`: no tiles are denser than the rest, so that a chunk of as many
+// tiles is as much work.
+//   bs 8   a step of the count takes 256 tiles: G(n, m) with 1.6M tiles count /
+//          min 15.3 / 19.1 us at 128 tiles, 14.6 / 17.6 at 256.  Where some tiles
+//          are dense the sweep ends with them up to some 4M (R-MAT with 3.7M
+//          count 37 / 42 us).
+//   bs 16  256 tiles make few rounds of waves and an uneven last one (G(n, m)
+//          with 8M min 95 / 103 us), with dense tiles up to 32M (R-MAT with 16.4M
+//          count 172 / 197 us, with 23.7M min-plus 351 / 373; G(n, m) with 24M
+//          488 / 479).
+//   bs 32, 64  the starts of chunks of 128 tiles lie 16 and 64 KB apart, where
+//          many waves read from the same memory channels at once: 96 / 128 tiles
+//          on G(n, m) with 1.1M at bs 64 min 98 / 112 us, with 1.2M at bs 32
+//          min-plus 37 / 43, R-MAT with 6.2M at bs 32 min-plus 309 / 337.  From
+//          some 6M on a sum loses by the rows that more chunks cut (R-MAT with
+//          7.7M at bs 64 799 / 771), from 12M on 256 are better still (G(n, m)
+//          with 16.6M at bs 32 sum 512 / 487 at 128 / 256).  Uniform tiles of bs
+//          32 that 8192 waves take in one round do so, in chunks of an odd
+//          multiple of 16 tiles, from 208 on of 256: count of G(n, m) with 0.93M
+//          28.0 / 25.3 us at 96 / 144, with 1.4M 36.7 / 35.4 at 96 / 176, with
+//          1.6M 40.5 / 40.4 / 37.9 at 96 / 208 / 256; beyond one round 96 again
+//          (with 2.3M min-plus 77 / 90 at 96 / 256).
+// Small ones: G(n, m) with 0.5M tiles bs 8 12.6 / 8.3 / 8.1 us at 32 / 128 / 256;
+// G(1024) bs 32 (1024 tiles) sum 9 / 18 / 59 us at 16 / 64 / 256.
+int default_chunk(int bs, int64_t tiles, bool uniform) {
+  const int64_t large = bs == 8 ? (uniform ? 1 : 4) : bs == 16 && !uniform ? 32 : 12;
+  if (tiles >= large << 20) return 256;
+  if (bs == 32 && uniform && tiles >= (512 << 10) && tiles <= (2ll << 20)) {
+    const int once = 16 * (int)((tiles / 8192 + 15) / 16 | 1);
+    return once > 192 ? 256 : once;
+  }
+  const int64_t most = bs >= 32 && tiles < (6ll << 20) ? 96 : 128;
   const int64_t c = (tiles / 4096 + 8) / 16 * 16;
-  return (int)std::min<int64_t>(128, std::max<int64_t>(c, 16));
+  return (int)std::min(most, std::max<int64_t>(c, 16));
 }
 
 // Above this many tiles the densest chunk ends long before the sweep does,
@@ -791,7 +814,7 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
     view_scratch(pv, A->bs, A->nblockrows, A->plan_even == 1);
     return GBO_OK;
   }
-  const int32_t chunk = default_chunk(A->bs, A->nblocks);
+  const int32_t chunk = default_chunk(A->bs, A->nblocks, true);
   const int64_t nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "too many chunks");
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
@@ -807,11 +830,11 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
 }
 
 int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st) {
-  const int32_t chunk = chunk_tiles > 0 ? chunk_tiles : default_chunk(A->bs, A->nblocks);
+  int32_t chunk = chunk_tiles > 0 ? chunk_tiles : default_chunk(A->bs, A->nblocks, false);
   // equal work needs the tiles' bits in 16-byte reads; the kernels that gain
   // from it need the same alignment
   bool even = chunk_tiles > 0 || A->nblocks == 0 || A->nblocks >= kEvenTiles || !A->tiles || ((uintptr_t)A->tiles & 15);
-  int64_t nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
+  int64_t nch = 0;
   Workspace mem(st);
   WorkCut w;
   if (!even) {
@@ -825,7 +848,9 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st
     if (rc) return rc;
     even = w.total == w.nunits * w.target / chunk * w.unit;  // no unit has more than its tiles' work
     if (!even) nch = w.nch;
+    else chunk = default_chunk(A->bs, A->nblocks, true);
   }
+  if (even) nch = std::max<int64_t>(1, (A->nblocks + chunk - 1) / chunk);
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "gbo_bsr_plan: too many chunks");
   bool whole = false;
   const int32_t longest = whole_row(A->bs, A->nblocks, chunk);

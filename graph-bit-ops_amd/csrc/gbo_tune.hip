@@ -78,7 +78,7 @@ int gbo_autotune(const int32_t* d_rowptr, const int32_t* d_colind, int32_t nrows
     GBO_HIP_CHECK(hipMalloc((void**)&cnt, sizeof(int64_t)));
     GBO_HIP_CHECK(hipMemsetAsync(x, 0x55, nw * bs / 8, st));   // half the frontier / x bits set
     GBO_HIP_CHECK(hipMemsetAsync(vis, 0, nw * bs / 8, st));
-    const int dc = default_chunk(bs, A.nblocks);
+    const int dc = default_chunk(bs, A.nblocks, true);
     const int chunks[3] = {dc, dc * 2, dc / 2};
     // kernel variants that differ for this block size and operation (bs 8
     // and 16 BFS: 3 is the dense count-based step; 2 would run variant 0)
