@@ -68,7 +68,9 @@ struct PlanGuard {
 
 // Device scratch of one call that waits for its stream before it returns:
 // blocks kept between calls (gbo_workspace.hip), given back on every return
-// path once the stream has been waited for.
+// path once the stream has been waited for.  What drop() is given is handed out
+// again to the same call, in the order of its stream: a loop of any length
+// holds the blocks of one turn.
 class Workspace {
  public:
   explicit Workspace(hipStream_t st) : st_(st) {}
@@ -82,6 +84,7 @@ class Workspace {
     *p = (T*)q;
     return rc;
   }
+  void drop(const void* p);
 
  private:
   int take(void** p, size_t bytes, const char* who);
@@ -90,6 +93,7 @@ class Workspace {
   int dev_ = -1;
   void* ptrs_[kMax];
   size_t bytes_[kMax];
+  bool spare_[kMax];  // dropped
   int n_ = 0;
 };
 // hipMalloc that gives the kept blocks back before it reports that memory is

@@ -79,8 +79,8 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(const TI* in, int64
 
 // The block sums' offsets of a scan of nb tiles (room for 2 nb + 1 int64 in
 // bsum), then the scan itself; nested through itself where nb needs it.
-template <class TI, class TO, class Alloc>
-static int scan_with(const TI* in, TO* out, int64_t n, hipStream_t st, Alloc alloc) {
+template <class TI, class TO, class Alloc, class Drop>
+static int scan_with(const TI* in, TO* out, int64_t n, hipStream_t st, Alloc alloc, Drop drop) {
   if (n <= 0) {
     GBO_HIP_CHECK(hipMemsetAsync(out, 0, sizeof(TO), st));
     return GBO_OK;
@@ -97,9 +97,10 @@ static int scan_with(const TI* in, TO* out, int64_t n, hipStream_t st, Alloc all
   int64_t* boff = bsum + nb;
   k_scan_reduce<TI><<<(unsigned)nb, kScanThreads, 0, st>>>(in, n, bsum);
   GBO_LAUNCH_CHECK();
-  if ((rc = scan_with<int64_t, int64_t>(bsum, boff, nb, st, alloc))) return rc;
+  if ((rc = scan_with<int64_t, int64_t>(bsum, boff, nb, st, alloc, drop))) return rc;
   k_scan_apply<TI, TO><<<(unsigned)nb, kScanThreads, 0, st>>>(in, n, boff, out);
   GBO_LAUNCH_CHECK();
+  drop(bsum);
   return GBO_OK;
 }
 
@@ -107,12 +108,14 @@ static int scan_with(const TI* in, TO* out, int64_t n, hipStream_t st, Alloc all
 template <class TI, class TO>
 int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st) {
   AsyncAllocs mem(st);
-  return scan_with(in, out, n, st, [&](int64_t** p, size_t bytes) { return mem.alloc(p, bytes, "scan"); });
+  return scan_with(in, out, n, st, [&](int64_t** p, size_t bytes) { return mem.alloc(p, bytes, "scan"); },
+                   [](const void*) {});
 }
 
 template <class TI, class TO>
 int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st, Workspace& mem) {
-  return scan_with(in, out, n, st, [&](int64_t** p, size_t bytes) { return mem.alloc(p, bytes, "scan"); });
+  return scan_with(in, out, n, st, [&](int64_t** p, size_t bytes) { return mem.alloc(p, bytes, "scan"); },
+                   [&](const void* p) { mem.drop(p); });
 }
 
 template int scan_exclusive<int32_t, int32_t>(const int32_t*, int32_t*, int64_t, hipStream_t);

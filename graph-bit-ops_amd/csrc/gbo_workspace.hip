@@ -127,9 +127,17 @@ Workspace::~Workspace() {
 
 int Workspace::take(void** p, size_t bytes, const char* who) {
   *p = nullptr;
+  const size_t want = rounded(bytes);
+  int s = -1;  // the smallest dropped block that fits
+  for (int i = 0; i < n_; ++i)
+    if (spare_[i] && bytes_[i] >= want && (s < 0 || bytes_[i] < bytes_[s])) s = i;
+  if (s >= 0) {
+    spare_[s] = false;
+    *p = ptrs_[s];
+    return GBO_OK;
+  }
   if (n_ == kMax) return set_error(GBO_EINVAL, "%s: too many scratch allocations", who);
   if (n_ == 0) GBO_HIP_CHECK(hipGetDevice(&dev_));
-  const size_t want = rounded(bytes);
   void* q = nullptr;
   size_t got = want;
   if (dev_ >= 0 && dev_ < kDevices) {
@@ -152,9 +160,15 @@ int Workspace::take(void** p, size_t bytes, const char* who) {
       return set_error(GBO_ENOMEM, "%s: device allocation of %zu bytes failed: %s", who, bytes, hipGetErrorString(e));
   }
   ptrs_[n_] = q;
+  spare_[n_] = false;
   bytes_[n_++] = got;
   *p = q;
   return GBO_OK;
+}
+
+void Workspace::drop(const void* p) {
+  for (int i = 0; i < n_; ++i)
+    if (ptrs_[i] == p) spare_[i] = true;
 }
 
 // ---- small host reads.  A copy into ordinary host memory is staged by the
