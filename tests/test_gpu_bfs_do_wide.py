@@ -23,3 +23,34 @@ def test_king_from_the_middle(gbo, m, bs):
         assert np.array_equal(lv, want), (x, y)
         assert np.array_equal(sizes, np.bincount(want)), (x, y)
     A.free()
+
+
+@pytest.mark.parametrize("bs", (8, 32))
+def test_wide_and_narrow_in_turn(gbo, po, bs):
+    """Four grids joined by paths: frontiers grow past what one workgroup takes
+    and shrink to one vertex again."""
+    m, path = 800, 40
+    step = m * m + path
+    k = gbo.gen_king(m)
+    row = np.repeat(np.arange(k.nrows), np.diff(k.rowptr))
+    u, v = [], []
+    for q in range(4):
+        o = q * step
+        u.append(row + o)
+        v.append(k.colind + o)
+        # from the last row's middle, over the path, to the middle of the next grid's first row
+        chain = np.concatenate([[o + m * (m - 1) + m // 2], o + m * m + np.arange(path), [o + step + m // 2]])
+        chain = chain[chain < 4 * step]
+        u += [chain[:-1], chain[1:]]
+        v += [chain[1:], chain[:-1]]
+    n = 4 * step
+    key = np.unique(np.concatenate(u).astype(np.int64) * n + np.concatenate(v))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(key // n, minlength=n))])
+    g = gbo.Csr(n, n, rp, key % n)
+    A = gbo.BsrMatrix.from_csr(g, bs)
+    for s in (m // 2 * m + m // 2, 0, n - 1):
+        want = po.bfs(n, g.rowptr, g.colind, s)
+        lv, sizes = gbo.bfs(A, s, max_levels=8192, A=A)
+        assert np.array_equal(lv, want), s
+        assert np.array_equal(sizes, np.bincount(want)), s
+    A.free()
