@@ -166,6 +166,7 @@ int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st, Workspace& 
 // `above` nonzeros: heavy_list finds them, heavy_count writes their tile counts
 // and raises PACKERR flags, heavy_fill writes their block columns and tiles
 // (from off, the first tile of each block row), for rows that raised none.
+// heavy_walks: how often each reads a block row, by the matrix's width.
 enum { PACKERR_COLRANGE = 1, PACKERR_UNSORTED = 2 };
 struct PackCsr {
   const int32_t *rp, *ci;
@@ -176,6 +177,7 @@ struct HeavyRows {
   int32_t* n = nullptr;  // device
   int32_t above = 0;
 };
+int64_t heavy_walks(int bs, int32_t ncols);
 int heavy_list(int bs, const PackCsr& A, Workspace& mem, HeavyRows* h, const char* who, hipStream_t st);
 int heavy_count(int bs, const PackCsr& A, const HeavyRows& h, int32_t* cnt, int* err, hipStream_t st);
 int heavy_fill(int bs, int dir, const PackCsr& A, const HeavyRows& h, int32_t nheavy, const int64_t* off, int64_t T,

@@ -11,7 +11,7 @@
 // column into its own row word -- which is directly word r of the tile in
 // the reference layout (MSB = column 0).  Two passes: count tiles, scan, then
 // fill colind/tiles.  No dense staging.  Block rows of many nonzeros are not
-// merged (gbo_pack_fill.hip).
+// merged (gbo_pack_fill.hip), or on very wide matrices merged in pieces.
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -128,7 +128,8 @@ template int scan_exclusive<int64_t, int64_t>(const int64_t*, int64_t*, int64_t,
 // ---------------------------------------------------------------- packing
 enum { PACK_COUNT = 0, PACK_ROW = 1, PACK_COL = 2, PACK_VALUES = 3 };
 
-// Where values follow the tiles' bits, a block row with more than kPieceNnz
+// Where values follow the tiles' bits, and on matrices of more than kMostWalks
+// walks, a block row with more than kPieceNnz
 // nonzeros is merged in pieces: ranges of block columns [lo, hi), one group
 // each, cut at evenly spaced entries of the block row's longest CSR row.  A
 // single group's merge over the hub block row of R-MAT s22 (129,447 tiles at
@@ -168,7 +169,9 @@ __device__ __forceinline__ int32_t first_blockcol_at_least(const int32_t* __rest
   return q0;
 }
 
-template <int BS, int MODE>
+// PIECES: by the table.  A kernel of its own, without the stage and the look at
+// each block row's length, which cost the merge of pieces a tenth.
+template <int BS, int MODE, bool PIECES>
 __global__ __launch_bounds__(256) void k_pack(const int32_t* __restrict__ rp,
                                               const int32_t* __restrict__ ci, int32_t nrows,
                                               int32_t ncols, int32_t nbr,
@@ -184,19 +187,19 @@ __global__ __launch_bounds__(256) void k_pack(const int32_t* __restrict__ rp,
   const int lane = lane_id();
   const int g = lane / BS, r = lane % BS;
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const int64_t npc = pc.row ? (int64_t)pc.n : (int64_t)nbr;
+  const int64_t npc = PIECES ? (int64_t)pc.n : (int64_t)nbr;
   const int64_t pi = wave * G + g;  // piece of this group
   if (wave * G >= npc) return;      // wave-uniform
   bool blk_ok = pi < npc;
-  const int64_t I = pc.row ? (blk_ok ? (int64_t)pc.row[pi] : 0) : pi;
+  const int64_t I = PIECES ? (blk_ok ? (int64_t)pc.row[pi] : 0) : pi;
   const int64_t row = I * BS + r;
-  if (blk_ok && pc.above != INT_MAX) blk_ok = rp[min((I + 1) * BS, (int64_t)nrows)] - rp[I * BS] <= pc.above;
+  if (!PIECES && blk_ok && pc.above != INT_MAX) blk_ok = rp[min((I + 1) * BS, (int64_t)nrows)] - rp[I * BS] <= pc.above;
   int32_t p = 0, pe = 0;
   if (blk_ok && row < nrows) {
     const int32_t r0 = rp[row], r1 = rp[row + 1];
     p = r0;
     pe = r1;
-    if (pc.row) {
+    if constexpr (PIECES) {
       const int32_t lo = pc.lo[pi], hi = pc.hi[pi];
       if (lo != INT_MIN) p = first_blockcol_at_least<BS>(ci, r0, r1, lo);
       if (hi != INT_MAX) pe = first_blockcol_at_least<BS>(ci, r0, r1, hi);
@@ -206,11 +209,12 @@ __global__ __launch_bounds__(256) void k_pack(const int32_t* __restrict__ rp,
     }
   }
   // the wave's rows are one run of the CSR: a short one is staged
-  __shared__ int32_t stage[256 / kWave][kStage];
-  int32_t* sci = stage[threadIdx.x / kWave];
   int32_t s0 = 0;
   bool staged = false;
-  if (!pc.row) {
+  int32_t* sci = nullptr;
+  if constexpr (!PIECES) {
+    __shared__ int32_t stage[256 / kWave][kStage];
+    sci = stage[threadIdx.x / kWave];
     const int64_t w0 = wave * G * BS;
     s0 = rp[w0];
     const int32_t s1 = rp[min(w0 + kWave, (int64_t)nrows)];
@@ -219,76 +223,80 @@ __global__ __launch_bounds__(256) void k_pack(const int32_t* __restrict__ rp,
       for (int32_t q = lane; q < s1 - s0; q += kWave) sci[q] = ci[s0 + q];
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
-  auto entry = [&](int32_t q) -> int32_t { return staged ? sci[q - s0] : ci[q]; };
-  auto blockcol = [&](int32_t q) -> int32_t {
-    const int32_t c = entry(q);
-    if (MODE == PACK_COUNT && (c < 0 || c >= ncols)) {
-      atomicOr(err, PACKERR_COLRANGE);
-      return INT_MAX - 1;  // poison: still terminates
-    }
-    return c / BS;
-  };
-  int32_t cur = (p < pe) ? blockcol(p) : INT_MAX;
   int64_t base = 0;
   if (MODE != PACK_COUNT && blk_ok) base = pc.base ? pc.base[pi] : bsr_rp[I];
   int32_t k = 0;
-  while (true) {
-    const int32_t m = group_min<BS>(cur);
-    if (__all(m == INT_MAX)) break;
-    uint64_t w = 0;
-    int32_t p0 = p;
-    if (m != INT_MAX) {
-      while (cur == m) {
-        w |= 1ull << (BS - 1 - (entry(p) % BS));
-        ++p;
-        const int32_t nxt = (p < pe) ? blockcol(p) : INT_MAX;
-        if (MODE == PACK_COUNT && nxt < cur) atomicOr(err, PACKERR_UNSORTED);
-        cur = nxt;
+  // one loop for staged entries, one for those in memory
+  auto merge = [&](auto entry) {
+    auto blockcol = [&](int32_t q) -> int32_t {
+      const int32_t c = entry(q);
+      if (MODE == PACK_COUNT && (c < 0 || c >= ncols)) {
+        atomicOr(err, PACKERR_COLRANGE);
+        return INT_MAX - 1;  // poison: still terminates
       }
-    }
-    if constexpr (MODE == PACK_ROW) {
+      return c / BS;
+    };
+    int32_t cur = (p < pe) ? blockcol(p) : INT_MAX;
+    while (true) {
+      const int32_t m = group_min<BS>(cur);
+      if (__all(m == INT_MAX)) break;
+      uint64_t w = 0;
+      int32_t p0 = p;
       if (m != INT_MAX) {
-        out_tiles[(base + k) * BS + r] = (W)w;
-        if (r == 0) out_col[base + k] = m;
+        while (cur == m) {
+          w |= 1ull << (BS - 1 - (entry(p) % BS));
+          ++p;
+          const int32_t nxt = (p < pe) ? blockcol(p) : INT_MAX;
+          if (MODE == PACK_COUNT && nxt < cur) atomicOr(err, PACKERR_UNSORTED);
+          cur = nxt;
+        }
       }
-    } else if constexpr (MODE == PACK_COL) {
-      // Transpose the group's bs x bs bit tile with one ballot per column:
-      // ballot bit (g*BS + r) = row r has column kk.
-      uint64_t mine = 0;
-      for (int kk = 0; kk < BS; ++kk) {
-        const uint64_t b = __ballot((w >> (BS - 1 - kk)) & 1ull);
-        const uint64_t grp = (b >> (g * BS)) & low_mask<BS>();
-        if (kk == r) mine = brev_low<BS>(grp);
-      }
-      if (m != INT_MAX) {
-        out_tiles[(base + k) * BS + r] = (W)mine;
-        if (r == 0) out_col[base + k] = m;
-      }
-    } else if constexpr (MODE == PACK_VALUES) {
-      // Rank of this row's first bit inside the tile = popcounts of the
-      // rows above it (exclusive prefix over the group).
-      int32_t cnt = (m != INT_MAX) ? popcw(w) : 0;
-      int32_t incl = cnt;
-      for (int off = 1; off < BS; off <<= 1) {
-        const int32_t o = __shfl_up(incl, off, BS);
-        if (r >= off) incl += o;
-      }
-      if (m != INT_MAX) {
-        int64_t pos = woff[base + k] + (incl - cnt);
-        for (int32_t q = p0; q < p; ++q) {
-          if (q > p0 && ci[q] == ci[q - 1]) {
-            tval[pos - 1] = min(tval[pos - 1], val[q]);
-          } else {
-            tval[pos++] = val[q];
+      if constexpr (MODE == PACK_ROW) {
+        if (m != INT_MAX) {
+          out_tiles[(base + k) * BS + r] = (W)w;
+          if (r == 0) out_col[base + k] = m;
+        }
+      } else if constexpr (MODE == PACK_COL) {
+        // Transpose the group's bs x bs bit tile with one ballot per column:
+        // ballot bit (g*BS + r) = row r has column kk.
+        uint64_t mine = 0;
+        for (int kk = 0; kk < BS; ++kk) {
+          const uint64_t b = __ballot((w >> (BS - 1 - kk)) & 1ull);
+          const uint64_t grp = (b >> (g * BS)) & low_mask<BS>();
+          if (kk == r) mine = brev_low<BS>(grp);
+        }
+        if (m != INT_MAX) {
+          out_tiles[(base + k) * BS + r] = (W)mine;
+          if (r == 0) out_col[base + k] = m;
+        }
+      } else if constexpr (MODE == PACK_VALUES) {
+        // Rank of this row's first bit inside the tile = popcounts of the
+        // rows above it (exclusive prefix over the group).
+        int32_t cnt = (m != INT_MAX) ? popcw(w) : 0;
+        int32_t incl = cnt;
+        for (int off = 1; off < BS; off <<= 1) {
+          const int32_t o = __shfl_up(incl, off, BS);
+          if (r >= off) incl += o;
+        }
+        if (m != INT_MAX) {
+          int64_t pos = woff[base + k] + (incl - cnt);
+          for (int32_t q = p0; q < p; ++q) {
+            if (q > p0 && ci[q] == ci[q - 1]) {
+              tval[pos - 1] = min(tval[pos - 1], val[q]);
+            } else {
+              tval[pos++] = val[q];
+            }
           }
         }
       }
+      if (m != INT_MAX) ++k;
     }
-    if (m != INT_MAX) ++k;
-  }
+  };
+  if (!PIECES && staged) merge([&](int32_t q) -> int32_t { return sci[q - s0]; });
+  else merge([&](int32_t q) -> int32_t { return ci[q]; });
   if constexpr (MODE == PACK_COUNT) {
     if (blk_ok && r == 0) {
-      if (pc.cnt) pc.cnt[pi] = k;
+      if constexpr (PIECES) pc.cnt[pi] = k;
       else bsr_rp[I] = k;
     }
   }
@@ -329,6 +337,13 @@ __global__ __launch_bounds__(256) void k_piece_fill(const int32_t* __restrict__ 
     plo[o + j] = j == 0 ? INT_MIN : ci[best + (int32_t)((int64_t)j * len / P)] / bs;
     phi[o + j] = j == P - 1 ? INT_MAX : ci[best + (int32_t)((int64_t)(j + 1) * len / P)] / bs;
   }
+}
+
+// off[I] = first tile of block row I's first piece (off[nbr] = total).
+__global__ __launch_bounds__(256) void k_piece_off(const int32_t* __restrict__ poff, const int64_t* __restrict__ toff,
+                                                   int32_t nbr, int64_t* __restrict__ off) {
+  const int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (I <= nbr) off[I] = toff[poff[I]];
 }
 
 // rowptr[I] = first tile of block row I (rowptr[nbr] = total).
@@ -557,8 +572,12 @@ static int launch_pack(const int32_t* rp, const int32_t* ci, int32_t nrows, int3
   const int64_t waves = (units + G - 1) / G;
   const int64_t blocks = (waves + 3) / 4;
   if (blocks == 0) return GBO_OK;
-  k_pack<BS, MODE><<<(unsigned)blocks, 256, 0, st>>>(rp, ci, nrows, ncols, nbr, bsr_rp, out_col,
-                                                     (word_t<BS>*)out_tiles, val, woff, tval, err, pc);
+  auto* kernel = k_pack<BS, MODE, true>;
+  if constexpr (MODE != PACK_VALUES) {  // values always come by the table
+    if (!pc.row) kernel = k_pack<BS, MODE, false>;
+  }
+  kernel<<<(unsigned)blocks, 256, 0, st>>>(rp, ci, nrows, ncols, nbr, bsr_rp, out_col, (word_t<BS>*)out_tiles, val,
+                                           woff, tval, err, pc);
   GBO_LAUNCH_CHECK();
   return GBO_OK;
 }
@@ -589,6 +608,7 @@ static int check_err_flag(int h, const char* who) {
 // owned by `mem`.
 struct PieceSet {
   PackPieces pc;
+  const int32_t* poff = nullptr;  // each block row's first piece, nbr + 1
   int64_t total = 0;
 };
 
@@ -637,13 +657,20 @@ static int make_pieces(int bs, const int32_t* d_rp, const int32_t* d_ci, int32_t
   pc.cnt = nullptr;
   pc.base = toff;
   ps->pc = pc;
+  ps->poff = poff;
   return GBO_OK;
 }
+
+// From how many walks on the bitmaps of the heavy block rows lose to merging
+// them in pieces (bs 8, pieces / bitmaps: R-MAT 2^23 of 12, 4 walks, 15.2 / 12.5
+// ms; 2^24 of 8, 8 walks, 19.9 / 22.3).
+constexpr int64_t kMostWalks = 4;
 
 // The tiles of every block row: off (nbr + 1 first tiles, owned by `mem`), the
 // heavy block rows and one read of what the host needs.  Checks the rows.
 struct PackCount {
   int64_t* off = nullptr;
+  PackPieces pieces;  // with a table: all block rows, and none is heavy
   HeavyRows heavy;
   PackSummary sum{};
 };
@@ -651,6 +678,17 @@ struct PackCount {
 static int pack_count(int bs, const PackCsr& A, const int32_t* d_given, Workspace& mem, PackCount* pk, const char* who,
                       hipStream_t st) {
   int rc;
+  if (heavy_walks(bs, A.ncols) > kMostWalks) {
+    PieceSet ps;
+    if ((rc = make_pieces(bs, A.rp, A.ci, A.nrows, A.ncols, A.nbr, mem, &ps, who, st)) ||
+        (rc = mem.alloc(&pk->off, sizeof(int64_t) * ((size_t)A.nbr + 1), who)))
+      return rc;
+    k_piece_off<<<(unsigned)(((int64_t)A.nbr + 256) / 256), 256, 0, st>>>(ps.poff, ps.pc.base, A.nbr, pk->off);
+    GBO_LAUNCH_CHECK();
+    pk->pieces = ps.pc;
+    pk->sum.total = ps.total;
+    return d_given ? read_back(&pk->sum.given, d_given, sizeof(int32_t), st) : GBO_OK;
+  }
   int32_t* cnt = nullptr;
   int* d_err = nullptr;
   PackSummary* d_sum = nullptr;
@@ -685,14 +723,16 @@ static int pack_rowptr(const PackCount& pk, int32_t nbr, int32_t* d_rowptr, hipS
 static int pack_fill(int bs, int dir, const PackCsr& A, const PackCount& pk, int32_t* d_col, void* d_tiles,
                      Workspace& mem, hipStream_t st) {
   if (pk.sum.total == 0) return GBO_OK;
-  PackPieces pc;
-  pc.above = pk.heavy.above;
-  pc.base = pk.off;
+  PackPieces pc = pk.pieces;
+  if (!pc.row) {
+    pc.above = pk.heavy.above;
+    pc.base = pk.off;
+  }
   const int rc = dir == 0 ? dispatch_pack<PACK_ROW>(bs, A.rp, A.ci, A.nrows, A.ncols, A.nbr, nullptr, d_col, d_tiles,
                                                     nullptr, nullptr, nullptr, nullptr, pc, st)
                           : dispatch_pack<PACK_COL>(bs, A.rp, A.ci, A.nrows, A.ncols, A.nbr, nullptr, d_col, d_tiles,
                                                     nullptr, nullptr, nullptr, nullptr, pc, st);
-  if (rc) return rc;
+  if (rc || pc.row) return rc;
   return heavy_fill(bs, dir, A, pk.heavy, pk.sum.heavy, pk.off, pk.sum.total, d_col, d_tiles, mem, st);
 }
 

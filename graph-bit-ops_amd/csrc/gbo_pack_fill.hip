@@ -502,13 +502,22 @@ int unsupported(int bs) { return set_error(GBO_EUNSUPPORTED, "block size %d not 
 
 }  // namespace
 
+int64_t heavy_walks(int bs, int32_t ncols) { return (((int64_t)ncols + bs - 1) / bs + kColWindow - 1) / kColWindow; }
+
 int heavy_list(int bs, const PackCsr& A, Workspace& mem, HeavyRows* h, const char* who, hipStream_t st) {
   // A merge's steps are the block row's tiles, unknown yet but at most its
-  // nonzeros.  At 128, 8 bs (king grid, 1M vertices, 8 nonzeros a row in few
-  // tiles): bs 64 merged 182 us, here 350; bs 32 182 and 500; bs 8 185 and 990.
-  // Above it (12 nonzeros a row at random, 2^20 rows): bs 64 3480 and 1560.  Any
-  // bound of 64 to 512 is within 20% of the best on R-MAT 2^20.
-  h->above = std::max(128, 8 * bs);
+  // nonzeros.  King grid, 1M vertices, 8 nonzeros a row in few tiles, merged and
+  // here: bs 64 182 and 350 us, bs 32 182 and 500, bs 8 185 and 990.  12 nonzeros a
+  // row at random, 2^20 rows: bs 64 3480 and 1560.  Bounds of 64 to 512 are within
+  // 20% of the best on R-MAT 2^20; 16 nonzeros a row at random at bs 8, block rows
+  // of 128: 2^20 rows 1033 us at a bound of 128, 640 at 256.
+  const int32_t least = std::max(256, 8 * bs);
+  // Each walk of a wider matrix costs a block row some 7 us of a workgroup whatever
+  // it holds (2^23 rows of 40 at random, bs 8: 29.4 ms at a bound of 128, 16.4 at 768),
+  // but a merge of a thousand tiles is as long as the rest of the pass (R-MAT 2^23 of
+  // 12: 11.8, 12.6 and 20.3 ms at 512, 768 and 1024).
+  const int64_t walks = heavy_walks(bs, A.ncols);
+  h->above = walks > 1 ? (int32_t)std::max<int64_t>(least, std::min<int64_t>(192 * walks, 768)) : least;
   int rc;
   if ((rc = mem.alloc(&h->list, sizeof(int32_t) * (size_t)std::max(A.nbr, 1), who)) ||
       (rc = mem.alloc(&h->n, sizeof(int32_t), who)))
