@@ -102,7 +102,8 @@ __global__ __launch_bounds__(kThreads) void k_block_count(const ColArgs a) {
       const int32_t s = a.rp[row0 + tid], e = a.rp[row0 + tid + 1];
       if (s > p0 && s < e && (a.ci[s - 1] >> S) > (a.ci[s] >> S)) --falls;
     }
-    for (int32_t w0 = 0; w0 < nbc; w0 += a.window) {
+    int32_t w0 = 0;
+    do {  // once where the matrix has no columns: the entries are out of range
       auto turn = [&](auto unroll, uint32_t p) {
         constexpr int U = unroll;
         int32_t b[U], before[U];
@@ -146,7 +147,8 @@ __global__ __launch_bounds__(kThreads) void k_block_count(const ColArgs a) {
         }
       }
       __syncthreads();
-    }
+      w0 += a.window;
+    } while (w0 < nbc);
     const int64_t sum = block_sum(((int64_t)falls << 32) + tiles, sh);
     if (tid == 0) {
       a.cnt[I] = (int32_t)sum;
