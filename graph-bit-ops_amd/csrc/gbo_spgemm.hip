@@ -732,21 +732,31 @@ int numeric_t(const gbo_bsr* A, const gbo_bsr* B, int64_t nc_expect, int32_t* d_
   return GBO_OK;
 }
 
-template <int BS>
-int valoff_t(const word_t<BS>* tiles, int64_t nc, int64_t* d_valoff, int64_t* nnz, hipStream_t st) {
-  Workspace mem(st);
+// `mem`: a Workspace, whose end waits for the stream, or AsyncAllocs.
+template <int BS, class Mem, class Scan>
+int valoff_with(const word_t<BS>* tiles, int64_t nc, Mem& mem, hipStream_t st, Scan scan) {
   int64_t* cnt = nullptr;
-  int rc = mem.alloc(&cnt, sizeof(int64_t) * (size_t)std::max<int64_t>(nc, 1), "gbo_bsrbmm_numeric");
+  const int rc = mem.alloc(&cnt, sizeof(int64_t) * (size_t)std::max<int64_t>(nc, 1), "gbo_bsrbmm_numeric");
   if (rc) return rc;
   if (nc > 0) {
     k_tile_popc64<BS><<<grid_for(nc, 256), 256, 0, st>>>(tiles, nc, cnt);
     GBO_LAUNCH_CHECK();
   }
-  if ((rc = scan_exclusive<int64_t, int64_t>(cnt, d_valoff, nc, st, mem))) return rc;
-  if (nnz) {
-    if ((rc = read_back(nnz, d_valoff + nc, sizeof(int64_t), st))) return rc;
+  return scan(cnt);
+}
+
+// Without a total the host has nothing to wait for, and does not.
+template <int BS>
+int valoff_t(const word_t<BS>* tiles, int64_t nc, int64_t* d_valoff, int64_t* nnz, hipStream_t st) {
+  if (!nnz) {
+    AsyncAllocs mem(st);
+    return valoff_with<BS>(tiles, nc, mem, st,
+                           [&](int64_t* cnt) { return scan_exclusive<int64_t, int64_t>(cnt, d_valoff, nc, st); });
   }
-  return GBO_OK;
+  Workspace mem(st);
+  const int rc = valoff_with<BS>(tiles, nc, mem, st,
+                                 [&](int64_t* cnt) { return scan_exclusive<int64_t, int64_t>(cnt, d_valoff, nc, st, mem); });
+  return rc ? rc : read_back(nnz, d_valoff + nc, sizeof(int64_t), st);
 }
 
 }  // namespace
