@@ -59,18 +59,19 @@ template <int BS>
 __global__ __launch_bounds__(256) void k_item_bits(const ItemArgs a) {
   constexpr int G = kWave / BS;
   const int lane = lane_id(), g = lane / BS, r = lane % BS;
-  const int64_t it = wave_index();
-  if (it >= a.itemptr[a.nbr]) return;
-  const int32_t R = a.itemrow[it];
-  const int64_t i0 = a.itemptr[R], m = a.itemptr[R + 1] - i0, k = it - i0;
-  const int64_t t0 = (int64_t)a.rowptr[R] + k * kItem<BS>;
-  const int64_t t1 = min(t0 + (int64_t)kItem<BS>, (int64_t)a.rowptr[R + 1]);
   const word_t<BS>* __restrict__ tiles = (const word_t<BS>*)a.tiles;
-  int c = 0;
+  const int64_t items = a.itemptr[a.nbr], nw = (int64_t)gridDim.x * (256 / kWave);
+  for (int64_t it = wave_index(); it < items; it += nw) {
+    const int32_t R = a.itemrow[it];
+    const int64_t i0 = a.itemptr[R], m = a.itemptr[R + 1] - i0, k = it - i0;
+    const int64_t t0 = (int64_t)a.rowptr[R] + k * kItem<BS>;
+    const int64_t t1 = min(t0 + (int64_t)kItem<BS>, (int64_t)a.rowptr[R + 1]);
+    int c = 0;
 #pragma unroll 8
-  for (int64_t t = t0 + g; t < t1; t += G) c += popcw(tiles[(a.perm ? (int64_t)a.perm[t] : t) * BS + r]);
-  for (int off = BS; off < kWave; off <<= 1) c += __shfl_xor(c, off);
-  if (g == 0) a.cnt[item_slot<BS>(i0, m, r, k)] = c;
+    for (int64_t t = t0 + g; t < t1; t += G) c += popcw(tiles[(a.perm ? (int64_t)a.perm[t] : t) * BS + r]);
+    for (int off = BS; off < kWave; off <<= 1) c += __shfl_xor(c, off);
+    if (g == 0) a.cnt[item_slot<BS>(i0, m, r, k)] = c;
+  }
 }
 
 template <int BS>
@@ -91,43 +92,44 @@ __global__ __launch_bounds__(256) void k_item_fill(const ItemArgs a) {
   constexpr int G = kWave / BS;
   constexpr int U = 4;  // tiles per lane whose words are loaded together
   const int lane = lane_id(), g = lane / BS, r = lane % BS;
-  const int64_t it = wave_index();
-  if (it >= a.itemptr[a.nbr]) return;
-  const int32_t R = a.itemrow[it];
-  const int64_t i0 = a.itemptr[R], m = a.itemptr[R + 1] - i0, k = it - i0;
-  const int64_t t0 = (int64_t)a.rowptr[R] + k * kItem<BS>;
-  const int64_t t1 = min(t0 + (int64_t)kItem<BS>, (int64_t)a.rowptr[R + 1]);
   const word_t<BS>* __restrict__ tiles = (const word_t<BS>*)a.tiles;
-  int64_t pos = a.pos[item_slot<BS>(i0, m, r, k)];
-  for (int64_t b = t0; b < t1; b += U * G) {  // wave-uniform
-    uint64_t w[U];
-    int32_t c[U];
+  const int64_t items = a.itemptr[a.nbr], nw = (int64_t)gridDim.x * (256 / kWave);
+  for (int64_t it = wave_index(); it < items; it += nw) {
+    const int32_t R = a.itemrow[it];
+    const int64_t i0 = a.itemptr[R], m = a.itemptr[R + 1] - i0, k = it - i0;
+    const int64_t t0 = (int64_t)a.rowptr[R] + k * kItem<BS>;
+    const int64_t t1 = min(t0 + (int64_t)kItem<BS>, (int64_t)a.rowptr[R + 1]);
+    int64_t pos = a.pos[item_slot<BS>(i0, m, r, k)];
+    for (int64_t b = t0; b < t1; b += U * G) {  // wave-uniform
+      uint64_t w[U];
+      int32_t c[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t t = b + u * G + g;
-      const int64_t tc = t < t1 ? t : t0;
-      const uint64_t wv = (uint64_t)tiles[(a.perm ? (int64_t)a.perm[tc] : tc) * BS + r];
-      c[u] = a.colind[tc];
-      w[u] = t < t1 ? wv : 0ull;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // bits of this row in the earlier tile slots of the step
-      const int own = popcw(w[u]);
-      int incl = own;
-#pragma unroll
-      for (int off = 1; off < G; off <<= 1) {
-        const int o = __shfl_up(incl, off * BS);
-        if (g >= off) incl += o;
+      for (int u = 0; u < U; ++u) {
+        const int64_t t = b + u * G + g;
+        const int64_t tc = t < t1 ? t : t0;
+        const uint64_t wv = (uint64_t)tiles[(a.perm ? (int64_t)a.perm[tc] : tc) * BS + r];
+        c[u] = a.colind[tc];
+        w[u] = t < t1 ? wv : 0ull;
       }
-      int64_t p = pos + incl - own;
-      uint64_t ww = w[u];
-      while (ww) {
-        const int bit = 63 - __builtin_clzll(ww);  // highest bit: lowest column
-        ww &= ~(1ull << bit);
-        a.col[p++] = c[u] * BS + (BS - 1 - bit);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // bits of this row in the earlier tile slots of the step
+        const int own = popcw(w[u]);
+        int incl = own;
+#pragma unroll
+        for (int off = 1; off < G; off <<= 1) {
+          const int o = __shfl_up(incl, off * BS);
+          if (g >= off) incl += o;
+        }
+        int64_t p = pos + incl - own;
+        uint64_t ww = w[u];
+        while (ww) {
+          const int bit = 63 - __builtin_clzll(ww);  // highest bit: lowest column
+          ww &= ~(1ull << bit);
+          a.col[p++] = c[u] * BS + (BS - 1 - bit);
+        }
+        pos += G > 1 ? __shfl(incl, kWave - BS + r) : incl;
       }
-      pos += G > 1 ? __shfl(incl, kWave - BS + r) : incl;
     }
   }
 }
@@ -135,6 +137,9 @@ __global__ __launch_bounds__(256) void k_item_fill(const ItemArgs a) {
 unsigned grid_of(int64_t items, int per_block) {
   return (unsigned)std::max<int64_t>(1, (items + per_block - 1) / per_block);
 }
+// A wave an item, past 2^24 of them several: a launch has less than 2^32
+// threads, a matrix up to 2^28 block rows.
+unsigned item_grid(int64_t cap) { return std::min(grid_of(cap, 4), 1u << 22); }
 
 template <int BS>
 int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
@@ -165,7 +170,7 @@ int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
   a.nbr = nbr;
   a.cnt = cnt;
   a.pos = pos;
-  k_item_bits<BS><<<grid_of(cap, 4), 256, 0, st>>>(a);
+  k_item_bits<BS><<<item_grid(cap), 256, 0, st>>>(a);
   GBO_LAUNCH_CHECK();
   // counts past the last item are never written; what they hold only moves
   // positions past the total, which nothing reads
@@ -177,7 +182,7 @@ int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
   int32_t* col = nullptr;
   if ((rc = mem.alloc(&col, sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1), who))) return rc;
   a.col = col;
-  k_item_fill<BS><<<grid_of(cap, 4), 256, 0, st>>>(a);
+  k_item_fill<BS><<<item_grid(cap), 256, 0, st>>>(a);
   GBO_LAUNCH_CHECK();
   out->rowptr = rowptr;
   out->col = col;

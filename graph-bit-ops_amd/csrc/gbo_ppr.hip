@@ -419,33 +419,38 @@ __global__ void k_ctl_init(Ctl* ctl) {
 __global__ __launch_bounds__(256) void k_pad(const float* __restrict__ src, int32_t n, int32_t K, int32_t ld,
                                              float* __restrict__ dst, const float* __restrict__ scale,
                                              float* __restrict__ xs) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t q4 = ld / 4;
-  if (idx >= n * q4) return;
-  const int64_t i = idx / q4;
-  const int k0 = (int)(idx % q4) * 4;
-  float v[4];
+  const int64_t q4 = ld / 4, nt = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n * q4; idx += nt) {
+    const int64_t i = idx / q4;
+    const int k0 = (int)(idx % q4) * 4;
+    float v[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) v[q] = k0 + q < K ? src[i * K + k0 + q] : 0.f;
-  if (dst) *(f32x4*)(dst + i * ld + k0) = f32x4{v[0], v[1], v[2], v[3]};
-  if (xs) {
-    const float s = scale[i];
-    *(f32x4*)(xs + i * ld + k0) = f32x4{v[0] * s, v[1] * s, v[2] * s, v[3] * s};
+    for (int q = 0; q < 4; ++q) v[q] = k0 + q < K ? src[i * K + k0 + q] : 0.f;
+    if (dst) *(f32x4*)(dst + i * ld + k0) = f32x4{v[0], v[1], v[2], v[3]};
+    if (xs) {
+      const float s = scale[i];
+      *(f32x4*)(xs + i * ld + k0) = f32x4{v[0] * s, v[1] * s, v[2] * s, v[3] * s};
+    }
   }
 }
 
 // dst [n][K] = a * src [n][ld].
 __global__ __launch_bounds__(256) void k_unpad(const float* __restrict__ src, int32_t n, int32_t K, int32_t ld, float a,
                                                float* __restrict__ dst) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)n * K) return;
-  const int64_t i = idx / K, k = idx % K;
-  dst[idx] = a * src[i * ld + k];
+  const int64_t nt = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < (int64_t)n * K; idx += nt) {
+    const int64_t i = idx / K, k = idx % K;
+    dst[idx] = a * src[i * ld + k];
+  }
 }
 
 unsigned grid_of(int64_t items, int per_block) {
   return (unsigned)std::max<int64_t>(1, (items + per_block - 1) / per_block);
 }
+
+// For k_pad and k_unpad, which go on past it: a launch has less than 2^32
+// threads, the arrays up to 2^31 rows of 64.
+unsigned grid_most(int64_t items) { return std::min(grid_of(items, 256), 1u << 22); }
 
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -606,7 +611,7 @@ int gbo_ppr_forward(const gbo_bsr* AT, const int32_t* d_outdeg, int32_t K, float
   if ((own && (rc = mem.alloc(&p, bytes, "gbo_ppr_forward"))) ||
       (rc = mem.alloc(&xs[0], bytes, "gbo_ppr_forward")) || (rc = mem.alloc(&xs[1], bytes, "gbo_ppr_forward")))
     return rc;
-  k_pad<<<grid_of((int64_t)n * (ld / 4), 256), 256, 0, st>>>(d_s, n, K, ld, p, s.inv, xs[0]);  // p_0 = s
+  k_pad<<<grid_most((int64_t)n * (ld / 4)), 256, 0, st>>>(d_s, n, K, ld, p, s.inv, xs[0]);  // p_0 = s
   GBO_LAUNCH_CHECK();
   if ((rc = col_norms(d_s, n, K, s, st))) return rc;
   SpmmArgs A{};
@@ -630,7 +635,7 @@ int gbo_ppr_forward(const gbo_bsr* AT, const int32_t* d_outdeg, int32_t K, float
   });
   if (rc) return rc;
   if (own) {
-    k_unpad<<<grid_of((int64_t)n * K, 256), 256, 0, st>>>(p, n, K, ld, 1.0f, d_p);
+    k_unpad<<<grid_most((int64_t)n * K), 256, 0, st>>>(p, n, K, ld, 1.0f, d_p);
     GBO_LAUNCH_CHECK();
     GBO_HIP_CHECK(hipStreamSynchronize(st));
   }
@@ -670,7 +675,7 @@ int gbo_ppr_adjoint(const gbo_bsr* A, const gbo_bsr* AT, const int32_t* d_outdeg
   float* lam[2] = {nullptr, nullptr};
   if ((rc = mem.alloc(&lam[0], bytes, "gbo_ppr_adjoint")) || (rc = mem.alloc(&lam[1], bytes, "gbo_ppr_adjoint")))
     return rc;
-  const unsigned padg = grid_of((int64_t)n * (ld / 4), 256);
+  const unsigned padg = grid_most((int64_t)n * (ld / 4));
   k_pad<<<padg, 256, 0, st>>>(d_w, n, K, ld, lam[0], nullptr, nullptr);
   GBO_LAUNCH_CHECK();
   if ((rc = col_norms(d_w, n, K, s, st))) return rc;
@@ -696,7 +701,7 @@ int gbo_ppr_adjoint(const gbo_bsr* A, const gbo_bsr* AT, const int32_t* d_outdeg
   const float* cur = lam[it & 1];
   float* xs = lam[(it + 1) & 1];
   // grad_s = (1 - alpha) * lambda
-  k_unpad<<<grid_of((int64_t)n * K, 256), 256, 0, st>>>(cur, n, K, ld, 1.0f - alpha, d_grad_s);
+  k_unpad<<<grid_most((int64_t)n * K), 256, 0, st>>>(cur, n, K, ld, 1.0f - alpha, d_grad_s);
   // dL/dalpha = sum_k lambda_k . (P^T p_k - s_k)
   k_pad<<<padg, 256, 0, st>>>(d_p, n, K, ld, nullptr, s.inv, xs);
   k_ctl_init<<<1, 1, 0, st>>>(s.ctl);

@@ -12,6 +12,7 @@ NOT_READY = 600  # hipErrorNotReady
 @pytest.mark.parametrize("scale,bs", [(8, 8), (16, 8), (14, 64)])
 def test_bit_offsets_without_a_total(gbo, scale, bs):
     L = gbo.lib()
+    gbo.lib()
     hip = ctypes.CDLL(gbo.hip_runtimes()[0])
     g = gbo.gen_rmat(scale, 8, seed=3)
     A = gbo.BsrMatrix.from_csr(g, bs)
