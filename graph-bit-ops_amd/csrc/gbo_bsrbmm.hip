@@ -176,6 +176,7 @@ struct ListTcArgs {
   const int32_t* ccol;
   int32_t nrows;        // rows of A
   int32_t nids;         // columns of A = rows of B: the ids in the sets
+  int32_t nkeys;        // columns of B; a key past them (padding bits of A) has no list
   const int64_t* hoff;  // heavy items before row i (scan), [nrows + 1]
   const int2* items;    // heavy items: row, first key
   unsigned long long* next;  // heavy items taken
@@ -212,6 +213,7 @@ template <class Has>
 __device__ __forceinline__ int64_t count_keys(const ListTcArgs& A, bool in, int32_t k, int64_t a0, int64_t di,
                                               bool searches, const Has& has) {
   const int lane = lane_id();
+  in = in && k < A.nkeys;
   const int64_t c0 = in ? A.crp[k] : 0;
   const int64_t dk = in ? A.crp[k + 1] - c0 : 0;
   int64_t hits = 0;
@@ -519,6 +521,7 @@ static int tc_lists(const gbo_bsr* A, const CsrList& a, const TileLists& cl, uns
   t.ccol = c.col;
   t.nrows = n;
   t.nids = A->ncols;
+  t.nkeys = cl.n;
   t.hoff = hoff;
   t.items = items;
   t.next = next;

@@ -43,7 +43,7 @@ struct ItemArgs {
   const int32_t* perm;     // nullable: where tile t lies in `tiles`
   const int64_t* itemptr;  // [nbr + 1]
   const int32_t* itemrow;  // [items]
-  int32_t nbr;
+  int32_t nbr, n;
   int32_t* cnt;            // [items * bs], see item_slot
   const int64_t* pos;      // its exclusive scan
   int32_t* col;
@@ -100,6 +100,7 @@ __global__ __launch_bounds__(256) void k_item_fill(const ItemArgs a) {
     const int64_t t0 = (int64_t)a.rowptr[R] + k * kItem<BS>;
     const int64_t t1 = min(t0 + (int64_t)kItem<BS>, (int64_t)a.rowptr[R + 1]);
     int64_t pos = a.pos[item_slot<BS>(i0, m, r, k)];
+    const bool own_row = (int64_t)R * BS + r < a.n;  // else past the total, with whatever bits the padding holds
     for (int64_t b = t0; b < t1; b += U * G) {  // wave-uniform
       uint64_t w[U];
       int32_t c[U];
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(256) void k_item_fill(const ItemArgs a) {
         const int64_t tc = t < t1 ? t : t0;
         const uint64_t wv = (uint64_t)tiles[(a.perm ? (int64_t)a.perm[tc] : tc) * BS + r];
         c[u] = a.colind[tc];
-        w[u] = t < t1 ? wv : 0ull;
+        w[u] = t < t1 && own_row ? wv : 0ull;
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -168,6 +169,7 @@ int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
   a.itemptr = itemptr;
   a.itemrow = itemrow;
   a.nbr = nbr;
+  a.n = n;
   a.cnt = cnt;
   a.pos = pos;
   k_item_bits<BS><<<item_grid(cap), 256, 0, st>>>(a);
