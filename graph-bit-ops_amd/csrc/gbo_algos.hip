@@ -1177,7 +1177,7 @@ int gbo_tc(int bs, int32_t nrows, const int32_t* h_rp, const int32_t* h_ci, uint
   gbo_free_host(tp);
   gbo_free_host(ti);
   uint64_t* d = nullptr;
-  if (rc == GBO_OK && hipMalloc((void**)&d, sizeof(uint64_t)) != hipSuccess) rc = set_error(GBO_ENOMEM, "gbo_tc: alloc");
+  if (rc == GBO_OK && device_malloc((void**)&d, sizeof(uint64_t)) != hipSuccess) rc = set_error(GBO_ENOMEM, "gbo_tc: alloc");
   if (rc == GBO_OK) rc = gbo_bsrbmm_tc(&L, &LT, d, stream);
   if (rc == GBO_OK && hipMemcpy(h_count, d, sizeof(uint64_t), hipMemcpyDeviceToHost) != hipSuccess)
     rc = set_error(GBO_EDEVICE, "gbo_tc: copy");

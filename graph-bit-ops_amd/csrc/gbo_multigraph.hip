@@ -777,7 +777,7 @@ static void batch_release(gbo_batch* b) {
 
 template <class T>
 static int upload(T** d, const std::vector<T>& h) {
-  GBO_HIP_CHECK(hipMalloc((void**)d, sizeof(T) * std::max<size_t>(h.size(), 1)));
+  GBO_HIP_CHECK(device_malloc((void**)d, sizeof(T) * std::max<size_t>(h.size(), 1)));
   if (!h.empty()) GBO_HIP_CHECK(hipMemcpy(*d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
   return GBO_OK;
 }
@@ -929,14 +929,14 @@ int gbo_batch_create(int bs, int32_t ngraphs, const int32_t* h_nrows, const int3
   }
   const size_t wb = (size_t)bs / 8 * ((size_t)b->A.nblockrows + 1);
   hipError_t e = hipSuccess;
-  e = e ? e : hipMalloc(&b->d_f0, wb);
-  e = e ? e : hipMalloc(&b->d_f1, wb);
-  e = e ? e : hipMalloc(&b->d_vis, wb);
-  e = e ? e : hipMalloc((void**)&b->d_lab, sizeof(int32_t) * nu);
-  e = e ? e : hipMalloc((void**)&b->d_gf, sizeof(int32_t) * nu);
-  e = e ? e : hipMalloc((void**)&b->d_act, sizeof(int32_t) * 2 * ngraphs);
-  e = e ? e : hipMalloc((void**)&b->d_sync, sizeof(GridSync));
-  e = e ? e : hipMalloc((void**)&b->d_src, sizeof(int32_t) * ngraphs);
+  e = e ? e : device_malloc(&b->d_f0, wb);
+  e = e ? e : device_malloc(&b->d_f1, wb);
+  e = e ? e : device_malloc(&b->d_vis, wb);
+  e = e ? e : device_malloc((void**)&b->d_lab, sizeof(int32_t) * nu);
+  e = e ? e : device_malloc((void**)&b->d_gf, sizeof(int32_t) * nu);
+  e = e ? e : device_malloc((void**)&b->d_act, sizeof(int32_t) * 2 * ngraphs);
+  e = e ? e : device_malloc((void**)&b->d_sync, sizeof(GridSync));
+  e = e ? e : device_malloc((void**)&b->d_src, sizeof(int32_t) * ngraphs);
   if (e != hipSuccess) {
     batch_release(b);
     return set_error(GBO_ENOMEM, "gbo_batch_create: scratch allocation failed");

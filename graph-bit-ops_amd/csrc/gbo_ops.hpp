@@ -96,10 +96,12 @@ class Workspace {
   bool spare_[kMax];  // dropped
   int n_ = 0;
 };
-// hipMalloc that gives the kept blocks back before it reports that memory is
-// out; gives all kept blocks of a device (-1: of each) back; counts the
-// matrices and plans the library has allocated.
+// hipMalloc and hipMallocAsync that give the kept blocks back before they report
+// that memory is out (every allocation of the library is one of them); gives all
+// kept blocks of a device (-1: of each) back; counts the matrices and plans the
+// library has allocated.
 hipError_t device_malloc(void** p, size_t bytes);
+hipError_t device_malloc_async(void** p, size_t bytes, hipStream_t st);
 void workspace_release(int dev);
 void workspace_live(int delta);
 // Copies a few bytes to the host and waits for the stream.
@@ -120,7 +122,7 @@ class AsyncAllocs {
     *p = nullptr;
     if (n_ == kMax) return set_error(GBO_EINVAL, "%s: too many scratch allocations", who);
     void* q = nullptr;
-    const hipError_t e = hipMallocAsync(&q, bytes ? bytes : 8, st_);
+    const hipError_t e = device_malloc_async(&q, bytes ? bytes : 8, st_);
     if (e != hipSuccess) return set_error(GBO_ENOMEM, "%s: device allocation of %zu bytes failed: %s", who, bytes,
                                           hipGetErrorString(e));
     ptrs_[n_++] = q;

@@ -862,7 +862,7 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
   if (nch >= INT_MAX) return set_error(GBO_ERANGE, "too many chunks");
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
   int32_t* plan = nullptr;
-  GBO_HIP_CHECK(hipMallocAsync((void**)&plan, L.bytes, st));
+  GBO_HIP_CHECK(device_malloc_async((void**)&plan, L.bytes, st));
   pv->plan = plan;
   pv->chunk = chunk;
   pv->nchunks = (int32_t)nch;
@@ -1073,8 +1073,8 @@ static int upload_csr(const int32_t* h_rp, const int32_t* h_ci, int32_t nrows, i
     for (int32_t r = 0; r < nrows; ++r) std::sort(copy.begin() + h_rp[r], copy.begin() + h_rp[r + 1]);
     src = copy.data();
   }
-  GBO_HIP_CHECK(hipMalloc((void**)d_rp, sizeof(int32_t) * ((size_t)nrows + 1)));
-  GBO_HIP_CHECK(hipMalloc((void**)d_ci, sizeof(int32_t) * std::max<int64_t>(nnz, 1)));
+  GBO_HIP_CHECK(device_malloc((void**)d_rp, sizeof(int32_t) * ((size_t)nrows + 1)));
+  GBO_HIP_CHECK(device_malloc((void**)d_ci, sizeof(int32_t) * std::max<int64_t>(nnz, 1)));
   GBO_HIP_CHECK(hipMemcpy(*d_rp, h_rp, sizeof(int32_t) * ((size_t)nrows + 1), hipMemcpyHostToDevice));
   if (nnz) GBO_HIP_CHECK(hipMemcpy(*d_ci, src, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
   return GBO_OK;
@@ -1088,7 +1088,7 @@ int gbo_csr2bsr_nnzb(int bs, const int32_t* h_rp, const int32_t* h_ci, int32_t n
   int32_t *d_rp = nullptr, *d_ci = nullptr, *d_brp = nullptr;
   int rc = upload_csr(h_rp, h_ci, nrows, ncols, &d_rp, &d_ci);
   const int32_t nbr = (nrows + bs - 1) / bs;
-  if (rc == GBO_OK && hipMalloc((void**)&d_brp, sizeof(int32_t) * ((size_t)nbr + 1)) != hipSuccess)
+  if (rc == GBO_OK && device_malloc((void**)&d_brp, sizeof(int32_t) * ((size_t)nbr + 1)) != hipSuccess)
     rc = set_error(GBO_ENOMEM, "allocation failed");
   if (rc == GBO_OK) rc = gbo_csr2bsr_nnzb_dev(bs, d_rp, d_ci, nrows, ncols, d_brp, nblocks, nullptr);
   (void)hipFree(d_rp);

@@ -72,10 +72,10 @@ int gbo_autotune(const int32_t* d_rowptr, const int32_t* d_colind, int32_t nrows
     const int64_t nw = (std::max(nrows, ncols) + bs - 1) / bs + 1;
     void *x = nullptr, *y = nullptr, *vis = nullptr;
     int64_t* cnt = nullptr;
-    GBO_HIP_CHECK(hipMalloc(&x, nw * bs / 8));
-    GBO_HIP_CHECK(hipMalloc(&vis, nw * bs / 8));
-    GBO_HIP_CHECK(hipMalloc(&y, std::max<size_t>((size_t)nrows * 4, nw * bs / 8)));
-    GBO_HIP_CHECK(hipMalloc((void**)&cnt, sizeof(int64_t)));
+    GBO_HIP_CHECK(device_malloc(&x, nw * bs / 8));
+    GBO_HIP_CHECK(device_malloc(&vis, nw * bs / 8));
+    GBO_HIP_CHECK(device_malloc(&y, std::max<size_t>((size_t)nrows * 4, nw * bs / 8)));
+    GBO_HIP_CHECK(device_malloc((void**)&cnt, sizeof(int64_t)));
     GBO_HIP_CHECK(hipMemsetAsync(x, 0x55, nw * bs / 8, st));   // half the frontier / x bits set
     GBO_HIP_CHECK(hipMemsetAsync(vis, 0, nw * bs / 8, st));
     const int dc = default_chunk(bs, A.nblocks, true);

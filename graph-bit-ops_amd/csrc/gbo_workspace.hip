@@ -84,17 +84,30 @@ void workspace_live(int delta) {
   if (last) workspace_release(-1);
 }
 
-hipError_t device_malloc(void** p, size_t bytes) {
-  hipError_t e = hipMalloc(p, bytes);
+namespace {
+
+template <class Alloc>
+hipError_t alloc_or_release(Alloc alloc) {
+  hipError_t e = alloc();
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     int dev = 0;
     (void)hipGetDevice(&dev);
     workspace_release(dev);
-    e = hipMalloc(p, bytes);
+    e = alloc();
   }
   if (e != hipSuccess) (void)hipGetLastError();
   return e;
+}
+
+}  // namespace
+
+hipError_t device_malloc(void** p, size_t bytes) {
+  return alloc_or_release([&] { return hipMalloc(p, bytes); });
+}
+
+hipError_t device_malloc_async(void** p, size_t bytes, hipStream_t st) {
+  return alloc_or_release([&] { return hipMallocAsync(p, bytes, st); });
 }
 
 Workspace::~Workspace() {
