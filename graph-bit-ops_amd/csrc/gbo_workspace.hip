@@ -15,7 +15,6 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
-#include <vector>
 
 #include "gbo_device.hpp"
 #include "gbo_ops.hpp"
@@ -24,7 +23,7 @@ namespace gbo {
 namespace {
 
 constexpr size_t kKeepBytes = (size_t)1 << 30;
-constexpr size_t kKeepBlocks = 128;
+constexpr int kKeepBlocks = 128;
 constexpr int kDevices = 64;
 
 struct Block {
@@ -32,18 +31,21 @@ struct Block {
   size_t bytes;
 };
 
-struct Pool {
-  std::mutex mu;
-  std::vector<Block> idle[kDevices];  // the longest unused first
-  size_t bytes[kDevices] = {};
-  int64_t live = 0;  // matrices and plans the library allocated
+// Arrays of fixed length: no call into the pool can throw.  Never destroyed (at
+// exit the runtime may be gone before it).
+struct Idle {
+  Block blocks[kKeepBlocks];  // the longest unused first
+  int n;
+  size_t bytes;
+  void remove(int i) {
+    bytes -= blocks[i].bytes;
+    std::copy(blocks + i + 1, blocks + n, blocks + i);
+    --n;
+  }
 };
-
-// Never destroyed: at exit the runtime may be gone before it.
-Pool& pool() {
-  static Pool* p = new Pool;
-  return *p;
-}
+std::mutex pool_mu;
+Idle pool_idle[kDevices];
+int64_t pool_live = 0;  // matrices and plans the library allocated
 
 // Sizes in steps of an eighth of a power of two (512 bytes at least), so that
 // calls of about the same size find each other's blocks.
@@ -53,33 +55,30 @@ size_t rounded(size_t bytes) {
   return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
 }
 
-void give_back(const std::vector<Block>& blocks) {
-  for (const Block& b : blocks) (void)hipFree(b.p);
-}
-
 }  // namespace
 
 void workspace_release(int dev) {
-  std::vector<Block> out;
-  {
-    Pool& P = pool();
-    std::lock_guard<std::mutex> lk(P.mu);
-    for (int d = dev < 0 ? 0 : dev; d < (dev < 0 ? kDevices : std::min(dev + 1, kDevices)); ++d) {
-      out.insert(out.end(), P.idle[d].begin(), P.idle[d].end());
-      P.idle[d].clear();
-      P.bytes[d] = 0;
+  for (int d = dev < 0 ? 0 : dev; d < (dev < 0 ? kDevices : std::min(dev + 1, kDevices)); ++d) {
+    Block out[kKeepBlocks];
+    int n = 0;
+    {
+      std::lock_guard<std::mutex> lk(pool_mu);
+      Idle& v = pool_idle[d];
+      n = v.n;
+      std::copy(v.blocks, v.blocks + n, out);
+      v.n = 0;
+      v.bytes = 0;
     }
+    for (int i = 0; i < n; ++i) (void)hipFree(out[i].p);
   }
-  give_back(out);
 }
 
 void workspace_live(int delta) {
   bool last = false;
   {
-    Pool& P = pool();
-    std::lock_guard<std::mutex> lk(P.mu);
-    P.live += delta;
-    last = delta < 0 && P.live <= 0;
+    std::lock_guard<std::mutex> lk(pool_mu);
+    pool_live += delta;
+    last = delta < 0 && pool_live <= 0;
   }
   if (last) workspace_release(-1);
 }
@@ -112,30 +111,31 @@ hipError_t device_malloc_async(void** p, size_t bytes, hipStream_t st) {
 
 Workspace::~Workspace() {
   if (n_ == 0) return;
-  const bool idle = hipStreamSynchronize(st_) == hipSuccess;
-  std::vector<Block> out;
+  const bool idle = hipStreamSynchronize(st_) == hipSuccess && dev_ >= 0 && dev_ < kDevices;
+  Block out[kMax + kKeepBlocks];
+  int drop = 0;
   {
-    Pool& P = pool();
-    std::lock_guard<std::mutex> lk(P.mu);
+    std::lock_guard<std::mutex> lk(pool_mu);
     for (int i = 0; i < n_; ++i) {
-      if (!idle || dev_ < 0 || dev_ >= kDevices) {
-        out.push_back({ptrs_[i], bytes_[i]});
+      const Block b{ptrs_[i], bytes_[i]};
+      if (!idle) {
+        out[drop++] = b;
         continue;
       }
-      P.idle[dev_].push_back({ptrs_[i], bytes_[i]});
-      P.bytes[dev_] += bytes_[i];
-    }
-    if (dev_ >= 0 && dev_ < kDevices) {
-      auto& v = P.idle[dev_];
-      size_t drop = 0;
-      while (drop < v.size() && (P.bytes[dev_] > kKeepBytes || v.size() - drop > kKeepBlocks)) {
-        P.bytes[dev_] -= v[drop].bytes;
-        out.push_back(v[drop++]);
+      Idle& v = pool_idle[dev_];
+      if (v.n == kKeepBlocks) {
+        out[drop++] = v.blocks[0];
+        v.remove(0);
       }
-      v.erase(v.begin(), v.begin() + (ptrdiff_t)drop);
+      v.blocks[v.n++] = b;
+      v.bytes += b.bytes;
+    }
+    while (idle && pool_idle[dev_].bytes > kKeepBytes) {
+      out[drop++] = pool_idle[dev_].blocks[0];
+      pool_idle[dev_].remove(0);
     }
   }
-  give_back(out);
+  for (int i = 0; i < drop; ++i) (void)hipFree(out[i].p);
 }
 
 int Workspace::take(void** p, size_t bytes, const char* who) {
@@ -154,17 +154,16 @@ int Workspace::take(void** p, size_t bytes, const char* who) {
   void* q = nullptr;
   size_t got = want;
   if (dev_ >= 0 && dev_ < kDevices) {
-    Pool& P = pool();
-    std::lock_guard<std::mutex> lk(P.mu);
-    auto& v = P.idle[dev_];
-    size_t best = v.size();
-    for (size_t i = 0; i < v.size(); ++i)  // the smallest that fits and is not twice too large
-      if (v[i].bytes >= want && v[i].bytes <= 2 * want && (best == v.size() || v[i].bytes < v[best].bytes)) best = i;
-    if (best < v.size()) {
-      q = v[best].p;
-      got = v[best].bytes;
-      P.bytes[dev_] -= got;
-      v.erase(v.begin() + (ptrdiff_t)best);
+    std::lock_guard<std::mutex> lk(pool_mu);
+    Idle& v = pool_idle[dev_];
+    int best = -1;
+    for (int i = 0; i < v.n; ++i)  // the smallest that fits and is not twice too large
+      if (v.blocks[i].bytes >= want && v.blocks[i].bytes <= 2 * want && (best < 0 || v.blocks[i].bytes < v.blocks[best].bytes))
+        best = i;
+    if (best >= 0) {
+      q = v.blocks[best].p;
+      got = v.blocks[best].bytes;
+      v.remove(best);
     }
   }
   if (!q) {
@@ -198,15 +197,12 @@ struct Slots {
   bool tried = false;
   uint32_t taken = 0;
 };
-Slots& slots() {
-  static Slots* s = new Slots;
-  return *s;
-}
+Slots slots;
 
 }  // namespace
 
 int read_back(void* h, const void* d, size_t bytes, hipStream_t st) {
-  Slots& S = slots();
+  Slots& S = slots;
   int k = -1;
   if (bytes <= kSlotBytes) {
     std::lock_guard<std::mutex> lk(S.mu);
