@@ -66,6 +66,9 @@ struct PlanGuard {
   PlanGuard& operator=(const PlanGuard&) = delete;
 };
 
+// Scratch kept between calls at most, per device.
+constexpr size_t kKeepBytes = (size_t)8 << 30;
+
 // Device scratch of one call that waits for its stream before it returns:
 // blocks kept between calls (gbo_workspace.hip), given back on every return
 // path once the stream has been waited for.  What drop() is given is handed out

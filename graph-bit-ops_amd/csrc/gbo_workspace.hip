@@ -9,7 +9,8 @@
 //   - a block enters the list only after the stream that used it has been
 //     waited for, so whichever thread or stream takes it next finds it idle;
 //   - the list holds at most kKeepBytes and kKeepBlocks per device, the
-//     longest unused go first; all of it goes back to the runtime when an
+//     longest unused go first, and a block of more than half of that is not kept
+//     (it would send all others off); all of it goes back to the runtime when an
 //     allocation fails and when the last matrix that the library allocated or
 //     planned is freed.
 #include <algorithm>
@@ -22,7 +23,6 @@
 namespace gbo {
 namespace {
 
-constexpr size_t kKeepBytes = (size_t)1 << 30;
 constexpr int kKeepBlocks = 128;
 constexpr int kDevices = 64;
 
@@ -118,7 +118,7 @@ Workspace::~Workspace() {
     std::lock_guard<std::mutex> lk(pool_mu);
     for (int i = 0; i < n_; ++i) {
       const Block b{ptrs_[i], bytes_[i]};
-      if (!idle) {
+      if (!idle || b.bytes > kKeepBytes / 2) {
         out[drop++] = b;
         continue;
       }

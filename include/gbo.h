@@ -378,7 +378,7 @@ int gbo_bfs_do(const gbo_bsr* AT, const gbo_bsr* A, int32_t source, int32_t* d_l
 
 /* The drivers below and gbo_bfs_multisource list the nonzeros of large sparse
  * matrices once per call and sweep the list: 12 (bs 8) to 64 (bs 64) bytes of
- * scratch per tile, kept between calls up to 1 GiB; without that memory they
+ * scratch per tile, kept between calls up to 8 GiB; without that memory they
  * sweep the tiles, with the same results. */
 /* SSSP (algorithm/sssp.cu:420-488) generalised to uint32 weights:
  * frontier Bellman-Ford on the min-plus semiring; dist = INF (0xFFFFFFFF)
