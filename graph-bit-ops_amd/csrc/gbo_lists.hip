@@ -466,8 +466,16 @@ unsigned grid_of(int64_t items, int per_block) {
   return (unsigned)std::max<int64_t>(1, (items + per_block - 1) / per_block);
 }
 
+// Rows from which on shortest paths at bs 8/16 over evenly spread columns (hardly
+// a tile of two nonzeros) go by the tiles, which skip the inactive ones: the list
+// gathers a word out of 8 MB and more for each nonzero on every sweep.  G(n, m),
+// lists / tiles: 2^21 of 16 bs 8 11.0 / 9.25 ms, 2^22 of 8 bs 8 18.0 / 12.4 and bs
+// 16 18.1 / 14.6, of 16 bs 16 33.5 / 25.6; lists / the sweeps over tiles of one look
+// each: 1.2M of 8 bs 16 2.4 / 4.0, R-MAT 2^22 of 4 bs 8 2.8 / 3.8.
+constexpr int32_t kSpreadRows = 3 << 19;
+
 template <int BS>
-int build_t(const gbo_bsr* A, Workspace& mem, ListView* out, hipStream_t st) {
+int build_t(const gbo_bsr* A, ListUse use, Workspace& mem, ListView* out, hipStream_t st) {
   const char* who = "edge lists";
   ListView l{};
   l.bs = BS;
@@ -494,7 +502,9 @@ int build_t(const gbo_bsr* A, Workspace& mem, ListView* out, hipStream_t st) {
   if ((rc = read_back(&h, info, sizeof(ListInfo), st))) return rc;
   unsigned long long bits = 0;
   for (int i = 0; i < kListSlots; ++i) bits += h.sample[i];
-  if (bits > (unsigned long long)(kRoom<BS> * (kSampleWaves * 64 / (BS * BS / 64)))) return GBO_OK;
+  constexpr unsigned long long kSampleTiles = kSampleWaves * 64 / (BS * BS / 64);
+  if (bits > kRoom<BS> * kSampleTiles) return GBO_OK;
+  if (use == ListUse::kPaths && BS <= 16 && l.n > kSpreadRows && bits * 10 < kSampleTiles * 11) return GBO_OK;
   if ((rc = mem.alloc(&edges, sizeof(uint32_t) * (size_t)room, who)) ||
       (rc = mem.alloc(&icnt, sizeof(int32_t) * (size_t)l.nwin, who)) ||
       (rc = mem.alloc(&first, sizeof(int64_t) * ((size_t)l.nwin + 1), who)) ||
@@ -581,10 +591,10 @@ void lists_build(const gbo_bsr* A, ListUse use, Workspace& mem, ListView* out, h
   }
   if (bytes < least || A->nrows > (1 << kColBits) || A->ncols > (1 << kColBits) || ((uintptr_t)A->tiles & 7)) return;
   switch (A->bs) {
-    case 8: (void)build_t<8>(A, mem, out, st); break;
-    case 16: (void)build_t<16>(A, mem, out, st); break;
-    case 32: (void)build_t<32>(A, mem, out, st); break;
-    case 64: (void)build_t<64>(A, mem, out, st); break;
+    case 8: (void)build_t<8>(A, use, mem, out, st); break;
+    case 16: (void)build_t<16>(A, use, mem, out, st); break;
+    case 32: (void)build_t<32>(A, use, mem, out, st); break;
+    case 64: (void)build_t<64>(A, use, mem, out, st); break;
   }
 }
 
