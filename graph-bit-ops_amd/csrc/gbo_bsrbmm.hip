@@ -490,6 +490,12 @@ static void lds_grid(size_t lds, bool wide, int* threads, int* blocks) {
   *blocks = 256 * std::max(1, (int)std::min<size_t>(2048 / *threads, ((size_t)158 << 10) / (lds + 1024)));
 }
 
+// A kernel's limit is every caller's: always the most that a call needs, so that
+// none lowers it between another's limit and launch.
+static hipError_t lds_limit(const void* kernel) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kWindow / 8));
+}
+
 // The list form: A's rows are in `a`, B's block lists by column in `cl`.
 static int tc_lists(const gbo_bsr* A, const CsrList& a, const TileLists& cl, unsigned long long* count,
                     Workspace& mem, hipStream_t st) {
@@ -529,7 +535,7 @@ static int tc_lists(const gbo_bsr* A, const CsrList& a, const TileLists& cl, uns
   const size_t lds = (size_t)(std::min<int64_t>(kWindow, A->ncols) + 31) / 32 * 4;
   int threads = 0, blocks = 0;
   lds_grid(lds, false, &threads, &blocks);
-  GBO_HIP_CHECK(hipFuncSetAttribute((const void*)k_tc_heavy, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  GBO_HIP_CHECK(lds_limit((const void*)k_tc_heavy));
   k_tc_heavy<<<blocks, threads, lds, st>>>(t);
   GBO_LAUNCH_CHECK();
   k_tc_light<<<(unsigned)std::min<int64_t>(2048, ((int64_t)n + 4 * kTinyRows - 1) / (4 * kTinyRows)), 256, 0, st>>>(t);
@@ -543,7 +549,7 @@ static int tc_tiles(const TileTcArgs& t, hipStream_t st) {
   const size_t lds = ((size_t)std::min<int64_t>(kWindow / 8 / (int64_t)X, t.nblocks) * X + 7) / 8 * 8;
   int threads = 0, blocks = 0;
   lds_grid(lds, t.nrows < 2048, &threads, &blocks);  // few rows: more waves on each
-  GBO_HIP_CHECK(hipFuncSetAttribute((const void*)k_tc_tiles<BS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  GBO_HIP_CHECK(lds_limit((const void*)k_tc_tiles<BS>));
   k_tc_tiles<BS><<<blocks, threads, lds, st>>>(t);
   GBO_LAUNCH_CHECK();
   return GBO_OK;
