@@ -9,8 +9,8 @@
 // sort of the tiles by block column on the device: csr2csc on blocks), and
 // the count is, over the set bits (i, k) of A, |A_i and C_k|: row i of A
 // against column k of B.  Sparse tiles are listed once as rows and columns of
-// ids (k_tc_light, k_tc_heavy), dense ones are intersected word by word
-// (k_tc_tiles).
+// ids (k_tc_light, k_tc_heavy), dense ones are counted by pairs of tiles
+// (k_tc_pairs).
 //
 // Plain product sum (bmm{N}_sparse, bsrbmm/bsrbmm.cu:296-555):
 //   sum_{i,k} (A B)_ik = sum_j colsum_A(j) * rowsum_B(j),
@@ -94,13 +94,13 @@ __global__ __launch_bounds__(256) void k_col_bounds(const int32_t* __restrict__ 
   ptr[c] = (int32_t)lower_bound_i32(keys, 0, T, (int32_t)c);
 }
 
-// row[i] = block row of tile tile[i]: the last J with rowptr[J] <= tile.
+// row[i] = block row of tile tile[i] (null: i): the last J with rowptr[J] <= tile.
 __global__ __launch_bounds__(256) void k_tile_block_row(const int32_t* __restrict__ rowptr, int32_t nbr,
                                                         const int32_t* __restrict__ tile, int64_t T,
                                                         int32_t* __restrict__ row) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= T) return;
-  const int32_t t = tile[i];
+  const int32_t t = tile ? tile[i] : (int32_t)i;
   int32_t lo = 0, hi = nbr;  // first J with rowptr[J + 1] > t
   while (lo < hi) {
     const int32_t mid = lo + (hi - lo) / 2;
@@ -394,106 +394,194 @@ __global__ __launch_bounds__(kHeavyThreads) void k_tc_heavy(const ListTcArgs A) 
 }
 
 // ------------------------------------------- triangle counting on tiles
-// Dense tiles: row i of A as a vector of bs-bit words in LDS (word J = row i of
-// tile (I,J)), against which the words of B's block column K are counted for
-// every mask tile (I,K) that has bits in row i: lane r holds column k = r of
-// the 64 / bs tiles of a step, one AND and popcount per bs ids.  At bs 8 the
-// vector holds the whole tiles of block row I, and one 64-bit AND and popcount
-// takes a column word against the rows of the mask's column.  A workgroup takes
-// one row (block row) after another from a counter; a matrix wider than the
-// vector window by window.
-struct TileTcArgs {
-  const int32_t *a_rowptr, *a_colind;
+// Dense tiles: a wave takes a mask tile (I,K), looks the block columns J of the
+// shorter one of A's block row I and B's block column K up in the other, 64 at a
+// time, and counts each match word against word under the mask: lane k holds
+// column k of B's tile and walks the rows of A's (bs 64, whose words are scalar
+// loads; bs 32, two matches at a time), or a lane counts a match of its own, a
+// 64-bit AND and popcount per four (bs 16) or eight rows.  Nothing in it is as
+// wide as the matrix: communities of 256 on 2^20 vertices at bs 8 / 16 / 64 take 1.4,
+// 0.95 and 0.30 ms (with a vector of each row in LDS 7.6, 16.7 and 14.5; the tile
+// pairs taken bit by bit before 4.6, 4.4 and 0.8), G(4096, 1) 0.22 to 0.37 ms (0.8 to
+// 1.3).
+struct PairTcArgs {
+  const int32_t *a_rowptr, *a_colind, *a_row;  // a_row: block row of each tile
   const void* a_tiles;
   const int32_t *bt_ptr, *bt_row, *bt_tile;  // block columns of B: rows J, tiles
   const void* b_tiles;
-  int32_t nrows, nblocks;  // rows (bs 8: block rows); block columns of A = block rows of B
-  unsigned long long *next, *count;
+  int64_t T;
+  unsigned long long* count;
 };
 
+// The tile's 32-bit words (bs 8: two, bs 16: eight), whatever its alignment.
 template <int BS>
-__global__ __launch_bounds__(kHeavyThreads) void k_tc_tiles(const TileTcArgs A) {
+__device__ __forceinline__ void load_words(const word_t<BS>* tiles, int64_t t, uint32_t (&w)[BS * BS / 32]) {
+  __builtin_memcpy(w, tiles + t * BS, BS * BS / 8);
+}
+
+// Mask bits up to which a lane takes a bit (row r, column k) of the mask and reads
+// the one word of A's and of B's tile that it needs, match after match, instead of
+// walking the rows: a turn of 64 bits is worth some 5 of 64 rows (communities of
+// 4096 at bs 64, 80 / 197 bits a tile: 0.62 / 1.03 ms, by rows 3.3; at bs 32 50 bits
+// 2.2, by rows 6.0).
+template <int BS>
+constexpr int kMaskBits = BS == 64 ? 768 : 320;
+
+template <int BS>
+__global__ __launch_bounds__(256) void k_tc_pairs(const PairTcArgs A) {
   using W = word_t<BS>;
-  using X = typename std::conditional<BS == 8, uint64_t, W>::type;  // an element of the vector
-  constexpr int G = kWave / BS;
-  extern __shared__ uint64_t xs64[];
-  X* __restrict__ xs = (X*)xs64;
-  __shared__ unsigned long long s_row;
-  const int tid = threadIdx.x, nt = blockDim.x, lane = lane_id(), g = lane / BS, r = lane % BS;
+  __shared__ uint16_t s_bits[256 / kWave][BS <= 16 ? 1 : kMaskBits<BS>];
+  uint16_t* __restrict__ bits = s_bits[threadIdx.x / kWave];
+  const int lane = lane_id();
   const W* __restrict__ at = (const W*)A.a_tiles;
   const W* __restrict__ bt = (const W*)A.b_tiles;
-  const int window = (int)min(kWindow / (8 * (int64_t)sizeof(X)), (int64_t)A.nblocks);
-  for (int s = tid; s < window; s += nt) xs[s] = (X)0;
+  const int64_t nw = (int64_t)gridDim.x * (256 / kWave);
   int64_t hits = 0;
-  while (true) {
-    __syncthreads();
-    if (tid == 0) s_row = atomicAdd(A.next, 1ull);
-    __syncthreads();
-    // the last rows first: those of a lower triangle are the longest
-    const int64_t i = A.nrows - 1 - (int64_t)s_row;
-    if (i < 0) break;  // each workgroup ends here: the counter only grows
-    const int64_t I = BS == 8 ? i : i / BS;
-    const int64_t t0 = A.a_rowptr[I], t1 = A.a_rowptr[I + 1];
-    auto own = [&](int64_t t) -> X {  // row i of tile t; bs 8: the tile
-      if constexpr (BS == 8) {
-        uint64_t w;
-        __builtin_memcpy(&w, at + t * 8, 8);
-        return w;
-      } else {
-        return at[t * BS + i % BS];
-      }
-    };
-    for (int64_t base = 0; base < A.nblocks; base += window) {
-      for (int64_t t = t0 + tid; t < t1; t += nt) {
-        const int64_t J = A.a_colind[t] - base;
-        if (J >= 0 && J < window) xs[J] = own(t);
-      }
-      __syncthreads();
-      for (int64_t t = t0 + tid / kWave; t < t1; t += nt / kWave) {  // wave-uniform
-        uint64_t m = (uint64_t)own(t);
-        if constexpr (BS == 8) {
-          // the bytes of the rows that have column r
-          m = ((m >> (7 - r)) & 0x0101010101010101ull) * 0xFFull;
-        } else {
-          if (m == 0) continue;
-          m = (m >> (BS - 1 - r)) & 1ull;
+  for (int64_t t = wave_index(); t < A.T; t += nw) {  // wave-uniform
+    const int32_t I = ld_uniform(A.a_row, t), K = ld_uniform(A.a_colind, t);
+    const int64_t a0 = ld_uniform(A.a_rowptr, I), a1 = ld_uniform(A.a_rowptr, I + 1);
+    const int64_t b0 = ld_uniform(A.bt_ptr, K), b1 = ld_uniform(A.bt_ptr, K + 1);
+    const bool a_short = a1 - a0 <= b1 - b0;
+    const int32_t* __restrict__ from = a_short ? A.a_colind : A.bt_row;
+    const int32_t* __restrict__ in = a_short ? A.bt_row : A.a_colind;
+    const int64_t f0 = a_short ? a0 : b0, f1 = a_short ? a1 : b1, i0 = a_short ? b0 : a0, i1 = a_short ? b1 : a1;
+    // the mask: at bs 8/16 its words (scalar), else the rows of this lane's column
+    // (bit r)
+    uint32_t ms[BS <= 16 ? BS * BS / 32 : 1] = {};
+    uint64_t m[1] = {};
+    int nbits = 0;  // of the mask, where they are listed; else past kMaskBits
+    if constexpr (BS <= 16) {
+      load_words<BS>(at, t, ms);
+#pragma unroll
+      for (auto& v : ms) v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    } else {
+      const W own = at[t * BS + lane % BS];
+      const int k = lane % BS;
+      const int mine = lane < BS ? popcw(own) : 0, incl = wave_incl_scan(mine);
+      nbits = __builtin_amdgcn_readlane(incl, kWave - 1);
+      if (nbits <= kMaskBits<BS>) {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        uint64_t w = lane < BS ? (uint64_t)own : 0;
+        for (int to = incl - mine; w; ++to) {
+          const int p = __builtin_ctzll(w);
+          w &= w - 1;
+          bits[to] = (uint16_t)(lane * BS + (BS - 1 - p));
         }
-        const int32_t K = A.a_colind[t];
-        const int64_t e1 = A.bt_ptr[K + 1];
-        int acc = 0;
-#pragma unroll 4
-        for (int64_t e = A.bt_ptr[K] + g; e < e1; e += G) {
-          const int64_t J = A.bt_row[e] - base;
-          if (J >= 0 && J < window) {
-            const W w = bt[(int64_t)A.bt_tile[e] * BS + r];
-            if constexpr (BS == 8) acc += __popcll(xs[J] & (w * 0x0101010101010101ull) & m);
-            else acc += popcw((W)(w & xs[J]));
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      }
+#pragma unroll
+      for (int r = 0; r < BS && nbits > kMaskBits<BS>; ++r) {
+        uint64_t row = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, r);
+        if constexpr (BS == 64) row |= (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)((uint64_t)own >> 32), r) << 32;
+        m[0] |= ((row >> (BS - 1 - k)) & 1ull) << r;
+      }
+    }
+    int acc = 0;
+    for (int64_t f = f0; f < f1; f += kWave) {
+      int32_t tA = -1, tB = -1;
+      if (f + lane < f1) {
+        const int32_t J = from[f + lane];
+        const int64_t at_ = lower_bound_i32(in, i0, i1, J);
+        if (at_ < i1 && in[at_] == J) {
+          tA = (int32_t)(a_short ? f + lane : at_);
+          tB = A.bt_tile[a_short ? at_ : f + lane];
+        }
+      }
+      uint64_t found = __ballot(tA >= 0);
+      if constexpr (BS <= 16) {
+        constexpr int Q = BS * BS / 32, F = 32 / BS;  // words of a tile, rows of a word
+        constexpr uint32_t kOnes = BS == 8 ? 0x01010101u : 0x00010001u;
+        uint32_t a[Q] = {}, b[Q] = {};
+        if (tA >= 0) {
+          load_words<BS>(at, tA, a);
+          load_words<BS>(bt, tB, b);
+        }
+        if (found) {
+#pragma unroll
+          for (int k = 0; k < BS; ++k) {
+            // column k of B's tile once for each row of a word
+            constexpr uint32_t kSel[4] = {0x00000000u, 0x01010101u, 0x02020202u, 0x03030303u};
+            const uint32_t bw = b[k / F];
+            const uint32_t col = BS == 8 ? __builtin_amdgcn_perm(bw, bw, kSel[k % F])
+                                         : __builtin_amdgcn_perm(bw, bw, k % F ? 0x03020302u : 0x01000100u);
+#pragma unroll
+            for (int q = 0; q < Q; ++q)  // under the rows of word q that have column k
+              acc += __popc(a[q] & col & (((ms[q] >> (BS - 1 - k)) & kOnes) * (uint32_t)low_mask<BS>()));
           }
         }
-        if (m) hits += acc;
+      } else {
+        constexpr int G = kWave / BS;
+        const int g = lane / BS, k = lane % BS;
+        while (found && nbits <= kMaskBits<BS>) {  // wave-uniform
+          constexpr int U = 4;
+          int64_t sa[U], sb[U];
+          int n = 0;
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            if (found) {
+              const int l = __builtin_ctzll(found);
+              found &= found - 1;
+              sa[u] = __builtin_amdgcn_readlane(tA, l);
+              sb[u] = __builtin_amdgcn_readlane(tB, l);
+              ++n;
+            } else {
+              sa[u] = sa[0], sb[u] = sb[0];
+            }
+          }
+          for (int p = lane; p - lane < nbits; p += kWave) {
+            const int e = bits[min(p, nbits - 1)];
+            W x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = at[sa[u] * BS + e / BS] & bt[sb[u] * BS + e % BS];
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc += p < nbits && u < n ? popcw(x[u]) : 0;
+          }
+        }
+        while (found) {
+          int mine = -1;
+          int64_t first = 0;  // bs 64: the match, wave-uniform
+#pragma unroll
+          for (int h = 0; h < G; ++h) {
+            if (found) {
+              const int l = __builtin_ctzll(found);
+              found &= found - 1;
+              if (g == h) mine = l;
+              first = l;
+            }
+          }
+          const int32_t sA = __shfl(tA, mine < 0 ? 0 : mine), sB = __shfl(tB, mine < 0 ? 0 : mine);
+          const W w = mine < 0 ? (W)0 : bt[(int64_t)sB * BS + k];
+          if constexpr (BS == 64) {
+            const int64_t ta = __builtin_amdgcn_readlane(tA, (int)first);
+#pragma unroll 16
+            for (int r = 0; r < BS; ++r) {
+              const uint64_t row = ld_uniform(at, ta * BS + r);
+              const uint32_t on = (uint32_t)((int32_t)((uint32_t)(m[0] >> (r & 32)) << (31 - (r & 31))) >> 31);
+              acc += __popc((uint32_t)w & (uint32_t)row & on) + __popc((uint32_t)(w >> 32) & (uint32_t)(row >> 32) & on);
+            }
+          } else {
+            const W own = mine < 0 ? (W)0 : at[(int64_t)sA * BS + k];
+#pragma unroll
+            for (int r = 0; r < BS; ++r) {
+              const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)own, r);
+              const uint32_t r1 = (uint32_t)__builtin_amdgcn_readlane((int)own, BS + r);
+              const uint32_t on = (uint32_t)((int32_t)((uint32_t)m[0] << (31 - r)) >> 31);
+              acc += __popc((uint32_t)w & (g ? r1 : r0) & on);
+            }
+          }
+        }
       }
-      __syncthreads();
-      for (int64_t t = t0 + tid; t < t1; t += nt) {
-        const int64_t J = A.a_colind[t] - base;
-        if (J >= 0 && J < window) xs[J] = (X)0;
-      }
-      __syncthreads();
     }
+    hits += acc;
   }
   add_count(hits, A.count);
 }
 
-// Workgroups and threads of a kernel whose workgroups hold `lds` bytes each:
-// as many as fit a CU's 160 KB of LDS and 32 waves (`wide`: of 16 waves each).
-static void lds_grid(size_t lds, bool wide, int* threads, int* blocks) {
-  *threads = wide || lds > ((size_t)40 << 10) ? kHeavyThreads : 256;
+// Workgroups and threads of k_tc_heavy, whose workgroups hold `lds` bytes each:
+// as many as fit a CU's 160 KB of LDS and 32 waves.
+static void lds_grid(size_t lds, int* threads, int* blocks) {
+  *threads = lds > ((size_t)40 << 10) ? kHeavyThreads : 256;
   *blocks = 256 * std::max(1, (int)std::min<size_t>(2048 / *threads, ((size_t)158 << 10) / (lds + 1024)));
-}
-
-// A kernel's limit is every caller's: always the most that a call needs, so that
-// none lowers it between another's limit and launch.
-static hipError_t lds_limit(const void* kernel) {
-  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kWindow / 8));
 }
 
 // The list form: A's rows are in `a`, B's block lists by column in `cl`.
@@ -534,8 +622,9 @@ static int tc_lists(const gbo_bsr* A, const CsrList& a, const TileLists& cl, uns
   t.count = count;
   const size_t lds = (size_t)(std::min<int64_t>(kWindow, A->ncols) + 31) / 32 * 4;
   int threads = 0, blocks = 0;
-  lds_grid(lds, false, &threads, &blocks);
-  GBO_HIP_CHECK(lds_limit((const void*)k_tc_heavy));
+  lds_grid(lds, &threads, &blocks);
+  // always the most that a call needs: none lowers it between another's limit and launch
+  GBO_HIP_CHECK(hipFuncSetAttribute((const void*)k_tc_heavy, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kWindow / 8)));
   k_tc_heavy<<<blocks, threads, lds, st>>>(t);
   GBO_LAUNCH_CHECK();
   k_tc_light<<<(unsigned)std::min<int64_t>(2048, ((int64_t)n + 4 * kTinyRows - 1) / (4 * kTinyRows)), 256, 0, st>>>(t);
@@ -544,27 +633,29 @@ static int tc_lists(const gbo_bsr* A, const CsrList& a, const TileLists& cl, uns
 }
 
 template <int BS>
-static int tc_tiles(const TileTcArgs& t, hipStream_t st) {
-  constexpr size_t X = BS == 8 ? 8 : BS / 8;  // bytes of an element of the vector
-  const size_t lds = ((size_t)std::min<int64_t>(kWindow / 8 / (int64_t)X, t.nblocks) * X + 7) / 8 * 8;
-  int threads = 0, blocks = 0;
-  lds_grid(lds, t.nrows < 2048, &threads, &blocks);  // few rows: more waves on each
-  GBO_HIP_CHECK(lds_limit((const void*)k_tc_tiles<BS>));
-  k_tc_tiles<BS><<<blocks, threads, lds, st>>>(t);
+static int tc_pairs(const PairTcArgs& t, hipStream_t st) {
+  k_tc_pairs<BS><<<(unsigned)std::min<int64_t>((t.T + 3) / 4, 4096), 256, 0, st>>>(t);  // one atomic each
   GBO_LAUNCH_CHECK();
   return GBO_OK;
 }
 
-// Whether the tiles are dense enough for the word form.  The lists' work falls
-// with the third power of the density, the words' hardly: G(4096, p), lists /
-// words: bs 8 p 0.1 (6 bits a tile) 496 / 648 us, 0.2 (13) 723 / 647; bs 16 0.2
-// (51) 693 / 861, 0.3 (77) 1049 / 858; bs 32 0.1 (102) 480 / 528, 0.2 (203) 708
-// / 551; bs 64 0.05 (202) 373 / 395, 0.1 (403) 514 / 427; p 1 6.1-7.2 ms / 0.8-
-// 1.3 (the tile-pair form before 1.6-6.1).  King grids, 0.8 bits a tile row,
-// belong to the lists.
-static bool tc_dense(int bs, int64_t nnz, int64_t tiles) {
-  const int64_t bits = bs == 8 ? 12 : bs == 16 ? 64 : bs == 32 ? 128 : 320;
-  return nnz > bits * tiles;
+// Nonzeros up to which the lists are counted, by the bits per tile: the lists' work
+// grows with the square of a row's length, the pairs' with its tiles.  ms, lists /
+// pairs:
+//   bs 8    communities of 512 on 2^18 vertices, 32 tiles a block row, 3.2 bits
+//           0.65 / 0.80, 6.0 1.64 / 0.80; of 4096, 256 tiles, 6.0 9.2 / 19.0; G(4096),
+//           6.3 0.49 / 0.38, 12.7 0.74 / 0.37: the search in long rows costs
+//   bs 16   512, 12 bits 0.61 / 0.58, 24 1.65 / 0.56; 4096, 12 4.5 / 5.0, 24 9.0 / 5.0;
+//           G(20000) 12.7 2.6 / 7.1
+//   bs 32   512, 19 bits 0.34 / 0.24, 47 0.53 / 0.24; 4096, 20 2.7 / 2.1, 97 9.2 /
+//           2.7; G(20000) 20 0.9 / 2.9, 51 2.6 / 3.0
+//   bs 64   512, 72 bits 0.32 / 0.20; 4096, 80 2.65 / 0.62; G(20000) 81 0.87 / 0.94, 204
+//           2.5 / 1.7
+// King grids hold 6 to 55 bits a tile (0.34 / 0.27 to 0.30 / 0.20), R-MAT up to 8 (2^18 2.2 /
+// 7.3 to 2.6 / 12.7).
+static int64_t tc_listed(int bs, int64_t tiles, int32_t nbr) {
+  const int64_t bits = bs == 8 ? (tiles <= 64 * (int64_t)nbr ? 5 : 8) : bs == 16 ? 16 : bs == 32 ? 32 : 48;
+  return bits * tiles;
 }
 
 extern "C" {
@@ -587,26 +678,30 @@ int gbo_bsrbmm_tc(const gbo_bsr* L, const gbo_bsr* LT, uint64_t* d_count, gbo_st
   int32_t *bt_ptr = nullptr, *bt_row = nullptr, *bt_tile = nullptr;
   unsigned long long* count = (unsigned long long*)d_count;
   CsrList a;
-  if ((rc = block_transpose(LT, mem, &bt_ptr, &bt_row, &bt_tile, st)) || (rc = expand_csr(L, mem, &a, st))) return rc;
-  if (tc_dense(L->bs, a.nnz, L->nblocks)) {
-    TileTcArgs t{};
+  if ((rc = block_transpose(LT, mem, &bt_ptr, &bt_row, &bt_tile, st)) || (rc = expand_csr(L, mem, &a, st, tc_listed(L->bs, L->nblocks, L->nblockrows))))
+    return rc;
+  if (!a.col) {
+    PairTcArgs t{};
+    int32_t* a_row = nullptr;
+    if ((rc = mem.alloc(&a_row, sizeof(int32_t) * (size_t)L->nblocks, "gbo_bsrbmm_tc"))) return rc;
+    k_tile_block_row<<<(unsigned)((L->nblocks + 255) / 256), 256, 0, st>>>(L->rowptr, L->nblockrows, nullptr,
+                                                                           L->nblocks, a_row);
+    GBO_LAUNCH_CHECK();
     t.a_rowptr = L->rowptr;
     t.a_colind = L->colind;
+    t.a_row = a_row;
     t.a_tiles = L->tiles;
     t.bt_ptr = bt_ptr;
     t.bt_row = bt_row;
     t.bt_tile = bt_tile;
     t.b_tiles = LT->tiles;
-    t.nrows = L->bs == 8 ? L->nblockrows : L->nrows;
-    t.nblocks = L->nblockcols;
+    t.T = L->nblocks;
     t.count = count;
-    if ((rc = mem.alloc(&t.next, sizeof(*t.next), "gbo_bsrbmm_tc"))) return rc;
-    GBO_HIP_CHECK(hipMemsetAsync(t.next, 0, sizeof(*t.next), st));
     switch (L->bs) {
-      case 8: rc = tc_tiles<8>(t, st); break;
-      case 16: rc = tc_tiles<16>(t, st); break;
-      case 32: rc = tc_tiles<32>(t, st); break;
-      case 64: rc = tc_tiles<64>(t, st); break;
+      case 8: rc = tc_pairs<8>(t, st); break;
+      case 16: rc = tc_pairs<16>(t, st); break;
+      case 32: rc = tc_pairs<32>(t, st); break;
+      case 64: rc = tc_pairs<64>(t, st); break;
     }
   } else {
     TileLists cl;

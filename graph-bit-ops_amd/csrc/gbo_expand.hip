@@ -143,7 +143,7 @@ unsigned grid_of(int64_t items, int per_block) {
 unsigned item_grid(int64_t cap) { return std::min(grid_of(cap, 4), 1u << 22); }
 
 template <int BS>
-int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
+int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st, int64_t most) {
   const int32_t nbr = A.nbr, n = A.n;
   const int64_t cap = (int64_t)nbr + A.T / kItem<BS> + 1;  // items
   int32_t *icnt = nullptr, *itemrow = nullptr, *cnt = nullptr;
@@ -181,30 +181,32 @@ int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
   GBO_LAUNCH_CHECK();
   int64_t nnz = 0;
   if ((rc = read_back(&nnz, rowptr + n, sizeof(int64_t), st))) return rc;
+  out->rowptr = rowptr;
+  out->col = nullptr;
+  out->nnz = nnz;
+  if (nnz > most) return GBO_OK;
   int32_t* col = nullptr;
   if ((rc = mem.alloc(&col, sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1), who))) return rc;
   a.col = col;
   k_item_fill<BS><<<item_grid(cap), 256, 0, st>>>(a);
   GBO_LAUNCH_CHECK();
-  out->rowptr = rowptr;
   out->col = col;
-  out->nnz = nnz;
   return GBO_OK;
 }
 
 }  // namespace
 
-int expand_lists(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st) {
+int expand_lists(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st, int64_t most) {
   switch (A.bs) {
-    case 8: return expand_t<8>(A, mem, out, st);
-    case 16: return expand_t<16>(A, mem, out, st);
-    case 32: return expand_t<32>(A, mem, out, st);
-    case 64: return expand_t<64>(A, mem, out, st);
+    case 8: return expand_t<8>(A, mem, out, st, most);
+    case 16: return expand_t<16>(A, mem, out, st, most);
+    case 32: return expand_t<32>(A, mem, out, st, most);
+    case 64: return expand_t<64>(A, mem, out, st, most);
   }
   return set_error(GBO_EUNSUPPORTED, "block size %d not supported", A.bs);
 }
 
-int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
+int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st, int64_t most) {
   TileLists l;
   l.bs = A->bs;
   l.nbr = A->nblockrows;
@@ -213,7 +215,7 @@ int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st) {
   l.ptr = A->rowptr;
   l.ind = A->colind;
   l.tiles = A->tiles;
-  return expand_lists(l, mem, out, st);
+  return expand_lists(l, mem, out, st, most);
 }
 
 }  // namespace gbo

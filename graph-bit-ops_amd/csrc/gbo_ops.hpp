@@ -142,13 +142,14 @@ class AsyncAllocs {
 int validate_bsr(const gbo_bsr* A, int want_dir, const char* who);
 
 // The nonzeros of a row-direction bit-BSR as CSR (rows in order, columns
-// ascending), in device memory owned by `mem`; one host read of the total.
+// ascending), in device memory owned by `mem`; one host read of the total.  More
+// than `most` are counted only.
 struct CsrList {
   const int64_t* rowptr = nullptr;  // [nrows + 1]
-  const int32_t* col = nullptr;     // [nnz]
+  const int32_t* col = nullptr;     // [nnz]; null past `most`
   int64_t nnz = 0;
 };
-int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st);
+int expand_csr(const gbo_bsr* A, Workspace& mem, CsrList* out, hipStream_t st, int64_t most = INT64_MAX);
 // The same for any block lists: list R (of nbr) holds the blocks ind[t], t in
 // [ptr[R], ptr[R+1]); word k of tile t (or perm[t]) holds list R * bs + k's
 // bits in block ind[t], top bit first.
@@ -159,7 +160,7 @@ struct TileLists {
   const void* tiles = nullptr;
   const int32_t* perm = nullptr;
 };
-int expand_lists(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st);
+int expand_lists(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st, int64_t most = INT64_MAX);
 
 template <class TI, class TO>
 int scan_exclusive(const TI* in, TO* out, int64_t n, hipStream_t st);
