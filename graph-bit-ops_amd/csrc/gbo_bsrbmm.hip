@@ -158,7 +158,8 @@ static int block_transpose(const gbo_bsr* B, Workspace& mem, int32_t** d_ptr, in
 // each.  Their sets are hash tables of the wave's own, a quarter full at most.
 // Longer rows: items of kHeavyKeys columns k, a workgroup takes one after
 // another from a counter, the set a bitmap of up to 2^20 ids (more: window by
-// window).  A bitmap probe is a load and a shift, a hash probe a loop, so the
+// window, each list going on where the last window ended: taken whole in each, R-MAT
+// 2^23 of 12 took 729 ms, 2^24 of 8 1724, now 202 and 320).  A bitmap probe is a load and a shift, a hash probe a loop, so the
 // line is low: R-MAT 2^18 2.2 / 3.1 / 3.7 ms at 32 / 64 / 128 columns.
 constexpr int kTinyRow = 8;
 constexpr int kTinyRows = kWave / kTinyRow;  // tiny rows per wave
@@ -208,20 +209,36 @@ __device__ __forceinline__ int64_t count_searched(const int32_t* __restrict__ a,
 // from a0: the elements of their C_k that has(element, lane) holds, this
 // lane's share.  Lists of 64 or more are streamed one after another by the
 // whole wave; the shorter ones are laid end to end, 64 elements a round
-// whatever lists they come from.
+// whatever lists they come from.  `cursor` (of this lane's key, in LDS; null: the
+// lists are taken whole): only elements below `until` are, and the key's next call
+// goes on after them.
 template <class Has>
 __device__ __forceinline__ int64_t count_keys(const ListTcArgs& A, bool in, int32_t k, int64_t a0, int64_t di,
-                                              bool searches, const Has& has) {
+                                              bool searches, const Has& has, int32_t* cursor = nullptr,
+                                              int64_t until = 0) {
   const int lane = lane_id();
   in = in && k < A.nkeys;
-  const int64_t c0 = in ? A.crp[k] : 0;
-  const int64_t dk = in ? A.crp[k + 1] - c0 : 0;
+  int64_t c0 = in ? A.crp[k] : 0;
+  int64_t dk = in ? A.crp[k + 1] - c0 : 0;
   int64_t hits = 0;
   const bool far = search_pays(dk, di);
   for (uint64_t m = __ballot(far && searches); m; m &= m - 1) {
     const int j = __builtin_ctzll(m);
     hits += count_searched(A.acol + __shfl((long long)a0, j), __shfl((long long)di, j),
                            A.ccol + __shfl((long long)c0, j), __shfl((long long)dk, j));
+  }
+  if (cursor && in && !far) {  // lists are ascending
+    const int64_t from = searches ? 0 : *cursor;
+    int64_t lo = from, hi = dk;
+    if (until >= A.nids) lo = hi;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (A.ccol[c0 + mid] < until) lo = mid + 1;
+      else hi = mid;
+    }
+    *cursor = (int32_t)lo;
+    c0 += from;
+    dk = lo - from;
   }
   for (uint64_t m = __ballot(!far && dk >= kWave); m; m &= m - 1) {
     const int j = __builtin_ctzll(m);
@@ -349,6 +366,7 @@ __global__ __launch_bounds__(256) void k_tc_items_fill(const int64_t* __restrict
 __global__ __launch_bounds__(kHeavyThreads) void k_tc_heavy(const ListTcArgs A) {
   extern __shared__ uint32_t bits[];
   __shared__ unsigned long long s_item;
+  __shared__ int32_t s_cursor[kHeavyKeys];  // windows: where each key's list goes on
   const int tid = threadIdx.x, nt = blockDim.x;
   const int64_t total = A.hoff[A.nrows];
   const int window = (int)min(kWindow, (int64_t)A.nids);
@@ -380,7 +398,8 @@ __global__ __launch_bounds__(kHeavyThreads) void k_tc_heavy(const ListTcArgs A) 
       for (int64_t k = k0 + (tid / kWave) * KW; k < k1; k += (nt / kWave) * KW) {
         const int64_t kk = k + lane_id();
         const bool in = lane_id() < KW && kk < k1;
-        hits += count_keys(A, in, in ? ai[kk] : 0, a0, d, base == 0, has);
+        hits += count_keys(A, in, in ? ai[kk] : 0, a0, d, base == 0, has,
+                           window < A.nids ? s_cursor + (in ? kk - k0 : 0) : nullptr, base + window);
       }
       __syncthreads();
       for (int64_t e = tid; e < d; e += nt) {
@@ -581,7 +600,7 @@ __global__ __launch_bounds__(256) void k_tc_pairs(const PairTcArgs A) {
 // as many as fit a CU's 160 KB of LDS and 32 waves.
 static void lds_grid(size_t lds, int* threads, int* blocks) {
   *threads = lds > ((size_t)40 << 10) ? kHeavyThreads : 256;
-  *blocks = 256 * std::max(1, (int)std::min<size_t>(2048 / *threads, ((size_t)158 << 10) / (lds + 1024)));
+  *blocks = 256 * std::max(1, (int)std::min<size_t>(2048 / *threads, ((size_t)158 << 10) / (lds + 3072)));
 }
 
 // The list form: A's rows are in `a`, B's block lists by column in `cl`.
