@@ -142,6 +142,7 @@ static int block_transpose(const gbo_bsr* B, Workspace& mem, int32_t** d_ptr, in
   GBO_LAUNCH_CHECK();
   k_tile_block_row<<<(unsigned)((T + 255) / 256), 256, 0, st>>>(B->rowptr, nbr, *d_tile, T, *d_row);
   GBO_LAUNCH_CHECK();
+  for (const void* p : {(const void*)keys, (const void*)idx, (const void*)tmp}) mem.drop(p);
   return GBO_OK;
 }
 

@@ -191,6 +191,8 @@ int expand_t(const TileLists& A, Workspace& mem, CsrList* out, hipStream_t st, i
   k_item_fill<BS><<<item_grid(cap), 256, 0, st>>>(a);
   GBO_LAUNCH_CHECK();
   out->col = col;
+  for (const void* p : {(const void*)icnt, (const void*)itemptr, (const void*)itemrow, (const void*)cnt, (const void*)pos})
+    mem.drop(p);
   return GBO_OK;
 }
 

@@ -91,6 +91,7 @@ class Workspace {
 
  private:
   int take(void** p, size_t bytes, const char* who);
+  bool free_dropped();
   static constexpr int kMax = 64;
   hipStream_t st_;
   int dev_ = -1;

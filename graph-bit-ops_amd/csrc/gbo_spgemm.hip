@@ -540,7 +540,10 @@ int count_rows(const gbo_bsr* A, const gbo_bsr* B, Workspace& mem, RowArgs* out,
   if ((rc = scan_exclusive<int32_t, int64_t>(a.cnt, off, a.nbr, st, mem))) return rc;
   int64_t h[2] = {0, 0};
   if ((rc = read_back(h, off + a.nbr, sizeof(h), st))) return rc;
-  if (h[1]) return GBO_OK;
+  if (h[1]) {
+    for (const void* p : {(const void*)a.cnt, (const void*)off, (const void*)am, (const void*)bm}) mem.drop(p);
+    return GBO_OK;
+  }
   a.off = off;
   *out = a;
   *nc = h[0];
@@ -624,6 +627,9 @@ int sorted_pairs(const gbo_bsr* A, const gbo_bsr* B, bool with_vals, Workspace& 
   } else {
     GBO_HIP_CHECK(rocprim::radix_sort_keys(sort_tmp, tb, k0, out->keys, (size_t)P, 0, end_bit, st));
   }
+  for (const void* p : {(const void*)k0, (const void*)v0, (const void*)sort_tmp, (const void*)wcount, (const void*)woff,
+                        (const void*)trow, (const void*)cnt, (const void*)coff, (const void*)amask, (const void*)bmask})
+    mem.drop(p);
   out->P = P;
   return GBO_OK;
 }
@@ -649,6 +655,8 @@ int key_runs(const Pairs& pr, Workspace& mem, int32_t** crow, int32_t* ccol, int
   }
   k_runs<<<grid_for(pr.P, 256), 256, 0, st>>>(pr.keys, head, rank, pr.P, pr.jbits, *crow, ccol, seg ? *seg : nullptr);
   GBO_LAUNCH_CHECK();
+  mem.drop(head);
+  mem.drop(rank);
   // the host value copied above must outlive the copy
   GBO_HIP_CHECK(hipStreamSynchronize(st));
   return GBO_OK;

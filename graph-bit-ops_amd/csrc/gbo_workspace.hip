@@ -167,7 +167,8 @@ int Workspace::take(void** p, size_t bytes, const char* who) {
     }
   }
   if (!q) {
-    const hipError_t e = device_malloc(&q, want);
+    hipError_t e = device_malloc(&q, want);
+    if (e == hipErrorOutOfMemory && free_dropped()) e = device_malloc(&q, want);
     if (e != hipSuccess)
       return set_error(GBO_ENOMEM, "%s: device allocation of %zu bytes failed: %s", who, bytes, hipGetErrorString(e));
   }
@@ -176,6 +177,25 @@ int Workspace::take(void** p, size_t bytes, const char* who) {
   bytes_[n_++] = got;
   *p = q;
   return GBO_OK;
+}
+
+// The dropped blocks back to the runtime; false if there are none.
+bool Workspace::free_dropped() {
+  int keep = 0;
+  bool any = false;
+  if (hipStreamSynchronize(st_) != hipSuccess) return false;
+  for (int i = 0; i < n_; ++i) {
+    if (spare_[i]) {
+      any = true;
+      (void)hipFree(ptrs_[i]);
+      continue;
+    }
+    ptrs_[keep] = ptrs_[i];
+    bytes_[keep] = bytes_[i];
+    spare_[keep++] = false;
+  }
+  n_ = keep;
+  return any;
 }
 
 void Workspace::drop(const void* p) {

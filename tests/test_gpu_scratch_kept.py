@@ -1,6 +1,7 @@
 """Blocks kept between calls: one too large to be kept sends no other off, and
 those of a call of some GB are there for the next."""
 import ctypes
+import gc
 import time
 
 import numpy as np
@@ -10,6 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 def test_large_blocks(gbo):
+    gc.collect()  # no matrix of another test
     gbo.lib()
     hip = ctypes.CDLL(gbo.hip_runtimes()[0])
 
