@@ -880,11 +880,11 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
   return plan_fill(A, chunk, true, false, nch, plan, st);
 }
 
-int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st) {
+static int plan_create_with(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bool cut, hipStream_t st) {
   int32_t chunk = chunk_tiles > 0 ? chunk_tiles : default_chunk(A->bs, A->nblocks, false);
   // equal work needs the tiles' bits in 16-byte reads; the kernels that gain
   // from it need the same alignment
-  bool even = chunk_tiles > 0 || A->nblocks == 0 || A->nblocks >= kEvenTiles || !A->tiles || ((uintptr_t)A->tiles & 15);
+  bool even = !cut || chunk_tiles > 0 || A->nblocks == 0 || A->nblocks >= kEvenTiles || !A->tiles || ((uintptr_t)A->tiles & 15);
   int64_t nch = 0;
   Workspace mem(st);
   WorkCut w;
@@ -937,6 +937,13 @@ int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st
   }
   const int rc = plan_fill(A, chunk, even, whole, nch, A->plan, st);
   if (rc) gbo_bsr_plan_free(A);
+  return rc;
+}
+
+int plan_create(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, hipStream_t st) {
+  int rc = plan_create_with(A, chunk_tiles, variant, true, st);
+  // no room for the prefix sums (20 bytes a unit): even chunks need none
+  if (rc == GBO_ENOMEM && chunk_tiles <= 0) rc = plan_create_with(A, chunk_tiles, variant, false, st);
   return rc;
 }
 

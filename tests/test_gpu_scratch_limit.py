@@ -106,3 +106,56 @@ def test_host_csr(gbo, hog):
     give()
     gbo._check(rc)
     assert nb.value == 1
+
+
+def test_own_plan_without_room(gbo):
+    """The library's own plan where its allocation fits and the prefix sums it is
+    cut by do not."""
+    gbo.lib()
+    hip = ctypes.CDLL(gbo.hip_runtimes()[0])
+    n, deg, bs = 1 << 21, 12, 8
+    g = gbo.gen_er_m(n, n * deg // 2, 1)
+    A = gbo.BsrMatrix.from_csr(g, bs, plan=False)
+    assert 20 << 20 < A.nblocks < 32 << 20
+    # in MB: row counts 4 n, per chunk of 256 plan, start, tail, partials; prefix sums 20 bytes per 16 tiles
+    plan = (4 * n + A.nblocks // 256 * (16 + 128)) >> 20
+    cut = A.nblocks // 16 * 20 >> 20
+    assert cut > 20
+    held, leave = [], plan + cut // 2
+
+    def grab(size):
+        p = ctypes.c_void_p()
+        if hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)):
+            hip.hipGetLastError()
+            return False
+        held.append((p, size))
+        return True
+
+    f, t = ctypes.c_size_t(), ctypes.c_size_t()
+    gbo._check(gbo.lib().gbo_bsr_plan(A.ref, 256, None))  # whatever a first plan sets up
+    gbo.lib().gbo_bsr_plan_free(A.ref)
+    gbo.synchronize()
+    assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+    assert grab(f.value - (1 << 30))
+    for size in (128 << 20, 2 << 20):
+        for _ in range(600):
+            if not grab(size):
+                break
+        else:
+            pytest.skip("no end of device memory")
+    # the kept blocks go with a failed allocation, and that is what there is then
+    given = 0
+    while held and given < leave << 20:
+        p, size = held.pop()
+        assert hip.hipFree(p) == 0
+        given += size
+    rc = gbo.lib().gbo_bsr_plan(A.ref, 0, None)
+    gbo.synchronize()
+    while held:
+        assert hip.hipFree(held.pop()[0]) == 0
+    gbo._check(rc)
+    x = gbo.pack_vec(bs, (np.arange(n) % 3 == 0).astype(np.float32))
+    y = gbo.bsrbmv_count(A, x)
+    want = np.bincount(np.repeat(np.arange(n), np.diff(g.rowptr))[g.colind % 3 == 0], minlength=n)
+    assert np.array_equal(y, want)
+    A.free()
