@@ -420,6 +420,7 @@ static SpmvArgs bfs_args(const gbo_bsr* A, const PlanView& pv) {
   a.start = pv.start;
   a.tail = pv.tail;
   a.whole = pv.whole;
+  a.dense = pv.dense;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -972,6 +973,7 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   a.start = pv.start;
   a.tail = pv.tail;
   a.whole = pv.whole;
+  a.dense = pv.dense;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -1041,6 +1043,7 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   a.start = pv.start;
   a.tail = pv.tail;
   a.whole = pv.whole;
+  a.dense = pv.dense;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -1125,6 +1128,7 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   a.start = pv.start;
   a.tail = pv.tail;
   a.whole = pv.whole;
+  a.dense = pv.dense;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

@@ -1928,7 +1928,18 @@ static void launch_value(const SpmvArgs& a, bool aligned, unsigned blocks, hipSt
   if constexpr (BS <= 16) {
     if (a.variant == 3 && aligned) return k_value_lpt<BS, OP, GO><<<blocks, 256, 0, st>>>(a);
   } else if constexpr (BS == 32 || OP == OP_MINPLUS) {
-    if (aligned && (BS == 32 || a.w)) return k_value_q<BS, OP, GO><<<blocks, 256, 0, st>>>(a);
+    if (aligned && (BS == 32 || a.w)) {
+      size_t lds = 0;
+      // Where tiles are dense each lane reads a weight cache line of its own: two
+      // workgroups to a compute unit (this much LDS asked for), as more of them throw
+      // out each other's lines (G(16384, 1) bs 32 4.37 -> 1.42 ms, bs 64 4.32 -> 1.47;
+      // one workgroup 1.36 and 1.42, but 0.43 against 0.32 ms on blocks of 256 on
+      // 2^18 vertices).
+      if constexpr (OP == OP_MINPLUS) {
+        if (a.w && a.dense) lds = 54 << 10;
+      }
+      return k_value_q<BS, OP, GO><<<blocks, 256, lds, st>>>(a);
+    }
   }
   k_spmv<BS, OP, GO><<<blocks, 256, 0, st>>>(a);
 }
@@ -2047,6 +2058,7 @@ static SpmvArgs base_args(const gbo_bsr* A, const PlanView& pv) {
   a.start = pv.start;
   a.tail = pv.tail;
   a.whole = pv.whole;
+  a.dense = pv.dense;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

@@ -46,6 +46,7 @@ struct PlanView {
   double* partial = nullptr;
   int32_t* bfs_counts = nullptr;  // the dense BFS step's row counts
   bool whole = false;             // no block row is cut
+  bool dense = false;             // an eighth of the tiles' bits are set, or more (equal work, bs 32/64)
 };
 
 // Most tiles per chunk of the library's own plans.
@@ -324,6 +325,7 @@ struct SpmvArgs {
   const unsigned long long* go;  // MINPLUS / SUM / MIN, BFS at bs 16 to 64: nothing is done where *go is 0 (nullable; kernels of their
                                  // own, the look costs a plain product 0.2 us a launch)
   int whole;            // no block row is cut by a chunk's end
+  int dense;            // see PlanView
   int prefilled;        // BFS / MINPLUS / MIN: `out` holds the identity where rows are split
 };
 

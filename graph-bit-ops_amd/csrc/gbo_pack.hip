@@ -448,9 +448,9 @@ __global__ __launch_bounds__(256) void k_even_starts(int64_t T, int32_t chunk, i
 // bit, the first few of a tile with its own load; the count and the BFS step,
 // whose tiles all cost the same, lose little to shorter chunks where tiles are
 // dense, and the sparse rest keeps even chunks).  A unit starts a chunk where
-// the prefix sum of the work passes a multiple of chunk * kTileWork.  Cut evenly, a power-law matrix has chunks of ten to
-// fifty times the mean number of bits, and one wave on the densest one sets
-// the time of a sweep: R-MAT 2^18, 256 tiles a chunk, weighted min-plus bs 64
+// the prefix sum of the work passes a multiple of a chunk's work.  Cut
+// evenly, a power-law matrix has chunks of ten to fifty times the mean number of
+// bits, and one wave on the densest one sets the time of a sweep: R-MAT 2^18, 256 tiles a chunk, weighted min-plus bs 64
 // 1.52 ms, sum bs 32 0.50 ms, against 0.15 and 0.08 ms of streaming.
 template <int BS>
 constexpr int kUnitTiles = BS == 64 ? 8 : 16;
@@ -493,22 +493,40 @@ __global__ __launch_bounds__(256) void k_unit_work(const uint4* __restrict__ til
   if (l == 0 && u < nunits) work[u] = UT * kTileWork<BS> + max(c - UT * kFreeBits, 0);
 }
 
+// Work of a chunk: that of `chunk` sparse tiles, and at bs 8/16 of as many mean
+// ones where these are denser.  There a step of the count takes 256 and 64 tiles
+// whatever they hold, and where all tiles are dense shorter chunks gain the value
+// products nothing (G(16384, 1): bs 8 count 77 us at the 32 tiles that hold the work
+// of 256 sparse ones, 24 at 256, min 1051 and 1007; bs 16 43 and 23, 1138 and 1011).
+struct UnitCut {
+  int32_t chunk, tile_work, unit;
+  bool mean;
+};
+__device__ __forceinline__ int64_t cut_target(const int64_t* __restrict__ pre, int64_t nunits, const UnitCut& u) {
+  const int64_t mean = u.mean ? pre[nunits] / (nunits * u.unit) : 0;
+  return u.chunk * max((int64_t)u.tile_work, mean);
+}
 __device__ __forceinline__ bool unit_starts(const int64_t* __restrict__ pre, int64_t u, int64_t target) {
   return u == 0 || pre[u] / target != pre[u - 1] / target;
 }
 
-__global__ __launch_bounds__(256) void k_unit_heads(const int64_t* __restrict__ pre, int64_t nunits, int64_t target,
-                                                    int32_t* __restrict__ head) {
+// *dense: units of more than one and a half times the mean work.
+__global__ __launch_bounds__(256) void k_unit_heads(const int64_t* __restrict__ pre, int64_t nunits, const UnitCut cut,
+                                                    int32_t* __restrict__ head,
+                                                    unsigned long long* __restrict__ dense) {
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u < nunits) head[u] = unit_starts(pre, u, target);
+  if (u < nunits) head[u] = unit_starts(pre, u, cut_target(pre, nunits, cut));
+  const bool more = u < nunits && (pre[u + 1] - pre[u]) * 2 * nunits > pre[nunits] * 3;
+  const int n = __syncthreads_count(more);
+  if (threadIdx.x == 0 && n) atomicAdd(dense, (unsigned long long)n);
 }
 
 __global__ __launch_bounds__(256) void k_unit_chunks(const int64_t* __restrict__ pre,
-                                                     const int64_t* __restrict__ rank, int64_t nunits, int64_t target,
-                                                     int unit_tiles, int64_t T, int64_t* __restrict__ start) {
+                                                     const int64_t* __restrict__ rank, int64_t nunits,
+                                                     const UnitCut cut, int64_t T, int64_t* __restrict__ start) {
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= nunits) return;
-  if (unit_starts(pre, u, target)) start[rank[u]] = u * unit_tiles;
+  if (unit_starts(pre, u, cut_target(pre, nunits, cut))) start[rank[u]] = u * cut.unit;
   if (u == 0) start[rank[nunits]] = T;
 }
 
@@ -821,32 +839,37 @@ static int plan_fill(const gbo_bsr* A, int32_t chunk, bool even, bool whole, int
 // prefix sums and ranks k_unit_chunks writes their starts from.
 struct WorkCut {
   int64_t *pre = nullptr, *rank = nullptr;
-  int64_t nunits = 0, target = 0, nch = 0, total = 0;
-  int unit = 0;
+  int64_t nunits = 0, nch = 0, total = 0, dense = 0;
+  UnitCut cut{};
 };
 
 template <int BS>
 static int work_cut(const gbo_bsr* A, int32_t chunk, Workspace& mem, WorkCut* w, hipStream_t st) {
   constexpr int UT = kUnitTiles<BS>, G = BS == 8 ? 8 : BS == 16 ? 2 : 1;  // units per wave
-  w->unit = UT;
   w->nunits = (A->nblocks + UT - 1) / UT;
-  w->target = (int64_t)chunk * kTileWork<BS>;
+  w->cut = {chunk, kTileWork<BS>, UT, BS <= 16};
   int32_t* work = nullptr;
   int rc;
   if ((rc = mem.alloc(&work, sizeof(int32_t) * (size_t)w->nunits, "gbo_bsr_plan")) ||
       (rc = mem.alloc(&w->pre, sizeof(int64_t) * ((size_t)w->nunits + 1), "gbo_bsr_plan")) ||
-      (rc = mem.alloc(&w->rank, sizeof(int64_t) * ((size_t)w->nunits + 1), "gbo_bsr_plan")))
+      (rc = mem.alloc(&w->rank, sizeof(int64_t) * ((size_t)w->nunits + 2), "gbo_bsr_plan")))
     return rc;
   const unsigned blocks = (unsigned)((w->nunits + 255) / 256);
   k_unit_work<BS><<<(unsigned)((w->nunits + 4 * G - 1) / (4 * G)), 256, 0, st>>>((const uint4*)A->tiles, A->nblocks,
                                                                                   w->nunits, work);
   GBO_LAUNCH_CHECK();
   if ((rc = scan_exclusive<int32_t, int64_t>(work, w->pre, w->nunits, st, mem))) return rc;
-  k_unit_heads<<<blocks, 256, 0, st>>>(w->pre, w->nunits, w->target, work);
+  GBO_HIP_CHECK(hipMemsetAsync(w->rank + w->nunits + 1, 0, sizeof(int64_t), st));
+  k_unit_heads<<<blocks, 256, 0, st>>>(w->pre, w->nunits, w->cut, work,
+                                       (unsigned long long*)(w->rank + w->nunits + 1));
   GBO_LAUNCH_CHECK();
   if ((rc = scan_exclusive<int32_t, int64_t>(work, w->rank, w->nunits, st, mem))) return rc;
   if ((rc = read_back(&w->total, w->pre + w->nunits, sizeof(int64_t), st))) return rc;
-  return read_back(&w->nch, w->rank + w->nunits, sizeof(int64_t), st);
+  int64_t h[2];
+  if ((rc = read_back(h, w->rank + w->nunits, sizeof(h), st))) return rc;
+  w->nch = h[0];
+  w->dense = h[1];
+  return GBO_OK;
 }
 
 // Plan for a matrix: uses A->plan (made by gbo_bsr_plan, with its scratch)
@@ -860,6 +883,7 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
     pv->variant = A->plan_variant;
     pv->owned = false;
     pv->whole = A->plan_even == 2;
+    pv->dense = A->plan_even == 3;
     view_scratch(pv, A->bs, A->nblockrows, A->plan_even == 1);
     return GBO_OK;
   }
@@ -897,7 +921,9 @@ static int plan_create_with(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bo
       case 64: rc = work_cut<64>(A, chunk, mem, &w, st); break;
     }
     if (rc) return rc;
-    even = w.total == w.nunits * w.target / chunk * w.unit;  // no unit has more than its tiles' work
+    // no unit has more than its tiles' work, or (bs 8/16) all have about as much
+    // (G(16384, 0.2) bs 8 count 32 -> 26 us)
+    even = w.total == w.nunits * w.cut.tile_work * w.cut.unit || (w.cut.mean && w.dense == 0);
     if (!even) nch = w.nch;
     else chunk = default_chunk(A->bs, A->nblocks, true);
   }
@@ -925,10 +951,13 @@ static int plan_create_with(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bo
   A->plan_chunk = chunk;
   A->plan_nchunks = (int32_t)nch;
   A->plan_variant = variant;
-  A->plan_even = whole ? 2 : even ? 1 : 0;
+  // an eighth of the bits or more (blocks of 512 with 10 % of their bits at bs 32, weighted min-plus
+  // 43 us, 49 where marked; of 2,048 with 20 % 278 and 156)
+  const int64_t full = w.nunits * w.cut.unit * (w.cut.tile_work + A->bs * A->bs / 8 - kFreeBits);
+  A->plan_even = whole ? 2 : even ? 1 : A->bs >= 32 && w.total >= full ? 3 : 0;
   if (!even) {
-    k_unit_chunks<<<(unsigned)((w.nunits + 255) / 256), 256, 0, st>>>(w.pre, w.rank, w.nunits, w.target, w.unit,
-                                                                      A->nblocks, (int64_t*)((char*)A->plan + L.start));
+    k_unit_chunks<<<(unsigned)((w.nunits + 255) / 256), 256, 0, st>>>(w.pre, w.rank, w.nunits, w.cut, A->nblocks,
+                                                                      (int64_t*)((char*)A->plan + L.start));
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
       gbo_bsr_plan_free(A);

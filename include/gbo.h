@@ -70,7 +70,8 @@ typedef struct gbo_bsr {
   int32_t plan_chunk;   /* tiles per chunk (about the most of any, where the library chose) */
   int32_t plan_nchunks;
   int32_t plan_variant; /* kernel variant for bs 8/16 (0 = default; see gbo_bsr_plan_ex) */
-  int32_t plan_even;    /* 1: every chunk holds plan_chunk tiles (the last one the rest); 2: chunks end at block rows */
+  int32_t plan_even;    /* 0, 3: chunks of about equal work (3: of dense tiles, bs 32/64);
+                           1: every chunk holds plan_chunk tiles (the last one the rest); 2: chunks end at block rows */
 } gbo_bsr;
 
 const char* gbo_last_error(void);
