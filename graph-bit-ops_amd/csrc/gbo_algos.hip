@@ -421,6 +421,7 @@ static SpmvArgs bfs_args(const gbo_bsr* A, const PlanView& pv) {
   a.tail = pv.tail;
   a.whole = pv.whole;
   a.dense = pv.dense;
+  a.count_plan = pv.count_plan;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -974,6 +975,7 @@ int gbo_sssp(const gbo_bsr* AT, const uint32_t* d_w, const int64_t* d_woff, int3
   a.tail = pv.tail;
   a.whole = pv.whole;
   a.dense = pv.dense;
+  a.count_plan = pv.count_plan;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -1044,6 +1046,7 @@ int gbo_pagerank(const gbo_bsr* AT, const int32_t* d_outdeg, float alpha, double
   a.tail = pv.tail;
   a.whole = pv.whole;
   a.dense = pv.dense;
+  a.count_plan = pv.count_plan;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;
@@ -1129,6 +1132,7 @@ int gbo_cc(const gbo_bsr* A, int32_t* d_label, int32_t* h_iters, gbo_stream_t st
   a.tail = pv.tail;
   a.whole = pv.whole;
   a.dense = pv.dense;
+  a.count_plan = pv.count_plan;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

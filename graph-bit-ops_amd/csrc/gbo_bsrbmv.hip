@@ -1975,6 +1975,18 @@ static int spmv_launch_t(const SpmvArgs& a, hipStream_t st) {
       return GBO_OK;
     }
   }
+  if constexpr (BS == 8 && OP == OP_COUNT) {
+    if (lean8 && a.count_plan) {
+      SpmvArgs e = a;
+      e.plan = a.count_plan;
+      e.nchunks = (int32_t)count_chunks(a.T);
+      e.tail = e.plan + e.nchunks;
+      e.start = nullptr;
+      e.chunk = kCountChunk;
+      e.count_plan = nullptr;
+      return spmv_launch_t<BS, OP>(e, st);
+    }
+  }
   const bool need_prefill = ((OP == OP_BFS || OP == OP_MINPLUS || OP == OP_MIN) && !a.prefilled) ||
                             (OP == OP_COUNT && !a.accumulate);
   if (need_prefill && a.nchunks > 1 && !a.whole) {
@@ -2059,6 +2071,7 @@ static SpmvArgs base_args(const gbo_bsr* A, const PlanView& pv) {
   a.tail = pv.tail;
   a.whole = pv.whole;
   a.dense = pv.dense;
+  a.count_plan = pv.count_plan;
   a.chunk = pv.chunk;
   a.nchunks = pv.nchunks;
   a.variant = pv.variant;

@@ -31,6 +31,16 @@ namespace gbo {
 struct PlanLayout {
   size_t start = 0, tail = 0, slots = 0, count = 0, partial = 0, bfs_counts = 0, bytes = 0;
 };
+// The count at bs 8 takes even chunks of kCountChunk tiles, on plans of equal
+// work from kCountTiles tiles on: their plan entries, then their tails, lie after
+// the rest.
+// All its tiles cost the same, and a look at the chunk's start before the first
+// tile is asked for costs more than equal work gains: R-MAT 2^19 of 16 (11M tiles) 107
+// -> 93 us, 2^20 of 12 143 -> 132, 2^21 of 8 208 -> 188 (2^18 of 28 67 -> 74); below,
+// 2^18 of 16 (5M tiles) 63 and 71.
+constexpr int64_t kCountTiles = 6 << 20;
+constexpr int32_t kCountChunk = 256;
+inline int64_t count_chunks(int64_t tiles) { return (tiles + kCountChunk - 1) / kCountChunk; }
 PlanLayout plan_layout(int bs, int64_t nchunks, int32_t nbr);
 
 struct PlanView {
@@ -45,6 +55,7 @@ struct PlanView {
   int64_t* count = nullptr;
   double* partial = nullptr;
   int32_t* bfs_counts = nullptr;  // the dense BFS step's row counts
+  const int32_t* count_plan = nullptr;  // even chunks of the count, where they are others; count_chunks tails behind
   bool whole = false;             // no block row is cut
   bool dense = false;             // an eighth of the tiles' bits are set, or more (equal work, bs 32/64)
 };
@@ -326,6 +337,7 @@ struct SpmvArgs {
                                  // own, the look costs a plain product 0.2 us a launch)
   int whole;            // no block row is cut by a chunk's end
   int dense;            // see PlanView
+  const int32_t* count_plan;  // see PlanView (nullable)
   int prefilled;        // BFS / MINPLUS / MIN: `out` holds the identity where rows are split
 };
 

@@ -816,6 +816,8 @@ __global__ __launch_bounds__(256) void k_whole_starts(const int32_t* __restrict_
   start[c] = rowptr[lo];
 }
 
+static bool counts_evenly(const gbo_bsr* A) { return A->bs == 8 && A->nblocks >= kCountTiles; }
+
 // Plan entries (of the chunks whose starts are in place, or of even chunks of
 // `chunk` tiles) and zeroed count slots.
 static int plan_fill(const gbo_bsr* A, int32_t chunk, bool even, bool whole, int64_t nch, int32_t* plan,
@@ -885,6 +887,8 @@ int acquire_plan(const gbo_bsr* A, PlanView* pv, hipStream_t st) {
     pv->whole = A->plan_even == 2;
     pv->dense = A->plan_even == 3;
     view_scratch(pv, A->bs, A->nblockrows, A->plan_even == 1);
+    if (A->plan_even == 0 && counts_evenly(A))
+      pv->count_plan = (const int32_t*)((char*)A->plan + plan_layout(A->bs, A->plan_nchunks, A->nblockrows).bytes);
     return GBO_OK;
   }
   // bs 64: 128 tiles gain a sweep nothing that a plan of twice the chunks does not
@@ -943,7 +947,8 @@ static int plan_create_with(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bo
   }
   gbo_bsr_plan_free(A);
   const PlanLayout L = plan_layout(A->bs, nch, A->nblockrows);
-  if (device_malloc((void**)&A->plan, L.bytes) != hipSuccess) {
+  const int64_t ncount = !even && !whole && counts_evenly(A) ? count_chunks(A->nblocks) : 0;
+  if (device_malloc((void**)&A->plan, L.bytes + 2 * sizeof(int32_t) * ncount) != hipSuccess) {
     A->plan = nullptr;
     return set_error(GBO_ENOMEM, "gbo_bsr_plan: allocation of %zu bytes failed", L.bytes);
   }
@@ -963,6 +968,12 @@ static int plan_create_with(gbo_bsr* A, int32_t chunk_tiles, int32_t variant, bo
       gbo_bsr_plan_free(A);
       return set_error(GBO_EDEVICE, "gbo_bsr_plan: %s", hipGetErrorString(e));
     }
+  }
+  if (ncount) {
+    int32_t* count_plan = (int32_t*)((char*)A->plan + L.bytes);
+    k_plan<true><<<(unsigned)((ncount + 255) / 256), 256, 0, st>>>(
+        A->rowptr, A->nblockrows, nullptr, kCountChunk, A->nblocks, (int32_t)ncount, count_plan, count_plan + ncount,
+        (unsigned long long*)((char*)A->plan + L.slots));
   }
   const int rc = plan_fill(A, chunk, even, whole, nch, A->plan, st);
   if (rc) gbo_bsr_plan_free(A);

@@ -48,3 +48,28 @@ def test_dense_tiles(gbo, po, bs, part, density):
         assert np.array_equal(gbo.bsrbmv_minplus(A, d), po.minplus(bs, n, rp, ci, tw, d))
         assert np.array_equal(gbo.bsrbmv_minplus(A, d, tv), po.minplus(bs, n, rp, ci, tw, d, otv, owo))
     A.free()
+
+
+def test_count_over_even_chunks(gbo):
+    """bs 8 from 6M tiles on: the count and the dense BFS step take chunks of their own."""
+    scale, bs = 18, 8
+    g = gbo.gen_rmat(scale, 24, seed=3)
+    n = g.nrows
+    A = gbo.BsrMatrix.from_csr(g, bs)
+    assert A.nblocks >= 6 << 20 and A.s.plan_even == 0
+    rng = np.random.default_rng(4)
+    x = rng.random(n) < 0.4
+    v = rng.random(n) < 0.3
+    xb, vb = (gbo.pack_vec(bs, t.astype(np.float32)) for t in (x, v))
+    want = np.diff(np.concatenate([[0], np.cumsum(x[g.colind], dtype=np.int64)])[g.rowptr]).astype(np.int32)
+    dist = rng.integers(0, 1000, n).astype(np.uint32)
+    first = gbo.bsrbmv_minplus(A, dist)
+    for _ in range(2):
+        assert np.array_equal(gbo.bsrbmv_count(A, xb), want)
+        nx, cnt = gbo.bsrbmv_bfs_step(A, xb, vb)
+        new = (want > 0) & ~v
+        assert cnt == new.sum() and np.array_equal(nx, gbo.pack_vec(bs, new.astype(np.float32)))
+    A.plan(100)
+    assert np.array_equal(gbo.bsrbmv_count(A, xb), want)
+    assert np.array_equal(gbo.bsrbmv_minplus(A, dist), first)
+    A.free()
