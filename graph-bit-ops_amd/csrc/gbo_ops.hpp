@@ -15,7 +15,8 @@ namespace gbo {
 // before the chunk is "split" and its partial results are combined across
 // chunks).  A chunk size given by the caller cuts evenly, chunk c starting at
 // tile c * chunk; the library's own plan (plan_create) makes chunks of about
-// equal work, at most `chunk` tiles.
+// equal work, at most `chunk` tiles, or moves their starts back to the start of a
+// block row where these are short (at most `chunk` and the longest row's tiles).
 //
 // The scratch the operations need besides their inputs and outputs is kept
 // in the plan's allocation, after the nchunks plan entries, so that a call
@@ -333,8 +334,9 @@ struct SpmvArgs {
   const uint64_t* active;  // MINPLUS: optional per-block-column activity bits (nullable)
   int accumulate;       // COUNT: add into y
   float scale, bias;    // SUM: y = scale * (A x) + bias  (scale 1, bias 0 for the plain op)
-  const unsigned long long* go;  // MINPLUS / SUM / MIN, BFS at bs 16 to 64: nothing is done where *go is 0 (nullable; kernels of their
-                                 // own, the look costs a plain product 0.2 us a launch)
+  const unsigned long long* go;  // MINPLUS / SUM / MIN (kernels of their own: the look costs a plain product 0.2 us a
+                                 // launch), BFS by columns (bs 16 to 64) and by a tile a lane (bs 8): nothing is
+                                 // done where *go is 0 (nullable)
   int whole;            // no block row is cut by a chunk's end
   int dense;            // see PlanView
   const int32_t* count_plan;  // see PlanView (nullable)

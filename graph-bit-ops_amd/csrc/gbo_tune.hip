@@ -80,14 +80,14 @@ int gbo_autotune(const int32_t* d_rowptr, const int32_t* d_colind, int32_t nrows
     GBO_HIP_CHECK(hipMemsetAsync(vis, 0, nw * bs / 8, st));
     const int dc = default_chunk(bs, A.nblocks, true);
     const int chunks[3] = {dc, dc * 2, dc / 2};
-    // kernel variants that differ for this block size and operation (bs 8
-    // and 16 BFS: 3 is the dense count-based step; 2 would run variant 0)
-    static const int kVarCount[] = {0, 1, 2, 3}, kVarBfs[] = {0, 1, 3}, kVarOne[] = {0};
+    // kernel variants that differ for this block size and operation (BFS: 3 is the
+    // dense count-based step, 2 would run variant 0, and at bs 16 so would 1)
+    static const int kVarCount[] = {0, 1, 2, 3}, kVarBfs8[] = {0, 1, 3}, kVarBfs16[] = {0, 3}, kVarOne[] = {0};
     const int* vars = kVarOne;
     int nvar = 1;
     if (bs <= 16) {
-      vars = op == 0 ? kVarCount : kVarBfs;
-      nvar = op == 0 ? 4 : 3;
+      vars = op == 0 ? kVarCount : bs == 8 ? kVarBfs8 : kVarBfs16;
+      nvar = op == 0 ? 4 : bs == 8 ? 3 : 2;
     }
     for (int vi = 0; vi < nvar && rc == GBO_OK; ++vi)
       for (int ci = 0; ci < 3 && rc == GBO_OK; ++ci) {
