@@ -685,6 +685,7 @@ __global__ __launch_bounds__(256) void k_spmv_lpt(const SpmvArgs a) {
           }
         }
       } else if constexpr (OP == OP_BFS) {
+        static_assert(BS == 8, "one 64-bit word a tile");
         W* nx = (W*)a.out;
         const W vword = ((const W*)a.visited)[R];
         const int64_t valid = (int64_t)a.nrows - (int64_t)R * BS;
@@ -693,16 +694,10 @@ __global__ __launch_bounds__(256) void k_spmv_lpt(const SpmvArgs a) {
           if (full && lane == 0) nx[R] = (W)0;
           continue;
         }
-        uint64_t hit[NW];
-#pragma unroll
-        for (int k = 0; k < NW; ++k) hit[k] = 0;
+        uint64_t hit = 0;
         // tiles and column indices of four steps are loaded before their
         // frontier words
-        auto or_tile = [&](const uint64_t* w, uint64_t f) {
-          const uint64_t xr = (BS == 8) ? f * 0x0101010101010101ull : f * 0x0001000100010001ull;
-#pragma unroll
-          for (int k = 0; k < NW; ++k) hit[k] |= w[k] & xr;
-        };
+        auto or_tile = [&](const uint64_t* w, uint64_t f) { hit |= w[0] & (f * 0x0101010101010101ull); };
         int64_t t = s + lane;
         for (; t + 3 * kWave < te; t += 4 * kWave) {
           uint64_t w[4][NW];
@@ -720,16 +715,12 @@ __global__ __launch_bounds__(256) void k_spmv_lpt(const SpmvArgs a) {
           load_tile<BS>(a.tiles, t, w);
           or_tile(w, (uint64_t)xb[colind[t]]);
         }
-#pragma unroll
-        for (int k = 0; k < NW; ++k)
-          hit[k] = wave_or64(hit[k]);
-        // row r hit <=> its byte (bs 8) / short (bs 16) of hit is non-zero
+        hit = wave_or64(hit);
+        // row r hit <=> its byte of hit is non-zero
         uint64_t word = 0;
 #pragma unroll
-        for (int r = 0; r < BS; ++r) {
-          const uint64_t field = (BS == 8) ? (hit[0] >> (8 * r)) & 0xFFull : (hit[r / 4] >> (16 * (r % 4))) & 0xFFFFull;
-          if (field) word |= 1ull << (BS - 1 - r);
-        }
+        for (int r = 0; r < BS; ++r)
+          if ((hit >> (8 * r)) & 0xFFull) word |= 1ull << (BS - 1 - r);
         word &= ~(uint64_t)vword & low_mask<BS>();
         if (lane == 0) {
           if (full) {
