@@ -458,13 +458,18 @@ template <int BS>
 constexpr int kTileWork = BS >= 32 ? 16 : 8;
 constexpr int kFreeBits = 4;
 
+// What the host reads: the number of chunks (the last rank), of units of more than
+// one and a half times the mean work, and all work.
+enum { UNIT_CHUNKS, UNIT_DENSE, UNIT_TOTAL, UNIT_SUMS };
+
 // Work of every unit.  Lanes take 16 bytes each: a unit is 8 lanes at bs 8,
 // 32 at bs 16, a wave twice over at bs 32.  At bs 64 a wave reads a quarter of
 // each tile, another quarter from tile to tile, and counts it four times: the
 // bits are only a measure of work.
 template <int BS>
 __global__ __launch_bounds__(256) void k_unit_work(const uint4* __restrict__ tiles, int64_t T, int64_t nunits,
-                                                   int32_t* __restrict__ work) {
+                                                   int32_t* __restrict__ work, unsigned long long* __restrict__ sums) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) sums[UNIT_DENSE] = 0;
   constexpr int UT = kUnitTiles<BS>, UL = BS == 8 ? 8 : BS == 16 ? 32 : 64;  // lanes per unit
   const int lane = lane_id();
   const int64_t u = (int64_t)wave_index() * (kWave / UL) + lane / UL;
@@ -510,15 +515,15 @@ __device__ __forceinline__ bool unit_starts(const int64_t* __restrict__ pre, int
   return u == 0 || pre[u] / target != pre[u - 1] / target;
 }
 
-// *dense: units of more than one and a half times the mean work.
 __global__ __launch_bounds__(256) void k_unit_heads(const int64_t* __restrict__ pre, int64_t nunits, const UnitCut cut,
                                                     int32_t* __restrict__ head,
-                                                    unsigned long long* __restrict__ dense) {
+                                                    unsigned long long* __restrict__ sums) {
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (u < nunits) head[u] = unit_starts(pre, u, cut_target(pre, nunits, cut));
   const bool more = u < nunits && (pre[u + 1] - pre[u]) * 2 * nunits > pre[nunits] * 3;
   const int n = __syncthreads_count(more);
-  if (threadIdx.x == 0 && n) atomicAdd(dense, (unsigned long long)n);
+  if (threadIdx.x == 0 && n) atomicAdd(&sums[UNIT_DENSE], (unsigned long long)n);
+  if (u == 0) sums[UNIT_TOTAL] = (unsigned long long)pre[nunits];
 }
 
 __global__ __launch_bounds__(256) void k_unit_chunks(const int64_t* __restrict__ pre,
@@ -854,23 +859,22 @@ static int work_cut(const gbo_bsr* A, int32_t chunk, Workspace& mem, WorkCut* w,
   int rc;
   if ((rc = mem.alloc(&work, sizeof(int32_t) * (size_t)w->nunits, "gbo_bsr_plan")) ||
       (rc = mem.alloc(&w->pre, sizeof(int64_t) * ((size_t)w->nunits + 1), "gbo_bsr_plan")) ||
-      (rc = mem.alloc(&w->rank, sizeof(int64_t) * ((size_t)w->nunits + 2), "gbo_bsr_plan")))
+      (rc = mem.alloc(&w->rank, sizeof(int64_t) * ((size_t)w->nunits + UNIT_SUMS), "gbo_bsr_plan")))
     return rc;
   const unsigned blocks = (unsigned)((w->nunits + 255) / 256);
+  auto* sums = (unsigned long long*)(w->rank + w->nunits);
   k_unit_work<BS><<<(unsigned)((w->nunits + 4 * G - 1) / (4 * G)), 256, 0, st>>>((const uint4*)A->tiles, A->nblocks,
-                                                                                  w->nunits, work);
+                                                                                  w->nunits, work, sums);
   GBO_LAUNCH_CHECK();
   if ((rc = scan_exclusive<int32_t, int64_t>(work, w->pre, w->nunits, st, mem))) return rc;
-  GBO_HIP_CHECK(hipMemsetAsync(w->rank + w->nunits + 1, 0, sizeof(int64_t), st));
-  k_unit_heads<<<blocks, 256, 0, st>>>(w->pre, w->nunits, w->cut, work,
-                                       (unsigned long long*)(w->rank + w->nunits + 1));
+  k_unit_heads<<<blocks, 256, 0, st>>>(w->pre, w->nunits, w->cut, work, sums);
   GBO_LAUNCH_CHECK();
   if ((rc = scan_exclusive<int32_t, int64_t>(work, w->rank, w->nunits, st, mem))) return rc;
-  if ((rc = read_back(&w->total, w->pre + w->nunits, sizeof(int64_t), st))) return rc;
-  int64_t h[2];
-  if ((rc = read_back(h, w->rank + w->nunits, sizeof(h), st))) return rc;
-  w->nch = h[0];
-  w->dense = h[1];
+  int64_t h[UNIT_SUMS];
+  if ((rc = read_back(h, sums, sizeof(h), st))) return rc;
+  w->nch = h[UNIT_CHUNKS];
+  w->dense = h[UNIT_DENSE];
+  w->total = h[UNIT_TOTAL];
   return GBO_OK;
 }
 
